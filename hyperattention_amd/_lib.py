@@ -15,6 +15,7 @@ _PKG = os.path.dirname(os.path.abspath(__file__))
 _CSRC = os.path.join(_PKG, "csrc")
 _BUILD = os.path.join(_PKG, "build")
 LIB_PATH = os.path.join(_PKG, "libhyperattn.so")
+HOST_PATH = os.path.join(_PKG, "_host.so")  # the module's host path on torch tensors (csrc/torch_host.cpp)
 
 SOURCES = ["api.hip", "lsh_hash.hip", "bucket_sort.hip", "gather_rows.hip", "lse_merge.hip", "attn_fwd.hip",
            "attn_bwd.hip", "power_probe.hip"]
@@ -35,14 +36,39 @@ SYMBOLS = [
 ]
 
 HA_F16, HA_BF16 = 0, 1
-ABI_VERSION = 6
+ABI_VERSION = 7
 HA_IDX_I32, HA_IDX_I64 = 0, 1
 
 
+def _host_commands(obj: str):
+    """The compiler's and the linker's command line of the torch binding (host code only)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    cxx = shutil.which("g++") or "g++"
+    compile_ = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                *[x for path in includes for x in ("-isystem", path)], "-c", os.path.join(_CSRC, "torch_host.cpp"), "-o", obj]
+    libs = cpp_extension.library_paths()
+    link = [cxx, "-shared", "-fPIC", obj, *[f"-L{path}" for path in libs], f"-L{_PKG}", "-l:libhyperattn.so", "-ltorch_python",
+            "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    return compile_, link
+
+
 def build(verbose: bool = False) -> str:
-    """Compile every HIP source for gfx950 and link libhyperattn.so next to this file."""
+    """Compile every HIP source for gfx950 and link libhyperattn.so next to this file, and beside it the torch
+    binding of the module's host path (_host.so)."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     os.makedirs(_BUILD, exist_ok=True)
+    host_obj = os.path.join(_BUILD, "torch_host.o")
+    host_compile, host_link = _host_commands(host_obj)
+
+    def compile_host() -> None:
+        res = subprocess.run(host_compile, capture_output=True, text=True)
+        if res.returncode != 0:
+            raise RuntimeError(f"g++ failed on torch_host.cpp:\n{res.stdout}\n{res.stderr}")
 
     def compile_one(src: str) -> str:
         obj = os.path.join(_BUILD, src.replace(".hip", ".o"))
@@ -54,14 +80,21 @@ def build(verbose: bool = False) -> str:
             print(res.stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as pool:
+        host = pool.submit(compile_host)
         objs = list(pool.map(compile_one, SOURCES))
+        host.result()
     tmp = LIB_PATH + ".tmp"
     res = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs],
                          capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    tmp = HOST_PATH + ".tmp"
+    res = subprocess.run([*host_link, "-o", tmp], capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of _host.so failed:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
     global _lib
     _lib = None
     return LIB_PATH
@@ -82,7 +115,7 @@ class AttnOperands(ctypes.Structure):
         ("q_seg_offset", ctypes.c_int64), ("k_seg_offset", ctypes.c_int64),
         ("o_seg_stride_rows", ctypes.c_int64), ("o_seg_offset", ctypes.c_int64),
         ("kv_group", ctypes.c_int64),
-        ("scale", ctypes.c_float), ("dtype", ctypes.c_int),
+        ("scale", ctypes.c_float), ("dtype", ctypes.c_int), ("lse_rows", ctypes.c_int64),
     ]
 
 
@@ -127,6 +160,7 @@ class ForwardArgs(ctypes.Structure):
         ("q_stride_b", ctypes.c_int64), ("q_stride_h", ctypes.c_int64), ("q_stride_n", ctypes.c_int64),
         ("k_stride_b", ctypes.c_int64), ("k_stride_h", ctypes.c_int64), ("k_stride_n", ctypes.c_int64),
         ("v_stride_b", ctypes.c_int64), ("v_stride_h", ctypes.c_int64), ("v_stride_n", ctypes.c_int64),
+        ("lse_rows", ctypes.c_int64),
     ]
 
 
@@ -191,6 +225,25 @@ def lib():
             raise RuntimeError("libhyperattn.so: ABI version mismatch")
         _lib = loaded
     return _lib
+
+
+_host_module = None
+
+
+def host():
+    """The module's host path on torch tensors (csrc/torch_host.cpp); raises if it has not been built."""
+    global _host_module
+    if _host_module is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`. "
+                               "There is no fallback path.")
+        import torch  # noqa: F401  (the binding's libraries)
+        from . import _host as loaded
+        if loaded.abi_version() != ABI_VERSION:
+            raise RuntimeError("_host.so: ABI version mismatch")
+        _host_module = loaded
+    return _host_module
 
 
 _ARG_ERRORS = {-1: ValueError, -2: AssertionError, -3: AssertionError, -4: AssertionError,

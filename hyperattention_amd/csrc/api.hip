@@ -34,6 +34,8 @@ int ha_check_operands(const ha_attn_operands& t, const char* who) {
              "%s: head dims must be multiples of 8 (got %lld and %lld)", who, (long long)t.d, (long long)t.dv);
   HA_REQUIRE(t.segs >= 1 && t.kv_group >= 1 && t.heads % t.kv_group == 0, HA_ERR_SHAPE,
              "%s: segs >= 1 and kv_group dividing heads required", who);
+  HA_REQUIRE(t.lse_rows == 0 || (t.lse_rows >= t.n_q && t.lse_rows <= (t.n_q + 127) / 128 * 128 && t.segs == 1), HA_ERR_SHAPE,
+             "%s: lse_rows between n_q and the next multiple of 128, without segments", who);
   HA_REQUIRE(t.scale > 0.f && isfinite(t.scale), HA_ERR_SHAPE, "%s: softmax scale must be positive and finite", who);
   const int64_t strides[] = {t.q_stride_b, t.q_stride_h, t.q_stride_n, t.k_stride_b, t.k_stride_h, t.k_stride_n,
                              t.v_stride_b, t.v_stride_h, t.v_stride_n, t.o_stride_b, t.o_stride_h, t.o_stride_n};
@@ -95,6 +97,7 @@ void fill_params(const ha_attn_operands& t, ha_attn_kernel_params& p) {
   p.block_tiles = 1; p.sample_chunks = 0; p.smooth = 0; p.accumulate = 0; p.idx64 = 0;
   p.sampled_pos = nullptr; p.sample_bias_raw = 0.f;
   p.n_q_last = (int)t.n_q;
+  p.lse_rows = (int)t.lse_rows;
   p.tiles_per_wg = 1;
   p.rag_levels = -1; p.rag_split = 0; p.rag_n = 0;
   for (int& c : p.rag_half) c = 0;
@@ -304,7 +307,8 @@ void forward_operands(const ha_forward_args& a, ha_attn_operands& t) {
   if (a.v_stride_b || a.v_stride_h || a.v_stride_n) {
     t.v_stride_b = a.v_stride_b; t.v_stride_h = a.v_stride_h; t.v_stride_n = a.v_stride_n;
   }
-  t.lse_stride_b = a.heads * a.n; t.lse_stride_h = a.n;
+  const int64_t lse_rows = a.lse_rows ? a.lse_rows : a.n;
+  t.lse_stride_b = a.heads * lse_rows; t.lse_stride_h = lse_rows;
   t.kv_group = a.heads / a.kv_heads;
   t.scale = a.scale;
   t.dtype = a.dtype;
@@ -506,6 +510,8 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     st = check_hashing(a, w, "ha_forward");
     if (st != HA_OK) return st;
   }
+  HA_REQUIRE(a.lse_rows == 0 || a.lse_rows == a.n || (!pl.any_hyper && pl.levels == 0), HA_ERR_SHAPE,
+             "ha_forward: padded lse rows are for passes of one exact call");
   unsigned char* ws = (unsigned char*)a.workspace;
 
   ha_attn_operands t;
@@ -551,6 +557,7 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     ha_attn_operands f = t;
     f.n_q = f.n_k = a.n;
     f.segs = 1; f.seg_stride_rows = a.n; f.q_seg_offset = f.k_seg_offset = 0;
+    f.lse_rows = a.lse_rows;
     return flash_attn(f, 0, 0, stream);
   }
 
@@ -565,6 +572,7 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     f.seg_stride_rows = leaves ? rows : 2 * rows;
     f.q_seg_offset = leaves ? 0 : rows;
     f.k_seg_offset = 0;
+    if (pl.levels == 0) f.lse_rows = a.lse_rows;
     if (!pl.ragged) return flash_attn(f, leaves ? 1 : 0, leaves ? 0 : 1, stream);
     Ragged rag = {};
     rag.levels = level;

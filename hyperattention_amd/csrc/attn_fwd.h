@@ -44,6 +44,7 @@ struct ha_attn_kernel_params {
   // past this number names a row that is not there (the zero row the causal recursion appends to an odd
   // length, hyper_attention.py:61-64); it is placed like any other row and its result is dropped.
   int n_q_last;
+  int lse_rows;  // exact kernels: lse rows n_q .. lse_rows - 1 are written as zeros (0: none)
   // first row of segment g in the out / lse tensors: o_seg_off + g * o_seg_stride (= the query side's unless
   // the caller packs the rows a call writes)
   int64_t o_seg_off, o_seg_stride;

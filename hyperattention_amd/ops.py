@@ -494,21 +494,6 @@ def causal_plan(n: int, min_seq_len: int):
     return halves, n
 
 
-def forward_plan_supported(n: int, min_seq_len: int, causal: bool, lsh_num_projs: int) -> bool:
-    """True when ha_forward covers this shape: any length, up to 16 projections."""
-    return lsh_num_projs <= 16
-
-
-def forward_plan_even(n: int, min_seq_len: int) -> bool:
-    """True when every level of the causal recursion has an even length (what the recursion under autograd,
-    which works on equal segments of the whole tensors, takes)."""
-    while n > min_seq_len:
-        if n % 2:
-            return False
-        n //= 2
-    return True
-
-
 def _forward_args(q, k, v, out, lse, proj, *, scale, causal, lsh_num_projs, block_size, sample_size, min_seq_len,
                   smooth_block, sampled_idx=None, workspace=None, stream=None):
     """ForwardArgs for (b,h,n,d) q and (b,h_kv,n,d) k, v with its workspace attached; the second result keeps

@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define HA_ABI_VERSION 6
+#define HA_ABI_VERSION 7
 
 typedef enum {
   HA_OK = 0,
@@ -131,6 +131,9 @@ typedef struct {
   int64_t kv_group; /* grouped-query: q head h reads k/v (and k_idx) head h / kv_group; 1 = plain */
   float scale;    /* softmax scale; <= 0 or NaN is an error (callers resolve the default)  */
   int dtype;      /* ha_dtype                                                               */
+  /* exact attention with segs == 1: rows n_q .. lse_rows - 1 of every head's lse are written as zeros (a caller
+   * whose lse rows are padded, at most up to the next multiple of 128); 0: only the n_q rows exist */
+  int64_t lse_rows;
 } ha_attn_operands;
 
 /* Sorted block-diagonal + sampled-column attention, forward.
@@ -315,6 +318,8 @@ typedef struct {
   int64_t q_stride_b, q_stride_h, q_stride_n;
   int64_t k_stride_b, k_stride_h, k_stride_n;
   int64_t v_stride_b, v_stride_h, v_stride_n;
+  int64_t lse_rows;  /* rows of lse per head: n (or 0), or, where the pass is one exact call, up to the next multiple
+                      * of 128, rows n .. lse_rows - 1 then being written as zeros */
 } ha_forward_args;
 
 int64_t ha_forward_workspace_bytes(const ha_forward_args* args);
