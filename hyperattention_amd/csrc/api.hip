@@ -337,15 +337,25 @@ int hash_and_sort(const ha_forward_args& a, const Plan& pl, const Workspace& w, 
   int st;
   if (w.units) {
     const int64_t qs[3] = {t.q_stride_b, t.q_stride_h, t.q_stride_n}, ks[3] = {t.k_stride_b, t.k_stride_h, t.k_stride_n};
+    // no hashed level has its queries in the first granule or its keys in the last one
+    const int64_t unused = a.causal ? w.grid.granule : 0;
     st = ha_hash_pair_u8(a.q, a.k, a.proj, ws + w.buckets_q, ws + w.buckets_k, a.batch, a.heads, a.kv_heads, pl.n_hashed,
-                         a.n, a.d, a.lsh_num_projs, qs, ks, a.dtype, stream);
+                         a.n, a.d, a.lsh_num_projs, qs, ks, unused, pl.n_hashed - unused, a.dtype, stream);
     if (st != HA_OK) return st;
     const uint8_t* ids[2] = {ws + w.buckets_q, ws + w.buckets_k};
     uint32_t* sorted[2] = {(uint32_t*)(ws + w.sorted_q), (uint32_t*)(ws + w.sorted_k)};
     uint32_t* hist[2] = {(uint32_t*)(ws + w.unit_hist_q), (uint32_t*)(ws + w.unit_hist_k)};
     const int64_t seqs[2] = {a.batch * a.heads, a.batch * a.kv_heads};
-    st = ha_rank_units(ids, sorted, hist, seqs, w.grid, stream);
-    if (st != HA_OK) return st;
+    const int first_unit[2] = {a.causal ? w.grid.units_per_granule : 0, 0};
+    const int num_units = w.grid.units_per_seq - first_unit[0];
+    // one unit per sequence is the one segment of the one hashed level: its rank is its order, nothing to place
+    int32_t* whole[2] = {nullptr, nullptr};
+    if (num_units == 1) {
+      whole[0] = (int32_t*)(ws + w.qidx[0]);
+      whole[1] = (int32_t*)(ws + w.kidx[0]);
+    }
+    st = ha_rank_units(ids, sorted, hist, seqs, w.grid, first_unit, num_units, whole, stream);
+    if (st != HA_OK || num_units == 1) return st;
     ha_place_jobs jobs;
     jobs.num_jobs = 0;
     jobs.grid = w.grid;

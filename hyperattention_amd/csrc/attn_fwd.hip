@@ -46,6 +46,9 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+#include <cmath>
+
 namespace {
 
 constexpr int WG_QUERIES = 256;  // sorted query positions per workgroup
@@ -241,6 +244,47 @@ __device__ __forceinline__ const unsigned char* piece_address(const unsigned cha
   return a;
 }
 
+// Rows of segment `seg`: how many queries and keys it has and where they start in the query-side, key-side and
+// out / lse tensors.
+struct SegmentRows {
+  int n_q, n_k;
+  int64_t q_row, k_row, o_row;
+};
+template <bool GATHER>
+__device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params& p, int seg) {
+  SegmentRows r;
+  r.n_q = p.n_q;
+  r.n_k = p.n_k;
+  r.q_row = p.q_seg_off + (int64_t)seg * p.seg_stride;
+  r.k_row = p.k_seg_off + (int64_t)seg * p.seg_stride;
+  r.o_row = p.o_seg_off + (int64_t)seg * p.o_seg_stride;
+  if (!GATHER && p.rag_levels >= 0) {
+    // walk down from the whole sequence: where the segment starts and how many of its rows exist
+    int start = 0, real = p.rag_n;
+    for (int i = 0; i < p.rag_levels; ++i) {
+      const int c = p.rag_half[i];
+      if ((seg >> (p.rag_levels - 1 - i)) & 1) {
+        start += c;
+        real = max(real - c, 0);
+      } else {
+        real = min(real, c);
+      }
+    }
+    if (p.rag_split) {
+      const int c = p.rag_half[p.rag_levels];
+      r.q_row = start + c;
+      r.k_row = start;
+      r.n_q = min(max(real - c, 0), c);
+      r.n_k = min(real, c);
+    } else {
+      r.q_row = r.k_row = start;
+      r.n_q = r.n_k = real;
+    }
+    r.o_row = r.q_row;
+  }
+  return r;
+}
+
 template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false>
 __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
@@ -296,34 +340,9 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   const int b = fast_div(bhk, p.div_kv_heads), hk = bhk - b * fast_div(p.heads, p.div_kv_group);
   const int h = hk * p.kv_group + hg;
 
-  // ---- rows of this segment -----------------------------------------------------------------------
-  int n_q = p.n_q, n_k = p.n_k;
-  int64_t seg_q_row = p.q_seg_off + (int64_t)seg * p.seg_stride, seg_k_row = p.k_seg_off + (int64_t)seg * p.seg_stride;
-  int64_t seg_o_row = p.o_seg_off + (int64_t)seg * p.o_seg_stride;  // first row of the segment in out / lse
-  if (!GATHER && p.rag_levels >= 0) {
-    // walk down from the whole sequence: where the segment starts and how many of its rows exist
-    int start = 0, real = p.rag_n;
-    for (int i = 0; i < p.rag_levels; ++i) {
-      const int c = p.rag_half[i];
-      if ((seg >> (p.rag_levels - 1 - i)) & 1) {
-        start += c;
-        real = max(real - c, 0);
-      } else {
-        real = min(real, c);
-      }
-    }
-    if (p.rag_split) {
-      const int c = p.rag_half[p.rag_levels];
-      seg_q_row = start + c;
-      seg_k_row = start;
-      n_q = min(max(real - c, 0), c);
-      n_k = min(real, c);
-    } else {
-      seg_q_row = seg_k_row = start;
-      n_q = n_k = real;
-    }
-    seg_o_row = seg_q_row;
-  }
+  const SegmentRows rows = segment_rows<GATHER>(p, seg);
+  const int n_q = rows.n_q, n_k = rows.n_k;
+  const int64_t seg_q_row = rows.q_row, seg_k_row = rows.k_row, seg_o_row = rows.o_row;
   // gathered kernel: entries of the query order from this number on name a row that does not exist
   const int q_rows_exist = (GATHER && seg == p.segs - 1) ? p.n_q_last : n_q;
 
@@ -347,6 +366,7 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
 }
 
 #include "attn_fwd_stream.inc"
+#include "attn_fwd_split.inc"
 
 namespace {
 
@@ -357,9 +377,23 @@ int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, con
   return ha_launch_status(what);
 }
 
+template <typename T, int D, bool GATHER, bool CAUSAL>
+int launch_split(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
+  if (p.qk_pieces != D / 8 || p.v_pieces != D / 8)
+    hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, true>), dim3(grid), dim3(SplitShape<D>::THREADS), 0, stream, p);
+  else
+    hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, false>), dim3(grid), dim3(SplitShape<D>::THREADS), 0, stream, p);
+  return ha_launch_status(what);
+}
+
 template <typename T, int D>
 int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, bool reweight, hipStream_t stream) {
   const bool narrow = p.qk_pieces != D / 8 || p.v_pieces != D / 8;
+  if (p.split_keys) {
+    if (gather) return launch_split<T, D, true, false>(p, grid, stream, "ha_block_attn_fwd");
+    if (causal) return launch_split<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
+    return launch_split<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
+  }
   if (gather && reweight)  // the entry point has checked that the head dims are the built ones
     return launch_one<T, D, true, false, false, false, true>(p, grid, stream, "ha_block_attn_fwd");
   if (gather) {
@@ -393,6 +427,32 @@ static ha_divisor make_divisor(int64_t y) {
   return d;
 }
 
+// Whether a launch is better off with the keys of its query tiles split over waves (attn_fwd_split.inc): estimated
+// times in us of the two kernels, from how many steps the longest workgroup takes and how many a CU has to take in
+// all.  Constants fitted to 130 shapes (4 to 128 heads, 500 to 4096 rows exact, 2048 to 16384 rows hashed): a step
+// of the 256-query kernel is 64 keys (0.95 us at d = 64; 1.4 us at d = 128 on a chip that is not full, 1.85 on a
+// full one), a step of a split workgroup 64 queries x 128 keys (0.6 us; 1.25 us), its set-up and the meeting of the
+// splits 2.75 steps.  24 causal heads of 1000 rows: 31 -> 12 us, of 2048 rows: 45 -> 29 us; 16 heads of 4096 rows
+// without mask stay (72 us, split 85).
+static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
+  const char* env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
+  if (env) return atoi(env) != 0;
+  const double cus = 256., vheads = (double)p.batch * p.heads * p.segs;
+  const double tiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES, split_tiles = (p.n_q + 63) / 64;
+  const bool paired = causal && !gather;
+  const double keys = gather ? 128. * p.block_tiles + 64. * p.sample_chunks : p.n_k;
+  const double per_cu = vheads * (paired ? std::ceil(tiles / 2) : tiles) / cus;
+  // steps of the longest workgroup (a pair of tiles where causal) and of all of a CU's
+  const double step = width == 64 ? 0.95 : 1.4 + 0.45 * std::min(1., per_cu), tail = paired ? 5. : 0.;
+  const double longest = (paired ? 4. * (tiles + 1) : keys / 64.) * step + tail;
+  const double all = vheads / cus * tiles * (paired ? 2. * (tiles + 1) : keys / 64.) * step + per_cu * tail;
+  const double whole = (gather ? 9. : 6.) + std::max(longest, all);  // gathered: a chain of row numbers, then rows
+  const double chain = std::ceil(keys / 128.), set_up = 2.75;
+  const double all_split = vheads / cus * split_tiles * ((paired ? chain / 2 + 0.5 : chain) + set_up) + (paired ? chain / 4 : 0.);
+  const double split = 5.5 + (width == 64 ? 0.6 : 1.25) * std::max(chain + set_up, all_split);
+  return split < 0.95 * whole;
+}
+
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,
                    bool reweight, hipStream_t stream) {
   ha_attn_kernel_params p = params;
@@ -413,7 +473,10 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   p.tiles_per_wg = 1;
   const char* stream_env = getenv("HA_STREAM_TILES");  // measurement aid: force the run length (1: off)
   const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0;
-  if (gather && !reweight && p.qk_pieces == width / 8 && p.v_pieces == width / 8 && p.n_q % WG_QUERIES == 0 && qtiles >= 2 &&
+  // (a forced run length asks for the 256-query kernels)
+  p.split_keys = !reweight && !(gather && stream_env) && use_split_keys(p, width, gather, causal);
+  if (p.split_keys) qtiles = (p.n_q + 63) / 64;
+  else if (gather && !reweight && p.qk_pieces == width / 8 && p.v_pieces == width / 8 && p.n_q % WG_QUERIES == 0 && qtiles >= 2 &&
       p.sample_chunks % 2 == 0 && p.n_k % (p.block_tiles * 128) == 0 && 2 * p.block_tiles + p.sample_chunks >= 4 &&
       (stream_env || (width == 128 && plain))) {
     const int64_t slots = 256 * (width == 64 ? 2 : 1);  // workgroups the chip holds at once

@@ -62,17 +62,22 @@ struct ha_place_jobs {
   ha_unit_grid grid;
 };
 
-// ids: byte-sized bucket ids of two tensors, (seqs[i], n) each
+// ids: byte-sized bucket ids of two tensors, (seqs[i], n) each.  Ranked are units first_unit[i] .. first_unit[i] +
+// num_units - 1 of every sequence.  With out[i] (num_units == 1: a unit is a whole segment) a unit's order is
+// written there, (seqs[i], unit) rows local to the unit, and nothing to sorted and hist.
 int ha_rank_units(const uint8_t* const ids[2], uint32_t* const sorted[2], uint32_t* const hist[2], const int64_t seqs[2],
-                  const ha_unit_grid& grid, hipStream_t stream);
+                  const ha_unit_grid& grid, const int (&first_unit)[2], int num_units, int32_t* const out[2],
+                  hipStream_t stream);
 int ha_place_units(const ha_place_jobs& jobs, int total_blocks, hipStream_t stream);
 
 // Bucket ids of the queries and keys of one forward pass as one byte each (at most 8 projections, one shared
 // projection matrix), one launch.  Strides: batch, head, row, in elements.  Defined in lsh_hash.hip.
-// Only the first n_read <= n rows of a sequence exist; the ids of the others are those of zero rows.
+// Only the first n_read <= n rows of a sequence exist; the ids of the others are those of zero rows.  Only the ids of
+// the queries from row q_first on and of the keys before row k_end are written.
 int ha_hash_pair_u8(const void* q, const void* k, const void* proj, uint8_t* ids_q, uint8_t* ids_k, int64_t batch,
                     int64_t heads, int64_t kv_heads, int64_t n, int64_t n_read, int64_t d, int64_t r,
-                    const int64_t (&q_strides)[3], const int64_t (&k_strides)[3], int dtype, hipStream_t stream);
+                    const int64_t (&q_strides)[3], const int64_t (&k_strides)[3], int64_t q_first, int64_t k_end, int dtype,
+                    hipStream_t stream);
 // ha_lsh_hash (int32 ids) with the same n / n_read distinction
 int ha_hash_i32(const void* x, const void* proj, int32_t* buckets, int64_t batch, int64_t heads, int64_t n,
                 int64_t n_read, int64_t d, int64_t r, int64_t x_stride_b, int64_t x_stride_h, int64_t x_stride_n,

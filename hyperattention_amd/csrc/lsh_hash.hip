@@ -32,8 +32,12 @@ struct HashMfma<bf16_t> {
   }
 };
 
-constexpr int HASH_TILES_PER_WAVE = 32;  // tiles of 512 elements (16 MFMA rows of 32 elements)
-constexpr int HASH_UNROLL = 8;           // tiles in flight per wave
+// Tiles of 512 elements (16 MFMA rows of 32 elements) per wave: as many as a launch of that size can have with the
+// chip full of workgroups, so that the projection's set-up is shared; a wave's groups of HASH_UNROLL tiles are one
+// memory round trip after the other (8 heads of 4096 rows at 32 tiles per wave: 32 workgroups, 19 us)
+constexpr int HASH_MAX_TILES_PER_WAVE = 32;
+constexpr int HASH_FULL_CHIP = 2048;  // workgroups
+constexpr int HASH_UNROLL = 8;        // tiles in flight per wave
 
 // A data row of D elements is cut into PARTS = D/32 MFMA rows of 32 elements, so that one load
 // instruction of the wave (16 bytes per lane) covers whole rows: 16/PARTS data rows of D*2 bytes.
@@ -50,9 +54,10 @@ struct HashTensors {
   int seqs0;           // batch * heads of the first tensor
   int seqs;            // sequences of both tensors together
   int64_t n_read;      // rows of a sequence that exist; rows from there up to n hash as zero rows
+  int64_t first[2], end[2];  // rows of every sequence whose ids are wanted
 };
 
-template <typename T, int D, bool OUT8>
+template <typename T, int D, bool OUT8, int TILES>
 __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors ten, const T* __restrict__ proj, int64_t n,
                                                             int r, int64_t psb, int64_t psh, int d_real) {
   typedef typename ElemTraits<T>::vec8 vec8;
@@ -74,6 +79,23 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   const int m = lane & 15, kg = lane >> 4;
   const int my_row = m / PARTS, my_part = m % PARTS;  // data row inside a tile, 32-element part of it
   const int j = m;                                    // projection slot of this lane's C registers
+
+  const int64_t end = ten.end[which];
+  const int64_t wave_row0 = ten.first[which] + ((int64_t)blockIdx.x * 4 + wave) * TILES * ROWS;
+  vec8 xf[HASH_UNROLL];
+  auto load_rows = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < HASH_UNROLL; ++u) {
+      const int64_t row = wave_row0 + (int64_t)(t0 + u) * ROWS + my_row;
+      vec8 z = {};
+      if (row < ten.n_read && my_part * 32 + 8 * kg < d_real) z = *reinterpret_cast<const vec8*>(xbase + row * sn + my_part * 32 + 8 * kg);
+      xf[u] = z;
+    }
+  };
+  // in flight while the projection is set up (a longer wave has them cost it registers that its own overlap of loads
+  // and arithmetic needs: 4 % of a launch over 16.8 M rows)
+  constexpr bool EARLY = TILES == HASH_UNROLL;
+  if (EARLY) load_rows(0);
 
   // the projection matrix goes through LDS once per block (one coalesced pass instead of a chain of
   // dependent 2-byte loads per lane)
@@ -98,21 +120,14 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   // A row's parts meet different B operands, but an MFMA has one B operand per lane column, not per
   // row: so the tile is multiplied once per part with the rows of the other parts zeroed.  (For
   // PARTS == 1 this is a single MFMA.)
-  const int64_t wave_row0 = ((int64_t)blockIdx.x * 4 + wave) * HASH_TILES_PER_WAVE * ROWS;
-  for (int t0 = 0; t0 < HASH_TILES_PER_WAVE; t0 += HASH_UNROLL) {
-    if (wave_row0 + (int64_t)t0 * ROWS >= n) break;
-    vec8 xf[HASH_UNROLL];
 #pragma unroll
-    for (int u = 0; u < HASH_UNROLL; ++u) {
-      const int64_t row = wave_row0 + (int64_t)(t0 + u) * ROWS + my_row;
-      vec8 z = {};
-      if (row < ten.n_read && my_part * 32 + 8 * kg < d_real) z = *reinterpret_cast<const vec8*>(xbase + row * sn + my_part * 32 + 8 * kg);
-      xf[u] = z;
-    }
+  for (int t0 = 0; t0 < TILES; t0 += HASH_UNROLL) {
+    if (wave_row0 + (int64_t)t0 * ROWS >= end) break;
+    if (!EARLY) load_rows(t0);
 #pragma unroll
     for (int u = 0; u < HASH_UNROLL; ++u) {
       const int64_t tile_row0 = wave_row0 + (int64_t)(t0 + u) * ROWS;
-      if (tile_row0 >= n) break;
+      if (tile_row0 >= end) break;
       f32x4 c = {0.f, 0.f, 0.f, 0.f}, ca = {0.f, 0.f, 0.f, 0.f};
       const u32x4 raw = __builtin_bit_cast(u32x4, xf[u]);
 #pragma unroll
@@ -155,7 +170,7 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
         bin = 0;
         for (int jj = 0; jj < r; ++jj) {
           double part = 0.0;
-          if (row < n)
+          if (row < end)
 #pragma unroll
             for (int e = 0; e < 8; ++e)
               part = __builtin_fma((double)ha_to_float(xf[u][e]),
@@ -178,7 +193,7 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
         for (int qq = 1; qq < NS; ++qq) sel = q == qq ? pos[qq] : sel;
         bin = (int)((sel >> (16 * g)) & ((1u << r) - 1u));
       }
-      if (lane < ROWS && tile_row0 + lane < n) {
+      if (lane < ROWS && tile_row0 + lane < end) {
         if (OUT8)
           obase8[tile_row0 + lane] = (uint8_t)(bin ^ (bin >> 1));
         else
@@ -191,13 +206,18 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
 template <typename T, int D, bool OUT8>
 int launch_hash_mfma(HashTensors ten, int64_t seqs, const void* proj, int64_t n, int64_t r, int64_t psb, int64_t psh,
                      int64_t d_real, hipStream_t stream) {
-  const int64_t rows_per_block = 4 * HASH_TILES_PER_WAVE * (16 / (D / 32));
   ten.seqs = (int)seqs;
+  for (int i = 0; i < 2; ++i)
+    if (ten.end[i] <= 0) ten.end[i] = n;
+  const int64_t rows = ten.end[0] - ten.first[0] > ten.end[1] - ten.first[1] ? ten.end[0] - ten.first[0] : ten.end[1] - ten.first[1];
+  int tiles = HASH_MAX_TILES_PER_WAVE;
+  while (tiles > HASH_UNROLL && (rows + 4 * tiles * (16 / (D / 32)) - 1) / (4 * tiles * (16 / (D / 32))) * seqs < HASH_FULL_CHIP) tiles /= 2;
+  const int64_t rows_per_block = 4 * tiles * (16 / (D / 32));
   if (ten.n_read <= 0 || ten.n_read > n) ten.n_read = n;
   const int64_t gy = seqs < 32768 ? seqs : 32768, gz = (seqs + gy - 1) / gy;
-  dim3 grid((unsigned)((n + rows_per_block - 1) / rows_per_block), (unsigned)gy, (unsigned)gz);
-  hipLaunchKernelGGL((lsh_hash_mfma_kernel<T, D, OUT8>), grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh,
-                     (int)d_real);
+  dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block), (unsigned)gy, (unsigned)gz);
+  auto kernel = tiles == 32 ? lsh_hash_mfma_kernel<T, D, OUT8, 32> : tiles == 16 ? lsh_hash_mfma_kernel<T, D, OUT8, 16> : lsh_hash_mfma_kernel<T, D, OUT8, 8>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh, (int)d_real);
   return ha_launch_status("ha_lsh_hash");
 }
 
@@ -246,10 +266,12 @@ int ha_hash_i32(const void* x, const void* proj, int32_t* buckets, int64_t batch
 
 // Bucket ids of the queries and keys of one forward pass as one byte each (r <= 8 projections, one shared
 // projection matrix), in one launch.  q: (batch, heads, n_read, d), k: (batch, kv_heads, n_read, d), d in {64, 128};
-// ids: n >= n_read per sequence, the ids past n_read being those of zero rows.
+// ids: n >= n_read per sequence, the ids past n_read being those of zero rows.  Wanted are the queries' from row q_first
+// on and the keys' before row k_end.
 int ha_hash_pair_u8(const void* q, const void* k, const void* proj, uint8_t* ids_q, uint8_t* ids_k, int64_t batch,
                     int64_t heads, int64_t kv_heads, int64_t n, int64_t n_read, int64_t d, int64_t r,
-                    const int64_t (&q_strides)[3], const int64_t (&k_strides)[3], int dtype, hipStream_t stream) {
+                    const int64_t (&q_strides)[3], const int64_t (&k_strides)[3], int64_t q_first, int64_t k_end, int dtype,
+                    hipStream_t stream) {
   HA_REQUIRE(r >= 1 && r <= 8, HA_ERR_UNSUPPORTED, "ha_forward: byte-sized bucket ids need at most 8 projections");
   HA_REQUIRE(batch * (heads + kv_heads) < (1ll << 30), HA_ERR_SHAPE, "ha_forward: batch*(heads + kv_heads) must be below 2^30");
   HashTensors ten = {};
@@ -259,6 +281,8 @@ int ha_hash_pair_u8(const void* q, const void* k, const void* proj, uint8_t* ids
   ten.heads[0] = (int)heads; ten.heads[1] = (int)kv_heads;
   ten.seqs0 = (int)(batch * heads);
   ten.n_read = n_read;
+  ten.first[0] = q_first; ten.end[0] = n;
+  ten.first[1] = 0; ten.end[1] = k_end;
   const int64_t seqs = batch * (heads + kv_heads);
 #define HA_HASH_PAIR(DD)                                                                                  \
   if (d <= DD) {                                                                                          \
