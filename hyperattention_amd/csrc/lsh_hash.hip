@@ -33,11 +33,14 @@ struct HashMfma<bf16_t> {
 };
 
 // Tiles of 512 elements (16 MFMA rows of 32 elements) per wave: as many as a launch of that size can have with the
-// chip full of workgroups, so that the projection's set-up is shared; a wave's groups of HASH_UNROLL tiles are one
-// memory round trip after the other (8 heads of 4096 rows at 32 tiles per wave: 32 workgroups, 19 us)
-constexpr int HASH_MAX_TILES_PER_WAVE = 32;
+// chip full of workgroups, so that the projection's set-up is shared; a wave's groups of tiles in flight are one
+// memory round trip after the other (8 heads of 4096 rows at 32 tiles per wave: 32 workgroups, 18.3 us; at 8: 10.5)
 constexpr int HASH_FULL_CHIP = 2048;  // workgroups
-constexpr int HASH_UNROLL = 8;        // tiles in flight per wave
+constexpr int HASH_SHORT = 8;         // tiles per wave of a launch that does not fill the chip, all in flight at once
+// tiles in flight per wave: at 8 the longer waves' registers cost them occupancy (4.2 M rows of 256 B: 4.1 TB/s
+// against 4.4 with 4, 16 tiles 3.1)
+template <int TILES>
+constexpr int hash_unroll() { return TILES == HASH_SHORT ? HASH_SHORT : 4; }
 
 // A data row of D elements is cut into PARTS = D/32 MFMA rows of 32 elements, so that one load
 // instruction of the wave (16 bytes per lane) covers whole rows: 16/PARTS data rows of D*2 bytes.
@@ -61,6 +64,7 @@ template <typename T, int D, bool OUT8, int TILES>
 __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors ten, const T* __restrict__ proj, int64_t n,
                                                             int r, int64_t psb, int64_t psh, int d_real) {
   typedef typename ElemTraits<T>::vec8 vec8;
+  constexpr int HASH_UNROLL = hash_unroll<TILES>();
   constexpr int PARTS = D / 32;
   constexpr int ROWS = 16 / PARTS;            // data rows per tile
   constexpr int NS = PARTS >= 4 ? 1 : 4 / PARTS;  // data rows per lane (sums of C registers)
@@ -82,18 +86,21 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
 
   const int64_t end = ten.end[which];
   const int64_t wave_row0 = ten.first[which] + ((int64_t)blockIdx.x * 4 + wave) * TILES * ROWS;
+  // The loads of a group have no condition, so that all of them are in flight together: rows and pieces that do not
+  // exist read the last row or the first piece, and are zeroed where the group is used (a condition on a load
+  // made the compiler wait for it before the next one).
+  const bool piece_exists = my_part * 32 + 8 * kg < d_real;
+  const T* const xlane = xbase + (piece_exists ? my_part * 32 + 8 * kg : 0);
+  const int64_t last_row = ten.n_read - 1;
   vec8 xf[HASH_UNROLL];
   auto load_rows = [&](int t0) {
 #pragma unroll
     for (int u = 0; u < HASH_UNROLL; ++u) {
       const int64_t row = wave_row0 + (int64_t)(t0 + u) * ROWS + my_row;
-      vec8 z = {};
-      if (row < ten.n_read && my_part * 32 + 8 * kg < d_real) z = *reinterpret_cast<const vec8*>(xbase + row * sn + my_part * 32 + 8 * kg);
-      xf[u] = z;
+      xf[u] = *reinterpret_cast<const vec8*>(xlane + (row < last_row ? row : last_row) * sn);
     }
   };
-  // in flight while the projection is set up (a longer wave has them cost it registers that its own overlap of loads
-  // and arithmetic needs: 4 % of a launch over 16.8 M rows)
+  // a short wave's rows are in flight while the projection is set up
   constexpr bool EARLY = TILES == HASH_UNROLL;
   if (EARLY) load_rows(0);
 
@@ -102,7 +109,10 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   __shared__ T lds_p[D * 16];
   // rows of d_real <= D elements: the missing elements of a row and the missing rows of the projection are
   // zeros (they add nothing to a dot product)
-  for (int i = threadIdx.x; i < D * r; i += blockDim.x) lds_p[i] = i < d_real * r ? pbase[i] : (T)0.f;
+  for (int i = threadIdx.x; i < D * r; i += 256) {
+    const T v = pbase[i < d_real * r ? i : 0];
+    lds_p[i] = i < d_real * r ? v : (T)0.f;
+  }
   __syncthreads();
   // B operands: P and |P| for every part: slot j, group kg holds P[part*32 + 8*kg + e][j]; slots >= r are zero
   vec8 pf[PARTS], pa[PARTS];
@@ -111,7 +121,10 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   for (int pt = 0; pt < PARTS; ++pt)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float v = j < r ? ha_to_float(lds_p[(pt * 32 + 8 * kg + e) * r + jc]) : 0.f;
+      // read by every lane (the slots past r a copy of slot 0) and then selected: a read under a condition waits for
+      // itself before the next one is issued
+      float v = ha_to_float(lds_p[(pt * 32 + 8 * kg + e) * r + jc]);
+      v = j < r ? v : 0.f;
       pf[pt][e] = (T)v;
       pa[pt][e] = (T)__builtin_fabsf(v);
     }
@@ -120,10 +133,18 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   // A row's parts meet different B operands, but an MFMA has one B operand per lane column, not per
   // row: so the tile is multiplied once per part with the rows of the other parts zeroed.  (For
   // PARTS == 1 this is a single MFMA.)
-#pragma unroll
+#pragma unroll 1  // unrolled, four copies of the group overflow the instruction cache
   for (int t0 = 0; t0 < TILES; t0 += HASH_UNROLL) {
     if (wave_row0 + (int64_t)t0 * ROWS >= end) break;
     if (!EARLY) load_rows(t0);
+    const bool all_exist = d_real == D && wave_row0 + (int64_t)(t0 + HASH_UNROLL) * ROWS <= ten.n_read;
+    if (!all_exist) {
+#pragma unroll
+      for (int u = 0; u < HASH_UNROLL; ++u) {
+        const bool exists = piece_exists && wave_row0 + (int64_t)(t0 + u) * ROWS + my_row <= last_row;
+        xf[u] = exists ? xf[u] : vec8{};
+      }
+    }
 #pragma unroll
     for (int u = 0; u < HASH_UNROLL; ++u) {
       const int64_t tile_row0 = wave_row0 + (int64_t)(t0 + u) * ROWS;
@@ -210,13 +231,16 @@ int launch_hash_mfma(HashTensors ten, int64_t seqs, const void* proj, int64_t n,
   for (int i = 0; i < 2; ++i)
     if (ten.end[i] <= 0) ten.end[i] = n;
   const int64_t rows = ten.end[0] - ten.first[0] > ten.end[1] - ten.first[1] ? ten.end[0] - ten.first[0] : ten.end[1] - ten.first[1];
-  int tiles = HASH_MAX_TILES_PER_WAVE;
-  while (tiles > HASH_UNROLL && (rows + 4 * tiles * (16 / (D / 32)) - 1) / (4 * tiles * (16 / (D / 32))) * seqs < HASH_FULL_CHIP) tiles /= 2;
+  constexpr int MOST = D >= 128 ? 64 : 32;
+  int tiles = MOST;
+  while (tiles > HASH_SHORT && (rows + 4 * tiles * (16 / (D / 32)) - 1) / (4 * tiles * (16 / (D / 32))) * seqs < HASH_FULL_CHIP) tiles /= 2;
   const int64_t rows_per_block = 4 * tiles * (16 / (D / 32));
   if (ten.n_read <= 0 || ten.n_read > n) ten.n_read = n;
   const int64_t gy = seqs < 32768 ? seqs : 32768, gz = (seqs + gy - 1) / gy;
   dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block), (unsigned)gy, (unsigned)gz);
-  auto kernel = tiles == 32 ? lsh_hash_mfma_kernel<T, D, OUT8, 32> : tiles == 16 ? lsh_hash_mfma_kernel<T, D, OUT8, 16> : lsh_hash_mfma_kernel<T, D, OUT8, 8>;
+  auto kernel = tiles == MOST ? lsh_hash_mfma_kernel<T, D, OUT8, MOST>
+                : tiles == 32 ? lsh_hash_mfma_kernel<T, D, OUT8, 32>
+                : tiles == 16 ? lsh_hash_mfma_kernel<T, D, OUT8, 16> : lsh_hash_mfma_kernel<T, D, OUT8, HASH_SHORT>;
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh, (int)d_real);
   return ha_launch_status("ha_lsh_hash");
 }
