@@ -31,13 +31,13 @@
 #include "attn_fwd.h"
 #include "attn_bwd.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
 
 constexpr int WG_THREADS = 256;
 constexpr int ST_ROWS = 128;       // stationary rows per workgroup
-constexpr int YC = 64;             // streamed rows per LDS tile
 constexpr int MAX_SMOOTH_TILES = 1024;  // query tiles that can attend one 128-key tile (smoothed blocks)
 
 // LDS layout of a streamed tile: row-major [64][D] 2-byte elements, the 16-byte pieces of a row XOR-ed
@@ -77,28 +77,56 @@ __device__ __forceinline__ typename ElemTraits<T>::vec8 bwd_read_tr(const unsign
 #endif
 }
 
+// Scheduling groups: M times one MFMA followed by its share of V plain vector instructions and E transcendentals, and,
+// from MFMA number 1 on, PER at a time of R LDS reads.  (Reads ahead of the first MFMA would be waited for by it: the
+// wait counter holds 15, and more younger reads than that cannot be told from the operands.)
+template <int M, int V, int E, int R, int PER, int I = 0>
+__device__ __forceinline__ void interleave_groups() {
+  if constexpr (I < M) {
+    constexpr int v = V * (I + 1) / M - V * I / M, e = E * (I + 1) / M - E * I / M;
+    constexpr int done = I > 0 ? (I - 1) * PER : 0, reads = I == 0 ? 0 : (R - done < PER ? R - done : PER);
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if constexpr (reads > 0) __builtin_amdgcn_sched_group_barrier(0x100, reads, 0);
+    if constexpr (v > 0) __builtin_amdgcn_sched_group_barrier(0x002, v, 0);
+    if constexpr (e > 0) __builtin_amdgcn_sched_group_barrier(0x400, e, 0);
+    interleave_groups<M, V, E, R, PER, I + 1>();
+  }
+}
+
 template <typename T, int D, int PASS, bool CAUSAL>
-__global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK ? 2 : 1)) void ha_attn_bwd_kernel(const ha_attn_bwd_params p) {
+__global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || PASS == HA_BWD_DQ_EXACT ? 2 : 1)) void ha_attn_bwd_kernel(const ha_attn_bwd_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr bool KEY_ST = PASS == HA_BWD_DKV_EXACT || PASS == HA_BWD_DKV_BLOCK || PASS == HA_BWD_DKV_SAMPLED;
-  // the gathered dK/dV passes start their dP accumulators from -D (below); the exact pass, at its register
-  // limit, subtracts D * scale per pair like the dQ passes
-  constexpr bool FOLD_D = PASS == HA_BWD_DKV_BLOCK || PASS == HA_BWD_DKV_SAMPLED;
   constexpr int KSTEPS = D / 16;  // MFMA k-steps over the head dim
   constexpr int DB = D / 32;      // 32-row blocks of the transposed gradients
   constexpr int PR = D / 8;       // 16-byte pieces per row
   constexpr int RPL = 64 / PR;    // rows per tile load (one load = 64 lanes x 16 bytes)
-  constexpr int LPW = PR / 4;     // tile loads per wave per tile
+  // Streamed rows per LDS tile and tiles in the ring: a step of 32 rows reads its own tile and the next step's, and
+  // the tile after that is in flight; two steps per tile at d = 64, one at d = 128 (the same bytes).
+  constexpr int YC = D <= 64 ? 64 : 32;
+  constexpr int NBUF = D <= 64 ? 3 : 4;
+  constexpr int CPT = 128 / YC;            // chunks per tile of 128 of the sorted order
+  constexpr int LPW = YC * PR / 64 / 4;    // tile loads per wave per tile
   constexpr int TILE_BYTES = YC * D * 2;
 
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_y1[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_y2[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) float lds_lse[2][YC];    // dK/dV passes: L (log2 units) of the streamed queries
-  __shared__ __attribute__((aligned(16))) float lds_delta[2][YC];  // and their -D (gathered passes) or D * scale (exact pass)
+  // The streamed tiles are separate LDS objects, named statically by the loop (unrolled over the ring of NBUF): the
+  // compiler then knows that the tile being filled from memory is not one being read.  As one array with the
+  // buffer's number as an index, every first read of a tile waited for the loads of the NEXT one, just issued.
+  __shared__ __attribute__((aligned(1024))) unsigned char y1_0[TILE_BYTES], y1_1[TILE_BYTES], y1_2[TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char y2_0[TILE_BYTES], y2_1[TILE_BYTES], y2_2[TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char y1_3[NBUF > 3 ? TILE_BYTES : 16], y2_3[NBUF > 3 ? TILE_BYTES : 16];
+  auto y1_tile = [&](int i) -> unsigned char* { return i == 0 ? y1_0 : i == 1 ? y1_1 : i == 2 ? y1_2 : y1_3; };
+  auto y2_tile = [&](int i) -> unsigned char* { return i == 0 ? y2_0 : i == 1 ? y2_1 : i == 2 ? y2_2 : y2_3; };
+  // dK/dV passes: -L / (scale log2 e) and -D of the streamed queries
+  constexpr int SN = KEY_ST ? YC : 4;
+  __shared__ __attribute__((aligned(16))) float lse_0[SN], lse_1[SN], lse_2[SN], lse_3[SN];
+  __shared__ __attribute__((aligned(16))) float delta_0[SN], delta_1[SN], delta_2[SN], delta_3[SN];
+  auto lse_tile = [&](int i) -> float* { return i == 0 ? lse_0 : i == 1 ? lse_1 : i == 2 ? lse_2 : lse_3; };
+  auto delta_tile = [&](int i) -> float* { return i == 0 ? delta_0 : i == 1 ? delta_1 : i == 2 ? delta_2 : delta_3; };
   constexpr bool STAGE_X = KEY_ST || D <= 64;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_x1[STAGE_X ? ST_ROWS * D * 2 : 16];  // staging of the
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_x2[STAGE_X ? ST_ROWS * D * 2 : 16];  // stationary rows
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_x2[STAGE_X ? ST_ROWS * D * 2 : 16];  // staging of the
+                                                                  // second stationary operand (prologue)
   __shared__ int lds_tiles[PASS == HA_BWD_DKV_BLOCK ? MAX_SMOOTH_TILES : 1];
   __shared__ int lds_ntiles;
 
@@ -379,12 +407,20 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
     hipLaunchKernelGGL(ha_bwd_zero_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, (f32x4*)w.dk32, n4);
     st = ha_launch_status("attention backward: clear");
     if (st != HA_OK) return st;
-    // every query attends every sampled key: the queries are cut into ranges, as long as possible (each
-    // range ends in one atomic add per element of the sampled rows) while two workgroups per CU remain
-    int64_t q_split = 8192;
-    while (q_split > 512 && bh * (a.sample_size / ST_ROWS) * ((t.n_q + q_split - 1) / q_split) < 512) q_split /= 2;
-    p.q_split = (int)q_split;
-    const int64_t splits = (t.n_q + q_split - 1) / q_split;
+    // Every query attends every sampled key: the queries are cut into ranges, one workgroup each per tile of sampled
+    // keys.  Taken is the number of ranges with the least time by the rounds of workgroups the chip needs and the
+    // rows of a round; setting up a workgroup and the atomic adds it ends in cost about as much as 384 rows.
+    const int64_t tiles = bh * (a.sample_size / ST_ROWS), slots = D <= 64 ? 512 : 256;
+    int64_t splits = 1, best = INT64_MAX;
+    for (int64_t n = 1; n <= std::min<int64_t>(64, (t.n_q + 511) / 512); ++n) {
+      const int64_t rows = ((t.n_q + n - 1) / n + 63) / 64 * 64;
+      const int64_t cost = (tiles * ((t.n_q + rows - 1) / rows) + slots - 1) / slots * (rows + 384);
+      if (cost < best) {
+        best = cost;
+        p.q_split = (int)rows;
+        splits = (t.n_q + rows - 1) / rows;
+      }
+    }
     st = launch_pass<T, D, HA_BWD_DKV_SAMPLED, false>(p, bh * (a.sample_size / ST_ROWS) * splits, stream,
                                                       "ha_block_attn_bwd: dk, dv of the sampled keys");
     if (st != HA_OK) return st;
