@@ -79,10 +79,10 @@ struct WaveShape {
 __device__ __forceinline__ int fast_div(int x, ha_divisor y) { return (int)(((uint64_t)(uint32_t)x * y.magic) >> y.shift); }
 
 // LDS byte offsets of one lane's operand reads, relative to a tile base (fixed for the whole kernel).
-template <int D>
+template <int DC>
 struct LaneOffsets {
-  int k[D / 16];  // Q / K operand piece of k-step ks for tile row lane%32 (add 32 rows for the upper half)
-  int v[D / 32];  // V^T operand word for dv block db, keys 0..3 (+4 for the upper lane half) of a 16-key half-step
+  int k[DC / 16];  // Q / K operand piece of k-step ks for tile row lane%32 (add 32 rows for the upper half)
+  int v[DC / 32];  // V^T operand word for dv block db, keys 0..3 (+4 for the upper lane half) of a 16-key half-step
 };
 
 // P of the 8 values of half-step H a lane holds per query block (elements 8H..8H+7 of its S^T
@@ -145,19 +145,19 @@ __device__ __forceinline__ void half_step_rescale(const f32x16 (&s_use)[NB], flo
 //           (k-steps H*KSTEPS/2 ..) of the next step's S^T, K rows k_row_off.. of k_tile
 //   VALU  : P of this half-step from s_use -> pb (for the next block) and the row sums
 //   LDS   : V^T of this half-step's keys (v_key_off.. of v_tile) -> vf (for the next block)
-template <typename T, int D, int H>
+template <typename T, int D, int H, int DC>
 __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB], f32x16 (&s_fill)[WaveShape<D>::NB],
                                           const unsigned char* k_tile, int k_row_off,
-                                          const unsigned char* v_tile, int v_key_off, const LaneOffsets<D>& lo,
-                                          const typename ElemTraits<T>::vec8 (&qf)[WaveShape<D>::NB][D / 16],
-                                          f32x16 (&acc)[D / 32][WaveShape<D>::NB], float (&m_run)[WaveShape<D>::NB],
+                                          const unsigned char* v_tile, int v_key_off, const LaneOffsets<DC>& lo,
+                                          const typename ElemTraits<T>::vec8 (&qf)[WaveShape<D>::NB][DC / 16],
+                                          f32x16 (&acc)[DC / 32][WaveShape<D>::NB], float (&m_run)[WaveShape<D>::NB],
                                           float (&l_run)[WaveShape<D>::NB],
                                           typename ElemTraits<T>::vec8 (&pb)[WaveShape<D>::NB],
-                                          typename ElemTraits<T>::vec8 (&vf)[D / 32], float scale_log2) {
+                                          typename ElemTraits<T>::vec8 (&vf)[DC / 32], float scale_log2) {
   typedef typename ElemTraits<T>::vec8 vec8;
   constexpr int NB = WaveShape<D>::NB;
-  constexpr int KH = D / 32;  // k-steps of this half
-  constexpr int DB = D / 32;
+  constexpr int KH = DC / 32;  // k-steps of this half
+  constexpr int DB = DC / 32;
 
   vec8 kf[KH];
 #pragma unroll
@@ -187,16 +187,16 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
   vec8 pn[NB];
   float sum[NB];
   half_step_p<T, NB, H>(s_use, m_run, scale_log2, pn, sum);
-  // Issue order of the block: each of its NB*D/16 large MFMAs is followed by a share of the P arithmetic (8 NB
+  // Issue order of the block: each of its NB*DC/16 large MFMAs is followed by a share of the P arithmetic (8 NB
   // multiply-adds, 4 NB conversions, 8 NB exponentials in all), so the soft-max fills the issue slots behind
   // every MFMA instead of running as one burst after the last of them.  Measured 3 % faster than the
   // scheduler's own order.
-  constexpr int MFMAS = NB * D / 16;
+  constexpr int MFMAS = NB * DC / 16;
 #pragma unroll
   for (int g = 0; g < MFMAS; ++g) {
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
     __builtin_amdgcn_sched_group_barrier(0x002, (12 * NB + MFMAS - 1) / MFMAS, 0);  // its share of plain VALU
-    __builtin_amdgcn_sched_group_barrier(0x400, 8 * NB / MFMAS, 0);             // and of the transcendentals
+    __builtin_amdgcn_sched_group_barrier(0x400, (8 * NB + MFMAS - 1) / MFMAS, 0);             // and of the transcendentals
   }
   // One compare for all query blocks: their sums are >= 0 or NaN, so the total is below the limit
   // only if every one is.  Not "total >= limit": a NaN (row that has seen nothing yet) must take the rare
@@ -234,6 +234,7 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
 // Head dims below the built width D (NARROW kernels): a row holds fewer 16-byte pieces than its LDS slot.
 // A lane whose piece lies past the end of the row fetches these zeros instead, so the tiles hold the rows
 // zero-padded to D: zero columns change neither q.k nor the other columns of the output.
+// Of the padded columns only the first DC (a multiple of 32) are computed with.
 __device__ __attribute__((aligned(16))) const unsigned char ha_zero_piece[16] = {0};
 
 template <bool NARROW>
@@ -285,7 +286,8 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
   return r;
 }
 
-template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false>
+template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
+          int DC = D>
 __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
@@ -293,9 +295,9 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   constexpr int QW = WaveShape<D>::QW;        // queries per wave
   constexpr int WAVES = WaveShape<D>::WAVES;  // waves per workgroup
   constexpr int DV = D;
-  constexpr int KSTEPS = D / 16;  // MFMA k-steps of Q.K^T
-  constexpr int DB = DV / 32;     // 32-row blocks of O^T
-  constexpr int PR = D / 8;       // 16-byte pieces per row
+  constexpr int KSTEPS = DC / 16;  // MFMA k-steps of Q.K^T
+  constexpr int DB = DC / 32;      // 32-row blocks of O^T
+  constexpr int PR = D / 8;        // 16-byte pieces per row
 
   // Separate LDS objects (two K tiles, two V tiles of KC rows, the query rows): the compiler then
   // knows that a tile being filled from HBM and a tile being read do not alias, and does not
@@ -370,32 +372,52 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
 
 namespace {
 
-template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false>
+template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
+          int DC = D>
 int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT>), dim3(grid), dim3(WaveShape<D>::THREADS), 0,
+  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT, DC>), dim3(grid),
+                     dim3(WaveShape<D>::THREADS), 0, stream, p);
+  return ha_launch_status(what);
+}
+
+template <typename T, int D, bool GATHER, bool CAUSAL, bool NARROW, int DC>
+int launch_split(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
+  hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, NARROW, DC>), dim3(grid), dim3(SplitShape<D>::THREADS), 0,
                      stream, p);
   return ha_launch_status(what);
 }
 
-template <typename T, int D, bool GATHER, bool CAUSAL>
-int launch_split(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  if (p.qk_pieces != D / 8 || p.v_pieces != D / 8)
-    hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, true>), dim3(grid), dim3(SplitShape<D>::THREADS), 0, stream, p);
-  else
-    hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, false>), dim3(grid), dim3(SplitShape<D>::THREADS), 0, stream, p);
-  return ha_launch_status(what);
+// Head dims below the built width.  At D = 128 the ones up to 96 (80 and 96 are models' head dims) compute with three
+// quarters of the row: a quarter of the MFMAs and LDS operand reads and 30 to 40 registers less.  16 heads of 20479
+// causal rows of d = 96: 546 -> 507 us (gathered level 87 -> 76, leaves 173 -> 151); 8 heads of 16384 rows without mask:
+// 896 -> 791 us.
+template <typename T, int D, int DC>
+int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, hipStream_t stream) {
+  if (p.split_keys) {
+    if (gather) return launch_split<T, D, true, false, true, DC>(p, grid, stream, "ha_block_attn_fwd");
+    if (causal) return launch_split<T, D, false, true, true, DC>(p, grid, stream, "ha_flash_attn_fwd");
+    return launch_split<T, D, false, false, true, DC>(p, grid, stream, "ha_flash_attn_fwd");
+  }
+  if (gather) return launch_one<T, D, true, false, false, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
+  if (causal) return launch_one<T, D, false, true, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
+  return launch_one<T, D, false, false, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
 }
 
 template <typename T, int D>
 int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, bool reweight, hipStream_t stream) {
-  const bool narrow = p.qk_pieces != D / 8 || p.v_pieces != D / 8;
-  if (p.split_keys) {
-    if (gather) return launch_split<T, D, true, false>(p, grid, stream, "ha_block_attn_fwd");
-    if (causal) return launch_split<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
-    return launch_split<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
-  }
   if (gather && reweight)  // the entry point has checked that the head dims are the built ones
     return launch_one<T, D, true, false, false, false, true>(p, grid, stream, "ha_block_attn_fwd");
+  if (p.qk_pieces != D / 8 || p.v_pieces != D / 8) {
+    if constexpr (D == 128) {
+      if (p.qk_pieces <= 12 && p.v_pieces <= 12) return launch_narrow<T, D, 96>(p, grid, gather, causal, stream);
+    }
+    return launch_narrow<T, D, D>(p, grid, gather, causal, stream);
+  }
+  if (p.split_keys) {
+    if (gather) return launch_split<T, D, true, false, false, D>(p, grid, stream, "ha_block_attn_fwd");
+    if (causal) return launch_split<T, D, false, true, false, D>(p, grid, stream, "ha_flash_attn_fwd");
+    return launch_split<T, D, false, false, false, D>(p, grid, stream, "ha_flash_attn_fwd");
+  }
   if (gather) {
     const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0 && p.n_q % WG_QUERIES == 0;
     if (p.tiles_per_wg > 1) {  // set by ha_attn_launch for the instances built below
@@ -403,13 +425,8 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
       else hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, false>), dim3(grid), dim3(WaveShape<D>::THREADS), 0, stream, p);
       return ha_launch_status("ha_block_attn_fwd");
     }
-    if (narrow) return launch_one<T, D, true, false, false, true>(p, grid, stream, "ha_block_attn_fwd");
     if (plain) return launch_one<T, D, true, false, true>(p, grid, stream, "ha_block_attn_fwd");
     return launch_one<T, D, true, false>(p, grid, stream, "ha_block_attn_fwd");
-  }
-  if (narrow) {
-    if (causal) return launch_one<T, D, false, true, false, true>(p, grid, stream, "ha_flash_attn_fwd");
-    return launch_one<T, D, false, false, false, true>(p, grid, stream, "ha_flash_attn_fwd");
   }
   if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
   return launch_one<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
