@@ -26,6 +26,7 @@
 // workgroup: stored like the exact pass's) and, if it is in the sample list, one from every query:
 // those are computed per range of queries and summed with atomics in small fp32 rows, one per slot of
 // the sample list, which a last kernel adds to the keys' rows of dK, dV.
+// Launches of the exact passes that are too small to fill the chip: split_steps.
 #include "ha_common.h"
 #include "attn_tiles.h"
 #include "attn_fwd.h"
@@ -93,8 +94,8 @@ __device__ __forceinline__ void interleave_groups() {
   }
 }
 
-template <typename T, int D, int PASS, bool CAUSAL>
-__global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || PASS == HA_BWD_DQ_EXACT ? 2 : 1)) void ha_attn_bwd_kernel(const ha_attn_bwd_params p) {
+template <typename T, int D, int PASS, bool CAUSAL, int HALVES>
+__global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || (PASS == HA_BWD_DQ_EXACT && HALVES == 1) ? 2 : 1)) void ha_attn_bwd_kernel(const ha_attn_bwd_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr bool KEY_ST = PASS == HA_BWD_DKV_EXACT || PASS == HA_BWD_DKV_BLOCK || PASS == HA_BWD_DKV_SAMPLED;
@@ -104,8 +105,13 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   constexpr int RPL = 64 / PR;    // rows per tile load (one load = 64 lanes x 16 bytes)
   // Streamed rows per LDS tile and tiles in the ring: a step of 32 rows reads its own tile and the next step's, and
   // the tile after that is in flight; two steps per tile at d = 64, one at d = 128 (the same bytes).
-  constexpr int YC = D <= 64 ? 64 : 32;
-  constexpr int NBUF = D <= 64 ? 3 : 4;
+  // HALVES == 2 (split_steps): 64 stationary rows per workgroup; of the two steps of a tile waves 0, 1 take the first
+  // and waves 2, 3 the second, and the two sums of a row meet in LDS at the end.
+  constexpr int YC = D <= 64 || HALVES == 2 ? 64 : 32;
+  constexpr int STEPS = YC / 32 / HALVES;  // steps that a wave takes from a tile
+  constexpr int NBUF = STEPS == 2 ? 3 : 4;
+  static_assert(HALVES == 1 || PASS == HA_BWD_DQ_EXACT || PASS == HA_BWD_DKV_EXACT, "built for the exact passes");
+  constexpr int ST = ST_ROWS / HALVES;
   constexpr int CPT = 128 / YC;            // chunks per tile of 128 of the sorted order
   constexpr int LPW = YC * PR / 64 / 4;    // tile loads per wave per tile
   constexpr int TILE_BYTES = YC * D * 2;
@@ -125,8 +131,8 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   auto lse_tile = [&](int i) -> float* { return i == 0 ? lse_0 : i == 1 ? lse_1 : i == 2 ? lse_2 : lse_3; };
   auto delta_tile = [&](int i) -> float* { return i == 0 ? delta_0 : i == 1 ? delta_1 : i == 2 ? delta_2 : delta_3; };
   constexpr bool STAGE_X = KEY_ST || D <= 64;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_x2[STAGE_X ? ST_ROWS * D * 2 : 16];  // staging of the
-                                                                  // second stationary operand (prologue)
+  // staging of the second stationary operand (prologue); with four tiles of 64 rows in the ring there is room in them
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_x2[STAGE_X && HALVES == 1 ? ST_ROWS * D * 2 : 16];
   __shared__ int lds_tiles[PASS == HA_BWD_DKV_BLOCK ? MAX_SMOOTH_TILES : 1];
   __shared__ int lds_ntiles;
 
@@ -134,20 +140,24 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   const int wave = tid >> 6, lane = tid & 63;
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   const int hi = lane >> 5, col = lane & 31;
+  const int half = HALVES == 2 ? wave_s >> 1 : 0;       // the step of a tile that the wave takes
+  const int st_wave = HALVES == 2 ? wave_s & 1 : wave_s;  // its 32 stationary rows of the tile
 
   // ---- which head, which stationary tile ------------------------------------------------------
   const int st_total = PASS == HA_BWD_DKV_SAMPLED ? p.sample_size : (KEY_ST ? p.n_k : p.n_q);
-  const int st_tiles = (st_total + ST_ROWS - 1) / ST_ROWS;
+  const int st_tiles = (st_total + ST - 1) / ST;
   const int splits = PASS == HA_BWD_DKV_SAMPLED ? (p.n_q + p.q_split - 1) / p.q_split : 1;
   // Exact causal attention: a workgroup takes the pair of stationary tiles (s, T-1-s), the one that streams more
   // rows first (the last query tile sees every key, the first key tile is seen by every query), so that every
   // workgroup of a launch streams the same number of rows.  The hardware hands out workgroups in order, and a
   // slot freed by a short one stays empty until the ones queued before it are placed.
-  constexpr bool PAIRED = CAUSAL && (PASS == HA_BWD_DQ_EXACT || PASS == HA_BWD_DKV_EXACT);
+  constexpr bool PAIRED = CAUSAL && HALVES == 1 && (PASS == HA_BWD_DQ_EXACT || PASS == HA_BWD_DKV_EXACT);
   const int wg_per_seq = PAIRED ? (st_tiles + 1) / 2 : st_tiles;
-  int rest = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int slot = rest % wg_per_seq;
-  rest /= wg_per_seq;
+  // Steps split over waves: no pairs; the tiles of all sequences that stream the most rows come first (tile-major)
+  const int n_vseq = HALVES == 2 ? gridDim.x / wg_per_seq : 1;
+  int rest = HALVES == 2 ? (int)blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);
+  const int slot = HALVES == 2 ? rest / n_vseq : rest % wg_per_seq;
+  rest = HALVES == 2 ? rest - slot * n_vseq : rest / wg_per_seq;
   const int split = rest % splits;
   const int vseq = rest / splits;   // (batch, head, segment)
   const int seg = vseq % p.segs;
@@ -201,7 +211,7 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   const int n_y = KEY_ST ? p.n_q : p.n_k;  // rows on the streamed side
 
   if constexpr (!PAIRED) {
-    const int tile = slot;
+    const int tile = HALVES == 2 && CAUSAL && PASS == HA_BWD_DQ_EXACT ? st_tiles - 1 - slot : slot;
 #include "attn_bwd_tile.inc"
   } else {
     const int t_long = PASS == HA_BWD_DQ_EXACT ? st_tiles - 1 - slot : slot;
@@ -282,11 +292,11 @@ __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __
   *dst_v = ov;
 }
 
-template <typename T, int D, int PASS, bool CAUSAL>
+template <typename T, int D, int PASS, bool CAUSAL, int HALVES = 1>
 int launch_pass(const ha_attn_bwd_params& p, int64_t grid, hipStream_t stream, const char* what) {
   if (grid <= 0) return HA_OK;
   if (grid >= (1ll << 31)) return ha_fail(HA_ERR_SHAPE, "%s: grid of %lld workgroups", what, (long long)grid);
-  hipLaunchKernelGGL((ha_attn_bwd_kernel<T, D, PASS, CAUSAL>), dim3((unsigned)grid), dim3(WG_THREADS), 0, stream, p);
+  hipLaunchKernelGGL((ha_attn_bwd_kernel<T, D, PASS, CAUSAL, HALVES>), dim3((unsigned)grid), dim3(WG_THREADS), 0, stream, p);
   return ha_launch_status(what);
 }
 
@@ -429,25 +439,58 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   return HA_OK;
 }
 
+// Whether a pass of exact attention is better off with the steps of its streamed tiles split over waves (HALVES = 2: 64
+// stationary rows per workgroup, half as many steps per wave).  What bounds a launch of few workgroups is the longest
+// chain of steps of one of them with CUs idle: a wave alone on its SIMD issues steps as fast as two together, so
+// smaller workgroups fill the idle CUs; on a full chip they do the same work slower (twice the set-up and tile loads
+// per row; dq at d = 128 also one workgroup per CU instead of two).  Estimated in steps of 32 streamed rows: rounds of
+// workgroups over the CUs times their chain, or, for causal tiles one by one (longest first), the longest chain or a CU's
+// share of all.  The weights are fitted to the times of both forms of both passes at 57 shapes per head dim (4 to 128
+// heads, grouped and not, 512 to 4096 rows): where the rule splits, it was never slower by more than they scatter.
+// Times in us, whole -> split, dq | dk, dv, bf16 causal: d 64, 24 heads of 2048 rows 40 -> 32 | 50 -> 39, 4 heads of 1000
+// 24 -> 13 | 29 -> 16, 8 query heads on 2 of 4096 61 -> 42 | 291 -> 189; d 128, 12 heads of 2048 75 -> 41 | 93 -> 49, 32
+// on 8 of 2048 78 (split 98: stays) | 320 -> 161.  Full: d 64, 48 heads of 4096 rows without mask 295 (split 335) | 387 (451).
+bool split_steps(int d, bool dkv, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal) {
+  const double cus = 256., set_up = 2., margin = 0.97;
+  // time of a step where a CU has several workgroups to take, against one alone
+  const double full_whole = d == 64 || dkv ? 0.95 : 0.8, full_split = d == 64 ? 1.25 : dkv ? 1. : 1.4;
+  const double tiles = (double)((rows + 127) / 128), split_tiles = (double)((rows + 63) / 64);
+  const double rounds = std::ceil(seqs * (causal ? std::ceil(tiles / 2) : tiles) / cus), split_wgs = seqs * split_tiles;
+  double whole, split;
+  if (causal) {
+    whole = (rounds > 1 ? full_whole : 1.) * rounds * 4 * (tiles + 1) * group + 2 * set_up * rounds;
+    split = std::max(split_tiles * group + set_up,
+                     full_split * split_wgs / cus * group * (split_tiles + 1) / 2 + set_up * std::max(1., split_wgs / cus));
+  } else {
+    const double streamed = (double)((streamed_rows + 127) / 128), split_rounds = std::ceil(split_wgs / cus);
+    whole = (rounds > 1 ? full_whole : 1.) * rounds * 4 * streamed * group + set_up * rounds;
+    split = (split_rounds > 1 ? full_split : 1.) * split_rounds * 2 * streamed * group + set_up * split_rounds;
+  }
+  return split < margin * whole;
+}
+
+// one pass of exact attention over `seqs` sequences with `rows` stationary rows each
+template <typename T, int D, int PASS>
+int launch_exact(const ha_attn_bwd_params& p, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal,
+                 hipStream_t stream, const char* what) {
+  if (split_steps(D, PASS == HA_BWD_DKV_EXACT, seqs, rows, streamed_rows, group, causal)) {
+    const int64_t grid = seqs * ((rows + 63) / 64);
+    return causal ? launch_pass<T, D, PASS, true, 2>(p, grid, stream, what) : launch_pass<T, D, PASS, false, 2>(p, grid, stream, what);
+  }
+  const int64_t tiles = (rows + ST_ROWS - 1) / ST_ROWS;
+  if (causal) return launch_pass<T, D, PASS, true>(p, seqs * ((tiles + 1) / 2), stream, what);  // pairs of tiles
+  return launch_pass<T, D, PASS, false>(p, seqs * tiles, stream, what);
+}
+
 template <typename T, int D>
 int run_flash_bwd(const ha_attn_operands& t, bool causal, const ha_attn_grads& g, hipStream_t stream) {
   const Workspace w = carve(t, 0, g.workspace);
-  int st;
   ha_attn_bwd_params p;
   fill_bwd_params(t, g, w, p);
   const int64_t bh = t.batch * t.heads * t.segs, bhk = t.batch * (t.heads / t.kv_group) * t.segs;
-  const int64_t q_tiles = (t.n_q + ST_ROWS - 1) / ST_ROWS, k_tiles = (t.n_k + ST_ROWS - 1) / ST_ROWS;
-  if (causal) {
-    // one workgroup per pair of stationary tiles
-    st = launch_pass<T, D, HA_BWD_DQ_EXACT, true>(p, bh * ((q_tiles + 1) / 2), stream, "ha_flash_attn_bwd: dq");
-    if (st != HA_OK) return st;
-    st = launch_pass<T, D, HA_BWD_DKV_EXACT, true>(p, bhk * ((k_tiles + 1) / 2), stream, "ha_flash_attn_bwd: dk, dv");
-  } else {
-    st = launch_pass<T, D, HA_BWD_DQ_EXACT, false>(p, bh * q_tiles, stream, "ha_flash_attn_bwd: dq");
-    if (st != HA_OK) return st;
-    st = launch_pass<T, D, HA_BWD_DKV_EXACT, false>(p, bhk * k_tiles, stream, "ha_flash_attn_bwd: dk, dv");
-  }
-  return st;
+  const int st = launch_exact<T, D, HA_BWD_DQ_EXACT>(p, bh, t.n_q, t.n_k, 1, causal, stream, "ha_flash_attn_bwd: dq");
+  if (st != HA_OK) return st;
+  return launch_exact<T, D, HA_BWD_DKV_EXACT>(p, bhk, t.n_k, t.n_q, t.kv_group, causal, stream, "ha_flash_attn_bwd: dk, dv");
 }
 
 }  // namespace
