@@ -34,13 +34,16 @@ struct HashMfma<bf16_t> {
 
 // Tiles of 512 elements (16 MFMA rows of 32 elements) per wave: as many as a launch of that size can have with the
 // chip full of workgroups, so that the projection's set-up is shared; a wave's groups of tiles in flight are one
-// memory round trip after the other (8 heads of 4096 rows at 32 tiles per wave: 32 workgroups, 18.3 us; at 8: 10.5)
+// memory round trip after the other.  8 sequences of 4096 rows of 128 bytes at 32 tiles per wave: 32 workgroups, 18.3 us;
+// at 8: 8.3, at 4: 6.4, at 2: 6.0, at 1: 6.6; 48 of 2048 rows at 8: 9.8, at 4: 9.1, at 2: 8.3, at 1: 8.9.  On a full chip
+// the set-up counts: 64 of 32768 rows at 32: 57.5, at 4: 64.7, at 2: 81.2
 constexpr int HASH_FULL_CHIP = 2048;  // workgroups
-constexpr int HASH_SHORT = 8;         // tiles per wave of a launch that does not fill the chip, all in flight at once
+constexpr int HASH_SHORT = 8;         // waves of up to this many tiles have them all in flight at once
+constexpr int HASH_LEAST = 2;         // tiles per wave of the smallest launches
 // tiles in flight per wave: at 8 the longer waves' registers cost them occupancy (4.2 M rows of 256 B: 4.1 TB/s
 // against 4.4 with 4, 16 tiles 3.1)
 template <int TILES>
-constexpr int hash_unroll() { return TILES == HASH_SHORT ? HASH_SHORT : 4; }
+constexpr int hash_unroll() { return TILES <= HASH_SHORT ? TILES : 4; }
 
 // A data row of D elements is cut into PARTS = D/32 MFMA rows of 32 elements, so that one load
 // instruction of the wave (16 bytes per lane) covers whole rows: 16/PARTS data rows of D*2 bytes.
@@ -233,14 +236,16 @@ int launch_hash_mfma(HashTensors ten, int64_t seqs, const void* proj, int64_t n,
   const int64_t rows = ten.end[0] - ten.first[0] > ten.end[1] - ten.first[1] ? ten.end[0] - ten.first[0] : ten.end[1] - ten.first[1];
   constexpr int MOST = D >= 128 ? 64 : 32;
   int tiles = MOST;
-  while (tiles > HASH_SHORT && (rows + 4 * tiles * (16 / (D / 32)) - 1) / (4 * tiles * (16 / (D / 32))) * seqs < HASH_FULL_CHIP) tiles /= 2;
+  while (tiles > HASH_LEAST && (rows + 4 * tiles * (16 / (D / 32)) - 1) / (4 * tiles * (16 / (D / 32))) * seqs < HASH_FULL_CHIP) tiles /= 2;
   const int64_t rows_per_block = 4 * tiles * (16 / (D / 32));
   if (ten.n_read <= 0 || ten.n_read > n) ten.n_read = n;
   const int64_t gy = seqs < 32768 ? seqs : 32768, gz = (seqs + gy - 1) / gy;
   dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block), (unsigned)gy, (unsigned)gz);
   auto kernel = tiles == MOST ? lsh_hash_mfma_kernel<T, D, OUT8, MOST>
                 : tiles == 32 ? lsh_hash_mfma_kernel<T, D, OUT8, 32>
-                : tiles == 16 ? lsh_hash_mfma_kernel<T, D, OUT8, 16> : lsh_hash_mfma_kernel<T, D, OUT8, HASH_SHORT>;
+                : tiles == 16 ? lsh_hash_mfma_kernel<T, D, OUT8, 16>
+                : tiles == 8  ? lsh_hash_mfma_kernel<T, D, OUT8, 8>
+                : tiles == 4  ? lsh_hash_mfma_kernel<T, D, OUT8, 4> : lsh_hash_mfma_kernel<T, D, OUT8, HASH_LEAST>;
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh, (int)d_real);
   return ha_launch_status("ha_lsh_hash");
 }

@@ -60,3 +60,10 @@ def test_padded_log_sum_exp_of_a_top_level_leaf_ends_in_zeros(ha, monkeypatch, s
     del filler
     _, lse = m(q, k, v, causal=True, return_lse=True)
     assert lse.shape == (1, 2, -(-n // 128) * 128) and float(lse[..., n:].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("heads,n", [(3, 130), (700, 257), (1030, 257), (1030, 600)])  # 2, 4, 8 and 16 tiles per wave
+def test_hash_at_every_wave_length(ha, heads, n):
+    x = _randn((1, heads, n, 64), 31, torch.bfloat16)
+    proj = _randn((1, 1, 64, 6), 32, torch.bfloat16)
+    assert torch.equal(ha.lsh_hash(x.cuda(), proj.cuda()).cpu(), torch.as_tensor(O.lsh_hash(x, proj[0, 0])).int())
