@@ -348,19 +348,25 @@ std::optional<std::pair<Tensor, Tensor>> forward(const Tensor& query, const Tens
           "query, key and value do not fit together");
   require(query.is_cuda() && key.device() == query.device() && value.device() == query.device(), "tensors must be on one GPU");
   require(query.scalar_type() == at::kHalf || query.scalar_type() == at::kBFloat16, "Only support fp16 and bf16");
-  require(key.scalar_type() == query.scalar_type() && value.scalar_type() == query.scalar_type() &&
-              proj.scalar_type() == query.scalar_type(),
+  require(key.scalar_type() == query.scalar_type() && value.scalar_type() == query.scalar_type(),
           "All tensors must have the same type");
   const int64_t d = query.size(3), dv = value.size(3);
   require(d <= 128 && dv <= 128, "FlashAttention only support head dimensions up to 128");
   const bool grad = wants_grad(query, key, value);
   if (d % 8 || dv % 8 || (grad && !(d == dv && (d == 64 || d == 128)))) return std::nullopt;
-  require(proj.device() == query.device() && proj.numel() == d * projs, "the projection does not fit the head dim");
-
   // the runtime's device is the tensors' one in all but a few programs: ask before paying for a guard
   c10::OptionalDeviceGuard guard;
   if (c10::hip::current_device() != query.device().index()) guard.reset_device(query.device());
   Config c{scale != 0. ? scale : 1. / std::sqrt((double)d), causal, projs, block, sample, min_seq, smooth};
+  // A pass that hashes nothing does not read the projection, wherever it is; one exact call with gradients does not ask
+  // for its type either.
+  const std::vector<Call> calls = calls_of(query.size(2) + (causal && query.size(2) > min_seq ? query.size(2) & 1 : 0), c);
+  const bool hashed = std::any_of(calls.begin(), calls.end(), [](const Call& x) { return x.hashed; });
+  if (hashed || !grad || calls.size() > 1) {
+    require(proj.scalar_type() == query.scalar_type(), "All three tensors must have the same type");
+    require(proj.numel() == d * projs, "the projection does not fit the head dim");
+  }
+  require(!hashed || proj.device() == query.device(), "the projection must be on the tensors' GPU");
   const Tensor p = proj.is_contiguous() ? proj : proj.contiguous();
   const Tensor sampled = sampled_idx ? *sampled_idx : Tensor();
   const int64_t n = query.size(2);

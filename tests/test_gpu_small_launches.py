@@ -67,3 +67,21 @@ def test_hash_at_every_wave_length(ha, heads, n):
     x = _randn((1, heads, n, 64), 31, torch.bfloat16)
     proj = _randn((1, 1, 64, 6), 32, torch.bfloat16)
     assert torch.equal(ha.lsh_hash(x.cuda(), proj.cuda()).cpu(), torch.as_tensor(O.lsh_hash(x, proj[0, 0])).int())
+
+
+def test_module_without_hashing_takes_a_projection_it_does_not_read(ha):
+    m = ha.HyperAttention(input_dim=64, min_seq_len=256)  # projection left in fp32 on the host
+    q, k, v = (_randn((1, 2, 200, 64), s, torch.float16).cuda().requires_grad_() for s in (41, 42, 43))
+    for causal in (True, False):
+        out = m(q, k, v, causal=causal)
+        ref, _ = O.exact_attention(*(x.detach().cpu() for x in (q, k, v)), None, causal)
+        assert_close(out, ref, "out", torch.float16)
+        torch.autograd.grad(out, q, torch.ones_like(out))
+    long = [torch.cat([x.detach()] * 2 + [x.detach()[:, :, :112]], dim=2) for x in (q, k, v)]  # 512 rows: hashed
+    with pytest.raises(AssertionError):
+        m(*long, causal=False)
+    m.lsh.proj_dir = m.lsh.proj_dir.half()  # the right type, still on the host
+    with pytest.raises(AssertionError):
+        m(*long, causal=False)
+    with torch.no_grad():
+        assert m(q, k, v, causal=True).shape == q.shape
