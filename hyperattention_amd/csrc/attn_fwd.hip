@@ -449,7 +449,7 @@ static ha_divisor make_divisor(int64_t y) {
 // all.  Constants fitted to 130 shapes (4 to 128 heads, 500 to 4096 rows exact, 2048 to 16384 rows hashed): a step
 // of the 256-query kernel is 64 keys (0.95 us at d = 64; 1.4 us at d = 128 on a chip that is not full, 1.85 on a
 // full one), a step of a split workgroup 64 queries x 128 keys (0.6 us; 1.25 us), its set-up and the meeting of the
-// splits 2.75 steps.  24 causal heads of 1000 rows: 31 -> 12 us, of 2048 rows: 45 -> 29 us; 16 heads of 4096 rows
+// splits 2.75 steps.  24 causal heads of 1000 rows: 32 -> 14.4 us, of 2048 rows: 46 -> 28 us; 16 heads of 4096 rows
 // without mask stay (72 us, split 85).
 static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   const char* env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
@@ -503,7 +503,9 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
     p.tiles_per_wg = r;
     qtiles = (qtiles + r - 1) / r;
   }
-  p.div_qtiles = make_divisor(qtiles);
+  // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
+  if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
+  p.div_qtiles = make_divisor(p.split_keys == 2 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);
   p.div_kv_heads = make_divisor(p.heads / p.kv_group);
