@@ -180,7 +180,7 @@ ha_block_attn_args block_args(const ha_attn_operands& t, const Tensor& ws, int64
 // What a forward leaves for its backward besides tensors.
 struct Saved : torch::CustomClassHolder {
   Config c;
-  Tensor proj, sampled;                     // the projection for the forward alone
+  Tensor proj, sampled;                     // for the forward alone (the backward's sample list is saved with the tensors)
   std::vector<Call> calls;
   std::vector<int64_t> q_idx_at, k_idx_at;  // per call: byte offsets of its orders in the sort's workspace
   int64_t n;                                // rows of the caller's tensors (an odd n runs with one row more)
@@ -267,8 +267,11 @@ class Attention : public torch::autograd::Function<Attention> {
       out = out.narrow(2, 0, s->n);
       lse = lse.narrow(2, 0, s->n);
     }
-    ctx->save_for_backward({q, k, v, o0, lse0_shifted, o_un, lse_un_shifted, ws});
+    // The sample list too: the backward reads it with the forward's log-sum-exps, so a list that was changed in place
+    // in between has to be an error.
+    ctx->save_for_backward({q, k, v, o0, lse0_shifted, o_un, lse_un_shifted, ws, any_hashed ? s->sampled : Tensor()});
     s->proj.reset();
+    s->sampled.reset();
     ctx->saved_data["s"] = c10::IValue::make_capsule(s);
     ctx->mark_non_differentiable({lse});
     ctx->set_materialize_grads(false);
@@ -314,7 +317,7 @@ class Attention : public torch::autograd::Function<Attention> {
       g.workspace = ws.data_ptr();
       g.workspace_bytes = ws.numel();
       if (s->calls[i].hashed) {
-        ha_block_attn_args a = block_args(ops[i], saved[7], s->q_idx_at[i], s->k_idx_at[i], s->sampled, c);
+        ha_block_attn_args a = block_args(ops[i], saved[7], s->q_idx_at[i], s->k_idx_at[i], saved[8], c);
         check(ha_block_attn_bwd(&a, &g, stream));
       } else {
         check(ha_flash_attn_bwd(&ops[i], s->calls[i].causal, &g, stream));

@@ -1,0 +1,66 @@
+"""GPU tests of the module under autograd as a training program calls it: explicit sample lists, tensors that are views
+of a layer's projections.  Gradients against torch autograd on the oracle."""
+import pytest
+import torch
+
+from oracle import hyper_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+from _util import _gen, _randn
+from test_gpu_backward import _check, _oracle_grads, ha  # noqa: F401
+
+BLOCK = SAMPLE = 128
+
+
+def _module(ha, d, dtype, min_seq_len, **kw):
+    m = ha.HyperAttention(input_dim=d, block_size=BLOCK, sample_size=SAMPLE, min_seq_len=min_seq_len, rng=_gen(95), **kw)
+    return m.to(device="cuda", dtype=dtype)
+
+
+def _reference(m, q, k, v, do, causal, sampled=None):
+    proj = m.lsh.proj_dir[0, 0].cpu()
+    expand = lambda x: x.repeat_interleave(q.shape[1] // x.shape[1], dim=1)
+    return _oracle_grads(lambda a, b, c: O.hyper_forward(a, expand(b), expand(c), proj, causal=causal, block_size=BLOCK,
+                                                         sample_size=SAMPLE, min_seq_len=m.min_seq_len, sampled_idx=sampled,
+                                                         detach_lse=True), q, k, v, do)
+
+
+# ------------------------------------------------------------------------------- explicit sample lists
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("idx_dtype", [torch.int32, torch.int64])
+def test_training_with_an_explicit_sample_list(ha, causal, idx_dtype):
+    """The gradients are those of the listed rows.  A list that is redrawn in place between forward and backward is an
+    error where the backward would read it (int32 on the GPU: taken as it is) and without effect where it was copied."""
+    dtype, h, n, d = torch.float16, 2, 1024, 64
+    q, k, v, do = (_randn((1, h, n, d), 60 + i, dtype) for i in range(4))
+    sampled = torch.randperm(256, generator=_gen(64))[:SAMPLE]
+    m = _module(ha, d, dtype, 256, sampled_idx=sampled.to(device="cuda", dtype=idx_dtype))
+    ref = _reference(m, q, k, v, do, causal, sampled)
+    leaves = [x.cuda().requires_grad_() for x in (q, k, v)]
+    out = m(*leaves, causal=causal)
+    for got, want, name in zip(torch.autograd.grad(out, leaves, do.cuda(), retain_graph=True), ref, ("dq", "dk", "dv")):
+        _check(got, want, name, dtype)
+    m.sampled_idx.add_(1)
+    if idx_dtype == torch.int32:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(out, leaves, do.cuda())
+    else:
+        for got, want, name in zip(torch.autograd.grad(out, leaves, do.cuda()), ref, ("dq", "dk", "dv")):
+            _check(got, want, name, dtype)
+
+
+def test_saved_tensor_hooks_see_the_sample_list(ha):
+    dtype, n, d = torch.float16, 512, 64
+    q, k, v, do = (_randn((1, 1, n, d), 70 + i, dtype).cuda() for i in range(4))
+    m = _module(ha, d, dtype, 256, sampled_idx=torch.arange(SAMPLE, dtype=torch.int32, device="cuda"))
+    leaves = [x.clone().requires_grad_() for x in (q, k, v)]
+    want = torch.autograd.grad(m(*leaves, causal=False), leaves, do)
+    with torch.autograd.graph.save_on_cpu():
+        out = m(*leaves, causal=False)
+    for a, b in zip(torch.autograd.grad(out, leaves, do), want):
+        _check(a, b, "gradient", dtype)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: packed.append(x) or x, lambda x: x):
+        m(*leaves, causal=False)
+    assert any(x.data_ptr() == m.sampled_idx.data_ptr() for x in packed)
