@@ -402,21 +402,22 @@ class HyperAttnFunc(torch.autograd.Function):
                 sampled_idx):
         o, lse = hyper_attn_func(q, k, v, q_sort_idx, k_sort_idx, block_size, sample_size, softmax_scale,
                                  smooth_block, sampled_idx=sampled_idx)
-        ctx.save_for_backward(q, k, v, q_sort_idx, k_sort_idx, o, lse)
+        # the sample list among them: the backward reads it with the forward's log-sum-exps, so a list that was
+        # changed in place in between has to be an error
+        ctx.save_for_backward(q, k, v, q_sort_idx, k_sort_idx, o, lse, sampled_idx)
         # no gradient is returned for lse: saying so up front keeps autograd from computing one
         ctx.mark_non_differentiable(lse)
-        ctx.sampled_idx = sampled_idx
         ctx.conf = (block_size, sample_size, softmax_scale or 1.0 / math.sqrt(q.shape[-1]), smooth_block)
         return o, lse
 
     @staticmethod
     def backward(ctx, do, dlse=None):
-        q, k, v, q_sort_idx, k_sort_idx, o, lse = ctx.saved_tensors
+        q, k, v, q_sort_idx, k_sort_idx, o, lse, sampled_idx = ctx.saved_tensors
         block_size, sample_size, softmax_scale, smooth_block = ctx.conf
         do = do.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         a, keep = _block_attn_args(q, k, v, o, lse, q_sort_idx, k_sort_idx, block_size, sample_size, softmax_scale,
-                                   smooth_block, ctx.sampled_idx)
+                                   smooth_block, sampled_idx)
         g, ws = _attn_grads(a.t, do, dq, dk, dv, sample_size=sample_size)
         with torch.cuda.device(q.device):
             _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), _stream(q)))

@@ -64,3 +64,15 @@ def test_saved_tensor_hooks_see_the_sample_list(ha):
     with torch.autograd.graph.saved_tensors_hooks(lambda x: packed.append(x) or x, lambda x: x):
         m(*leaves, causal=False)
     assert any(x.data_ptr() == m.sampled_idx.data_ptr() for x in packed)
+
+
+def test_the_operator_refuses_a_sample_list_changed_before_its_backward(ha):
+    dtype, n, d = torch.float16, 512, 64
+    q, k, v, do = (_randn((1, n, 1, d), 80 + i, dtype).cuda() for i in range(4))
+    order = torch.randperm(n, generator=_gen(84)).view(1, n, 1).cuda()
+    sampled = torch.arange(SAMPLE, device="cuda")
+    leaf = q.requires_grad_()
+    out, _ = ha.hyper_attn_func(leaf, k, v, order, order, BLOCK, SAMPLE, sampled_idx=sampled)
+    sampled.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out, leaf, do)
