@@ -349,13 +349,17 @@ std::optional<std::pair<Tensor, Tensor>> forward(const Tensor& query, const Tens
   require(value.size(2) == key.size(2) && value.size(1) == key.size(1) && value.size(0) == key.size(0) &&
               query.size(0) == key.size(0) && query.size(3) == key.size(3),
           "query, key and value do not fit together");
+  const bool grad = wants_grad(query, key, value);
+  // no length is below a negative min_seq_len, so the causal recursion would not end; without mask there is nothing to
+  // end, and a call with gradients hashes, as with zero
+  require(min_seq >= 0 || (grad && !causal), "min_seq_len must not be negative");
+  min_seq = std::max<int64_t>(min_seq, 0);
   require(query.is_cuda() && key.device() == query.device() && value.device() == query.device(), "tensors must be on one GPU");
   require(query.scalar_type() == at::kHalf || query.scalar_type() == at::kBFloat16, "Only support fp16 and bf16");
   require(key.scalar_type() == query.scalar_type() && value.scalar_type() == query.scalar_type(),
           "All tensors must have the same type");
   const int64_t d = query.size(3), dv = value.size(3);
   require(d <= 128 && dv <= 128, "FlashAttention only support head dimensions up to 128");
-  const bool grad = wants_grad(query, key, value);
   if (d % 8 || dv % 8 || (grad && !(d == dv && (d == 64 || d == 128)))) return std::nullopt;
   // the runtime's device is the tensors' one in all but a few programs: ask before paying for a guard
   c10::OptionalDeviceGuard guard;

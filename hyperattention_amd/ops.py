@@ -170,7 +170,7 @@ def smallest_hashed_key_length(n: int, min_seq_len: int, causal: bool):
     if not causal:
         return None if min_seq_len > n else n
     smallest = None
-    while n > min_seq_len:
+    while n > max(min_seq_len, 1):  # one row is not cut in two
         n = (n + 1) // 2
         if not min_seq_len > n:
             smallest = n
@@ -489,7 +489,7 @@ def causal_plan(n: int, min_seq_len: int):
     (:61-64); leaf the length the recursion stops at.  Only n itself can be odd in a shape the kernels take:
     hashed halves are multiples of 128, and a level with shorter halves is the last."""
     halves = []
-    while n > min_seq_len:
+    while n > max(min_seq_len, 1):  # one row is not cut in two
         n = (n + 1) // 2
         halves.append(n)
     return halves, n

@@ -309,3 +309,23 @@ def test_sampled_idx_bounds_of_an_inference_tensor():
     with pytest.raises(AssertionError, match="sampled_idx must lie in"):
         ops.check_sampled_idx(idx, 100)
     assert not hasattr(idx, "_ha_bounds")
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("sampled", [False, True])
+def test_a_negative_min_seq_len_is_refused(grad, sampled):
+    """The causal recursion halves until a length is at most min_seq_len: with a negative one it would not end."""
+    import torch
+    from hyperattention_amd import HyperAttention
+    q, k, v = (torch.zeros((1, 1, 256, 64), dtype=torch.float16, requires_grad=grad) for _ in range(3))
+    m = HyperAttention(input_dim=64, min_seq_len=-1, sample_size=128, sampled_idx=torch.zeros(128, dtype=torch.int32) if sampled else None)
+    with pytest.raises(AssertionError, match="min_seq_len must not be negative"):
+        m(q, k, v, causal=True)
+
+
+@pytest.mark.parametrize("min_seq_len", [-1, 0, 1])
+def test_the_plan_of_the_recursion_ends_at_one_row(min_seq_len):
+    from hyperattention_amd import ops
+    assert ops.causal_plan(8, min_seq_len) == ([4, 2, 1], 1)
+    assert ops.smallest_hashed_key_length(8, min_seq_len, True) == 1
+    assert ops.smallest_hashed_key_length(8, min_seq_len, False) == 8

@@ -76,3 +76,15 @@ def test_the_operator_refuses_a_sample_list_changed_before_its_backward(ha):
     sampled.add_(1)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(out, leaf, do)
+
+
+def test_training_without_mask_takes_a_negative_min_seq_len(ha):
+    dtype, n, d = torch.float16, 256, 64
+    q, k, v, do = (_randn((1, 1, n, d), 90 + i, dtype) for i in range(4))
+    m = _module(ha, d, dtype, -1)
+    leaves = [x.cuda().requires_grad_() for x in (q, k, v)]
+    grads = torch.autograd.grad(m(*leaves, causal=False), leaves, do.cuda())
+    for got, want, name in zip(grads, _reference(m, q, k, v, do, False), ("dq", "dk", "dv")):
+        _check(got, want, name, dtype)
+    with torch.no_grad(), pytest.raises(AssertionError, match="min_seq_len"):
+        m(*leaves, causal=False)
