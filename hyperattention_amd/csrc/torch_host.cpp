@@ -173,6 +173,10 @@ ha_block_attn_args block_args(const ha_attn_operands& t, const Tensor& ws, int64
   a.q_idx_stride_b = t.heads * rows; a.q_idx_stride_h = rows; a.q_idx_stride_n = 1;
   a.k_idx_stride_b = kv_heads * rows; a.k_idx_stride_h = rows; a.k_idx_stride_n = 1;
   a.sampled_idx = sampled.defined() ? sampled.data_ptr() : nullptr;
+  if (sampled.defined() && sampled.dim() > 1) {  // a list per k/v head: hyper_attention.py lets it through without mask
+    a.sampled_stride_h = c.sample;
+    a.sampled_stride_b = sampled.dim() > 2 ? kv_heads * c.sample : 0;
+  }
   a.block_size = c.block; a.sample_size = c.sample; a.smooth_block = c.smooth;
   return a;
 }

@@ -28,7 +28,8 @@ class HyperAttention(torch.nn.Module):
         - block_size and sample_size must be divisible by 128
         Optional keyword hooks (not in the reference, for reproducible runs): `rng` (torch.Generator
         for the projection), `proj_dir` (explicit (input_dim, lsh_num_projs) projection) and
-        `sampled_idx` (explicit sampled key rows, shape (sample_size,)).
+        `sampled_idx` (explicit sampled key rows, shape (sample_size,); with gradients and without mask also a list
+        per key/value head, (heads, sample_size) or (batch, heads, sample_size)).
         `residual_estimator=True` (not in the reference either; the estimator of the HyperAttention paper):
         every hashed call weights its sampled keys by n_key / sample_size and leaves out those that are
         already among the block keys of the query.  Forward only, head dims 64 and 128.
@@ -63,7 +64,7 @@ class HyperAttention(torch.nn.Module):
         proj = self.lsh.proj_dir
         if self.residual_estimator:
             return self._forward_residual_estimator(query, key, value, scale or dim ** (-0.5), causal, return_lse)
-        sampled = self._sampled(query, causal) if self.sampled_idx is not None else None
+        sampled = self._sampled(query, key, value, causal) if self.sampled_idx is not None else None
         run = _lib.host().forward
         result = run(query, key, value, proj, sampled, scale or 0.0, causal is not False, self.lsh_num_projs,
                      self.block_size, self.sample_size, self.min_seq_len, bool(self.smooth_block))
@@ -80,15 +81,19 @@ class HyperAttention(torch.nn.Module):
             result = attn[..., :dim_v], lse
         return result if return_lse else result[0]
 
-    def _sampled(self, query, causal):
+    def _sampled(self, query, key, value, causal):
         """The module's explicit sample list as an int32 device tensor, checked against the shortest hashed call (the
-        list serves every level); None where no call is hashed."""
+        list serves every level); None where no call is hashed.  One list for all heads; the one call of a pass with
+        gradients and without mask takes a list per key/value head too, as hyper_attn_func does."""
         shortest = ops.smallest_hashed_key_length(query.shape[2], self.min_seq_len, causal is not False)
         if shortest is None:
             return None
         ops.check_sampled_idx(self.sampled_idx, shortest)
         sampled = self.sampled_idx.to(device=query.device, dtype=torch.int32).contiguous()
-        assert sampled.shape == (self.sample_size,), "the module's sampled_idx is one (sample_size,) list"
+        shapes, heads = [(self.sample_size,)], key.shape[1]
+        if causal is False and ops._wants_grad(query, key, value):
+            shapes += [(heads, self.sample_size), (key.shape[0], heads, self.sample_size)]
+        assert sampled.shape in shapes, f"the module's sampled_idx must have one of the shapes {shapes}"
         return sampled
 
     def _forward_residual_estimator(self, query, key, value, scale, causal, return_lse):

@@ -50,6 +50,26 @@ def test_training_with_an_explicit_sample_list(ha, causal, idx_dtype):
             _check(got, want, name, dtype)
 
 
+@pytest.mark.parametrize("per_batch", [False, True])
+def test_training_without_mask_takes_a_sample_list_per_key_head(ha, per_batch):
+    dtype, b, h, hk, n, d = torch.float16, 2, 4, 2, 512, 64
+    q, do = (_randn((b, h, n, d), 65 + i, dtype) for i in range(2))
+    k, v = (_randn((b, hk, n, d), 67 + i, dtype) for i in range(2))
+    lists = torch.stack([torch.randperm(n, generator=_gen(i))[:SAMPLE] for i in range(b * hk)]).view(b, hk, SAMPLE)
+    if not per_batch:
+        lists = lists[0]
+    m = _module(ha, d, dtype, 256, sampled_idx=lists.cuda())
+    of_q_heads = lists.expand(b, hk, SAMPLE).repeat_interleave(h // hk, dim=1)
+    leaves = [x.cuda().requires_grad_() for x in (q, k, v)]
+    grads = torch.autograd.grad(m(*leaves, causal=False), leaves, do.cuda())
+    for got, want, name in zip(grads, _reference(m, q, k, v, do, False, of_q_heads), ("dq", "dk", "dv")):
+        _check(got, want, name, dtype)
+    with pytest.raises(AssertionError):  # the recursion's calls share one list, and so does the one-call forward
+        m(*leaves, causal=True)
+    with torch.no_grad(), pytest.raises(AssertionError):
+        m(*leaves, causal=False)
+
+
 def test_saved_tensor_hooks_see_the_sample_list(ha):
     dtype, n, d = torch.float16, 512, 64
     q, k, v, do = (_randn((1, 1, n, d), 70 + i, dtype).cuda() for i in range(4))
