@@ -62,6 +62,13 @@ bool readable(const Tensor& t) {
 }
 Tensor as_readable(const Tensor& t) { return readable(t) ? t : t.contiguous(); }
 
+// A row's address is its head's plus 32 bits, the row number times a stride below 16 MiB (include/hyperattn.h).  With
+// gradients wider views are copied; a forward alone leaves them to the library, which refuses them.
+bool addressable(const Tensor& t) {
+  return t.stride(2) < (int64_t(1) << 23) && (t.size(2) - 1) * t.stride(2) * 2 + 256 <= (int64_t(1) << 32);
+}
+Tensor as_addressable(const Tensor& t) { return readable(t) && addressable(t) ? t : t.contiguous(); }
+
 struct Config {
   double scale;
   bool causal;
@@ -293,7 +300,7 @@ class Attention : public torch::autograd::Function<Attention> {
     c10::OptionalDeviceGuard guard(q.device());
     void* const stream = stream_of(q);
     const int64_t n = q.size(2);
-    dout = n != s->n ? at::constant_pad_nd(dout, {0, 0, 0, n - s->n}) : as_readable(dout);
+    dout = n != s->n ? at::constant_pad_nd(dout, {0, 0, 0, n - s->n}) : as_addressable(dout);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     // A call's gradients are linear in the output gradient it is given, and that enters only through
     // P = exp(s - lse): weighting a row's output gradient by the call's merge weight w equals giving the call the
@@ -388,7 +395,7 @@ std::optional<std::pair<Tensor, Tensor>> forward(const Tensor& query, const Tens
     s->c = c;
     s->proj = p;
     s->sampled = sampled;
-    const variable_list r = Attention::apply(as_readable(query), as_readable(key), as_readable(value), s);
+    const variable_list r = Attention::apply(as_addressable(query), as_addressable(key), as_addressable(value), s);
     out = r[0];
     lse = r[1];
   } else {

@@ -108,3 +108,21 @@ def test_training_without_mask_takes_a_negative_min_seq_len(ha):
         _check(got, want, name, dtype)
     with torch.no_grad(), pytest.raises(AssertionError, match="min_seq_len"):
         m(*leaves, causal=False)
+
+
+# ------------------------------------------------------------------------------- layouts
+@pytest.mark.parametrize("wide", ["query", "gradient"])
+def test_training_copies_rows_that_lie_too_far_apart_to_be_addressed(ha, wide):
+    """Rows 16 MiB apart, 4 GiB in all: past the kernels' limits, so the module works on a copy."""
+    dtype, n, d = torch.float16, 256, 64
+    q, k, v, do = (_randn((1, 1, n, d), 100 + i, dtype) for i in range(4))
+    far = torch.empty((1, 1, n, 1 << 23), dtype=dtype, device="cuda")[..., :d]
+    m = _module(ha, d, dtype, 128)
+    leaves = [x.cuda().requires_grad_() for x in (q, k, v)]
+    if wide == "query":
+        leaves[0] = far.copy_(q.cuda()).requires_grad_()
+        out, dout = m(*leaves, causal=True), do.cuda()
+    else:
+        out, dout = m(*leaves, causal=True), far.copy_(do.cuda())
+    for got, want, name in zip(torch.autograd.grad(out, leaves, dout), _reference(m, q, k, v, do, True), ("dq", "dk", "dv")):
+        _check(got, want, name, dtype)
