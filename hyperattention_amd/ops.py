@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import weakref
 
 import torch
 
@@ -138,7 +139,8 @@ def padded_head_dim(d):
     return 64 if d <= 64 else 128
 
 
-_SAMPLED_BOUNDS = {}  # bounds of explicit sample lists already looked at
+# bounds of explicit sample lists already looked at: id -> (weak reference, (address, shape, version), smallest, largest)
+_SAMPLED_BOUNDS = {}
 
 
 def check_sampled_idx(sampled_idx, n_k: int):
@@ -149,20 +151,21 @@ def check_sampled_idx(sampled_idx, n_k: int):
     tensor: pass the list once before capturing a graph)."""
     if sampled_idx is None:
         return
-    # keyed by the tensor's identity, storage and version; an inference tensor has no version counter and is
-    # checked on every call
+    # An id and an address are given out again as soon as a list dies, so an entry counts only while its tensor lives;
+    # an inference tensor has no version counter and is looked at on every call
     version = None if sampled_idx.is_inference() else sampled_idx._version
-    key = (id(sampled_idx), sampled_idx.data_ptr(), tuple(sampled_idx.shape), version)
-    cached = _SAMPLED_BOUNDS.get(key) if version is not None else None
-    if cached is None:
+    state = (sampled_idx.data_ptr(), tuple(sampled_idx.shape), version)
+    cached = _SAMPLED_BOUNDS.get(id(sampled_idx)) if version is not None else None
+    if cached is None or cached[0]() is not sampled_idx or cached[1] != state:
         lo, hi = (int(sampled_idx.min()), int(sampled_idx.max())) if sampled_idx.numel() else (0, -1)
-        cached = (version, lo, hi)
+        cached = (weakref.ref(sampled_idx), state, lo, hi)
         if version is not None:
             if len(_SAMPLED_BOUNDS) > 64:
                 _SAMPLED_BOUNDS.clear()
-            _SAMPLED_BOUNDS[key] = cached
-    assert cached[1] >= 0 and cached[2] < n_k, \
-        f"sampled_idx must lie in [0, {n_k}) (the key length of the shortest hashed call); got [{cached[1]}, {cached[2]}]"
+            _SAMPLED_BOUNDS[id(sampled_idx)] = cached
+    lo, hi = cached[2:]
+    assert lo >= 0 and hi < n_k, \
+        f"sampled_idx must lie in [0, {n_k}) (the key length of the shortest hashed call); got [{lo}, {hi}]"
 
 
 def smallest_hashed_key_length(n: int, min_seq_len: int, causal: bool):

@@ -329,3 +329,18 @@ def test_the_plan_of_the_recursion_ends_at_one_row(min_seq_len):
     assert ops.causal_plan(8, min_seq_len) == ([4, 2, 1], 1)
     assert ops.smallest_hashed_key_length(8, min_seq_len, True) == 1
     assert ops.smallest_hashed_key_length(8, min_seq_len, False) == 8
+
+
+def test_bounds_of_a_sample_list_are_not_those_of_a_dead_one():
+    """A list drawn anew for every call often lies where the last one lay, under the same id and version."""
+    import torch
+    from hyperattention_amd import HyperAttention, ops
+    module = HyperAttention(input_dim=64)
+    for _ in range(20):
+        module.sampled_idx = None
+        module.sampled_idx = torch.randint(0, 5, (128,))
+        ops.check_sampled_idx(module.sampled_idx, 1024)
+        module.sampled_idx = None
+        module.sampled_idx = torch.randint(5000, 6000, (128,))
+        with pytest.raises(AssertionError, match="sampled_idx must lie in"):
+            ops.check_sampled_idx(module.sampled_idx, 1024)
