@@ -32,3 +32,23 @@ def test_exact_backward_at_tile_edges(ha, dtype, d, heads, causal, nq, nk):
         got = (grads[0][:, h], grads[1][:, kv:kv + 1], grads[2][:, kv:kv + 1])
         for g, r, name in zip(got, ref, ("dq", "dk", "dv")):
             _check(g, r, f"{name} of key head {kv}", dtype)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("heads,n", [(2, 65), (1024, 512)])
+def test_fp16_dk_of_large_gradients(ha, d, heads, n):
+    """P (dP - D) of the first rows is past 65504 and scale times it is not: dK comes from the latter."""
+    sign = torch.where(_randn((1, heads, n, 1), 41, torch.float32) > 0, 1., -1.)
+    v = (24 * sign).expand(1, heads, n, d).half()
+    do = torch.full((1, heads, n, d), 160.).half()
+    q, k = ((_randn((1, heads, n, d), s, torch.float32) * a).half() for s, a in ((42, 0.05), (43, 0.01)))
+    h = slice(0, 2)
+    ref = _oracle_grads(lambda a, b, c: O.exact_attention(a, b, c, None, True), q[:, h], k[:, h], v[:, h], do[:, h])
+    dp = torch.einsum("bhid,bhjd->bhij", do[:, h].double(), v[:, h].double())
+    p = torch.softmax((torch.einsum("bhid,bhjd->bhij", q[:, h].double(), k[:, h].double()) * d ** -0.5)
+                      .masked_fill(torch.ones(n, n).triu(1).bool(), float("-inf")), dim=-1)
+    ds = (p * (dp - (p * dp).sum(-1, keepdim=True))).abs().max()
+    assert 65504 < ds and ds * d ** -0.5 < 65504
+    _, dk, dv = _gpu_grads(lambda a, b, c: ha.flash_attn_func(a, b, c, None, True), q, k, v, do)[2:]
+    _check(dk[:, h], ref[1], "dk", torch.float16)
+    _check(dv[:, h], ref[2], "dv", torch.float16)
