@@ -445,29 +445,46 @@ static ha_divisor make_divisor(int64_t y) {
 }
 
 // Whether a launch is better off with the keys of its query tiles split over waves (attn_fwd_split.inc): estimated
-// times in us of the two kernels, from how many steps the longest workgroup takes and how many a CU has to take in
-// all.  Constants fitted to 130 shapes (4 to 128 heads, 500 to 4096 rows exact, 2048 to 16384 rows hashed): a step
-// of the 256-query kernel is 64 keys (0.95 us at d = 64; 1.4 us at d = 128 on a chip that is not full, 1.85 on a
-// full one), a step of a split workgroup 64 queries x 128 keys (0.6 us; 1.25 us), its set-up and the meeting of the
-// splits 2.75 steps.  24 causal heads of 1000 rows: 32 -> 14.4 us, of 2048 rows: 46 -> 28 us; 16 heads of 4096 rows
-// without mask stay (72 us, split 85).
+// times in us of the two kernels, from how many steps a workgroup takes and how many workgroups a CU has to take.  A step
+// of the 256-query kernel is 64 keys, one of a split workgroup 64 queries x 128 keys.  What the estimates have to catch:
+// - 256-query workgroups: up to one per CU the launch takes as long as one of them; the first ones past 256 cost most
+//   of a second round (48 causal heads of 3000 rows, 288 pairs: 97 us, 24 heads 66).  At d = 64 a CU works on two at a
+//   time, so beyond that it is the CU's share that counts; at d = 128 equal workgroups go in whole rounds.
+// - split workgroups: the longest one, or a CU's share of all; causal ones run longest first, so a CU's share ends with
+//   short ones and some of the set-up hides behind other workgroups; at d = 128 equal ones go in whole rounds.
+// Constants fitted to the kernels' times inside calls of the module, 645 launches at d <= 64 and 648 above (2 to 256
+// heads, grouped and not, 300 to 4133 rows exact, 2048 to 16384 rows hashed): the chosen kernel is within 3 % of the
+// better one at all but 10 of them, within 10 % at all.  Times whole | split in us, d = 64 causal: 24 heads of 1000
+// rows 31 | 13, of 2048 45 | 27, of 4096 81 | 72; 48 of 2048 48 | 45, of 4096 129 | 139; without mask 16 of 4096 rows
+// 75 | 86; d = 128, 12 heads of 2048 rows, blocks and samples of 256: 20 | 26.
 static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   const char* env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
   if (env) return atoi(env) != 0;
+  struct Fit {
+    double step, pair, start, crowd, second, share, rest;    // 256-query kernel
+    double split_step, split_start, set_up, hidden;          // split kernel
+  };
+  const Fit f = width == 64 ? Fit{0.97, 4.4, 6.2, 0.08, 1.85, 0.94, 0.45, 0.56, 5.6, 4.3, 0.34}
+                            : Fit{1.25, 2.0, 7.0, 0.37, 1.47, 1.58, 0.29, 1.23, 1.3, 5.4, 0.22};
+  const bool paired = causal && !gather;
   const double cus = 256., vheads = (double)p.batch * p.heads * p.segs;
   const double tiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES, split_tiles = (p.n_q + 63) / 64;
-  const bool paired = causal && !gather;
   const double keys = gather ? 128. * p.block_tiles + 64. * p.sample_chunks : p.n_k;
+
   const double per_cu = vheads * (paired ? std::ceil(tiles / 2) : tiles) / cus;
-  // steps of the longest workgroup (a pair of tiles where causal) and of all of a CU's
-  const double step = width == 64 ? 0.95 : 1.4 + 0.45 * std::min(1., per_cu), tail = paired ? 5. : 0.;
-  const double longest = (paired ? 4. * (tiles + 1) : keys / 64.) * step + tail;
-  const double all = vheads / cus * tiles * (paired ? 2. * (tiles + 1) : keys / 64.) * step + per_cu * tail;
-  const double whole = (gather ? 9. : 6.) + std::max(longest, all);  // gathered: a chain of row numbers, then rows
-  const double chain = std::ceil(keys / 128.), set_up = 2.75;
-  const double all_split = vheads / cus * split_tiles * ((paired ? chain / 2 + 0.5 : chain) + set_up) + (paired ? chain / 4 : 0.);
-  const double split = 5.5 + (width == 64 ? 0.6 : 1.25) * std::max(chain + set_up, all_split);
-  return split < 0.95 * whole;
+  const double one = paired ? 4. * (tiles + 1) * f.step + f.pair : std::ceil(keys / 64.) * f.step;  // a workgroup
+  double rounds;
+  if (per_cu <= 1) rounds = 1 + f.crowd * per_cu;
+  else if (width == 64 || paired) rounds = std::max(f.second, f.share * per_cu + f.rest);
+  else rounds = f.second * std::ceil(per_cu);
+  const double whole = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
+
+  const double chain = std::ceil(keys / 128.), split_per_cu = vheads * split_tiles / cus;
+  double all;
+  if (paired) all = split_per_cu * (chain / 2 + 0.5 + f.set_up) - f.hidden * chain;
+  else all = (width == 64 ? split_per_cu : std::ceil(split_per_cu)) * (chain + f.set_up);
+  const double split = f.split_start + f.split_step * std::max(chain + f.set_up, all);
+  return split < whole;
 }
 
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,
