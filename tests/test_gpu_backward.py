@@ -265,7 +265,7 @@ def test_backward_grouped_query_heads_through_the_c_abi(ha, kind):
 @pytest.mark.parametrize("causal,n,min_seq_len,block,sample,smooth,kv_heads", [
     (False, 1024, 256, 128, 128, False, 2),
     (True, 1024, 256, 128, 128, False, 2),    # two hashed levels, on views with accumulated gradients
-    (True, 1025, 600, 128, 128, False, 2),    # odd length: the operator-by-operator recursion, padded
+    (True, 1025, 600, 128, 128, False, 2),    # odd length: a zero row appended
     (True, 2048, 512, 256, 256, True, 2),     # smoothed blocks
     (True, 1024, 600, 128, 128, False, 2),    # the off-diagonal call is exact (min_seq_len > n/2)
     (True, 2048, 256, 128, 128, False, 1),    # three levels; two query heads on one key/value head

@@ -111,6 +111,65 @@ def test_training_without_mask_takes_a_negative_min_seq_len(ha):
 
 
 # ------------------------------------------------------------------------------- layouts
+LAYOUTS = {
+    # what a layer has in memory for b batches, h query heads, hk key/value heads, and the views it calls the module with
+    "transposed": (lambda b, h, hk, n, d: [(b, n, h, d), (b, n, hk, d), (b, n, hk, d)],
+                   lambda t, h, hk: [x.transpose(1, 2) for x in t]),
+    "packed": (lambda b, h, hk, n, d: [(b, n, h + 2 * hk, d)],
+               lambda t, h, hk: [x.transpose(1, 2) for x in t[0].split((h, hk, hk), dim=2)]),
+    "rows_first": (lambda b, h, hk, n, d: [(n, b, h, d), (n, b, hk, d), (n, b, hk, d)],
+                   lambda t, h, hk: [x.permute(1, 2, 0, 3) for x in t]),
+    "expanded": (lambda b, h, hk, n, d: [(b, h, n, d), (b, 1, n, d), (b, 1, n, d)],
+                 lambda t, h, hk: [t[0]] + [x.expand(-1, h, -1, -1) for x in t[1:]]),
+}
+
+
+def _layouts(layout, b, h, hk, n, d, dtype):
+    shapes, views = LAYOUTS[layout]
+    leaves = [_randn(s, 110 + i, dtype).cuda().requires_grad_() for i, s in enumerate(shapes(b, h, hk, n, d))]
+    return leaves, views(leaves, h, hk)
+
+
+@pytest.mark.parametrize("layout", ["transposed", "packed", "rows_first", "expanded"])
+@pytest.mark.parametrize("dtype,d,causal,n", [(torch.float16, 64, True, 511), (torch.bfloat16, 128, True, 512),
+                                              (torch.float16, 64, False, 512), (torch.bfloat16, 96, True, 512),
+                                              (torch.float16, 64, True, 200)])
+@pytest.mark.parametrize("gradient", ["rows", "heads", "broadcast"])
+def test_training_on_views(ha, layout, dtype, d, causal, n, gradient):
+    """Inputs and output gradients are read where they lie; the gradients are those of the same values laid out plainly."""
+    b, h, hk = 2, 4, 2
+    m = _module(ha, d, dtype, 256)
+    leaves, call = _layouts(layout, b, h, hk, n, d, dtype)
+    out = m(*call, causal=causal)
+    do = _randn((b, h, n, d), 120, dtype).cuda()
+    if gradient == "heads":  # (batch, rows, heads, dim) in memory: what the layer's output projection hands back
+        do = do.transpose(1, 2).contiguous().transpose(1, 2)
+    elif gradient == "broadcast":
+        do = do[:, :, :1, :1].expand(b, h, n, d)
+    grads = torch.autograd.grad(out, leaves, do)
+    plain = [x.detach().contiguous().requires_grad_() for x in call]
+    out_plain = m(*plain, causal=causal)
+    assert torch.equal(out.detach(), out_plain.detach())
+    want = torch.autograd.grad(out_plain, plain, do.contiguous())
+    # back through the views alone
+    want = torch.autograd.grad(LAYOUTS[layout][1](leaves, h, hk), leaves, want)
+    for got, ref in zip(grads, want):
+        # (the sampled keys' sums are added up by atomics, in an order that can differ between runs)
+        assert ((got.double() - ref.double()).norm() / ref.double().norm()).item() < (2e-3 if dtype == torch.bfloat16 else 5e-4)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_training_on_packed_rows_against_the_oracle(ha, causal):
+    dtype, b, h, hk, n, d = torch.float16, 1, 2, 1, 512, 64
+    m = _module(ha, d, dtype, 256)
+    (leaf,), call = _layouts("packed", b, h, hk, n, d, dtype)
+    do = _randn((b, n, h, d), 121, dtype).transpose(1, 2)
+    got = torch.autograd.grad(m(*call, causal=causal), leaf, do.cuda())[0].split((h, hk, hk), dim=2)
+    ref = _reference(m, *(x.detach().cpu() for x in call), do, causal)
+    for g, r, name in zip(got, ref, ("dq", "dk", "dv")):
+        _check(g.transpose(1, 2), r, name, dtype)
+
+
 @pytest.mark.parametrize("wide", ["query", "gradient"])
 def test_training_copies_rows_that_lie_too_far_apart_to_be_addressed(ha, wide):
     """Rows 16 MiB apart, 4 GiB in all: past the kernels' limits, so the module works on a copy."""
