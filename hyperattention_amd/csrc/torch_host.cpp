@@ -360,6 +360,8 @@ std::optional<std::pair<Tensor, Tensor>> forward(const Tensor& query, const Tens
   require(value.size(2) == key.size(2) && value.size(1) == key.size(1) && value.size(0) == key.size(0) &&
               query.size(0) == key.size(0) && query.size(3) == key.size(3),
           "query, key and value do not fit together");
+  // what the attention calls of a pass with gradients are given is the quotient
+  require(key.size(1) > 0 && query.size(1) % key.size(1) == 0, "the key/value heads must divide the query heads");
   const bool grad = wants_grad(query, key, value);
   // no length is below a negative min_seq_len, so the causal recursion would not end; without mask there is nothing to
   // end, and a call with gradients hashes, as with zero

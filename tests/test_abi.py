@@ -344,3 +344,16 @@ def test_bounds_of_a_sample_list_are_not_those_of_a_dead_one():
         module.sampled_idx = torch.randint(5000, 6000, (128,))
         with pytest.raises(AssertionError, match="sampled_idx must lie in"):
             ops.check_sampled_idx(module.sampled_idx, 1024)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(3, 2), (2, 3), (2, 0)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_key_heads_that_do_not_divide_the_query_heads_are_refused(heads, kv_heads, grad):
+    """With the quotient rounded down the last query heads would read and write past the key/value heads."""
+    import torch
+    from hyperattention_amd import HyperAttention
+    q = torch.zeros((1, heads, 256, 64), dtype=torch.float16, requires_grad=grad)
+    k, v = (torch.zeros((1, kv_heads, 256, 64), dtype=torch.float16, requires_grad=grad) for _ in range(2))
+    for causal in (True, False):
+        with pytest.raises(AssertionError, match="must divide the query heads"):
+            HyperAttention(input_dim=64)(q, k, v, causal=causal)
