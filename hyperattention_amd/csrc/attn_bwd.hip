@@ -13,8 +13,9 @@
 // the sample list counts twice.  P and dS are rounded to the input type before the products, as the
 // reference does.
 //
-// One kernel body serves five passes.  A workgroup of 4 waves keeps 128 "stationary" rows (32 per
-// wave, as B operands in registers) and streams tiles of 64 rows of the other side through LDS:
+// One kernel body serves five passes.  A workgroup of 4 waves keeps 128 "stationary" rows (32 per wave, as B operands in
+// registers; 64 rows where the steps are split over waves) and streams the rows of the other side through LDS, in tiles
+// of 64 rows at d = 64 and of 32 at d = 128 (64 where the steps are split):
 //   dQ passes    stationary = queries (Q, dO), streamed = keys (K, V):      dQ^T += K^T dS^T
 //   dK/dV passes stationary = keys (K, V),     streamed = queries (Q, dO):  dK^T += Q^T dS, dV^T += dO^T P
 // Both compute S' = Y1 X1^T and dP' = Y2 X2^T (streamed rows as MFMA rows, stationary rows as MFMA
