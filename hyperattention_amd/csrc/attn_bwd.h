@@ -48,5 +48,10 @@ struct ha_attn_bwd_params {
   int smooth, idx64;
   int accumulate;  // add to dq / dk / dv instead of overwriting them
   int q_split;  // sampled-key pass: queries per workgroup
-  float scale, scale_log2;
+  int run_blocks;  // fused kernel of blocks and samples: consecutive blocks per workgroup
+  float scale, scale_log2, neg_inv_scale;  // scale * log2(e), -1 / scale
 };
+
+// dq, dk, dv of blocks and the sums of the sampled keys (dk32, dv32, cleared before) in one launch (attn_bwd_block.hip)
+bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d);
+int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream);

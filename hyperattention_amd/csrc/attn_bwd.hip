@@ -27,11 +27,13 @@
 // workgroup: stored like the exact pass's) and, if it is in the sample list, one from every query:
 // those are computed per range of queries and summed with atomics in small fp32 rows, one per slot of
 // the sample list, which a last kernel adds to the keys' rows of dK, dV.
-// Launches of the exact passes that are too small to fill the chip: split_steps.
+// Launches of the exact passes that are too small to fill the chip: split_steps.  Plain blocks of 256 at head dim 64 take
+// the one kernel of attn_bwd_block.hip in the place of the three gathered passes.
 #include "ha_common.h"
 #include "attn_tiles.h"
 #include "attn_fwd.h"
 #include "attn_bwd.h"
+#include "attn_bwd_tiles.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -41,43 +43,6 @@ namespace {
 constexpr int WG_THREADS = 256;
 constexpr int ST_ROWS = 128;       // stationary rows per workgroup
 constexpr int MAX_SMOOTH_TILES = 1024;  // query tiles that can attend one 128-key tile (smoothed blocks)
-
-// LDS layout of a streamed tile: row-major [64][D] 2-byte elements, the 16-byte pieces of a row XOR-ed
-// with a function of the row number chosen so that BOTH ways the tile is read are free of bank
-// conflicts (the LDS serves 16 lanes, 64 banks of 4 bytes, at a time):
-//   row reads (ds_read_b128): 16 lanes read the same piece of 16 consecutive rows -> the 16 rows
-//     must land in 16 different 16-byte slots of the 256-byte bank window;
-//   transposing reads (ds_read_b64_tr_b16): 16 lanes read 2 adjacent pieces of 4 consecutive rows
-//     (starting at a multiple of 4) -> the four pairs must differ in a bit above the lowest.
-// d = 64 (a row is half a bank window, so rows of equal parity compete for 8 slots): the bits 1,2,3
-// of the row number, in reversed order.  d = 128 (16 slots per row): the low four bits of the row
-// number with the two pairs of bits exchanged.
-template <int D>
-__device__ __forceinline__ int bwd_swizzle(int row) {
-  if (D == 64) return (((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1) | ((row >> 3) & 1);
-  return ((row & 3) << 2) | ((row >> 2) & 3);
-}
-template <int D>
-__device__ __forceinline__ int bwd_tile_offset(int row, int piece) {
-  return row * D * 2 + ((piece ^ bwd_swizzle<D>(row)) << 4);
-}
-
-// 8 streamed rows x 1 column, transposed by the LDS unit: rows 0..3 and 8..11 (+4 for the upper lane
-// half) relative to the row the offsets were computed for
-template <typename T>
-__device__ __forceinline__ typename ElemTraits<T>::vec8 bwd_read_tr(const unsigned char* tile, int off_lo, int off_hi) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef short s16x8 __attribute__((ext_vector_type(8)));
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off_lo));
-  const s16x4 hi8 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off_hi));
-  const s16x8 both = __builtin_shufflevector(lo, hi8, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(typename ElemTraits<T>::vec8, both);
-#else
-  return typename ElemTraits<T>::vec8{};
-#endif
-}
 
 // Scheduling groups: M times one MFMA followed by its share of V plain vector instructions and E transcendentals, and,
 // from MFMA number 1 on, PER at a time of R LDS reads.  (Reads ahead of the first MFMA would be waited for by it: the
@@ -375,6 +340,7 @@ void fill_bwd_params(const ha_attn_operands& t, const ha_attn_grads& g, const Wo
   p.q_split = (int)t.n_q;
   p.scale = t.scale;
   p.scale_log2 = t.scale * LOG2E;
+  p.neg_inv_scale = -1.f / t.scale;
 }
 
 // the sampled keys' sums onto their rows of dk, dv
@@ -408,16 +374,23 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   p.smooth = a.smooth_block != 0;
   p.idx64 = a.idx_type == HA_IDX_I64;
   const int64_t bh = t.batch * t.heads * t.segs, bhk = t.batch * (t.heads / t.kv_group) * t.segs;
-  st = launch_pass<T, D, HA_BWD_DQ_BLOCK, false>(p, bh * (t.n_q / ST_ROWS), stream, "ha_block_attn_bwd: dq");
-  if (st != HA_OK) return st;
-  st = launch_pass<T, D, HA_BWD_DKV_BLOCK, false>(p, bhk * (t.n_k / ST_ROWS), stream, "ha_block_attn_bwd: dk, dv of the blocks");
-  if (st != HA_OK) return st;
   if (a.sample_size > 0) {
     // the two arrays of sums lie one behind the other in the workspace (each a multiple of 256 bytes): one fill
     const int64_t n4 = (int64_t)(((char*)w.dv32 - (char*)w.dk32) + align256(w.acc_floats * 4)) / 16;
     hipLaunchKernelGGL(ha_bwd_zero_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, (f32x4*)w.dk32, n4);
     st = ha_launch_status("attention backward: clear");
     if (st != HA_OK) return st;
+  }
+  if (ha_block_bwd_fused_takes(p, D)) {
+    st = ha_launch_block_bwd_fused(p, std::is_same<T, f16_t>::value, stream);
+    if (st != HA_OK || a.sample_size == 0) return st;
+    return launch_add_samples<T, D>(a, g, w, stream);
+  }
+  st = launch_pass<T, D, HA_BWD_DQ_BLOCK, false>(p, bh * (t.n_q / ST_ROWS), stream, "ha_block_attn_bwd: dq");
+  if (st != HA_OK) return st;
+  st = launch_pass<T, D, HA_BWD_DKV_BLOCK, false>(p, bhk * (t.n_k / ST_ROWS), stream, "ha_block_attn_bwd: dk, dv of the blocks");
+  if (st != HA_OK) return st;
+  if (a.sample_size > 0) {
     // Every query attends every sampled key: the queries are cut into ranges, one workgroup each per tile of sampled
     // keys.  Taken is the number of ranges with the least time by the rounds of workgroups the chip needs and the
     // rows of a round; setting up a workgroup and the atomic adds it ends in cost about as much as 384 rows.

@@ -1,0 +1,607 @@
+// Backward of the sorted blocks and the sampled keys in ONE kernel: plain blocks of 256 at head dim 64, as many key/value
+// heads as query heads (the three passes of attn_bwd.hip serve everything else; see ha_block_bwd_fused_takes).
+//
+// The passes gather a level's rows three times (4.0 GB at 24 heads of 65536 rows with gradients added to; dq 447 us, dk/dv of
+// the blocks 403, of the sampled keys 229) and compute the scores twice (7 products per pair).  Here a workgroup gathers the
+// q, k, v, dO, O rows of a block of 256 queries and 256 keys once, computes every score once (5 products) and leaves dq, dk,
+// dv of the block and adds to the sampled keys' sums: 2.9 GB, 875 us in the same launch (without adding, 24 heads of 16384:
+// 285 -> 250 us).  What bounds it now: the board's power limit (1.9 to 2.1 GHz); of a block's 73k cycles 50k are the steps.
+//
+// A workgroup: 8 waves, a run of consecutive blocks of one (head, segment).  A block has a phase for its own keys and one
+// per 256 sampled keys.  In a phase a wave keeps 32 keys (k, v rows as MFMA B operands, sums of dK^T, dV^T in registers) and
+// goes through the block's queries in 8 steps of 32, their q and dO rows in LDS for the whole block (64 KB: 256 queries are
+// what fits).  dS of a step, 32 queries x 256 keys, goes through LDS once; of dq^T = sum K^T dS^T a wave sums 16 elements of
+// the head dim of 16 queries of every step over all keys.  All sums of a block are complete in registers: 64 (dk, dv) and 32
+// (dq) of them.  Of the sampled keys' sums a flush costs 64 KB of atomics per tensor, so two blocks in a row share one.
+// The next block's rows come in while this one is worked on: q and dO rows into a step's place once the step is done for the
+// last time, k rows into an LDS stage, v rows through registers, O rows (for D) four queries of a step per wave.
+#include "ha_common.h"
+#include "attn_tiles.h"
+#include "attn_bwd_tiles.h"
+#include "attn_bwd.h"
+
+#include <algorithm>
+
+namespace {
+
+constexpr int FUSED_WAVES = 8, FUSED_THREADS = 64 * FUSED_WAVES;
+constexpr int FUSED_ROWS = 256;  // queries, and keys of a phase, per workgroup
+constexpr int FD = 64;           // head dim
+constexpr int FUSED_MAX_SAMPLES = 1024;  // their row numbers are kept in LDS
+constexpr int STEPS = FUSED_ROWS / 32;
+
+template <typename T>
+struct Mfma16;
+template <>
+struct Mfma16<f16_t> {
+  static __device__ __forceinline__ f32x4 run(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Mfma16<bf16_t> {
+  static __device__ __forceinline__ f32x4 run(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+};
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// A barrier that waits for this wave's LDS operations but not for its loads and stores in memory
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// What lanes of one wave write to LDS and others read: the wave's LDS operations stay in this order
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
+// LDS, by address: q rows (4 KB) and dO rows (4 KB) of the eight steps; dS of three steps, [key][query of the step]; the k
+// rows of a phase; -L / scale and -D of a block's queries and the next one's; query and key rows of a block and the next
+// one; rows of the sampled keys.  As numbers, so that all but a few of the loop's addresses are a register and an offset
+// in the instruction.
+constexpr uint32_t TILES = 0, DS = TILES + STEPS * 8192, KEYS = DS + 3 * 16384, LSE = KEYS + 32768, DELTA = LSE + 2 * FUSED_ROWS * 4,
+                   ROWS = DELTA + 2 * FUSED_ROWS * 4, SAMPLE_ROWS = ROWS + 4 * FUSED_ROWS * 4, LDS_BYTES = SAMPLE_ROWS + FUSED_MAX_SAMPLES * 4;
+static_assert(LDS_BYTES <= 163840, "one workgroup per CU");
+
+template <typename V>
+__device__ __forceinline__ V lds_get(uint32_t address) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const __attribute__((address_space(3))) V*)address;
+#else
+  return V{};
+#endif
+}
+template <typename V>
+__device__ __forceinline__ void lds_put(uint32_t address, V value) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  *(__attribute__((address_space(3))) V*)address = value;
+#endif
+}
+// 8 rows x 1 column, transposed by the LDS unit, from two blocks of 4 rows
+template <typename T>
+__device__ __forceinline__ typename ElemTraits<T>::vec8 lds_get_tr(uint32_t lo, uint32_t hi) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)lo), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)hi);
+  return __builtin_bit_cast(typename ElemTraits<T>::vec8, (s16x8)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+#else
+  return typename ElemTraits<T>::vec8{};
+#endif
+}
+
+// 16 bytes per lane from base + offset to LDS at lds_dst + 16 * lane.  In assembly: the compiler, which does not know what
+// such a load writes, would wait for it before LDS accesses that have nothing to do with it.  It also does not count it, so
+// a wait that it puts in for one of its own loads waits for these loads too if they were issued later.
+__device__ __forceinline__ void load_to_lds(const unsigned char* base, uint32_t offset, uint32_t lds_dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" 
+               ::"s"(__builtin_amdgcn_readfirstlane(lds_dst)), "v"(offset), "s"(base) : "memory", "m0");
+#endif
+}
+
+template <typename T, bool ACC>
+__global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(const ha_attn_bwd_params p) {
+  typedef typename ElemTraits<T>::vec8 vec8;
+  typedef typename ElemTraits<T>::vec4 vec4;
+  constexpr int KSTEPS = FD / 16;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds_block[];  // LDS_BYTES, from address 0 on
+  (void)lds_block;
+  const uint32_t tid = threadIdx.x, hi = (tid >> 5) & 1, col = tid & 31;
+  uint32_t lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // ---- which run of blocks ----
+  const int n = p.n_q, blocks = (n + FUSED_ROWS - 1) / FUSED_ROWS;
+  const int runs = (blocks + p.run_blocks - 1) / p.run_blocks;
+  const int id = xcd_contiguous_id(blockIdx.x, gridDim.x);
+  const int vseq = id / runs, run = id - vseq * runs;
+  const int seg = vseq % p.segs, bh = vseq / p.segs, b = bh / p.heads, h = bh - b * p.heads;
+  const int first_block = run * p.run_blocks, end_block = min(first_block + p.run_blocks, blocks);
+  const int n_phases = 1 + p.sample_size / FUSED_ROWS;
+
+  const int64_t q_row0 = p.q_seg_off + (int64_t)seg * p.seg_stride, k_row0 = p.k_seg_off + (int64_t)seg * p.seg_stride;
+  const int64_t o_row0 = p.o_seg_off + (int64_t)seg * p.o_seg_stride;
+  const unsigned char* const qb = (const unsigned char*)((const T*)p.q + b * p.q_sb + h * p.q_sh + q_row0 * p.q_sn);
+  const unsigned char* const dob = (const unsigned char*)((const T*)p.dout + b * p.do_sb + h * p.do_sh + q_row0 * p.do_sn);
+  const unsigned char* const kb = (const unsigned char*)((const T*)p.k + b * p.k_sb + h * p.k_sh + k_row0 * p.k_sn);
+  const unsigned char* const vb = (const unsigned char*)((const T*)p.v + b * p.v_sb + h * p.v_sh + k_row0 * p.v_sn);
+  const unsigned char* const ob = (const unsigned char*)((const T*)p.out + b * p.o_sb + h * p.o_sh + o_row0 * p.o_sn);
+  const float* const lseb = p.lse + b * p.lse_sb + h * p.lse_sh + o_row0;
+  unsigned char* const dqb = (unsigned char*)((T*)p.dq + b * p.dq_sb + h * p.dq_sh + q_row0 * p.dq_sn);
+  unsigned char* const dkb = (unsigned char*)((T*)p.dk + b * p.dk_sb + h * p.dk_sh + k_row0 * p.dk_sn);
+  unsigned char* const dvb = (unsigned char*)((T*)p.dv + b * p.dv_sb + h * p.dv_sh + k_row0 * p.dv_sn);
+  const uint32_t q_rb = (uint32_t)p.q_sn * 2, k_rb = (uint32_t)p.k_sn * 2, v_rb = (uint32_t)p.v_sn * 2,
+                 do_rb = (uint32_t)p.do_sn * 2, o_rb = (uint32_t)p.o_sn * 2, dq_rb = (uint32_t)p.dq_sn * 2,
+                 dk_rb = (uint32_t)p.dk_sn * 2, dv_rb = (uint32_t)p.dv_sn * 2;
+  const int64_t sums0 = (((int64_t)b * p.heads + h) * p.segs + seg) * p.sample_size * FD;
+
+  // ---- row numbers: of a block and the next one, of the sampled keys ----
+  const int idx_shift = p.idx64 ? 3 : 2;
+  // threads 0..255 fetch query rows, 256..511 key rows
+  const unsigned char* const idx_b =
+      wave < 4 ? (const unsigned char*)p.q_idx + ((b * p.qi_sb + h * p.qi_sh + (int64_t)seg * n * p.qi_sn) << idx_shift)
+               : (const unsigned char*)p.k_idx + ((b * p.ki_sb + h * p.ki_sh + (int64_t)seg * n * p.ki_sn) << idx_shift);
+  const uint32_t idx_rb = (uint32_t)(wave < 4 ? p.qi_sn : p.ki_sn) << idx_shift;
+  auto opaque_lane = [&]() -> uint32_t {  // offsets made from it are not kept in registers across the loop
+    asm volatile("" : "+v"(lane));
+    return lane;
+  };
+  auto fetch_row = [&](int bl) -> int {
+    const int pos = min(bl * FUSED_ROWS + (int)((wave & 3) * 64 + opaque_lane()), n - 1);
+    return *reinterpret_cast<const int*>(row_address(idx_b, pos, idx_rb, 0));
+  };
+  auto rows_of = [&](int bl) -> uint32_t { return ROWS + (bl & 1) * (2 * FUSED_ROWS * 4); };  // query rows, then key rows
+  auto keep_row = [&](int bl, int row) { lds_put<int>(rows_of(bl) + (wave * 64 + opaque_lane()) * 4, row); };
+  auto query_row = [&](int bl, uint32_t r) -> uint32_t { return lds_get<int>(rows_of(bl) + r * 4); };
+  auto key_row = [&](int bl, int ph, uint32_t r) -> uint32_t {
+    return lds_get<int>((ph == 0 ? rows_of(bl) + FUSED_ROWS * 4 : SAMPLE_ROWS + (ph - 1) * (FUSED_ROWS * 4)) + r * 4);
+  };
+
+  // ---- loads ----
+  // q or dO rows of step u: waves 0..3 eight q rows each, waves 4..7 eight dO rows
+  const unsigned char* const fill_b = wave < 4 ? qb : dob;
+  const uint32_t fill_rb = wave < 4 ? q_rb : do_rb;
+  const uint32_t fill_row_at = ((wave & 3) * 8 + lane / 8) * 4, stats_row_at = (wave * 4 + lane / 16) * 4;  // in a step's rows
+  const uint32_t fill_piece = ((lane & 7) ^ bwd_swizzle<FD>((wave & 3) * 8 + lane / 8)) << 4;
+  auto fill_tile = [&](int u, uint32_t row) { load_to_lds(fill_b, __umul24(row, fill_rb) + fill_piece, TILES + u * 8192 + wave * 1024); };
+  // the wave's 32 k rows of a phase
+  auto stage_keys = [&](int bl, int ph) {
+    const uint32_t ln = opaque_lane();
+    uint32_t rows[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) rows[j] = key_row(bl, ph, wave * 32 + j * 8 + ln / 8);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j)
+      load_to_lds(kb, __umul24(rows[j], k_rb) + (((ln & 7) ^ bwd_swizzle<FD>(j * 8 + ln / 8)) << 4), KEYS + wave * 4096 + j * 1024);
+  };
+  // -L / scale and -D of a block's queries, four queries of 32 per wave: loaded, and a step later put in place.
+  // A query past the end has L = inf: its weights are zero.
+  struct Stats {
+    vec4 o, g;
+    float l;
+  };
+  auto load_stats = [&](uint32_t row) -> Stats {
+    const uint32_t piece = (opaque_lane() & 15) * 8;
+    Stats st;
+    st.o = *reinterpret_cast<const vec4*>(row_address(ob, row, o_rb, piece));
+    st.g = *reinterpret_cast<const vec4*>(row_address(dob, row, do_rb, piece));
+    st.l = lseb[row];
+    return st;
+  };
+  auto keep_stats = [&](int bl, int u, const Stats& st) {
+    const uint32_t ln = opaque_lane(), r = u * 32 + wave * 4 + ln / 16;
+    float d = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d = __builtin_fmaf((float)st.o[e], (float)st.g[e], d);
+    d += dpp<0xB1>(d);   // lane ^ 1
+    d += dpp<0x4E>(d);   // lane ^ 2
+    d += dpp<0x141>(d);  // the other four lanes of eight
+    d += dpp<0x140>(d);  // the other eight lanes of sixteen
+    if ((ln & 15) == 0) {
+      const uint32_t at = LSE + (bl & 1) * (FUSED_ROWS * 4) + r * 4;
+      lds_put<float>(at, (bl * FUSED_ROWS + (int)r < n ? st.l : __builtin_inff()) * p.neg_inv_scale);
+      lds_put<float>(at + (DELTA - LSE), -d);
+    }
+  };
+
+  // ---- LDS addresses of the operand reads: of step 0 ----
+  uint32_t row_at = TILES + bwd_tile_offset<FD>(col, hi), tr_at;
+  {  // 32x32 operands: as in attn_bwd_tile.inc
+    const uint32_t g = lane >> 4, sl = lane & 15, key = (g >> 1) * 4 + (sl >> 2), w = sl & 3;
+    tr_at = TILES + bwd_tile_offset<FD>(key, (g & 1) * 2 + (w >> 1)) + (w & 1) * 8;  // rows 8 further on: 1024 further, another swizzle
+  }
+  // dS of a step is [256 keys][32 queries]: a lane's 16 queries (8g + 4 hi + e) side by side, the 16-byte pieces of a row
+  // XOR-ed with two bits of the key number
+  uint32_t ds_write = DS + (wave * 32 + col) * 64 + (((2 * hi) ^ ((col >> 2) & 3)) << 4);
+  const uint32_t qw = wave & 1, dw = wave >> 1;  // the 16 queries of a step, the 16 elements of the head dim whose dq the wave sums
+  uint32_t ds_at;
+  {
+    const uint32_t g = lane >> 4, sl = lane & 15, key = 8 * g + (sl >> 2), w = sl & 3, piece = 2 * qw + (w >> 1);
+    ds_at = DS + key * 64 + ((piece ^ ((key >> 2) & 3)) << 4) + (w & 1) * 8;  // keys 4 further on: 256 further, another swizzle
+  }
+
+  // ---- first block ----
+  keep_row(first_block, fetch_row(first_block));
+  for (int i = tid; i < p.sample_size; i += FUSED_THREADS)
+    lds_put<int>(SAMPLE_ROWS + i * 4, p.sampled_idx ? ha_load_idx(p.sampled_idx, b * p.si_sb + h * p.si_sh + i, p.idx64) : i);
+  __syncthreads();
+  // v rows of the wave's keys: loaded whole rows at a time, then turned through 4 KB of LDS into the products' operands
+  vec8 x2f[KSTEPS];
+  auto load_v = [&](int bl, int ph) {
+    const uint32_t ln = opaque_lane();
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j)
+      x2f[j] = *reinterpret_cast<const vec8*>(row_address(vb, key_row(bl, ph, wave * 32 + j * 8 + ln / 8), v_rb, (ln & 7) * 16));
+  };
+  const uint32_t turn = DS + (wave < 4 ? 0 : 2 * 16384) + (wave & 3) * 4096;  // dq of a phase's last step is read from between
+  auto turn_v = [&]() {
+    const uint32_t ln = opaque_lane();
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) lds_put<vec8>(turn + (j * 8 + ln / 8) * 128 + (((ln & 7) ^ bwd_swizzle<FD>(j * 8 + ln / 8)) << 4), x2f[j]);
+    wave_lds_order();
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) x2f[ks] = lds_get<vec8>(turn + (row_at ^ (ks << 5)));
+    wave_lds_order();
+  };
+  stage_keys(first_block, 0);
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) fill_tile(u, lds_get<int>(rows_of(first_block) + fill_row_at + u * 128));
+  load_v(first_block, 0);
+  Stats first_stats[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) first_stats[u] = load_stats(lds_get<int>(rows_of(first_block) + stats_row_at + u * 128));
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) keep_stats(first_block, u, first_stats[u]);
+  int row_ahead = fetch_row(first_block + 1);  // of the block after the next one, from the first block on
+  turn_v();
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+
+  f32x16 acc1[2], acc2[2];  // dK^T, dV^T of the wave's keys
+  for (int bl = first_block; bl < end_block; ++bl) {
+    const int n_waves = min(n - bl * FUSED_ROWS, FUSED_ROWS) / 32;  // with rows that exist; 4 or 8: n is a multiple of 128
+    const bool more_blocks = bl + 1 < end_block;
+    keep_row(bl + 1, row_ahead);
+    row_ahead = fetch_row(bl + 2);
+    f32x4 dq[STEPS];
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u) dq[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // every other block goes through its phases backwards: two blocks in a row then share the sums of their sampled keys
+    const bool backwards = (bl - first_block) & 1;
+    for (int i_ph = 0; i_ph < n_phases; ++i_ph) {
+      const int ph = backwards ? n_phases - 1 - i_ph : i_ph;
+      const bool last_phase = i_ph + 1 == n_phases, more = !last_phase || more_blocks;
+      const int next_bl = last_phase ? bl + 1 : bl, next_ph = last_phase ? ph : backwards ? ph - 1 : ph + 1;
+      // ---- the phase's keys ----
+      lds_barrier();
+      vec8 x1f[KSTEPS], kt[STEPS];  // k rows of the wave's keys; 16 elements of every key's row, for dq
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) x1f[ks] = lds_get<vec8>(KEYS - TILES + wave * 4096 + (row_at ^ (ks << 5)));
+      {
+        const uint32_t ln = opaque_lane(), g = ln >> 4, sl = ln & 15, key = 8 * g + (sl >> 2), w = sl & 3;
+        const uint32_t lo = KEYS + bwd_tile_offset<FD>(key, 2 * dw + (w >> 1)) + (w & 1) * 8, hi4 = KEYS + bwd_tile_offset<FD>(key + 4, 2 * dw + (w >> 1)) + (w & 1) * 8;
+#pragma unroll
+        for (int ks = 0; ks < STEPS; ++ks) kt[ks] = lds_get_tr<T>(lo + ks * 4096, hi4 + ks * 4096);
+        if (ph == 0 && n_waves < FUSED_WAVES) {  // keys that do not exist take no part in dq
+#pragma unroll
+          for (int ks = STEPS / 2; ks < STEPS; ++ks) kt[ks] = vec8{};
+        }
+      }
+      if (i_ph > 0 || ph == 0 || bl == first_block) {
+#pragma unroll
+        for (int d2 = 0; d2 < 2; ++d2)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc1[d2][i] = acc2[d2][i] = 0.f;
+      }
+
+      // ---- 32 queries a step ----
+      f32x16 s, dp;
+      vec8 rq[KSTEPS], rg[KSTEPS];   // q and dO rows of a step
+      uint32_t stats_at = LSE + (bl & 1) * (FUSED_ROWS * 4) + hi * 16;
+      const uint32_t next_rows = rows_of(bl + 1);
+      auto read_statistics = [&](int u, int g) {
+        const f32x4 l = lds_get<f32x4>(stats_at + u * 128 + g * 32), nd = lds_get<f32x4>(stats_at + (DELTA - LSE) + u * 128 + g * 32);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[g * 4 + e] = l[e];
+          dp[g * 4 + e] = nd[e];
+        }
+      };
+      Stats st = {};
+      vec8 old1[4], old2[4], old3[4];  // what the call adds to: rows of dk, dv (blocks), of dq (last phase)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) old1[j] = old2[j] = old3[j] = vec8{};
+      auto load_old = [&](vec8 (&old)[4], const unsigned char* base, uint32_t rb, uint32_t list) {
+        const uint32_t ln = opaque_lane();
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+          const uint32_t row = query_row(bl, list + wave * 32 + j * 8 + ln / 8);
+          old[j] = *reinterpret_cast<const vec8*>(row_address(base, row, rb, (ln & 7) * 16));
+        }
+      };
+      vec8 pn[2], dsn[2], tq[2][2], tg[2][2];
+      // the operands' addresses: not known here, so that a step's offset stays in the instructions and what an address and
+      // an offset add up to is not kept in registers of its own
+      auto opaque_addresses = [&]() {
+        asm volatile("" : "+v"(row_at), "+v"(tr_at), "+v"(ds_write), "+v"(ds_at), "+v"(stats_at));
+      };
+      // P and dS of step u, dS into LDS; what the products of the step need is read
+      auto weights = [&](int u) {
+        opaque_addresses();
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float pv = __builtin_amdgcn_exp2f(s[kk * 8 + i] * p.scale_log2);
+            pn[kk][i] = (T)pv;
+            dsn[kk][i] = (T)(pv * dp[kk * 8 + i]);
+          }
+#pragma unroll
+          for (int d2 = 0; d2 < 2; ++d2) {
+            const uint32_t at = u * 8192 + kk * 16 * FD * 2;
+            const uint32_t lo = tr_at ^ (d2 << 6), hi8 = (tr_at ^ (d2 << 6) ^ 16) + 1024;
+            tq[kk][d2] = lds_get_tr<T>(lo + at, hi8 + at);
+            tg[kk][d2] = lds_get_tr<T>(lo + at + 4096, hi8 + at + 4096);
+          }
+          lds_put<vec8>((ds_write ^ (kk << 4)) + u % 3 * 16384, dsn[kk]);
+          asm volatile("" : "+v"(pn[kk]), "+v"(dsn[kk]));  // rounded here, not behind a branch
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      vec8 rs[STEPS];
+      auto read_ds = [&](int u, int ks) {  // of 32 keys
+        rs[ks] = lds_get_tr<T>(ds_at + u % 3 * 16384 + ks * 2048, (ds_at ^ 16) + 256 + u % 3 * 16384 + ks * 2048);
+      };
+      auto add_dq = [&](int u, int ks) { dq[u] = Mfma16<T>::run(kt[ks], rs[ks], dq[u]); };
+      auto add_dkv = [&](int kk, int which) {  // four products
+        if (which & 1) acc2[which >> 1] = Mfma<T>::run(tg[kk][which >> 1], pn[kk], acc2[which >> 1]);
+        else acc1[which >> 1] = Mfma<T>::run(tq[kk][which >> 1], dsn[kk], acc1[which >> 1]);
+      };
+      auto read_rows = [&](int u, int ks) {
+        rq[ks] = lds_get<vec8>((row_at ^ (ks << 5)) + u * 8192);
+        rg[ks] = lds_get<vec8>((row_at ^ (ks << 5)) + u * 8192 + 4096);
+      };
+      auto add_scores = [&]() {
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          s = Mfma<T>::run(rq[ks], x1f[ks], s);
+          dp = Mfma<T>::run(rg[ks], x2f[ks], dp);
+        }
+      };
+      auto in_order = [&]() { __builtin_amdgcn_sched_barrier(0); };
+      // the products: dk, dv of step u, dq of step u-1, the scores of step u+1, in the order written: behind each a few LDS
+      // reads (more at once would leave the matrix pipe idle while they are issued), of operands that are used four or more
+      // products later
+      auto products = [&](int u) {
+        __builtin_amdgcn_s_setprio(1);  // of the two waves on a SIMD the one with matrix work first
+        const bool more_steps = u + 1 < STEPS;
+        auto read = [&](int ds_ks, int stat_g, int rows_ks) {
+          if (ds_ks >= 0 && u > 0) read_ds(u - 1, ds_ks);
+          if (more_steps && stat_g >= 0) read_statistics(u + 1, stat_g);
+          if (more_steps && rows_ks >= 0) read_rows(u + 1, rows_ks);
+          in_order();
+        };
+        auto dq_of = [&](int ks) {
+          if (u > 0) add_dq(u - 1, ks);
+        };
+        in_order();
+        add_dkv(0, 0);
+        read(0, -1, -1);
+        read(1, -1, -1);
+        add_dkv(0, 1);
+        read(2, -1, -1);
+        add_dkv(0, 2);
+        read(3, -1, -1);
+        add_dkv(0, 3);
+        read(-1, 0, -1);
+        add_dkv(1, 0);
+        read(4, 1, -1);
+        add_dkv(1, 1);
+        read(5, 2, -1);
+        dq_of(0);
+        dq_of(1);
+        read(-1, 3, -1);
+        dq_of(2);
+        dq_of(3);
+        read(-1, -1, 0);
+        add_dkv(1, 2);
+        read(6, -1, -1);
+        read(7, -1, -1);
+        dq_of(4);
+        read(-1, -1, 1);
+        dq_of(5);
+        add_dkv(1, 3);
+        read(-1, -1, 2);
+        if (u + 1 == STEPS) {
+          // the scores are done: their registers take the v rows of the next phase and what this one adds to
+          load_v(more ? next_bl : bl, next_ph);
+          if (ACC && ph == 0) load_old(old1, dkb, dk_rb, FUSED_ROWS);
+          in_order();
+        }
+        dq_of(6);
+        dq_of(7);
+        read(-1, -1, 3);
+        uint32_t frow = 0, srow;  // rows of the next block
+        if (u > 0) frow = lds_get<int>(next_rows + fill_row_at + (u - 1) * 128);
+        srow = lds_get<int>(next_rows + stats_row_at + u * 128);
+        in_order();
+        if (more_steps) add_scores();
+        __builtin_amdgcn_s_setprio(0);
+        in_order();
+        if (__builtin_expect(i_ph == 0, true)) {  // the next block's statistics
+          if (u > 0) keep_stats(bl + 1, u - 1, st);
+          // the last tiles of this block, loaded since the end of the one before, have landed as well
+          if (u == 1) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+          st = load_stats(srow);
+        }
+        if (u == 1 && more) stage_keys(next_bl, next_ph);  // every wave is done with the keys of this phase
+        if (u > 0 && __builtin_expect(last_phase && more_blocks, true)) fill_tile(u - 1, frow);  // every wave is done with step u-1
+        in_order();
+        if (u + 1 == STEPS) {
+          if (ACC && ph == 0) load_old(old2, dvb, dv_rb, FUSED_ROWS);
+          in_order();
+        }
+      };
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        read_rows(0, i);
+        read_statistics(0, i);
+      }
+      add_scores();
+      // One barrier a step; of the two waves on a SIMD one has it behind the weights and one behind the products, so that
+      // the one's vector work meets the other's matrix work.
+      weights(0);
+#pragma unroll
+      for (int u = 0; u < STEPS; ++u) {
+        products(u);
+        if (wave >= 4 || u + 1 == STEPS) lds_barrier();
+        if (u + 1 < STEPS) {
+          weights(u + 1);
+          if (wave < 4) lds_barrier();
+        }
+      }
+      const uint32_t frow = lds_get<int>(next_rows + fill_row_at + (STEPS - 1) * 128);
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ++ks) read_ds(STEPS - 1, ks);
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ++ks) add_dq(STEPS - 1, ks);
+      if (i_ph == 0) keep_stats(bl + 1, STEPS - 1, st);
+      if (ACC && last_phase) load_old(old3, dqb, dq_rb, 0);
+      // the next phase's v rows have landed, and with them all loads into LDS; not to be waited for behind the stores
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(x2f[ks]));
+      asm volatile("" : "+v"(row_ahead));
+      if (ACC && ph == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(old1[j]), "+v"(old2[j]));
+      }
+      if (last_phase && more_blocks) fill_tile(STEPS - 1, frow);
+      turn_v();
+      // ---- the keys' gradients: turned around in the wave's 4 KB of the dS tiles ----
+      const uint32_t ln = opaque_lane();
+      if (ph == 0) {
+        uint32_t rows[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) rows[j] = key_row(bl, 0, wave * 32 + j * 8 + ln / 8);
+        if (wave < (uint32_t)n_waves) {
+          auto store = [&](const f32x16 (&acc)[2], float factor, unsigned char* base, uint32_t rb, const vec8 (&old)[4]) {
+#pragma unroll
+            for (int d2 = 0; d2 < 2; ++d2)
+#pragma unroll
+              for (int g = 0; g < 4; ++g) {
+                vec4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = (T)(acc[d2][g * 4 + e] * factor);
+                lds_put<vec4>(turn + (ln & 31) * 128 + (((4 * d2 + g) ^ (ln & 7)) << 4) + (ln >> 5) * 8, o);
+              }
+            wave_lds_order();
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+              const uint32_t r = j * 8 + ln / 8;
+              vec8 o = lds_get<vec8>(turn + r * 128 + (((ln & 7) ^ (r & 7)) << 4));
+              if constexpr (ACC) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = (T)((float)o[e] + (float)old[j][e]);
+              }
+              *reinterpret_cast<vec8*>(base + (uint32_t)(__umul24(rows[j], rb) + (ln & 7) * 16)) = o;
+            }
+          };
+          store(acc1, p.scale, dkb, dk_rb, old1);
+          wave_lds_order();
+          store(acc2, 1.f, dvb, dv_rb, old2);
+        }
+      } else if (!last_phase || !more_blocks) {  // else the next block goes on with the same sampled keys
+        const int64_t slot0 = sums0 + (int64_t)((ph - 1) * FUSED_ROWS + wave * 32) * FD;
+#pragma unroll
+        for (int which = 0; which < 2; ++which) {
+          float* const dst = (which == 0 ? p.dk32 : p.dv32) + slot0;
+          const float factor = which == 0 ? p.scale : 1.f;
+#pragma unroll
+          for (uint32_t part = 0; part < 2; ++part) {  // 16 keys at a time
+            if ((ln & 31) >> 4 == part) {
+#pragma unroll
+              for (int d2 = 0; d2 < 2; ++d2)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                  const f32x16& a = which == 0 ? acc1[d2] : acc2[d2];
+                  const uint32_t piece = (8 * d2 + 2 * g + (ln >> 5)) ^ (ln & 15);
+                  lds_put<f32x4>(turn + (ln & 15) * (FD * 4) + piece * 16,
+                                 f32x4{a[g * 4] * factor, a[g * 4 + 1] * factor, a[g * 4 + 2] * factor, a[g * 4 + 3] * factor});
+                }
+            }
+            wave_lds_order();
+#pragma unroll
+            for (uint32_t r = 0; r < 16; ++r)
+              unsafeAtomicAdd(dst + (part * 16 + r) * FD + ln, lds_get<float>(turn + r * (FD * 4) + (((ln >> 2) ^ r) << 4) + (ln & 3) * 4));
+            wave_lds_order();
+          }
+        }
+      }
+      // ---- dq ----
+      if (last_phase) {
+        lds_barrier();  // every wave is done with its part of the dS tiles
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u) {
+          vec4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (T)(dq[u][e] * p.scale);
+          const uint32_t q = (u & 3) * 32 + 8 * ((ln & 15) >> 2) + 4 * qw + (ln & 3);
+          lds_put<vec4>(DS + (u < 4 ? 0 : 2 * 16384) + q * 128 + (((2 * dw + (ln >> 5)) ^ (q & 7)) << 4) + ((ln >> 4) & 1) * 8, o);
+        }
+        uint32_t rows[4];  // behind the barrier other waves may put the next rows in their place
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) rows[j] = query_row(bl, wave * 32 + j * 8 + ln / 8);
+        lds_barrier();
+        if (wave < (uint32_t)n_waves) {
+#pragma unroll
+          for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t r = (wave & 3) * 32 + j * 8 + ln / 8;
+            vec8 o = lds_get<vec8>(DS + (wave < 4 ? 0 : 2 * 16384) + r * 128 + (((ln & 7) ^ (r & 7)) << 4));
+            if constexpr (ACC) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) o[e] = (T)((float)o[e] + (float)old3[j][e]);
+            }
+            *reinterpret_cast<vec8*>(dqb + (uint32_t)(__umul24(rows[j], dq_rb) + (ln & 7) * 16)) = o;
+          }
+        }
+      }
+    }
+  }
+}
+
+}  // namespace
+
+// What the registers and LDS are laid out for: 256 keys and queries per block; with grouped queries a block's dk, dv would
+// have to be kept over the query heads beside the sampled keys' sums.  At every size measured (1 to 32 heads of 2048 to 65536
+// rows) the one kernel is the faster one or equal, but for three workgroups' worth of blocks per CU (24 x 8192: 178 against 168
+// us): 1 x 4096 37 against 45 us, 12 x 4096 64 against 74, 24 x 4096 85 against 106, 32 x 32768 578 against 775.
+bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d) {
+  return d == FD && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
+         p.sample_size <= FUSED_MAX_SAMPLES;
+}
+
+int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream) {
+  const int64_t vseqs = (int64_t)p.batch * p.heads * p.segs, blocks = (p.n_q + FUSED_ROWS - 1) / FUSED_ROWS;
+  // Blocks per workgroup, one workgroup per CU: the run with the least time by the rounds of workgroups; starting and ending
+  // one takes as long as two fifths of a block (41 us each in a full launch)
+  int64_t best = INT64_MAX;
+  p.run_blocks = 1;
+  for (int64_t r = 1; r <= std::min<int64_t>(blocks, 32); ++r) {
+    const int64_t cost = (vseqs * ((blocks + r - 1) / r) + 255) / 256 * (5 * r + 2);
+    if (cost < best) {
+      best = cost;
+      p.run_blocks = (int)r;
+    }
+  }
+  const int64_t grid = vseqs * ((blocks + p.run_blocks - 1) / p.run_blocks);
+  if (grid >= (1ll << 31)) return ha_fail(HA_ERR_SHAPE, "ha_block_attn_bwd: grid of %lld workgroups", (long long)grid);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FUSED_THREADS), LDS_BYTES, stream, p); };
+  if (is_f16) p.accumulate ? launch(ha_block_bwd_fused_kernel<f16_t, true>) : launch(ha_block_bwd_fused_kernel<f16_t, false>);
+  else p.accumulate ? launch(ha_block_bwd_fused_kernel<bf16_t, true>) : launch(ha_block_bwd_fused_kernel<bf16_t, false>);
+  return ha_launch_status("ha_block_attn_bwd: blocks and sampled keys");
+}

@@ -1,0 +1,61 @@
+"""The one-kernel backward of plain blocks of 256 at head dim 64 (csrc/attn_bwd_block.hip) at the edges of what it takes:
+one block and many, a last block of half the rows, runs of blocks that do not divide a sequence, phases of sampled keys,
+index types and layouts, results added to what is there."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import hyper_oracle as O
+from test_gpu_backward import _check, _gpu_grads, _oracle_grads, _perms, ha  # noqa: F401 (fixture)
+from _util import _gen, _randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,h,n,sample,idx", [
+    (torch.float16, 1, 128, 0, torch.int64),       # half a block, nothing else
+    (torch.bfloat16, 2, 256, 256, torch.int32),    # one block
+    (torch.float16, 1, 384, 256, torch.int32),     # the last block is half
+    (torch.bfloat16, 3, 1152, 512, torch.int64),   # two phases of sampled keys
+    (torch.float16, 1, 1024, 1024, torch.int32),   # the most sampled keys
+    (torch.float16, 5, 16512, 256, torch.int32),   # 65 blocks in runs of two: the last run has one, of half the rows
+])
+def test_blocks_and_samples(ha, dtype, h, n, sample, idx):  # noqa: F811
+    q, k, v, do = (_randn((1, h, n, 64), s, dtype) for s in (31, 32, 33, 34))
+    qi, ki = _perms(1, h, n, 35), _perms(1, h, n, 36)
+    ref = _oracle_grads(lambda a, b, c: O.block_sampled_attention(a, b, c, qi, ki, 256, sample, None, False), q, k, v, do)
+    qi_g, ki_g = (x.cuda().to(idx).transpose(1, 2) for x in (qi, ki))
+    _, _, *got = _gpu_grads(lambda a, b, c: ha.hyper_attn_func(a, b, c, qi_g, ki_g, 256, sample, None, False), q, k, v, do)
+    for g, want, name in zip(got, ref, ("dq", "dk", "dv")):
+        _check(g, want, f"{name}, {h} x {n}, {sample} samples", dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_adds_to_gradients_in_transposed_layout_and_keeps_an_explicit_list(ha, dtype):  # noqa: F811
+    """Gradients added to (bnhd layout, repeated rows in an int64 sample list), a short last block: the result is
+    what was there and the plain gradient, up to the rounding of the sum."""
+    from hyperattention_amd import _lib, ops
+    b, h, n, sample, scale = 2, 2, 896, 256, 0.11
+    q, k, v, do = (_randn((b, n, h, 64), s, dtype).cuda() for s in (41, 42, 43, 44))
+    qi, ki = (_perms(b, h, n, s).cuda().int().transpose(1, 2) for s in (45, 46))
+    sl = torch.randint(0, n, (sample,), generator=_gen(47)).cuda()
+    sl[1] = sl[0]
+    o, lse = ops.hyper_attn_func(q, k, v, qi, ki, 256, sample, scale, False, sampled_idx=sl)
+    ref = _oracle_grads(lambda x, y, z: O.block_sampled_attention(x, y, z, qi.transpose(1, 2).cpu().long(), ki.transpose(1, 2).cpu().long(),
+                                                                  256, sample, scale, False, sampled_idx=sl.cpu()),
+                        *(x.transpose(1, 2).cpu() for x in (q, k, v, do)))
+    there = [_randn((b, n, h, 64), s, dtype).cuda() for s in (48, 49, 50)]
+    grads = [x.clone() for x in there]
+    a, _keep = ops._block_attn_args(q, k, v, o, lse, qi, ki, 256, sample, scale, False, sl)
+    g, ws = ops._attn_grads(a.t, do, *grads, sample_size=sample)
+    g.accumulate = 1
+    _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), ops._stream(q)))
+    torch.cuda.synchronize()
+    # the sum is rounded to the type once more: half a unit of its last place, of values of N(0, 1) plus the gradient
+    unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    for got, was, want, name in zip(grads, there, ref, ("dq", "dk", "dv")):
+        total = was.double().cpu().transpose(1, 2) + want
+        err = (got.double().cpu().transpose(1, 2) - total).norm() / total.norm()
+        assert err <= unit + (3e-3 if dtype == torch.float16 else 8e-3), f"{name}: {err:.2e}"
+        assert torch.isfinite(got).all()
