@@ -28,3 +28,17 @@ def test_windows(ha, monkeypatch, dtype, d, n, block, sample, smooth):  # noqa: 
     ro, rl = O.block_sampled_attention(q, k, v, qi, ki, block, sample, None, smooth)
     assert_close(o, ro, "out", dtype)
     assert_close(lse, rl, "lse")
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 40), (torch.bfloat16, 96), (torch.float16, 120)])
+def test_plain_blocks_of_narrow_heads_resumed(ha, monkeypatch, dtype, d):  # noqa: F811
+    monkeypatch.setenv("HA_SPLIT", "0")
+    q, k, v, qi, ki = _sorted_inputs(1, 2, 768, d, dtype, 70)
+    o0, l0 = O.exact_attention(q, v, v, None, False)
+    o0, l0 = o0.to(dtype), l0.float()
+    c = lambda t: t.cuda().transpose(1, 2)
+    o, lse = ha.hyper_attn_func(c(q), c(k), c(v), c(qi), c(ki), 256, 128, None, False, resume=(c(o0).contiguous(), l0.cuda()))
+    ro, rl = O.block_sampled_attention(q, k, v, qi, ki, 256, 128, None, False)
+    mo, ml = O.add_self_attentions(o0.double(), l0.double().unsqueeze(-1), ro, rl.unsqueeze(-1))
+    assert_close(o.transpose(1, 2), mo, "merged out", dtype)
+    assert_close(lse, ml.squeeze(-1), "merged lse")
