@@ -55,3 +55,7 @@ struct ha_attn_bwd_params {
 // dq, dk, dv of blocks and the sums of the sampled keys (dk32, dv32, cleared before) in one launch (attn_bwd_block.hip)
 bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d);
 int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream);
+
+// dk, dv of exact attention or of plain blocks (multiples of 256 keys) at head dim 128, 256 keys per workgroup
+// (attn_bwd_wide.hip); grid: workgroups
+int ha_launch_bwd_wide(const ha_attn_bwd_params& p, int pass, bool causal, int is_f16, int64_t grid, hipStream_t stream, const char* what);

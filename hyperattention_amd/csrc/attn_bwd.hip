@@ -27,7 +27,7 @@
 // workgroup: stored like the exact pass's) and, if it is in the sample list, one from every query:
 // those are computed per range of queries and summed with atomics in small fp32 rows, one per slot of
 // the sample list, which a last kernel adds to the keys' rows of dK, dV.
-// Launches of the exact passes that are too small to fill the chip: split_steps.  Plain blocks of 256 at head dim 64 take
+// The forms of the exact passes: exact_form.  Plain blocks of 256 at head dim 64 take
 // the one kernel of attn_bwd_block.hip in the place of the three gathered passes.
 #include "ha_common.h"
 #include "attn_tiles.h"
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   constexpr int RPL = 64 / PR;    // rows per tile load (one load = 64 lanes x 16 bytes)
   // Streamed rows per LDS tile and tiles in the ring: a step of 32 rows reads its own tile and the next step's, and
   // the tile after that is in flight; two steps per tile at d = 64, one at d = 128 (the same bytes).
-  // HALVES == 2 (split_steps): 64 stationary rows per workgroup; of the two steps of a tile waves 0, 1 take the first
+  // HALVES == 2 (SPLIT): 64 stationary rows per workgroup; of the two steps of a tile waves 0, 1 take the first
   // and waves 2, 3 the second, and the two sums of a row meet in LDS at the end.
   constexpr int YC = D <= 64 || HALVES == 2 ? 64 : 32;
   constexpr int STEPS = YC / 32 / HALVES;  // steps that a wave takes from a tile
@@ -388,7 +388,16 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   }
   st = launch_pass<T, D, HA_BWD_DQ_BLOCK, false>(p, bh * (t.n_q / ST_ROWS), stream, "ha_block_attn_bwd: dq");
   if (st != HA_OK) return st;
-  st = launch_pass<T, D, HA_BWD_DKV_BLOCK, false>(p, bhk * (t.n_k / ST_ROWS), stream, "ha_block_attn_bwd: dk, dv of the blocks");
+  // 256 keys per workgroup where their tiles are all of one block, smooth windows apart, and more than half the chip
+  // has work.  dk, dv of the blocks in us, d 128, 128 -> 256 keys, workgroups of 256 in brackets: 8 heads of 4096 rows
+  // in blocks of 256 (128) 20.7 -> 24.8, 9 heads (144) 35.9 -> 25.5, 17 (272) 56.7 -> 49.3, 32 query heads on 8 of 4096
+  // (128) 53 -> 61, of 4224 (136) 76 -> 61, of 16384 (512) 225 -> 159; blocks of 512, 32 on 8 of 8320 (264) 221 -> 162.
+  const int64_t wide_wgs = bhk * ((t.n_k + 255) / 256);
+  if (D == 128 && !p.smooth && p.block_tiles % 2 == 0 && wide_wgs > 128)
+    st = ha_launch_bwd_wide(p, HA_BWD_DKV_BLOCK, false, std::is_same<T, f16_t>::value, wide_wgs, stream,
+                            "ha_block_attn_bwd: dk, dv of the blocks");
+  else
+    st = launch_pass<T, D, HA_BWD_DKV_BLOCK, false>(p, bhk * (t.n_k / ST_ROWS), stream, "ha_block_attn_bwd: dk, dv of the blocks");
   if (st != HA_OK) return st;
   if (a.sample_size > 0) {
     // Every query attends every sampled key: the queries are cut into ranges, one workgroup each per tile of sampled
@@ -405,7 +414,7 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
         splits = (t.n_q + rows - 1) / rows;
       }
     }
-    st = launch_pass<T, D, HA_BWD_DKV_SAMPLED, false>(p, bh * (a.sample_size / ST_ROWS) * splits, stream,
+    st = launch_pass<T, D, HA_BWD_DKV_SAMPLED, false>(p, tiles * splits, stream,
                                                       "ha_block_attn_bwd: dk, dv of the sampled keys");
     if (st != HA_OK) return st;
     return launch_add_samples<T, D>(a, g, w, stream);
@@ -413,18 +422,26 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   return HA_OK;
 }
 
-// Whether a pass of exact attention is better off with the steps of its streamed tiles split over waves (HALVES = 2: 64
-// stationary rows per workgroup, half as many steps per wave).  What bounds a launch of few workgroups is the longest
-// chain of steps of one of them with CUs idle: a wave alone on its SIMD issues steps as fast as two together, so
-// smaller workgroups fill the idle CUs; on a full chip they do the same work slower (twice the set-up and tile loads
-// per row; dq at d = 128 also one workgroup per CU instead of two).  Estimated in steps of 32 streamed rows: rounds of
-// workgroups over the CUs times their chain, or, for causal tiles one by one (longest first), the longest chain or a CU's
-// share of all.  The weights are fitted to the times of both forms of both passes at 57 shapes per head dim (4 to 128
-// heads, grouped and not, 512 to 4096 rows): where the rule splits, it was never slower by more than they scatter.
+// The form of a pass of exact attention with the least estimated time.
+//   WHOLE: 128 stationary rows per workgroup, causal tiles in pairs.
+//   SPLIT: 64, the steps of the streamed tiles split over waves (HALVES = 2), half as many steps per wave.
+//   WIDE: 256 (attn_bwd_wide.hip; dk, dv at d = 128).
+// What bounds a launch of few workgroups is the longest chain of steps of one of them with CUs idle: a wave alone on its
+// SIMD issues steps as fast as two together, so smaller workgroups fill the idle CUs; on a full chip they do the same
+// work slower (twice the set-up and tile loads per row; dq at d = 128 also one workgroup per CU instead of two).
+// Estimated in steps of 32 streamed rows: rounds of workgroups over the CUs times their chain, or, for causal tiles one
+// by one (longest first), the longest chain or a CU's share of all.  The weights are fitted to the times of WHOLE and
+// SPLIT of both passes at 57 shapes per head dim (4 to 128 heads, grouped and not, 512 to 4096 rows): where the rule
+// splits, it was never slower by more than they scatter.
 // Times in us, whole -> split, dq | dk, dv, bf16 causal: d 64, 24 heads of 2048 rows 40 -> 32 | 50 -> 39, 4 heads of 1000
 // 24 -> 13 | 29 -> 16, 8 query heads on 2 of 4096 61 -> 42 | 291 -> 189; d 128, 12 heads of 2048 75 -> 41 | 93 -> 49, 32
 // on 8 of 2048 78 (split 98: stays) | 320 -> 161.  Full: d 64, 48 heads of 4096 rows without mask 295 (split 335) | 387 (451).
-bool split_steps(int d, bool dkv, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal) {
+// A wide step is 1.05 whole steps long on an idle chip and 1.3 on a full one, for twice the pairs.  The better of the other
+// two -> wide, dk, dv in us at 35 shapes, among them (causal) 24 heads of 4096 rows 307 -> 223, 32 387 -> 271, of 8192 1347
+// -> 972, 256 of 256 41 -> 32; (not causal) 24 of 2048 147 -> 108, 32 of 4096 684 -> 477; 32 on 8, 300 on 8192 rows 124 ->
+// 84.  Where the chip is not full the others stay: causal 32 on 8 heads of 4096 413 (wide 696), 12 of 2048 56 (103).
+enum ExactForm { WHOLE, SPLIT, WIDE };
+ExactForm exact_form(int d, bool dkv, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal) {
   const double cus = 256., set_up = 2., margin = 0.97;
   // time of a step where a CU has several workgroups to take, against one alone
   const double full_whole = d == 64 || dkv ? 0.95 : 0.8, full_split = d == 64 ? 1.25 : dkv ? 1. : 1.4;
@@ -440,14 +457,24 @@ bool split_steps(int d, bool dkv, int64_t seqs, int64_t rows, int64_t streamed_r
     whole = (rounds > 1 ? full_whole : 1.) * rounds * 4 * streamed * group + set_up * rounds;
     split = (split_rounds > 1 ? full_split : 1.) * split_rounds * 2 * streamed * group + set_up * split_rounds;
   }
-  return split < margin * whole;
+  const ExactForm narrow = split < margin * whole ? SPLIT : WHOLE;
+  if (d != 128 || !dkv) return narrow;
+  const double wide_tiles = (double)((rows + 255) / 256), wide_wgs = seqs * wide_tiles, chain = (double)((streamed_rows + 31) / 32) * group;
+  const double step = 1.05 + 0.25 * std::min(1., wide_wgs / cus), wide_rounds = std::ceil(wide_wgs / cus), wide_set_up = 3.;
+  const double wide = causal ? std::max(1.05 * chain + wide_set_up, 1.3 * wide_wgs / cus * std::max(chain / 2, chain - 4 * (wide_tiles - 1) * group) +
+                                                                        wide_set_up * std::max(1., wide_wgs / cus))
+                             : wide_rounds * (step * chain + wide_set_up);
+  return wide < margin * std::min(whole, split) ? WIDE : narrow;
 }
 
 // one pass of exact attention over `seqs` sequences with `rows` stationary rows each
 template <typename T, int D, int PASS>
 int launch_exact(const ha_attn_bwd_params& p, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal,
                  hipStream_t stream, const char* what) {
-  if (split_steps(D, PASS == HA_BWD_DKV_EXACT, seqs, rows, streamed_rows, group, causal)) {
+  const ExactForm form = exact_form(D, PASS == HA_BWD_DKV_EXACT, seqs, rows, streamed_rows, group, causal);
+  if (form == WIDE)
+    return ha_launch_bwd_wide(p, PASS, causal, std::is_same<T, f16_t>::value, seqs * ((rows + 255) / 256), stream, what);
+  if (form == SPLIT) {
     const int64_t grid = seqs * ((rows + 63) / 64);
     return causal ? launch_pass<T, D, PASS, true, 2>(p, grid, stream, what) : launch_pass<T, D, PASS, false, 2>(p, grid, stream, what);
   }

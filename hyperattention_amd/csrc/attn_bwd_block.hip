@@ -46,12 +46,6 @@ __device__ __forceinline__ float dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// A barrier that waits for this wave's LDS operations but not for its loads and stores in memory
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// What lanes of one wave write to LDS and others read: the wave's LDS operations stay in this order
-__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
-
 // LDS, by address: q rows (4 KB) and dO rows (4 KB) of the eight steps; dS of three steps, [key][query of the step]; the k
 // rows of a phase; -L / scale and -D of a block's queries and the next one's; query and key rows of a block and the next
 // one; rows of the sampled keys.  As numbers, so that all but a few of the loop's addresses are a register and an offset
@@ -59,44 +53,6 @@ __device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory")
 constexpr uint32_t TILES = 0, DS = TILES + STEPS * 8192, KEYS = DS + 3 * 16384, LSE = KEYS + 32768, DELTA = LSE + 2 * FUSED_ROWS * 4,
                    ROWS = DELTA + 2 * FUSED_ROWS * 4, SAMPLE_ROWS = ROWS + 4 * FUSED_ROWS * 4, LDS_BYTES = SAMPLE_ROWS + FUSED_MAX_SAMPLES * 4;
 static_assert(LDS_BYTES <= 163840, "one workgroup per CU");
-
-template <typename V>
-__device__ __forceinline__ V lds_get(uint32_t address) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return *(const __attribute__((address_space(3))) V*)address;
-#else
-  return V{};
-#endif
-}
-template <typename V>
-__device__ __forceinline__ void lds_put(uint32_t address, V value) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  *(__attribute__((address_space(3))) V*)address = value;
-#endif
-}
-// 8 rows x 1 column, transposed by the LDS unit, from two blocks of 4 rows
-template <typename T>
-__device__ __forceinline__ typename ElemTraits<T>::vec8 lds_get_tr(uint32_t lo, uint32_t hi) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef short s16x8 __attribute__((ext_vector_type(8)));
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)lo), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)hi);
-  return __builtin_bit_cast(typename ElemTraits<T>::vec8, (s16x8)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
-#else
-  return typename ElemTraits<T>::vec8{};
-#endif
-}
-
-// 16 bytes per lane from base + offset to LDS at lds_dst + 16 * lane.  In assembly: the compiler, which does not know what
-// such a load writes, would wait for it before LDS accesses that have nothing to do with it.  It also does not count it, so
-// a wait that it puts in for one of its own loads waits for these loads too if they were issued later.
-__device__ __forceinline__ void load_to_lds(const unsigned char* base, uint32_t offset, uint32_t lds_dst) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" 
-               ::"s"(__builtin_amdgcn_readfirstlane(lds_dst)), "v"(offset), "s"(base) : "memory", "m0");
-#endif
-}
 
 template <typename T, bool ACC>
 __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(const ha_attn_bwd_params p) {

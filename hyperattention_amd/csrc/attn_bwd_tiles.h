@@ -42,4 +42,57 @@ __device__ __forceinline__ typename ElemTraits<T>::vec8 bwd_read_tr(const unsign
 #endif
 }
 
+// ---- LDS by address: kernels whose whole LDS is one dynamic block from address 0 on ----
+// A barrier that waits for this wave's LDS operations but not for its loads and stores in memory
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// What lanes of one wave write to LDS and others read: the wave's LDS operations stay in this order
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
+template <typename V>
+__device__ __forceinline__ V lds_get(uint32_t address) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const __attribute__((address_space(3))) V*)address;
+#else
+  return V{};
+#endif
+}
+template <typename V>
+__device__ __forceinline__ void lds_put(uint32_t address, V value) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  *(__attribute__((address_space(3))) V*)address = value;
+#endif
+}
+// 8 rows x 1 column, transposed by the LDS unit, from two blocks of 4 rows
+template <typename T>
+__device__ __forceinline__ typename ElemTraits<T>::vec8 lds_get_tr(uint32_t lo, uint32_t hi) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)lo), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)hi);
+  return __builtin_bit_cast(typename ElemTraits<T>::vec8, (s16x8)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+#else
+  return typename ElemTraits<T>::vec8{};
+#endif
+}
+
+// 16 bytes per lane from base + offset to LDS at lds_dst + 16 * lane.  In assembly: the compiler, which does not know what
+// such a load writes, would wait for it before LDS accesses that have nothing to do with it.  It also does not count it, so
+// a wait that it puts in for one of its own loads waits for these loads too if they were issued later.
+__device__ __forceinline__ void load_to_lds(const unsigned char* base, uint32_t offset, uint32_t lds_dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" 
+               ::"s"(__builtin_amdgcn_readfirstlane(lds_dst)), "v"(offset), "s"(base) : "memory", "m0");
+#endif
+}
+
+// As load_to_lds, 4 bytes per lane to lds_dst + 4 * lane
+__device__ __forceinline__ void load_to_lds_4(const unsigned char* base, uint32_t offset, uint32_t lds_dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               ::"s"(__builtin_amdgcn_readfirstlane(lds_dst)), "v"(offset), "s"(base) : "memory", "m0");
+#endif
+}
+
 }  // namespace

@@ -1,0 +1,100 @@
+"""dk, dv with 256 keys per workgroup at head dim 128 (csrc/attn_bwd_wide.hip): launches that fill the chip with few rows
+per head, at the edges of its tiles of 256 keys and 32 queries.  The shapes are ones that its dispatch rules take."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import hyper_oracle as O
+from test_gpu_backward import _check, _gpu_grads, _oracle_grads, ha  # noqa: F401 (fixture)
+from _util import _gen, _randn
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def _orders(h, n, seed):
+    return torch.rand((1, h, n), generator=_gen(seed)).argsort(-1)
+
+
+def _grouped(fn, group):
+    """An oracle with `group` query heads on each key head."""
+    return lambda q, k, v: fn(q, k.repeat_interleave(group, 1), v.repeat_interleave(group, 1))
+
+
+@pytest.mark.parametrize("dtype,h,hk,nq,nk,causal", [
+    (torch.float16, 300, 300, 128, 128, True),     # half the waves have no keys
+    (torch.bfloat16, 300, 300, 192, 192, False),
+    (torch.float16, 300, 300, 77, 500, False),     # ragged on both sides
+    (torch.bfloat16, 200, 200, 1001, 250, False),
+    (torch.float16, 400, 200, 300, 300, True),     # two query heads, a last tile with 44 keys
+    (torch.bfloat16, 300, 300, 300, 500, True),    # keys that nothing attends
+    (torch.float16, 300, 300, 300, 256, True),     # queries after the last key
+    (torch.bfloat16, 600, 200, 20, 260, False),    # one step per query head
+])
+def test_exact(ha, dtype, h, hk, nq, nk, causal):  # noqa: F811
+    q, do = (_randn((1, h, nq, D), s, dtype) for s in (51, 52))
+    k, v = (_randn((1, hk, nk, D), s, dtype) for s in (53, 54))
+    ref = _oracle_grads(_grouped(lambda a, b, c: O.exact_attention(a, b, c, None, causal), h // hk), q, k, v, do)
+    _, _, *got = _gpu_grads(lambda a, b, c: ha.flash_attn_func(a, b, c, None, causal), q, k, v, do)
+    for g, want, name in zip(got, ref, ("dq", "dk", "dv")):
+        _check(g, want, name, dtype)
+
+
+@pytest.mark.parametrize("dtype,h,hk,n,block,sample,idx", [
+    (torch.float16, 130, 130, 128, 256, 0, torch.int64),     # half a block
+    (torch.bfloat16, 65, 65, 384, 256, 128, torch.int32),    # the last block is half
+    (torch.float16, 44, 44, 640, 512, 256, torch.int32),     # two tiles of a block, a short block
+    (torch.bfloat16, 132, 44, 640, 256, 0, torch.int64),     # three query heads on each key head
+    (torch.float16, 44, 22, 1280, 1024, 0, torch.int32),     # four tiles of a block, two of a short one
+])
+def test_blocks(ha, dtype, h, hk, n, block, sample, idx):  # noqa: F811
+    q, do = (_randn((1, h, n, D), s, dtype) for s in (61, 62))
+    k, v = (_randn((1, hk, n, D), s, dtype) for s in (63, 64))
+    qi, ki = _orders(h, n, 65), _orders(hk, n, 66)
+    group = h // hk
+    ref = _oracle_grads(_grouped(lambda a, b, c: O.block_sampled_attention(a, b, c, qi, ki.repeat_interleave(group, 1), block, sample), group),
+                        q, k, v, do)
+    qi_g, ki_g = (x.cuda().to(idx).transpose(1, 2) for x in (qi, ki))
+    _, _, *got = _gpu_grads(lambda a, b, c: ha.hyper_attn_func(a, b, c, qi_g, ki_g, block, sample, None, False), q, k, v, do)
+    for g, want, name in zip(got, ref, ("dq", "dk", "dv")):
+        _check(g, want, name, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("exact", [False, True])
+def test_adds_to_what_is_there(ha, dtype, exact):  # noqa: F811
+    """Gradients added to (bnhd layout): the result is what was there and the plain gradient, up to the rounding of the sum."""
+    from hyperattention_amd import _lib, ops
+    h, n = (300, 200) if exact else (70, 384)
+    q, k, v, do = (_randn((1, n, h, D), s, dtype).cuda() for s in (71, 72, 73, 74))
+    qi, ki = _orders(h, n, 75), _orders(h, n, 76)
+    back = lambda x: x.transpose(1, 2).cpu()  # noqa: E731
+    if exact:
+        fn = lambda a, b, c: O.exact_attention(a, b, c, None, False)  # noqa: E731
+        o, lse = ops.flash_attn_func(q, k, v)
+        t, entry = ops._operands(q, k, v, o, lse, D ** -0.5, layout_bnhd=True, lse_row_stride=lse.shape[-1]), _lib.lib().ha_flash_attn_bwd
+    else:
+        fn = lambda a, b, c: O.block_sampled_attention(a, b, c, qi, ki, 256)  # noqa: E731
+        qi_g, ki_g = (x.cuda().int().transpose(1, 2) for x in (qi, ki))
+        o, lse = ops.hyper_attn_func(q, k, v, qi_g, ki_g, 256, 0, None, False)
+        a, _keep = ops._block_attn_args(q, k, v, o, lse, qi_g, ki_g, 256, 0, D ** -0.5, False, None)
+        t, entry = a.t, _lib.lib().ha_block_attn_bwd
+    ref = _oracle_grads(fn, *(back(x) for x in (q, k, v, do)))
+    there = [_randn((1, n, h, D), s, dtype).cuda() for s in (77, 78, 79)]
+    grads = [x.clone() for x in there]
+    g, ws = ops._attn_grads(t, do, *grads, sample_size=0)
+    g.accumulate = 1
+    if exact:
+        _lib.check(entry(ctypes.byref(t), 0, ctypes.byref(g), ops._stream(q)))
+    else:
+        _lib.check(entry(ctypes.byref(a), ctypes.byref(g), ops._stream(q)))
+    torch.cuda.synchronize()
+    # the sum is rounded to the type once more: half a unit of its last place, of values of N(0, 1) plus the gradient
+    unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    for got, was, want, name in zip(grads, there, ref, ("dq", "dk", "dv")):
+        total = back(was).double() + want
+        err = (back(got).double() - total).norm() / total.norm()
+        assert err <= unit + (3e-3 if dtype == torch.float16 else 8e-3), f"{name}: {err:.2e}"
+        assert torch.isfinite(got).all()
