@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(_PKG, "libhyperattn.so")
 HOST_PATH = os.path.join(_PKG, "_host.so")  # the module's host path on torch tensors (csrc/torch_host.cpp)
 
 SOURCES = ["api.hip", "lsh_hash.hip", "bucket_sort.hip", "gather_rows.hip", "lse_merge.hip", "attn_fwd.hip",
-           "attn_bwd.hip", "attn_bwd_block.hip", "attn_bwd_wide.hip", "power_probe.hip"]
+           "attn_bwd.hip", "attn_bwd_block.hip", "attn_bwd_wide.hip", "attn_bwd_wide_dq.hip", "power_probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -59,3 +59,6 @@ int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stre
 // dk, dv of exact attention or of plain blocks (multiples of 256 keys) at head dim 128, 256 keys per workgroup
 // (attn_bwd_wide.hip); grid: workgroups
 int ha_launch_bwd_wide(const ha_attn_bwd_params& p, int pass, bool causal, int is_f16, int64_t grid, hipStream_t stream, const char* what);
+
+// dq of exact attention at head dim 128, 256 queries per workgroup (attn_bwd_wide_dq.hip)
+int ha_launch_bwd_wide_dq(const ha_attn_bwd_params& p, bool causal, int is_f16, int64_t grid, hipStream_t stream, const char* what);

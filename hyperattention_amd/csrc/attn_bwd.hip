@@ -425,7 +425,7 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
 // The form of a pass of exact attention with the least estimated time.
 //   WHOLE: 128 stationary rows per workgroup, causal tiles in pairs.
 //   SPLIT: 64, the steps of the streamed tiles split over waves (HALVES = 2), half as many steps per wave.
-//   WIDE: 256 (attn_bwd_wide.hip; dk, dv at d = 128).
+//   WIDE: 256 (d = 128; dk, dv: attn_bwd_wide.hip, dq: attn_bwd_wide_dq.hip).
 // What bounds a launch of few workgroups is the longest chain of steps of one of them with CUs idle: a wave alone on its
 // SIMD issues steps as fast as two together, so smaller workgroups fill the idle CUs; on a full chip they do the same
 // work slower (twice the set-up and tile loads per row; dq at d = 128 also one workgroup per CU instead of two).
@@ -440,8 +440,15 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
 // two -> wide, dk, dv in us at 35 shapes, among them (causal) 24 heads of 4096 rows 307 -> 223, 32 387 -> 271, of 8192 1347
 // -> 972, 256 of 256 41 -> 32; (not causal) 24 of 2048 147 -> 108, 32 of 4096 684 -> 477; 32 on 8, 300 on 8192 rows 124 ->
 // 84.  Where the chip is not full the others stay: causal 32 on 8 heads of 4096 413 (wide 696), 12 of 2048 56 (103).
+// dq: wide where its workgroups occupy more than half of the CUs, unless their chains are so short (128 keys without mask)
+// that all there is is their start.  The better of the others -> wide in us at 43 shapes, workgroups of 256 in brackets:
+// causal, 16 heads of 2048 rows (128) 55 -> 68, 24 (192) 82 -> 73, 8 heads of 4096 (128) 91 -> 122, 12 (192) 138 -> 129, 16
+// (256) 142 -> 141, 32 (512) 223 -> 190, 8 segments of 2048 with 32 heads (2048) 500 -> 466, 256 of 256 (256) 31 -> 25, 2048
+// of 128 (2048) 174 -> 115; without mask, 16 of 2000 (128) 62 -> 64, 17 (136) 82 -> 66, 33 of 2048 (264) 149 -> 151, 32 of
+// 4096 (512) 376 -> 342, of 4096 on 256 keys (512) 51 -> 52, on 128 42 -> 44, 2048 of 128 (2048) 108 -> 121.
 enum ExactForm { WHOLE, SPLIT, WIDE };
 ExactForm exact_form(int d, bool dkv, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal) {
+  if (d == 128 && !dkv && seqs * ((rows + 255) / 256) > 128 && (causal || streamed_rows > 128)) return WIDE;
   const double cus = 256., set_up = 2., margin = 0.97;
   // time of a step where a CU has several workgroups to take, against one alone
   const double full_whole = d == 64 || dkv ? 0.95 : 0.8, full_split = d == 64 ? 1.25 : dkv ? 1. : 1.4;
@@ -472,8 +479,11 @@ template <typename T, int D, int PASS>
 int launch_exact(const ha_attn_bwd_params& p, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal,
                  hipStream_t stream, const char* what) {
   const ExactForm form = exact_form(D, PASS == HA_BWD_DKV_EXACT, seqs, rows, streamed_rows, group, causal);
-  if (form == WIDE)
-    return ha_launch_bwd_wide(p, PASS, causal, std::is_same<T, f16_t>::value, seqs * ((rows + 255) / 256), stream, what);
+  if (form == WIDE) {
+    constexpr int is_f16 = std::is_same<T, f16_t>::value;
+    const int64_t grid = seqs * ((rows + 255) / 256);
+    return PASS == HA_BWD_DQ_EXACT ? ha_launch_bwd_wide_dq(p, causal, is_f16, grid, stream, what) : ha_launch_bwd_wide(p, PASS, causal, is_f16, grid, stream, what);
+  }
   if (form == SPLIT) {
     const int64_t grid = seqs * ((rows + 63) / 64);
     return causal ? launch_pass<T, D, PASS, true, 2>(p, grid, stream, what) : launch_pass<T, D, PASS, false, 2>(p, grid, stream, what);

@@ -1,4 +1,5 @@
-"""dk, dv with 256 keys per workgroup at head dim 128 (csrc/attn_bwd_wide.hip): launches that fill the chip with few rows
+"""dk, dv with 256 keys and dq with 256 queries per workgroup at head dim 128 (csrc/attn_bwd_wide.hip,
+attn_bwd_wide_dq.hip): launches that fill the chip with few rows
 per head, at the edges of its tiles of 256 keys and 32 queries.  The shapes are ones that its dispatch rules take."""
 import ctypes
 
@@ -32,6 +33,7 @@ def _grouped(fn, group):
     (torch.bfloat16, 300, 300, 300, 500, True),    # keys that nothing attends
     (torch.float16, 300, 300, 300, 256, True),     # queries after the last key
     (torch.bfloat16, 600, 200, 20, 260, False),    # one step per query head
+    (torch.float16, 130, 130, 40, 33, True),       # two steps, half of the waves without queries
 ])
 def test_exact(ha, dtype, h, hk, nq, nk, causal):  # noqa: F811
     q, do = (_randn((1, h, nq, D), s, dtype) for s in (51, 52))
