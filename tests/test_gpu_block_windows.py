@@ -20,6 +20,8 @@ pytestmark = pytest.mark.gpu
     (640, 512, 0, True),     # windows wrap around the sequence
     (256, 512, 128, True),   # a block longer than the sequence
     (1024, 128, 128, True),  # windows of one tile, 64 keys off
+    (640, 256, 128, False),  # the plain instance with one tile in the last workgroup
+    (128, 512, 0, False),    # and in the only one
 ])
 def test_windows(ha, monkeypatch, dtype, d, n, block, sample, smooth):  # noqa: F811
     monkeypatch.setenv("HA_SPLIT", "0")
