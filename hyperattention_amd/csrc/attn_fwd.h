@@ -49,7 +49,8 @@ struct ha_attn_kernel_params {
   // the caller packs the rows a call writes)
   int64_t o_seg_off, o_seg_stride;
   // Streaming gathered kernel: consecutive query tiles of one (virtual) head per workgroup (the last
-  // workgroup of a head may have fewer); 1: the one-tile kernels
+  // workgroup of a head may have fewer); 1: the one-tile kernels.  Exact causal kernel: 0 for one tile per
+  // workgroup, longest first, instead of pairs
   int tiles_per_wg;
   int split_keys;  // the keys of a query tile are split over the waves of a workgroup, 2: longest tiles first (filled by
                    // ha_attn_launch)

@@ -326,18 +326,32 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   // Workgroup number = (((batch, kv head), segment), tile, query head inside the kv group), the last one
   // fastest: the query heads that share a kv head work on the same tile side by side, on one XCD, so that the
   // K and V rows of the tile (the same for all of them) come from HBM once and from L2 after that.
-  const int wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
+  int wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
   const int qtiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES;
-  // Exact causal attention: a workgroup takes the tile pair (qtiles-1-s, s), so that every workgroup of the
+  // Exact causal attention, many workgroups: one takes the tile pair (qtiles-1-s, s), so that every workgroup of the
   // launch has the same number of key chunks to go through.  The hardware hands out workgroups in order and
   // a slot freed by a short one stays empty until the ones queued before it are placed: with one tile per
   // workgroup (4 to 32 chunks in a 2048-row leaf) the slots of a CU stood empty for 8 us at a time.
+  // Few workgroups (p.tiles_per_wg == 0, see single_tiles): one tile each, the tiles of all sequences, longest first, at
+  // head dim 64, where a CU holds two workgroups, the second 256 in reversed order (see ha_attn_fwd_split_kernel).
   constexpr bool PAIRED = CAUSAL && !GATHER;
   const int wg_per_seq = PAIRED ? (qtiles + 1) / 2 : qtiles;  // what p.div_qtiles divides by
-  const int wg_tile = fast_div(wg, p.div_kv_group);
-  const int hg = wg - wg_tile * p.kv_group;
-  const int vseq = fast_div(wg_tile, p.div_qtiles);
-  const int slot = wg_tile - vseq * wg_per_seq;
+  const bool single = PAIRED && p.tiles_per_wg == 0;
+  int hg, vseq, slot;
+  if (single) {
+    const int second = min((int)gridDim.x, 512);
+    wg = blockIdx.x;
+    if (D <= 64 && wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
+    slot = fast_div(wg, p.div_qtiles);
+    wg -= slot * (p.batch * p.heads * p.segs);  // what p.div_qtiles divides by here
+    vseq = fast_div(wg, p.div_kv_group);
+    hg = wg - vseq * p.kv_group;
+  } else {
+    const int wg_tile = fast_div(wg, p.div_kv_group);
+    hg = wg - wg_tile * p.kv_group;
+    vseq = fast_div(wg_tile, p.div_qtiles);
+    slot = wg_tile - vseq * wg_per_seq;
+  }
   const int bhk = fast_div(vseq, p.div_segs);
   const int seg = vseq - bhk * p.segs;
   const int b = fast_div(bhk, p.div_kv_heads), hk = bhk - b * fast_div(p.heads, p.div_kv_group);
@@ -361,7 +375,7 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
       const int qt = t_long;
 #include "attn_fwd_tile.inc"
     }
-    if (slot != t_long && slot * WG_QUERIES < n_q) {  // an odd number of tiles: the middle one has no partner
+    if (!single && slot != t_long && slot * WG_QUERIES < n_q) {  // an odd number of tiles: the middle one has no partner
       const int qt = slot;
 #include "attn_fwd_tile.inc"
     }
@@ -460,8 +474,9 @@ static ha_divisor make_divisor(int64_t y) {
 // Constants fitted to the kernels' times inside calls of the module, 645 launches at d <= 64 and 648 above (2 to 256
 // heads, grouped and not, 300 to 4133 rows exact, 2048 to 16384 rows hashed): the chosen kernel is within 3 % of the
 // better one at all but 10 of them, within 10 % at all.  Times whole | split in us, d = 64 causal: 24 heads of 1000
-// rows 31 | 13, of 2048 45 | 27, of 4096 81 | 72; 48 of 2048 48 | 45, of 4096 129 | 139; without mask 16 of 4096 rows
+// rows 31 | 13, of 2048 39 | 28, of 4096 72 | 72; 48 of 2048 41 | 45, of 4096 116 | 143; without mask 16 of 4096 rows
 // 75 | 86; d = 128, 12 heads of 2048 rows, blocks and samples of 256: 20 | 26.
+static bool single_tiles(const ha_attn_kernel_params& p, int width);
 static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   const char* env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
   if (env) return atoi(env) != 0;
@@ -482,7 +497,14 @@ static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gathe
   if (per_cu <= 1) rounds = 1 + f.crowd * per_cu;
   else if (width == 64 || paired) rounds = std::max(f.second, f.share * per_cu + f.rest);
   else rounds = f.second * std::ceil(per_cu);
-  const double whole = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
+  double whole = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
+  if (paired && single_tiles(p, width)) {
+    // one tile per workgroup, longest first: the longest chain, slowed by its neighbours, or a CU's share of all
+    const double longest = 4. * tiles, share = vheads * 2. * tiles * (tiles + 1) / cus, wgs = vheads * tiles / cus;
+    const double crowd = width == 64 ? 0.1 * share : 0.3 * std::min(longest, share);
+    whole = f.start + std::max(f.step * (longest + crowd), (width == 64 ? 0.97 : 1.9) * share + 2. * wgs);
+    if (width == 128) whole *= 0.93;  // the other estimate is that much too low beside this one (48 heads of 685 rows: 24 us | split 30)
+  }
 
   const double chain = std::ceil(keys / 128.), split_per_cu = vheads * split_tiles / cus;
   double all;
@@ -490,6 +512,19 @@ static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gathe
   else all = (width == 64 ? split_per_cu : std::ceil(split_per_cu)) * (chain + f.set_up);
   const double split = f.split_start + f.split_step * std::max(chain + f.set_up, all);
   return split < whole;
+}
+
+// Whether exact causal attention takes one query tile per workgroup, longest first, instead of a pair of tiles.  Pairs
+// leave CUs idle in a last round that is not full; single tiles fill it, but read a sequence's keys at times
+// far apart, which costs where there are many rounds.  At head dim 128, with one workgroup per CU, full rounds of pairs
+// are as fast or faster.  Times in us, pairs | single, 256-query pairs per CU in brackets: d = 64, 48 heads of 2048 rows
+// (0.75) 49.9 | 43.0, 80 (1.25) 74.1 | 58.1, 96 of 1024 (0.75) 32.8 | 26.8, 128 of 2048 (2) 82.9 | 81.2, 200 (3.1) 151 |
+// 130, 256 (4) 170 | 175, 700 (11) 448 | 490, 2048 (32) 1292 | 1462; d = 128, 24 of 2048 (0.38) 64 | 55, 64 (1) 78 | 78, 96
+// (1.5) 136 | 117, 128 (2) 154 | 156, 256 of 1024 (2) 99 | 106, 200 of 2048 (3.1) 285 | 263, 300 (4.7) 402 | 417, 512 (8)
+// 659 | 736.
+static bool single_tiles(const ha_attn_kernel_params& p, int width) {
+  const double pairs = (double)p.batch * p.heads * p.segs * ((p.n_q + 2 * WG_QUERIES - 1) / (2 * WG_QUERIES)) / 256.;
+  return width == 64 ? pairs <= 3.5 : pairs < 4 && std::ceil(pairs) > 1.05 * pairs;
 }
 
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,
@@ -501,7 +536,8 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   p.qk_pieces = d / 8;
   p.v_pieces = dv / 8;
   int64_t qtiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES;
-  if (causal && !gather) qtiles = (qtiles + 1) / 2;  // exact causal attention: one workgroup per pair of tiles
+  const bool single = causal && !gather && single_tiles(p, width);
+  if (causal && !gather && !single) qtiles = (qtiles + 1) / 2;  // one workgroup per pair of tiles
   // Gathered attention with whole 256-query tiles, whole key blocks and an even number of at least four key
   // chunks per tile can run as a stream: a workgroup takes a run of tiles of its head
   // (ha_attn_fwd_stream_kernel), as long a run as still leaves every CU its full set of resident workgroups.
@@ -527,7 +563,8 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   }
   // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
   if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
-  p.div_qtiles = make_divisor(p.split_keys == 2 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
+  if (single && !p.split_keys) p.tiles_per_wg = 0;
+  p.div_qtiles = make_divisor(p.split_keys == 2 || p.tiles_per_wg == 0 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);
   p.div_kv_heads = make_divisor(p.heads / p.kv_group);
