@@ -48,6 +48,7 @@ struct ha_attn_bwd_params {
   int smooth, idx64;
   int accumulate;  // add to dq / dk / dv instead of overwriting them
   int q_split;  // sampled-key pass: queries per workgroup
+  int single_tiles;  // exact causal passes: one tile per workgroup, longest first, instead of pairs
   int run_blocks;  // fused kernel of blocks and samples: consecutive blocks per workgroup
   float scale, scale_log2, neg_inv_scale;  // scale * log2(e), -1 / scale
 };

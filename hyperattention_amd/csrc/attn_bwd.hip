@@ -116,14 +116,21 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   // Exact causal attention: a workgroup takes the pair of stationary tiles (s, T-1-s), the one that streams more
   // rows first (the last query tile sees every key, the first key tile is seen by every query), so that every
   // workgroup of a launch streams the same number of rows.  The hardware hands out workgroups in order, and a
-  // slot freed by a short one stays empty until the ones queued before it are placed.
+  // slot freed by a short one stays empty until the ones queued before it are placed.  Few tiles (single_tiles) come one by
+  // one, the ones of all sequences that stream the most rows first, at d = 64, two workgroups per CU, the second 256 reversed.
   constexpr bool PAIRED = CAUSAL && HALVES == 1 && (PASS == HA_BWD_DQ_EXACT || PASS == HA_BWD_DKV_EXACT);
-  const int wg_per_seq = PAIRED ? (st_tiles + 1) / 2 : st_tiles;
+  const bool single = PAIRED && p.single_tiles;
+  const int wg_per_seq = PAIRED && !single ? (st_tiles + 1) / 2 : st_tiles;
   // Steps split over waves: no pairs; the tiles of all sequences that stream the most rows come first (tile-major)
-  const int n_vseq = HALVES == 2 ? gridDim.x / wg_per_seq : 1;
-  int rest = HALVES == 2 ? (int)blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int slot = HALVES == 2 ? rest / n_vseq : rest % wg_per_seq;
-  rest = HALVES == 2 ? rest - slot * n_vseq : rest / wg_per_seq;
+  const bool tile_major = HALVES == 2 || single;
+  const int n_vseq = tile_major ? gridDim.x / wg_per_seq : 1;
+  int rest = tile_major ? (int)blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);
+  if (single && D <= 64) {
+    const int second = min((int)gridDim.x, 512);
+    if (rest >= 256 && rest < second) rest = 256 + second - 1 - rest;
+  }
+  const int slot = tile_major ? rest / n_vseq : rest % wg_per_seq;
+  rest = tile_major ? rest - slot * n_vseq : rest / wg_per_seq;
   const int split = rest % splits;
   const int vseq = rest / splits;   // (batch, head, segment)
   const int seg = vseq % p.segs;
@@ -186,7 +193,7 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
       const int tile = t_long;
 #include "attn_bwd_tile.inc"
     }
-    if (t_short != t_long) {  // an odd number of tiles: the middle one has no partner
+    if (!single && t_short != t_long) {  // an odd number of tiles: the middle one has no partner
       // the first tile's last reads of the staging areas and the streamed tiles are behind every wave
       __syncthreads();
       const int tile = t_short;
@@ -337,6 +344,7 @@ void fill_bwd_params(const ha_attn_operands& t, const ha_attn_grads& g, const Wo
   p.n_q = (int)t.n_q; p.n_k = (int)t.n_k;
   p.block_tiles = 1; p.sample_size = 0; p.smooth = 0; p.idx64 = 0;
   p.accumulate = g.accumulate != 0;
+  p.single_tiles = 0;
   p.q_split = (int)t.n_q;
   p.scale = t.scale;
   p.scale_log2 = t.scale * LOG2E;
@@ -424,36 +432,57 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
 
 // The form of a pass of exact attention with the least estimated time.
 //   WHOLE: 128 stationary rows per workgroup, causal tiles in pairs.
+//   SINGLE: causal tiles one by one, longest first.
 //   SPLIT: 64, the steps of the streamed tiles split over waves (HALVES = 2), half as many steps per wave.
 //   WIDE: 256 (d = 128; dk, dv: attn_bwd_wide.hip, dq: attn_bwd_wide_dq.hip).
 // What bounds a launch of few workgroups is the longest chain of steps of one of them with CUs idle: a wave alone on its
 // SIMD issues steps as fast as two together, so smaller workgroups fill the idle CUs; on a full chip they do the same
 // work slower (twice the set-up and tile loads per row; dq at d = 128 also one workgroup per CU instead of two).
-// Estimated in steps of 32 streamed rows: rounds of workgroups over the CUs times their chain, or, for causal tiles one
-// by one (longest first), the longest chain or a CU's share of all.  The weights are fitted to the times of WHOLE and
-// SPLIT of both passes at 57 shapes per head dim (4 to 128 heads, grouped and not, 512 to 4096 rows): where the rule
-// splits, it was never slower by more than they scatter.
-// Times in us, whole -> split, dq | dk, dv, bf16 causal: d 64, 24 heads of 2048 rows 40 -> 32 | 50 -> 39, 4 heads of 1000
-// 24 -> 13 | 29 -> 16, 8 query heads on 2 of 4096 61 -> 42 | 291 -> 189; d 128, 12 heads of 2048 75 -> 41 | 93 -> 49, 32
-// on 8 of 2048 78 (split 98: stays) | 320 -> 161.  Full: d 64, 48 heads of 4096 rows without mask 295 (split 335) | 387 (451).
-// A wide step is 1.05 whole steps long on an idle chip and 1.3 on a full one, for twice the pairs.  The better of the other
-// two -> wide, dk, dv in us at 35 shapes, among them (causal) 24 heads of 4096 rows 307 -> 223, 32 387 -> 271, of 8192 1347
-// -> 972, 256 of 256 41 -> 32; (not causal) 24 of 2048 147 -> 108, 32 of 4096 684 -> 477; 32 on 8, 300 on 8192 rows 124 ->
-// 84.  Where the chip is not full the others stay: causal 32 on 8 heads of 4096 413 (wide 696), 12 of 2048 56 (103).
-// dq: wide where its workgroups occupy more than half of the CUs, unless their chains are so short (128 keys without mask)
-// that all there is is their start.  The better of the others -> wide in us at 43 shapes, workgroups of 256 in brackets:
-// causal, 16 heads of 2048 rows (128) 55 -> 68, 24 (192) 82 -> 73, 8 heads of 4096 (128) 91 -> 122, 12 (192) 138 -> 129, 16
-// (256) 142 -> 141, 32 (512) 223 -> 190, 8 segments of 2048 with 32 heads (2048) 500 -> 466, 256 of 256 (256) 31 -> 25, 2048
-// of 128 (2048) 174 -> 115; without mask, 16 of 2000 (128) 62 -> 64, 17 (136) 82 -> 66, 33 of 2048 (264) 149 -> 151, 32 of
-// 4096 (512) 376 -> 342, of 4096 on 256 keys (512) 51 -> 52, on 128 42 -> 44, 2048 of 128 (2048) 108 -> 121.
-enum ExactForm { WHOLE, SPLIT, WIDE };
+//
+// Pairs of causal tiles are equal workgroups, which leave CUs idle in a last round that is not full.  Single ones fill it,
+// but read a sequence's rows at times far apart: up to 4.5 pairs per CU they are never slower.  Pairs | split | single, dq,
+// then dk, dv, in us at d = 64, pairs per CU in brackets: 24 heads of 2048 rows (0.75) 40 | 33 | 36, 58 | 41 | 53; 48 (1.5) 60
+// | 55 | 51, 80 | 71 | 67; 80 (2.5) 88 | 87 | 74, 125 | 113 | 105; 128 (4) 119 | 139 | 114, 161 | 179 | 154; 300 (9.4) 292 |
+// 426 | 299, 405 | 482 | 411; 700 (22) 670 | 1077 | 773, 920 | 1206 | 998; 24 of 4096 (1.5) 105 | 97 | 89, 141 | 129 | 117; 32
+// query heads on 8 of 2048 (1, dk, dv 0.25) 39 | 40 | 38, 178 | 101 | 162.  d = 128: 24 of 2048 83 | 83 | 67, 108 | 99 | 95.
+// Their estimates in us at d = 64: the longest chain and a part of the load beside it, or a CU's share of the steps and
+// starts; within 10 % of the times at 27 shapes.
+//
+// The others are estimated in steps of 32 streamed rows: rounds of workgroups over the CUs times their chain, or, for causal
+// tiles one by one (longest first), the longest chain or a CU's share of all.  The weights are fitted to the times of WHOLE
+// and SPLIT of both passes at 57 shapes per head dim (4 to 128 heads, grouped and not, 512 to 4096 rows).
+// Times in us, whole -> split, dq | dk, dv, bf16 causal: d 64, 4 heads of 1000 rows 24 -> 13 | 29 -> 16; d 128, 12 heads of
+// 2048 75 -> 41 | 93 -> 49, 32 on 8 of 2048 78 (split 98: stays) | 320 -> 161.  Full: d 64, 48 heads of 4096 rows without
+// mask 295 (split 335) | 387 (451).
+// A wide step of dk, dv is 1.05 whole steps long on an idle chip and 1.3 on a full one, for twice the pairs.  The better of
+// the others -> wide, dk, dv in us at 35 shapes, among them (causal) 24 heads of 4096 rows 307 -> 223, 32 387 -> 271, of 8192
+// 1347 -> 972, 256 of 256 41 -> 32; (not causal) 24 of 2048 147 -> 108, 32 of 4096 684 -> 477; 32 on 8, 300 on 8192 rows 124
+// -> 84.  Where the chip is not full the others stay: causal 32 on 8 heads of 4096 413 (wide 696), 12 of 2048 56 (103).
+// dq: causal, wide from two and a half tiles of 128 rows per CU on, the better of the others -> wide in us: 24 heads of 2048
+// rows (1.5) 67 -> 71, 32 of 2048 (2) 71 -> 75, 300 of 256 (2.3) 35 -> 37, 20 of 4096 (2.5) 140 -> 144, 80 of 1024 (2.5) 55 ->
+// 46, 24 of 4096 (3) 161 -> 154, 128 of 1024 (4) 72 -> 68, 32 of 4096 (4) 209 -> 185, 2048 of 128 (8) 174 -> 115, 8 segments of
+// 2048 with 32 heads (16) 500 -> 466.  Without mask, where wide workgroups occupy more than half of the CUs (in brackets)
+// and have more than 128 keys: 16 of 2000 (128) 62 -> 64, 17 (136) 82 -> 66, 33 of 2048 (264) 149 -> 151, 32 of 4096 (512)
+// 376 -> 342, of 4096 on 256 keys (512) 51 -> 52, on 128 42 -> 44, 2048 of 128 (2048) 108 -> 121.
+enum ExactForm { WHOLE, SINGLE, SPLIT, WIDE };
 ExactForm exact_form(int d, bool dkv, int64_t seqs, int64_t rows, int64_t streamed_rows, int64_t group, bool causal) {
-  if (d == 128 && !dkv && seqs * ((rows + 255) / 256) > 128 && (causal || streamed_rows > 128)) return WIDE;
   const double cus = 256., set_up = 2., margin = 0.97;
+  const double tiles = (double)((rows + 127) / 128), split_tiles = (double)((rows + 63) / 64), split_wgs = seqs * split_tiles;
+  if (d == 128 && !dkv && (causal ? seqs * tiles >= 2.5 * cus : seqs * ((rows + 255) / 256) > cus / 2 && streamed_rows > 128)) return WIDE;
+  const bool few_pairs = causal && seqs * std::ceil(tiles / 2) <= 4.5 * cus;
+  if (d == 64 && causal) {
+    if (!few_pairs) return WHOLE;
+    const double wgs = seqs * tiles, share = 2. * group * wgs * (tiles + 1) / cus, chain = 4. * group * tiles;
+    const double split_share = group * split_wgs * (split_tiles + 1) / 2 / cus, split_chain = group * split_tiles;
+    const double single = dkv ? std::max(0.61 * chain + 0.06 * share + 8, 0.53 * share + 1.6 * wgs / cus + 5)
+                              : std::max(0.43 * chain + 0.06 * share + 5, 0.39 * share + 1.6 * wgs / cus + 5);
+    const double split = dkv ? std::max(0.75 * split_chain + 7, 0.58 * split_share + 1.5 * split_wgs / cus + 5)
+                             : std::max(0.56 * split_chain + 6, 0.43 * split_share + 1.7 * split_wgs / cus + 5);
+    return split < single ? SPLIT : SINGLE;
+  }
   // time of a step where a CU has several workgroups to take, against one alone
   const double full_whole = d == 64 || dkv ? 0.95 : 0.8, full_split = d == 64 ? 1.25 : dkv ? 1. : 1.4;
-  const double tiles = (double)((rows + 127) / 128), split_tiles = (double)((rows + 63) / 64);
-  const double rounds = std::ceil(seqs * (causal ? std::ceil(tiles / 2) : tiles) / cus), split_wgs = seqs * split_tiles;
+  const double rounds = std::ceil(seqs * (causal ? std::ceil(tiles / 2) : tiles) / cus);
   double whole, split;
   if (causal) {
     whole = (rounds > 1 ? full_whole : 1.) * rounds * 4 * (tiles + 1) * group + 2 * set_up * rounds;
@@ -464,7 +493,7 @@ ExactForm exact_form(int d, bool dkv, int64_t seqs, int64_t rows, int64_t stream
     whole = (rounds > 1 ? full_whole : 1.) * rounds * 4 * streamed * group + set_up * rounds;
     split = (split_rounds > 1 ? full_split : 1.) * split_rounds * 2 * streamed * group + set_up * split_rounds;
   }
-  const ExactForm narrow = split < margin * whole ? SPLIT : WHOLE;
+  const ExactForm narrow = split < margin * whole ? SPLIT : few_pairs ? SINGLE : WHOLE;
   if (d != 128 || !dkv) return narrow;
   const double wide_tiles = (double)((rows + 255) / 256), wide_wgs = seqs * wide_tiles, chain = (double)((streamed_rows + 31) / 32) * group;
   const double step = 1.05 + 0.25 * std::min(1., wide_wgs / cus), wide_rounds = std::ceil(wide_wgs / cus), wide_set_up = 3.;
@@ -489,7 +518,12 @@ int launch_exact(const ha_attn_bwd_params& p, int64_t seqs, int64_t rows, int64_
     return causal ? launch_pass<T, D, PASS, true, 2>(p, grid, stream, what) : launch_pass<T, D, PASS, false, 2>(p, grid, stream, what);
   }
   const int64_t tiles = (rows + ST_ROWS - 1) / ST_ROWS;
-  if (causal) return launch_pass<T, D, PASS, true>(p, seqs * ((tiles + 1) / 2), stream, what);  // pairs of tiles
+  if (causal && form == SINGLE) {
+    ha_attn_bwd_params single = p;
+    single.single_tiles = 1;
+    return launch_pass<T, D, PASS, true>(single, seqs * tiles, stream, what);
+  }
+  if (causal) return launch_pass<T, D, PASS, true>(p, seqs * ((tiles + 1) / 2), stream, what);
   return launch_pass<T, D, PASS, false>(p, seqs * tiles, stream, what);
 }
 
