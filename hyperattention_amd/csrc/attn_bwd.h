@@ -24,7 +24,7 @@ struct ha_attn_bwd_params {
                  // by the dq pass of a call for the dk/dv passes that follow it
   void* dq;
   void *dk, *dv;       // written directly by the exact and the block passes
-  float *dk32, *dv32;  // fp32 (batch, heads / kv_group, sample_size, d): sums of the sampled keys, by slot
+  float *dk32, *dv32;  // fp32 (batch, heads / kv_group, segs, shares, sample_size, d): sums of the sampled keys, by slot
   int64_t q_sb, q_sh, q_sn;
   int64_t k_sb, k_sh, k_sn;
   int64_t v_sb, v_sh, v_sn;

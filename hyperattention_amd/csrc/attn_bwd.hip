@@ -25,8 +25,9 @@
 // queries of a key (of every query head of the key head's group, streamed one head after the other)
 // and stores dK, dV.  With sorted blocks a key gets one contribution from its block (complete in one
 // workgroup: stored like the exact pass's) and, if it is in the sample list, one from every query:
-// those are computed per range of queries and summed with atomics in small fp32 rows, one per slot of
-// the sample list, which a last kernel adds to the keys' rows of dK, dV.
+// those are computed per range of queries and summed in small fp32 rows, one per slot of
+// the sample list (with atomics, or one share per range, see writes_shares), which a last kernel adds to the keys' rows of
+// dK, dV.
 // The forms of the exact passes: exact_form.  Plain blocks of 256 at head dim 64 take
 // the one kernel of attn_bwd_block.hip in the place of the three gathered passes.
 #include "ha_common.h"
@@ -207,41 +208,36 @@ __global__ __launch_bounds__(256) void ha_bwd_zero_kernel(f32x4* __restrict__ bu
   if (i < n4) buf[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// Sums of the sampled keys (fp32, one row per slot of the sample list) added to the rows of dk, dv, 8
-// elements per lane.  A row that is listed several times is handled by its first slot alone, which adds
+// Sums of the sampled keys (fp32, `shares` rows per slot of the sample list) added to the rows of dk (blockIdx.y = 0) or dv,
+// 4 elements per lane.  A row that is listed several times is handled by its first slot alone, which adds
 // the sums of all of them: no two lanes write the same row, whatever the list holds.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __restrict__ sk32, const float* __restrict__ sv32,
                                                                  T* __restrict__ dk, T* __restrict__ dv,
                                                                  const void* __restrict__ sampled_idx, int idx64,
                                                                  int64_t si_sb, int64_t si_sh, int kv_heads, int sample_size,
-                                                                 int64_t dk_sb, int64_t dk_sh, int64_t dk_sn, int64_t dv_sb,
-                                                                 int64_t dv_sh, int64_t dv_sn, int64_t total_slots,
+                                                                 int shares, int64_t dk_sb, int64_t dk_sh, int64_t dk_sn,
+                                                                 int64_t dv_sb, int64_t dv_sh, int64_t dv_sn, int64_t total_slots,
                                                                  int segs, int64_t seg_stride, int64_t k_seg_off) {
-  typedef typename ElemTraits<T>::vec8 vec8;
-  constexpr int PR = D / 8;
+  typedef typename ElemTraits<T>::vec4 vec4;
+  constexpr int PR = D / 4;
   const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t gslot = item / PR;
   const int piece = (int)(item % PR);
   if (gslot >= total_slots) return;
+  const bool is_v = blockIdx.y != 0;
   const int64_t bhs = gslot / sample_size;   // (batch, kv head, segment)
   const int slot = (int)(gslot - bhs * sample_size);
   const int64_t bh = bhs / segs, seg = bhs - bh * segs;
   const int64_t b = bh / kv_heads, h = bh - b * kv_heads;
   const int64_t row0 = k_seg_off + seg * seg_stride;
   int row = slot;
-  float sum_k[8], sum_v[8];
-  const float* const bk = sk32 + (bhs * sample_size) * D + piece * 8;
-  const float* const bv = sv32 + (bhs * sample_size) * D + piece * 8;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  const float* const base = (is_v ? sv32 : sk32) + bhs * shares * sample_size * D + piece * 4;
   auto add_slot = [&](int s2) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      sum_k[e] += bk[(int64_t)s2 * D + e];
-      sum_v[e] += bv[(int64_t)s2 * D + e];
-    }
+#pragma unroll 8
+    for (int k = 0; k < shares; ++k) sum += *reinterpret_cast<const f32x4*>(base + ((int64_t)k * sample_size + s2) * D);
   };
-#pragma unroll
-  for (int e = 0; e < 8; ++e) sum_k[e] = sum_v[e] = 0.f;
   if (sampled_idx) {
     const int64_t list = b * si_sb + h * si_sh;
     row = ha_load_idx(sampled_idx, list + slot, idx64);
@@ -253,16 +249,12 @@ __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __
   } else {
     add_slot(slot);
   }
-  vec8* const dst_k = reinterpret_cast<vec8*>(dk + b * dk_sb + h * dk_sh + (row0 + row) * dk_sn + piece * 8);
-  vec8* const dst_v = reinterpret_cast<vec8*>(dv + b * dv_sb + h * dv_sh + (row0 + row) * dv_sn + piece * 8);
-  vec8 ok = *dst_k, ov = *dst_v;
+  vec4* const dst = reinterpret_cast<vec4*>(is_v ? dv + b * dv_sb + h * dv_sh + (row0 + row) * dv_sn + piece * 4
+                                                 : dk + b * dk_sb + h * dk_sh + (row0 + row) * dk_sn + piece * 4);
+  vec4 o = *dst;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    ok[e] = (T)((float)ok[e] + sum_k[e]);
-    ov[e] = (T)((float)ov[e] + sum_v[e]);
-  }
-  *dst_k = ok;
-  *dst_v = ov;
+  for (int e = 0; e < 4; ++e) o[e] = (T)((float)o[e] + sum[e]);
+  *dst = o;
 }
 
 template <typename T, int D, int PASS, bool CAUSAL, int HALVES = 1>
@@ -275,18 +267,49 @@ int launch_pass(const ha_attn_bwd_params& p, int64_t grid, hipStream_t stream, c
 
 inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
+// Every query attends every sampled key: the queries are cut into ranges, one workgroup each per tile of sampled
+// keys.  Taken is the number of ranges with the least time by the rounds of workgroups the chip needs and the
+// rows of a round; setting up a workgroup and the adds it ends in cost about as much as 384 rows.
+struct QueryRanges {
+  int64_t rows, count;
+};
+QueryRanges query_ranges(int64_t n_q, int64_t tiles, int64_t slots) {
+  QueryRanges r = {n_q, 1};
+  int64_t best = INT64_MAX;
+  for (int64_t n = 1; n <= std::min<int64_t>(64, (n_q + 511) / 512); ++n) {
+    const int64_t rows = ((n_q + n - 1) / n + 63) / 64 * 64, count = (n_q + rows - 1) / rows;
+    const int64_t cost = (tiles * count + slots - 1) / slots * (rows + 384);
+    if (cost < best) {
+      best = cost;
+      r = {rows, count};
+    }
+  }
+  return r;
+}
+
+// Whether the sampled keys' sums are made by workgroups of 256 keys that write their share of them (rows of a range of one
+// query head's queries) to the workspace, to be added up at the end, instead of adding them there with atomics, which took
+// 54 us of a pass for the 64 MB of 256 workgroups; to write and read them takes about 20.  This pass, clearing and final adds together, in us at d = 128, atomics -> shares (256 samples): 32 query heads
+// on 8 of 4096 rows 99 -> 61, of 8192 146 -> 97, 32 of 8192 149 -> 96, 33 of 2048 64 -> 45; small launches: 4 of 2048 rows 34.3
+// -> 35.0, 2 of 8192 41 -> 36, 64 of 512 41 -> 41, 8 of 4096 49 -> 38.  Ranges as many as with atomics.
+bool writes_shares(const ha_attn_operands& t, int64_t sample_size, QueryRanges& r) {
+  if (t.d != 128 || sample_size == 0 || sample_size % 256 != 0) return false;
+  r = query_ranges(t.n_q, t.batch * t.heads * t.segs * (sample_size / 256), 256);
+  return true;
+}
+
 struct Workspace {
   f32x2* stats;  // per query {L * log2(e), -D}
-  float* dk32;  // sums of the sampled keys, (batch, kv_heads, sample_size, d) fp32
+  float* dk32;  // sums of the sampled keys, (batch, kv_heads, segs, shares, sample_size, d) fp32
   float* dv32;
   int64_t acc_floats;  // per accumulator
   int64_t bytes;
 };
 
-Workspace carve(const ha_attn_operands& t, int64_t sample_size, void* base) {
+Workspace carve(const ha_attn_operands& t, int64_t sample_size, int64_t shares, void* base) {
   Workspace w;
   const int64_t delta_bytes = align256(t.batch * t.heads * t.segs * t.n_q * 8);
-  w.acc_floats = t.batch * (t.heads / t.kv_group) * t.segs * sample_size * t.d;
+  w.acc_floats = t.batch * (t.heads / t.kv_group) * t.segs * shares * sample_size * t.d;
   const int64_t acc_bytes = align256(w.acc_floats * 4);
   w.stats = (f32x2*)base;
   w.dk32 = (float*)((char*)base + delta_bytes);
@@ -313,7 +336,7 @@ int check_grads(const ha_attn_operands& t, int64_t sample_size, const ha_attn_gr
     HA_REQUIRE((row_counts[i] - 1) * row_strides[i] * 2 + t.d * 2 <= (1ll << 32), HA_ERR_UNSUPPORTED,
                "%s: one head of a gradient tensor may span 4 GiB at most", who);
   }
-  const Workspace w = carve(t, sample_size, nullptr);
+  const Workspace w = carve(t, sample_size, 1, nullptr);  // what every form can work in
   HA_REQUIRE(g.workspace && g.workspace_bytes >= w.bytes && ((uintptr_t)g.workspace % 256) == 0, HA_ERR_WORKSPACE,
              "%s: workspace of %lld bytes (256-byte aligned) required", who, (long long)w.bytes);
   return HA_OK;
@@ -353,14 +376,14 @@ void fill_bwd_params(const ha_attn_operands& t, const ha_attn_grads& g, const Wo
 
 // the sampled keys' sums onto their rows of dk, dv
 template <typename T, int D>
-int launch_add_samples(const ha_block_attn_args& a, const ha_attn_grads& g, const Workspace& w, hipStream_t stream) {
+int launch_add_samples(const ha_block_attn_args& a, const ha_attn_grads& g, const Workspace& w, int64_t shares, hipStream_t stream) {
   const ha_attn_operands& t = a.t;
   const int64_t kv_heads = t.heads / t.kv_group;
   const int64_t slots = t.batch * kv_heads * t.segs * a.sample_size;
-  const int64_t items = slots * (D / 8);
-  hipLaunchKernelGGL((ha_bwd_add_samples_kernel<T, D>), dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream,
+  const int64_t items = slots * (D / 4);
+  hipLaunchKernelGGL((ha_bwd_add_samples_kernel<T, D>), dim3((unsigned)((items + 255) / 256), 2), dim3(256), 0, stream,
                      w.dk32, w.dv32, (T*)g.dk, (T*)g.dv, a.sampled_idx, (int)(a.idx_type == HA_IDX_I64),
-                     a.sampled_stride_b, a.sampled_stride_h, (int)kv_heads, (int)a.sample_size, g.dk_stride_b,
+                     a.sampled_stride_b, a.sampled_stride_h, (int)kv_heads, (int)a.sample_size, (int)shares, g.dk_stride_b,
                      g.dk_stride_h, g.dk_stride_n, g.dv_stride_b, g.dv_stride_h, g.dv_stride_n, slots, (int)t.segs,
                      t.seg_stride_rows, t.k_seg_offset);
   return ha_launch_status("attention backward: sampled keys");
@@ -369,7 +392,13 @@ int launch_add_samples(const ha_block_attn_args& a, const ha_attn_grads& g, cons
 template <typename T, int D>
 int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream_t stream) {
   const ha_attn_operands& t = a.t;
-  const Workspace w = carve(t, a.sample_size, g.workspace);
+  QueryRanges ranges;
+  const bool shared_out = writes_shares(t, a.sample_size, ranges);
+  const int64_t wanted = shared_out ? t.kv_group * ranges.count : 1;
+  // (a workspace for the sums alone takes the atomics)
+  const int64_t shares = carve(t, a.sample_size, wanted, nullptr).bytes <= g.workspace_bytes ? wanted : 1;
+  const bool wide_samples = shared_out && shares == wanted;
+  const Workspace w = carve(t, a.sample_size, shares, g.workspace);
   int st;
   ha_attn_bwd_params p;
   fill_bwd_params(t, g, w, p);
@@ -382,7 +411,7 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   p.smooth = a.smooth_block != 0;
   p.idx64 = a.idx_type == HA_IDX_I64;
   const int64_t bh = t.batch * t.heads * t.segs, bhk = t.batch * (t.heads / t.kv_group) * t.segs;
-  if (a.sample_size > 0) {
+  if (a.sample_size > 0 && !wide_samples) {
     // the two arrays of sums lie one behind the other in the workspace (each a multiple of 256 bytes): one fill
     const int64_t n4 = (int64_t)(((char*)w.dv32 - (char*)w.dk32) + align256(w.acc_floats * 4)) / 16;
     hipLaunchKernelGGL(ha_bwd_zero_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, (f32x4*)w.dk32, n4);
@@ -392,7 +421,7 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   if (ha_block_bwd_fused_takes(p, D)) {
     st = ha_launch_block_bwd_fused(p, std::is_same<T, f16_t>::value, stream);
     if (st != HA_OK || a.sample_size == 0) return st;
-    return launch_add_samples<T, D>(a, g, w, stream);
+    return launch_add_samples<T, D>(a, g, w, shares, stream);
   }
   st = launch_pass<T, D, HA_BWD_DQ_BLOCK, false>(p, bh * (t.n_q / ST_ROWS), stream, "ha_block_attn_bwd: dq");
   if (st != HA_OK) return st;
@@ -408,24 +437,18 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
     st = launch_pass<T, D, HA_BWD_DKV_BLOCK, false>(p, bhk * (t.n_k / ST_ROWS), stream, "ha_block_attn_bwd: dk, dv of the blocks");
   if (st != HA_OK) return st;
   if (a.sample_size > 0) {
-    // Every query attends every sampled key: the queries are cut into ranges, one workgroup each per tile of sampled
-    // keys.  Taken is the number of ranges with the least time by the rounds of workgroups the chip needs and the
-    // rows of a round; setting up a workgroup and the atomic adds it ends in cost about as much as 384 rows.
-    const int64_t tiles = bh * (a.sample_size / ST_ROWS), slots = D <= 64 ? 512 : 256;
-    int64_t splits = 1, best = INT64_MAX;
-    for (int64_t n = 1; n <= std::min<int64_t>(64, (t.n_q + 511) / 512); ++n) {
-      const int64_t rows = ((t.n_q + n - 1) / n + 63) / 64 * 64;
-      const int64_t cost = (tiles * ((t.n_q + rows - 1) / rows) + slots - 1) / slots * (rows + 384);
-      if (cost < best) {
-        best = cost;
-        p.q_split = (int)rows;
-        splits = (t.n_q + rows - 1) / rows;
-      }
+    if (wide_samples) {
+      p.q_split = (int)ranges.rows;
+      st = ha_launch_bwd_wide(p, HA_BWD_DKV_SAMPLED, false, std::is_same<T, f16_t>::value, bh * (a.sample_size / 256) * ranges.count, stream,
+                              "ha_block_attn_bwd: dk, dv of the sampled keys");
+    } else {
+      const int64_t tiles = bh * (a.sample_size / ST_ROWS);
+      const QueryRanges r = query_ranges(t.n_q, tiles, D <= 64 ? 512 : 256);
+      p.q_split = (int)r.rows;
+      st = launch_pass<T, D, HA_BWD_DKV_SAMPLED, false>(p, tiles * r.count, stream, "ha_block_attn_bwd: dk, dv of the sampled keys");
     }
-    st = launch_pass<T, D, HA_BWD_DKV_SAMPLED, false>(p, tiles * splits, stream,
-                                                      "ha_block_attn_bwd: dk, dv of the sampled keys");
     if (st != HA_OK) return st;
-    return launch_add_samples<T, D>(a, g, w, stream);
+    return launch_add_samples<T, D>(a, g, w, shares, stream);
   }
   return HA_OK;
 }
@@ -529,7 +552,7 @@ int launch_exact(const ha_attn_bwd_params& p, int64_t seqs, int64_t rows, int64_
 
 template <typename T, int D>
 int run_flash_bwd(const ha_attn_operands& t, bool causal, const ha_attn_grads& g, hipStream_t stream) {
-  const Workspace w = carve(t, 0, g.workspace);
+  const Workspace w = carve(t, 0, 1, g.workspace);
   ha_attn_bwd_params p;
   fill_bwd_params(t, g, w, p);
   const int64_t bh = t.batch * t.heads * t.segs, bhk = t.batch * (t.heads / t.kv_group) * t.segs;
@@ -544,7 +567,8 @@ extern "C" int64_t ha_attn_bwd_workspace_bytes(const ha_attn_operands* t, int64_
   if (!t || t->batch <= 0 || t->heads <= 0 || t->n_q <= 0 || t->n_k <= 0 || t->d <= 0 || t->kv_group <= 0 ||
       t->heads % t->kv_group != 0 || sample_size < 0 || t->segs < 1)
     return ha_fail(HA_ERR_SHAPE, "ha_attn_bwd_workspace_bytes: sizes must be positive, kv_group dividing heads, segs >= 1");
-  return carve(*t, sample_size, nullptr).bytes;
+  QueryRanges r;
+  return carve(*t, sample_size, writes_shares(*t, sample_size, r) ? t->kv_group * r.count : 1, nullptr).bytes;
 }
 
 extern "C" int ha_block_attn_bwd(const ha_block_attn_args* args, const ha_attn_grads* grads, void* stream) {

@@ -1,4 +1,4 @@
-// dk, dv of exact attention and of plain blocks at head dim 128, 256 keys per workgroup.
+// dk, dv of exact attention, of plain blocks and of sampled keys at head dim 128, 256 keys per workgroup.
 //
 // Same sums as the passes of attn_bwd.hip, which keep 128 keys in 4 waves, one on each SIMD, with 480 registers each.
 // There the 32 matrix products of a step of 32 queries (1080 cycles) and its soft-max and LDS reads (about 700) follow one
@@ -17,7 +17,8 @@
 // Bound by the matrix cores and what does not overlap them: 32 products of 34 cycles and two waves on each SIMD are 0.9 us
 // at 2.4 GHz of a step's 1.3 us (half the chip at work) to 1.9 us (all of it).  Measured, bf16, 128 -> 256 keys: exact
 // causal, 8 segments of 2048 rows, 32 query heads on 8, 753 -> 540 us (1.0 PFLOP/s of the visible pairs); 32 heads of 4096
-// rows without mask 684 -> 477 (1.15); blocks of 256 of 16384 rows, 32 heads on 8, 225 -> 159.
+// rows without mask 684 -> 477 (1.15); blocks of 256 of 16384 rows, 32 heads on 8, 225 -> 159; 256 sampled keys of 8192
+// queries, 32 heads, 128 -> 75 (with atomic adds instead of stores at the end 122).
 #include "ha_common.h"
 #include "attn_tiles.h"
 #include "attn_bwd_tiles.h"
@@ -40,7 +41,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int KSTEPS = WD / 16, DB = WD / 32;
-  constexpr bool EXACT = PASS == HA_BWD_DKV_EXACT, BLOCK = PASS == HA_BWD_DKV_BLOCK;
+  constexpr bool EXACT = PASS == HA_BWD_DKV_EXACT, BLOCK = PASS == HA_BWD_DKV_BLOCK, SAMPLED = PASS == HA_BWD_DKV_SAMPLED;
   // in fp16 the exact pass rounds dS with its factor `scale`: see attn_bwd_tile.inc
   constexpr bool SCALE_DS = EXACT && std::is_same<T, f16_t>::value;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds_block[];  // WIDE_LDS_BYTES, from address 0 on
@@ -50,20 +51,25 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   // ---- which keys, which queries ----
-  const int st_total = p.n_k, st_tiles = (st_total + WIDE_KEYS - 1) / WIDE_KEYS;
-  int tile, vseq;
+  const int st_total = SAMPLED ? p.sample_size : p.n_k, st_tiles = (st_total + WIDE_KEYS - 1) / WIDE_KEYS;
+  const int splits = SAMPLED ? (p.n_q + p.q_split - 1) / p.q_split : 1;
+  int tile, vseq, split = 0;
   if (EXACT && CAUSAL) {  // the tiles that stream the most queries first, over all sequences
     const int n_vseq = gridDim.x / st_tiles;
     tile = blockIdx.x / n_vseq;
     vseq = blockIdx.x - tile * n_vseq;
   } else {
-    const int id = xcd_contiguous_id(blockIdx.x, gridDim.x);
-    vseq = id / st_tiles;
-    tile = id - vseq * st_tiles;
+    int rest = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    tile = rest % st_tiles;
+    rest /= st_tiles;
+    split = rest % splits;
+    vseq = rest / splits;
   }
   const int seg = vseq % p.segs, bh = vseq / p.segs, kv_heads = p.heads / p.kv_group;
-  const int n_group = p.kv_group;  // complete sums over the query heads of a group
-  const int b = bh / kv_heads, hk = bh - b * kv_heads, h0 = hk * n_group;
+  // complete sums over the query heads of a group, or (sampled keys) the share of a range of one query head's queries
+  const int n_group = SAMPLED ? 1 : p.kv_group;
+  const int b = SAMPLED ? bh / p.heads : bh / kv_heads;
+  const int h0 = SAMPLED ? bh - b * p.heads : (bh - b * kv_heads) * p.kv_group, hk = h0 / p.kv_group;
 
   const int64_t q_row0 = p.q_seg_off + (int64_t)seg * p.seg_stride, k_row0 = p.k_seg_off + (int64_t)seg * p.seg_stride;
   const unsigned char* const q0 = (const unsigned char*)((const T*)p.q + b * p.q_sb + h0 * p.q_sh + q_row0 * p.q_sn);
@@ -85,6 +91,10 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
     y_first = block_id * p.block_tiles * 128;
     y_end = min(y_first + p.block_tiles * 128, p.n_q);
   }
+  if (SAMPLED) {
+    y_first = split * p.q_split;
+    y_end = min(y_first + p.q_split, p.n_q);
+  }
   const int ns = y_end > y_first ? (y_end - y_first + 31) / 32 : 0, n_t = ns * n_group;
 
   // the wave's keys
@@ -92,6 +102,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
   auto key_row = [&](uint32_t r) -> uint32_t {  // row of key r of the wave, clamped
     const int pos = min(st_lo + (int)r, st_total - 1);
     if (BLOCK) return *reinterpret_cast<const int*>(row_address(k_idx, pos, ki_rb, 0));
+    if (SAMPLED && p.sampled_idx) return ha_load_idx(p.sampled_idx, b * p.si_sb + hk * p.si_sh + pos, p.idx64);
     return pos;
   };
 
@@ -336,6 +347,36 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
   }
   const uint32_t stage = STAGE + wave * 8192;
   if (st_lo >= st_total) return;
+  if (SAMPLED) {
+    // this share's rows: [(batch, key head, segment)][share][slot], written whole
+    const int shares = p.kv_group * splits, share = (h0 - hk * p.kv_group) * splits + split;
+    const int64_t slot0 = (((((int64_t)b * kv_heads + hk) * p.segs + seg) * shares + share) * p.sample_size + st_lo) * WD;
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      float* const dst = (which == 0 ? p.dk32 : p.dv32) + slot0;
+#pragma unroll
+      for (uint32_t part = 0; part < 2; ++part) {  // 16 keys at a time
+        if (col >> 4 == part) {
+#pragma unroll
+          for (int d2 = 0; d2 < DB; ++d2)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const f32x16& a = which == 0 ? acc1[d2] : acc2[d2];
+              const uint32_t piece = (8 * d2 + 2 * g + hi) ^ (col & 15);
+              lds_put<f32x4>(stage + (col & 15) * (WD * 4) + piece * 16, f32x4{a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]});
+            }
+        }
+        wave_lds_order();
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+          const uint32_t r = j * 2 + hi;
+          *reinterpret_cast<f32x4*>(dst + (part * 16 + r) * WD + col * 4) = lds_get<f32x4>(stage + r * (WD * 4) + ((col ^ r) << 4));
+        }
+        wave_lds_order();
+      }
+    }
+    return;
+  }
   unsigned char* const dkb = (unsigned char*)((T*)p.dk + b * p.dk_sb + hk * p.dk_sh + k_row0 * p.dk_sn);
   unsigned char* const dvb = (unsigned char*)((T*)p.dv + b * p.dv_sb + hk * p.dv_sh + k_row0 * p.dv_sn);
   // turned around in LDS: 16 lanes write a whole row
@@ -385,6 +426,7 @@ int ha_launch_bwd_wide(const ha_attn_bwd_params& p, int pass, bool causal, int i
   auto typed = [&](auto t) {
     typedef decltype(t) T;
     if (pass == HA_BWD_DKV_BLOCK) launch(ha_attn_bwd_wide_kernel<T, HA_BWD_DKV_BLOCK, false>);
+    else if (pass == HA_BWD_DKV_SAMPLED) launch(ha_attn_bwd_wide_kernel<T, HA_BWD_DKV_SAMPLED, false>);
     else if (causal) launch(ha_attn_bwd_wide_kernel<T, HA_BWD_DKV_EXACT, true>);
     else launch(ha_attn_bwd_wide_kernel<T, HA_BWD_DKV_EXACT, false>);
   };

@@ -64,6 +64,41 @@ def test_blocks(ha, dtype, h, hk, n, block, sample, idx):  # noqa: F811
         _check(g, want, name, dtype)
 
 
+@pytest.mark.parametrize("dtype,h,hk,n,sample,smooth", [
+    (torch.float16, 130, 130, 384, 256, False),    # one share: the sums themselves
+    (torch.bfloat16, 33, 33, 2048, 256, True),     # ranges of a head's queries
+    (torch.float16, 44, 11, 1664, 512, False),     # and four heads; two tiles of sampled keys
+])
+def test_sampled_keys(ha, dtype, h, hk, n, sample, smooth):  # noqa: F811
+    """Sums of the sampled keys from shares in the workspace, and, in a workspace without room for them, by atomics; a row
+    listed twice."""
+    from hyperattention_amd import _lib, ops
+    q, do = (_randn((1, n, h, D), s, dtype).cuda() for s in (101, 102))
+    k, v = (_randn((1, n, hk, D), s, dtype).cuda() for s in (103, 104))
+    qi, ki = _orders(h, n, 105), _orders(hk, n, 106)
+    sl = torch.randint(0, n, (sample,), generator=_gen(107))
+    sl[sample - 1] = sl[3]
+    group = h // hk
+    ref = _oracle_grads(_grouped(lambda a, b, c: O.block_sampled_attention(a, b, c, qi, ki.repeat_interleave(group, 1), 256, sample,
+                                                                           None, smooth, sampled_idx=sl), group),
+                        *(x.transpose(1, 2).cpu() for x in (q, k, v, do)))
+    qi_g, ki_g = (x.cuda().int().transpose(1, 2) for x in (qi, ki))
+    o, lse = ops.hyper_attn_func(q, k, v, qi_g, ki_g, 256, sample, None, smooth, sampled_idx=sl.cuda())
+    a, _keep = ops._block_attn_args(q, k, v, o, lse, qi_g, ki_g, 256, sample, D ** -0.5, smooth, sl.cuda())
+    sums = (h * n * 8 + 255) // 256 * 256 + 2 * hk * sample * D * 4  # statistics, one row of dk and dv per slot
+    for room in (True, False):
+        grads = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        g, ws = ops._attn_grads(a.t, do, *grads, sample_size=sample)
+        assert g.workspace_bytes >= sums and (group == 1 or g.workspace_bytes > sums)
+        ws.fill_(255)  # NaN: nothing is read that has not been written
+        if not room:
+            g.workspace_bytes = sums
+        _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), ops._stream(q)))
+        torch.cuda.synchronize()
+        for got, want, name in zip(grads, ref, ("dq", "dk", "dv")):
+            _check(got.transpose(1, 2), want, f"{name}, room {room}", dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("exact", [False, True])
 def test_adds_to_what_is_there(ha, dtype, exact):  # noqa: F811
