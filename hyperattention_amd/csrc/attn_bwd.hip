@@ -61,6 +61,14 @@ __device__ __forceinline__ void interleave_groups() {
   }
 }
 
+// sum over the 16 lanes of a row of lanes
+__device__ __forceinline__ float row16_sum(float v) {
+  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));  // row_ror:8
+  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xf, 0xf, true));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x122, 0xf, 0xf, true));
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x121, 0xf, 0xf, true));
+}
+
 template <typename T, int D, int PASS, bool CAUSAL, int HALVES>
 __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || (PASS == HA_BWD_DQ_EXACT && HALVES == 1) ? 2 : 1)) void ha_attn_bwd_kernel(const ha_attn_bwd_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
@@ -97,7 +105,7 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   __shared__ __attribute__((aligned(16))) float delta_0[SN], delta_1[SN], delta_2[SN], delta_3[SN];
   auto lse_tile = [&](int i) -> float* { return i == 0 ? lse_0 : i == 1 ? lse_1 : i == 2 ? lse_2 : lse_3; };
   auto delta_tile = [&](int i) -> float* { return i == 0 ? delta_0 : i == 1 ? delta_1 : i == 2 ? delta_2 : delta_3; };
-  constexpr bool STAGE_X = KEY_ST || D <= 64;
+  constexpr bool STAGE_X = KEY_ST || D <= 64, STAGE_TURNS = !STAGE_X && HALVES == 1;
   // staging of the second stationary operand (prologue); with four tiles of 64 rows in the ring there is room in them
   __shared__ __attribute__((aligned(1024))) unsigned char lds_x2[STAGE_X && HALVES == 1 ? ST_ROWS * D * 2 : 16];
   __shared__ int lds_tiles[PASS == HA_BWD_DKV_BLOCK ? MAX_SMOOTH_TILES : 1];
