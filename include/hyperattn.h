@@ -200,7 +200,8 @@ int ha_flash_attn_fwd(const ha_attn_operands* t, int causal, void* stream);
  * Segments (segs, seg_stride_rows and the offsets) as in the forward; dout, dq follow q's segment
  * layout, dk, dv that of k, v.  Built for d == dv in {64, 128} (HA_ERR_UNSUPPORTED otherwise).
  * workspace: ha_attn_bwd_workspace_bytes(t, sample_size) bytes (sample_size = 0 for exact attention),
- * 256-byte aligned: two floats per query, and fp32 sums of the sampled keys, cleared by the call.
+ * 256-byte aligned: two floats per query, and fp32 sums of the sampled keys (at d = 128 shares of them, added up
+ * by the call; a workspace with room for the sums alone is accepted and takes atomics), overwritten by the call.
  */
 typedef struct {
   const void* dout;  /* (.., n_q, dv)                          */
