@@ -128,6 +128,8 @@ __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || 
   // slot freed by a short one stays empty until the ones queued before it are placed.  Few tiles (single_tiles) come one by
   // one, the ones of all sequences that stream the most rows first, at d = 64, two workgroups per CU, the second 256 reversed.
   constexpr bool PAIRED = CAUSAL && HALVES == 1 && (PASS == HA_BWD_DQ_EXACT || PASS == HA_BWD_DKV_EXACT);
+  // (dq at d = 128 gets no pairs: so many tiles go to the wide pass.  Compiled without the pair's second copy of the tile its
+  // loop spills: 24 heads of 2048 rows 67 -> 75 us.)
   const bool single = PAIRED && p.single_tiles;
   const int wg_per_seq = PAIRED && !single ? (st_tiles + 1) / 2 : st_tiles;
   // Steps split over waves: no pairs; the tiles of all sequences that stream the most rows come first (tile-major)
