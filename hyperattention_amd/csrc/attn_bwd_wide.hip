@@ -8,7 +8,7 @@
 //     dP of step t + 1, operands read 4 products ahead.  Its vector stage: P, dS of step t + 1 and the first operands.
 //     Waves 0-3 pass the step's one barrier after the vector stage, waves 4-7 after the matrix stage, which keeps the two
 //     waves of a SIMD (w, w + 4) in different stages.
-//   - Registers: 128 accumulators, 64 for the keys' k and v, 64 for S, dP, P, dS, 32 operands: 256, no spills.
+//   - Registers: 128 accumulators, 64 for the keys' k and v, 64 for S, dP, P, dS, 32 operands: 256 (the sampled pass spills one).
 //   - LDS, 136 KB: four tiles of 32 q and dO rows, filled three steps ahead by loads that bypass the registers, four
 //     steps' statistics, eight steps' row numbers.  The compiler must not see those loads (it would wait for all of them at
 //     every LDS access): assembly, counted by hand, the step's end waits for all but the last tile's two.
@@ -347,6 +347,19 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
   }
   const uint32_t stage = STAGE + wave * 8192;
   if (st_lo >= st_total) return;
+  // fp32 sums through the stage, 16 of the wave's keys at a time: rows [16][WD], 16-byte pieces XOR-ed with the row number
+  auto turn = [&](const f32x16 (&acc)[DB], uint32_t part) {
+    if (col >> 4 == part) {
+#pragma unroll
+      for (int d2 = 0; d2 < DB; ++d2)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          lds_put<f32x4>(stage + (col & 15) * (WD * 4) + (((8 * d2 + 2 * g + hi) ^ (col & 15)) << 4),
+                         f32x4{acc[d2][g * 4], acc[d2][g * 4 + 1], acc[d2][g * 4 + 2], acc[d2][g * 4 + 3]});
+    }
+    wave_lds_order();
+  };
+  auto turned = [&](uint32_t r, uint32_t piece) { return lds_get<f32x4>(stage + r * (WD * 4) + ((piece ^ r) << 4)); };
   if (SAMPLED) {
     // this share's rows: [(batch, key head, segment)][share][slot], written whole
     const int shares = p.kv_group * splits, share = (h0 - hk * p.kv_group) * splits + split;
@@ -355,22 +368,12 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
     for (int which = 0; which < 2; ++which) {
       float* const dst = (which == 0 ? p.dk32 : p.dv32) + slot0;
 #pragma unroll
-      for (uint32_t part = 0; part < 2; ++part) {  // 16 keys at a time
-        if (col >> 4 == part) {
-#pragma unroll
-          for (int d2 = 0; d2 < DB; ++d2)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const f32x16& a = which == 0 ? acc1[d2] : acc2[d2];
-              const uint32_t piece = (8 * d2 + 2 * g + hi) ^ (col & 15);
-              lds_put<f32x4>(stage + (col & 15) * (WD * 4) + piece * 16, f32x4{a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]});
-            }
-        }
-        wave_lds_order();
+      for (uint32_t part = 0; part < 2; ++part) {
+        turn(which == 0 ? acc1 : acc2, part);
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
           const uint32_t r = j * 2 + hi;
-          *reinterpret_cast<f32x4*>(dst + (part * 16 + r) * WD + col * 4) = lds_get<f32x4>(stage + r * (WD * 4) + ((col ^ r) << 4));
+          *reinterpret_cast<f32x4*>(dst + (part * 16 + r) * WD + col * 4) = turned(r, col);
         }
         wave_lds_order();
       }
@@ -384,10 +387,27 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
 #pragma unroll
   for (uint32_t j = 0; j < 8; ++j) rows[j] = key_row(j * 4 + lane / 16);
   auto store = [&](const f32x16 (&acc)[DB], unsigned char* base, int64_t row_bytes) {
-    vec8 old[8];
+    // What is there and the fp32 sum are rounded once, together, as in the passes of 128 keys (rounded to 16 bits for the
+    // turn first, 320 heads of 256 causal rows take 95 us instead of 97 for all gradients, 256 of 1280 rows 753 and 759).
     if (p.accumulate) {
+      vec8 old[8];
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) old[j] = *reinterpret_cast<const vec8*>(base + rows[j] * row_bytes + (lane & 15) * 16);
+#pragma unroll
+      for (uint32_t part = 0; part < 2; ++part) {
+        turn(acc, part);
+#pragma unroll
+        for (uint32_t j = part * 4; j < part * 4 + 4; ++j) {
+          const uint32_t r = j * 4 + lane / 16;
+          const f32x4 lo = turned(r & 15, 2 * (lane & 15)), up = turned(r & 15, 2 * (lane & 15) + 1);
+          vec8 o;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = (T)((e < 4 ? lo[e & 3] : up[e & 3]) + (float)old[j][e]);
+          if (st_lo + (int)r < st_total) *reinterpret_cast<vec8*>(base + rows[j] * row_bytes + (lane & 15) * 16) = o;
+        }
+        wave_lds_order();
+      }
+      return;
     }
 #pragma unroll
     for (int d2 = 0; d2 < DB; ++d2)
@@ -402,12 +422,8 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) {
       const uint32_t r = j * 4 + lane / 16;
-      vec8 o = lds_get<vec8>(stage + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
-      if (p.accumulate) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (T)((float)o[e] + (float)old[j][e]);
-      }
-      if (st_lo + (int)r < st_total) *reinterpret_cast<vec8*>(base + rows[j] * row_bytes + (lane & 15) * 16) = o;
+      if (st_lo + (int)r < st_total)
+        *reinterpret_cast<vec8*>(base + rows[j] * row_bytes + (lane & 15) * 16) = lds_get<vec8>(stage + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
     }
     wave_lds_order();
   };

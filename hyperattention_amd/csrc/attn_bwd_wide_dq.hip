@@ -273,10 +273,38 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_dq_kernel(co
   uint32_t rows[8];
 #pragma unroll
   for (uint32_t j = 0; j < 8; ++j) rows[j] = query_row(j * 4 + lane / 16);
-  vec8 old[8];
   if (p.accumulate) {
+    // what is there and the fp32 sum are rounded once, together: 16 rows at a time, [16][WD] fp32, 16-byte pieces XOR-ed
+    // with the row number
+    vec8 old[8];
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) old[j] = *reinterpret_cast<const vec8*>(dqb + rows[j] * dq_rb + (lane & 15) * 16);
+#pragma unroll
+    for (uint32_t part = 0; part < 2; ++part) {
+      if (col >> 4 == part) {
+#pragma unroll
+        for (int d2 = 0; d2 < DB; ++d2)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            f32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = acc[d2][g * 4 + e] * p.scale;
+            lds_put<f32x4>(stage + (col & 15) * (WD * 4) + (((8 * d2 + 2 * g + hi) ^ (col & 15)) << 4), o);
+          }
+      }
+      wave_lds_order();
+#pragma unroll
+      for (uint32_t j = part * 4; j < part * 4 + 4; ++j) {
+        const uint32_t r = j * 4 + lane / 16, at = stage + (r & 15) * (WD * 4), piece = 2 * (lane & 15);
+        const f32x4 lo = lds_get<f32x4>(at + ((piece ^ (r & 15)) << 4)), up = lds_get<f32x4>(at + (((piece + 1) ^ (r & 15)) << 4));
+        vec8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (T)((e < 4 ? lo[e & 3] : up[e & 3]) + (float)old[j][e]);
+        if (st_lo + (int)r < p.n_q) *reinterpret_cast<vec8*>(dqb + rows[j] * dq_rb + (lane & 15) * 16) = o;
+      }
+      wave_lds_order();
+    }
+    return;
   }
 #pragma unroll
   for (int d2 = 0; d2 < DB; ++d2)
@@ -291,12 +319,8 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_dq_kernel(co
 #pragma unroll
   for (uint32_t j = 0; j < 8; ++j) {
     const uint32_t r = j * 4 + lane / 16;
-    vec8 o = lds_get<vec8>(stage + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
-    if (p.accumulate) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (T)((float)o[e] + (float)old[j][e]);
-    }
-    if (st_lo + (int)r < p.n_q) *reinterpret_cast<vec8*>(dqb + rows[j] * dq_rb + (lane & 15) * 16) = o;
+    if (st_lo + (int)r < p.n_q)
+      *reinterpret_cast<vec8*>(dqb + rows[j] * dq_rb + (lane & 15) * 16) = lds_get<vec8>(stage + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
   }
 }
 

@@ -135,3 +135,38 @@ def test_adds_to_what_is_there(ha, dtype, exact):  # noqa: F811
         err = (back(got).double() - total).norm() / total.norm()
         assert err <= unit + (3e-3 if dtype == torch.float16 else 8e-3), f"{name}: {err:.2e}"
         assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("h,n,causal", [(300, 200, False), (320, 200, True), (4, 200, True)])  # the last not in 256 rows
+@pytest.mark.parametrize("dead", ["q", "k"])
+def test_a_sum_added_to_what_is_there_is_rounded_once(ha, dtype, h, n, causal, dead):  # noqa: F811
+    """Gradients of exact attention added to.  The inputs make every fp32 sum exact and not representable in 16 bits: with
+    q or k zero and log-sum-exps of log(256) all weights are 1/256, O is zero (D = 0), v has one column of -1, 0, 1, and dO
+    and the other of q and k are whole numbers whose products stay below 2^24.  So the one rounding, of the sum with what
+    is there, is known to the bit."""
+    from hyperattention_amd import _lib, ops
+    gen, top = _gen(81), 1000 if dtype == torch.float16 else 100
+    whole = lambda limit: torch.randint(-limit, limit + 1, (1, n, h, D), generator=gen).double()  # noqa: E731
+    q, k, do, v = whole(63), whole(63), whole(top), whole(1)
+    v[..., 1:] = 0
+    (q if dead == "q" else k).zero_()
+    heads = lambda x: x.transpose(1, 2)  # noqa: E731
+    weight = torch.ones(n, n, dtype=torch.float64) / 256
+    if causal:
+        weight = weight.tril()
+    scale = 0.125
+    ds = weight * (heads(do) @ heads(v).transpose(-1, -2).contiguous()) * scale
+    sums = [ds @ heads(k), ds.transpose(-1, -2).contiguous() @ heads(q), weight.T.contiguous() @ heads(do)]
+    there = [(torch.randn((1, n, h, D), generator=gen) * max(x.std().item(), 1.)).to(dtype) for x in sums]
+    q_g, k_g, v_g, do_g = (x.to(dtype).cuda() for x in (q, k, v, do))
+    lse = torch.full((1, h, n), 256., device="cuda").log()
+    out = torch.zeros_like(q_g)
+    t = ops._operands(q_g, k_g, v_g, out, lse, scale, layout_bnhd=True, lse_row_stride=n)
+    grads = [x.cuda() for x in there]
+    g, ws = ops._attn_grads(t, do_g, *grads, accumulate=True)
+    _lib.check(_lib.lib().ha_flash_attn_bwd(ctypes.byref(t), int(causal), ctypes.byref(g), ops._stream(q_g)))
+    torch.cuda.synchronize()
+    for got, was, want, name in zip(grads, there, sums, ("dq", "dk", "dv")):
+        total = (was.float() + heads(want).float()).to(dtype)
+        assert torch.equal(got.cpu(), total), f"{name}: {(got.cpu() != total).float().mean().item():.3f} of the elements differ"
