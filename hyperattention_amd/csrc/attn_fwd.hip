@@ -39,7 +39,14 @@
 // (or is not a number: nothing seen yet) is the row maximum computed, m raised, the accumulators
 // rescaled and the half-step redone; below that bound every value is finite in fp16 and the result
 // does not depend on m beyond rounding.  m only ever grows, and starts from the true maximum of the
-// first keys or from the log-sum-exp of the partial result that is being resumed.
+// first keys or from the log-sum-exp of the partial result that is being resumed.  What rounding it depends on: the
+// key whose score is m has a weight of exactly 1, and the split kernel (attn_fwd_split.inc) has four such keys per row.  Where
+// single causal tiles of this kernel take its place, m follows the row maximum in a sequence's first tile (p.follow_max),
+// whose rows of few keys are most of the error.  Error against float64 over that of the split kernel, without | with, 16-bit
+// types, N(0,1) and clustered data: d = 64, 100 heads of 600 rows to 32 of 4096 1.015 to 1.024 | 0.992 to 0.997, d = 128, 48 of
+// 685 to 16 of 4096 1.010 to 1.024 | 0.994 to 1.000.  It costs nothing where a launch has longer tiles than CUs to hide the
+// first ones behind (48 of 2048 rows 43 us, d = 128 44 of 1024 32) and up to 3 us elsewhere (d = 64 130 of 1024 35.3 -> 37.7,
+// 100 of 700 21.2 -> 23.8; the split kernel 59 and 27).
 #include "ha_common.h"
 #include "attn_tiles.h"
 #include "attn_fwd.h"
@@ -119,7 +126,7 @@ __device__ __forceinline__ void half_step_p(const f32x16 (&s_use)[NB], const flo
 template <typename T, int NB, int H>
 __device__ __forceinline__ void half_step_rescale(const f32x16 (&s_use)[NB], float scale_log2,
                                                   float (&alpha)[NB], float (&m_run)[NB], float (&l_run)[NB],
-                                                  typename ElemTraits<T>::vec8 (&pn)[NB], float (&sum)[NB]) {
+                                                  typename ElemTraits<T>::vec8 (&pn)[NB], float (&sum)[NB], bool follow) {
   float m_use[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
@@ -128,6 +135,10 @@ __device__ __forceinline__ void half_step_rescale(const f32x16 (&s_use)[NB], flo
     float v = s_use[nb][H * 8];
 #pragma unroll
     for (int e = 1; e < 8; ++e) v = fmaxf(v, s_use[nb][H * 8 + e]);
+    if (H == 0 && follow) {  // the whole step's: its second half goes on under the same exponents
+#pragma unroll
+      for (int e = 8; e < 16; ++e) v = fmaxf(v, s_use[nb][e]);
+    }
     v = ha_max_xor32(v) * scale_log2;
     const float m_new = fmaxf(m_run[nb], v);
     // 2^(old - new) <= 1; nothing is accumulated yet under the floor exponent of a fresh row
@@ -144,6 +155,7 @@ __device__ __forceinline__ void half_step_rescale(const f32x16 (&s_use)[NB], flo
 //   MFMAs : P.V of the previous half-step (operands vf, pb, both in registers) and this half's share
 //           (k-steps H*KSTEPS/2 ..) of the next step's S^T, K rows k_row_off.. of k_tile
 //   VALU  : P of this half-step from s_use -> pb (for the next block) and the row sums
+//   follow: the reference exponents follow the rows' maxima, raised at every step of 32 keys
 //   LDS   : V^T of this half-step's keys (v_key_off.. of v_tile) -> vf (for the next block)
 template <typename T, int D, int H, int DC>
 __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB], f32x16 (&s_fill)[WaveShape<D>::NB],
@@ -153,7 +165,8 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
                                           f32x16 (&acc)[DC / 32][WaveShape<D>::NB], float (&m_run)[WaveShape<D>::NB],
                                           float (&l_run)[WaveShape<D>::NB],
                                           typename ElemTraits<T>::vec8 (&pb)[WaveShape<D>::NB],
-                                          typename ElemTraits<T>::vec8 (&vf)[DC / 32], float scale_log2) {
+                                          typename ElemTraits<T>::vec8 (&vf)[DC / 32], float scale_log2,
+                                          bool follow = false) {
   typedef typename ElemTraits<T>::vec8 vec8;
   constexpr int NB = WaveShape<D>::NB;
   constexpr int KH = DC / 32;  // k-steps of this half
@@ -204,10 +217,10 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
   float total = sum[0];
 #pragma unroll
   for (int nb = 1; nb < NB; ++nb) total += sum[nb];
-  const bool redo = !(total < HALF_SUM_LIMIT);
+  const bool redo = (H == 0 && follow) || !(total < HALF_SUM_LIMIT);
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) != 0, false)) {
     float alpha[NB];
-    half_step_rescale<T, NB, H>(s_use, scale_log2, alpha, m_run, l_run, pn, sum);
+    half_step_rescale<T, NB, H>(s_use, scale_log2, alpha, m_run, l_run, pn, sum, follow);
     // the accumulators hold everything up to the previous half-step (its P.V was issued above; the
     // P.V of this half-step is added by the next block, under the new exponents)
 #pragma unroll
@@ -476,10 +489,10 @@ static ha_divisor make_divisor(int64_t y) {
 // better one at all but 10 of them, within 10 % at all.  Times whole | split in us, d = 64 causal: 24 heads of 1000
 // rows 31 | 13, of 2048 39 | 28, of 4096 72 | 72; 48 of 2048 41 | 45, of 4096 116 | 143; without mask 16 of 4096 rows
 // 75 | 86; d = 128, 12 heads of 2048 rows, blocks and samples of 256: 20 | 26.
-static bool single_tiles(const ha_attn_kernel_params& p, int width);
-static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
-  const char* env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
-  if (env) return atoi(env) != 0;
+struct LaunchTimes {
+  double whole, single, split;  // the 256-query kernel (exact causal: pairs of tiles), its single tiles, the split kernel
+};
+static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   struct Fit {
     double step, pair, start, crowd, second, share, rest;    // 256-query kernel
     double split_step, split_start, set_up, hidden;          // split kernel
@@ -497,21 +510,22 @@ static bool use_split_keys(const ha_attn_kernel_params& p, int width, bool gathe
   if (per_cu <= 1) rounds = 1 + f.crowd * per_cu;
   else if (width == 64 || paired) rounds = std::max(f.second, f.share * per_cu + f.rest);
   else rounds = f.second * std::ceil(per_cu);
-  double whole = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
-  if (paired && single_tiles(p, width)) {
+  LaunchTimes t;
+  t.whole = t.single = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
+  if (paired) {
     // one tile per workgroup, longest first: the longest chain, slowed by its neighbours, or a CU's share of all
     const double longest = 4. * tiles, share = vheads * 2. * tiles * (tiles + 1) / cus, wgs = vheads * tiles / cus;
     const double crowd = width == 64 ? 0.1 * share : 0.3 * std::min(longest, share);
-    whole = f.start + std::max(f.step * (longest + crowd), (width == 64 ? 0.97 : 1.9) * share + 2. * wgs);
-    if (width == 128) whole *= 0.93;  // the other estimate is that much too low beside this one (48 heads of 685 rows: 24 us | split 30)
+    t.single = f.start + std::max(f.step * (longest + crowd), (width == 64 ? 0.97 : 1.9) * share + 2. * wgs);
+    if (width == 128) t.single *= 0.93;  // the other estimate is that much too low beside this one (48 heads of 685 rows: 24 us | split 30)
   }
 
   const double chain = std::ceil(keys / 128.), split_per_cu = vheads * split_tiles / cus;
   double all;
   if (paired) all = split_per_cu * (chain / 2 + 0.5 + f.set_up) - f.hidden * chain;
   else all = (width == 64 ? split_per_cu : std::ceil(split_per_cu)) * (chain + f.set_up);
-  const double split = f.split_start + f.split_step * std::max(chain + f.set_up, all);
-  return split < whole;
+  t.split = f.split_start + f.split_step * std::max(chain + f.set_up, all);
+  return t;
 }
 
 // Whether exact causal attention takes one query tile per workgroup, longest first, instead of a pair of tiles.  Pairs
@@ -548,8 +562,10 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   p.tiles_per_wg = 1;
   const char* stream_env = getenv("HA_STREAM_TILES");  // measurement aid: force the run length (1: off)
   const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0;
+  const LaunchTimes t = launch_times(p, width, gather, causal);
+  const char* split_env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
   // (a forced run length asks for the 256-query kernels)
-  p.split_keys = !reweight && !(gather && stream_env) && use_split_keys(p, width, gather, causal);
+  p.split_keys = !reweight && !(gather && stream_env) && (split_env ? atoi(split_env) != 0 : t.split < (single ? t.single : t.whole));
   if (p.split_keys) qtiles = (p.n_q + 63) / 64;
   else if (gather && !reweight && p.qk_pieces == width / 8 && p.v_pieces == width / 8 && p.n_q % WG_QUERIES == 0 && qtiles >= 2 &&
       p.sample_chunks % 2 == 0 && p.n_k % (p.block_tiles * 128) == 0 && 2 * p.block_tiles + p.sample_chunks >= 4 &&
@@ -564,6 +580,7 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
   if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
   if (single && !p.split_keys) p.tiles_per_wg = 0;
+  p.follow_max = single && t.split < t.whole;
   p.div_qtiles = make_divisor(p.split_keys == 2 || p.tiles_per_wg == 0 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);
