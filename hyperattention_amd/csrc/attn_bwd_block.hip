@@ -27,7 +27,7 @@ namespace {
 constexpr int FUSED_WAVES = 8, FUSED_THREADS = 64 * FUSED_WAVES;
 constexpr int FUSED_ROWS = 256;  // queries, and keys of a phase, per workgroup
 constexpr int FD = 64;           // head dim
-constexpr int FUSED_MAX_SAMPLES = 1024;  // their row numbers are kept in LDS
+constexpr int FUSED_MAX_SAMPLES = 512;  // their row numbers are kept in LDS
 constexpr int STEPS = FUSED_ROWS / 32;
 
 template <typename T>
@@ -533,22 +533,29 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 }  // namespace
 
 // What the registers and LDS are laid out for: 256 keys and queries per block; with grouped queries a block's dk, dv would
-// have to be kept over the query heads beside the sampled keys' sums.  At every size measured (1 to 32 heads of 2048 to 65536
-// rows) the one kernel is the faster one or equal, but for three workgroups' worth of blocks per CU (24 x 8192: 178 against 168
-// us): 1 x 4096 37 against 45 us, 12 x 4096 64 against 74, 24 x 4096 85 against 106, 32 x 32768 578 against 775.
+// have to be kept over the query heads beside the sampled keys' sums.  How many sampled keys: two blocks in a row share the
+// sums of one phase, those of the others are added to memory by every block, while the passes add them once per range of
+// queries.  Three passes | this kernel, the whole call in us where it writes the gradients, 38 launches of 64 to 6144 blocks
+// (0.25 to 24 per CU): up to 256 samples it is the faster one at all (4 heads x 4096 rows 44 | 40, 24 x 4096 98 | 79, 24 x 8192
+// 156 | 131, 32 x 16384 361 | 267, 24 x 65536 1038 | 744; without samples 20.4 | 19.3 to 692 | 424; where it adds to them
+// too, but for 16 x 2048 without samples, 22.8 | 23.2); 512: 8 x 2048 51 | 54, 24 x 2048 82 | 79, 10 x 16384 172 | 178, 130 x 2048
+// 294 | 306, then within 5 % to both sides up to 1600 blocks, 28 x 16384 (1792) 453 | 382, 24 x 65536 1402 | 1118; 1024 never:
+// 8 x 2048 66 | 82, 24 x 65536 2027 | 2247.
 bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d) {
+  const int64_t blocks = (int64_t)p.batch * p.heads * p.segs * ((p.n_q + FUSED_ROWS - 1) / FUSED_ROWS);
   return d == FD && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
-         p.sample_size <= FUSED_MAX_SAMPLES;
+         (p.sample_size <= FUSED_ROWS || (p.sample_size <= FUSED_MAX_SAMPLES && blocks >= 1792));
 }
 
 int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream) {
   const int64_t vseqs = (int64_t)p.batch * p.heads * p.segs, blocks = (p.n_q + FUSED_ROWS - 1) / FUSED_ROWS;
   // Blocks per workgroup, one workgroup per CU: the run with the least time by the rounds of workgroups; starting and ending
-  // one takes as long as two fifths of a block (41 us each in a full launch)
+  // one takes as long as two thirds of a block.  Within 0.2 % of the best run of 1 to 8, 10 and 12 at every one of those
+  // launches, samples or not; as two fifths of a block it chose three rounds of one block for 24 x 8192, 175 us.
   int64_t best = INT64_MAX;
   p.run_blocks = 1;
-  for (int64_t r = 1; r <= std::min<int64_t>(blocks, 32); ++r) {
-    const int64_t cost = (vseqs * ((blocks + r - 1) / r) + 255) / 256 * (5 * r + 2);
+  for (int64_t r = 1; r <= std::min<int64_t>(blocks, 12); ++r) {
+    const int64_t cost = (vseqs * ((blocks + r - 1) / r) + 255) / 256 * (3 * r + 2);
     if (cost < best) {
       best = cost;
       p.run_blocks = (int)r;

@@ -17,8 +17,8 @@ pytestmark = pytest.mark.gpu
     (torch.float16, 1, 128, 0, torch.int64),       # half a block, nothing else
     (torch.bfloat16, 2, 256, 256, torch.int32),    # one block
     (torch.float16, 1, 384, 256, torch.int32),     # the last block is half
-    (torch.bfloat16, 3, 1152, 512, torch.int64),   # two phases of sampled keys
-    (torch.float16, 1, 1024, 1024, torch.int32),   # the most sampled keys
+    (torch.bfloat16, 3, 1152, 512, torch.int64),   # two phases of sampled keys: few blocks take the three passes
+    (torch.float16, 1, 1024, 1024, torch.int32),   # and so does what is above
     (torch.float16, 5, 16512, 256, torch.int32),   # 65 blocks in runs of two: the last run has one, of half the rows
 ])
 def test_blocks_and_samples(ha, dtype, h, n, sample, idx):  # noqa: F811
@@ -29,6 +29,22 @@ def test_blocks_and_samples(ha, dtype, h, n, sample, idx):  # noqa: F811
     _, _, *got = _gpu_grads(lambda a, b, c: ha.hyper_attn_func(a, b, c, qi_g, ki_g, 256, sample, None, False), q, k, v, do)
     for g, want, name in zip(got, ref, ("dq", "dk", "dv")):
         _check(g, want, f"{name}, {h} x {n}, {sample} samples", dtype)
+
+
+@pytest.mark.parametrize("dtype,h,n,idx", [
+    (torch.float16, 896, 512, torch.int32),   # 1792 blocks, the fewest with two phases of sampled keys; runs of two
+    (torch.bfloat16, 600, 640, torch.int64),  # runs of three: the last block has half the rows
+])
+def test_two_phases_of_samples(ha, dtype, h, n, idx):  # noqa: F811
+    """Many heads, four different ones in turn."""
+    q, k, v, do = (_randn((1, 4, n, 64), s, dtype) for s in (31, 32, 33, 34))
+    qi, ki = _perms(1, 4, n, 35), _perms(1, 4, n, 36)
+    ref = _oracle_grads(lambda a, b, c: O.block_sampled_attention(a, b, c, qi, ki, 256, 512, None, False), q, k, v, do)
+    many = lambda x: x.repeat(1, h // 4, *[1] * (x.dim() - 2))  # noqa: E731
+    qi_g, ki_g = (many(x).cuda().to(idx).transpose(1, 2) for x in (qi, ki))
+    _, _, *got = _gpu_grads(lambda a, b, c: ha.hyper_attn_func(a, b, c, qi_g, ki_g, 256, 512, None, False), *(many(x) for x in (q, k, v, do)))
+    for g, want, name in zip(got, ref, ("dq", "dk", "dv")):
+        _check(g, many(want), f"{name}, {h} x {n}", dtype)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
