@@ -1,6 +1,6 @@
 """dk, dv with 256 keys and dq with 256 queries per workgroup at head dim 128 (csrc/attn_bwd_wide.hip,
 attn_bwd_wide_dq.hip): launches that fill the chip with few rows
-per head, at the edges of its tiles of 256 keys and 32 queries.  The shapes are ones that its dispatch rules take."""
+per head, at the edges of its tiles of 256 keys and 32 queries.  The shapes are ones that its dispatch rules take, or say so."""
 import ctypes
 
 import pytest
@@ -25,7 +25,10 @@ def _grouped(fn, group):
 
 
 @pytest.mark.parametrize("dtype,h,hk,nq,nk,causal", [
-    (torch.float16, 300, 300, 128, 128, True),     # half the waves have no keys
+    (torch.bfloat16, 640, 640, 128, 128, True),    # half the waves have no queries; dk, dv stay with the narrow pass
+    (torch.float16, 640, 640, 64, 128, True),      # no queries, no keys, keys that nothing attends
+    (torch.float16, 640, 640, 40, 33, True),       # two steps of dq, six waves without queries
+    (torch.float16, 300, 300, 128, 128, True),     # too few for the wide passes
     (torch.bfloat16, 300, 300, 192, 192, False),
     (torch.float16, 300, 300, 77, 500, False),     # ragged on both sides
     (torch.bfloat16, 200, 200, 1001, 250, False),
@@ -33,7 +36,7 @@ def _grouped(fn, group):
     (torch.bfloat16, 300, 300, 300, 500, True),    # keys that nothing attends
     (torch.float16, 300, 300, 300, 256, True),     # queries after the last key
     (torch.bfloat16, 600, 200, 20, 260, False),    # one step per query head
-    (torch.float16, 130, 130, 40, 33, True),       # two steps, half of the waves without queries
+    (torch.float16, 130, 130, 40, 33, True),       # nor these
 ])
 def test_exact(ha, dtype, h, hk, nq, nk, causal):  # noqa: F811
     q, do = (_randn((1, h, nq, D), s, dtype) for s in (51, 52))
@@ -49,7 +52,8 @@ def test_exact(ha, dtype, h, hk, nq, nk, causal):  # noqa: F811
     (torch.bfloat16, 65, 65, 384, 256, 128, torch.int32),    # the last block is half
     (torch.float16, 44, 44, 640, 512, 256, torch.int32),     # two tiles of a block, a short block
     (torch.bfloat16, 132, 44, 640, 256, 0, torch.int64),     # three query heads on each key head
-    (torch.float16, 44, 22, 1280, 1024, 0, torch.int32),     # four tiles of a block, two of a short one
+    (torch.float16, 52, 26, 1280, 1024, 0, torch.int32),     # four tiles of a block, two of a short one
+    (torch.float16, 44, 22, 1280, 1024, 0, torch.int32),     # too few for the wide pass
 ])
 def test_blocks(ha, dtype, h, hk, n, block, sample, idx):  # noqa: F811
     q, do = (_randn((1, h, n, D), s, dtype) for s in (61, 62))
