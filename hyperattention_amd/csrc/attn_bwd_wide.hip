@@ -8,7 +8,7 @@
 //     dP of step t + 1, operands read 4 products ahead.  Its vector stage: P, dS of step t + 1 and the first operands.
 //     Waves 0-3 pass the step's one barrier after the vector stage, waves 4-7 after the matrix stage, which keeps the two
 //     waves of a SIMD (w, w + 4) in different stages.
-//   - Registers: 128 accumulators, 64 for the keys' k and v, 64 for S, dP, P, dS, 32 operands: 256 (the sampled pass spills one).
+//   - Registers: 128 accumulators, 64 for the keys' k and v, 64 for S, dP, P, dS, 32 operands: 256 (the sampled pass spills one, outside its loop).
 //   - LDS, 136 KB: four tiles of 32 q and dO rows, filled three steps ahead by loads that bypass the registers, four
 //     steps' statistics, eight steps' row numbers.  The compiler must not see those loads (it would wait for all of them at
 //     every LDS access): assembly, counted by hand, the step's end waits for all but the last tile's two.
