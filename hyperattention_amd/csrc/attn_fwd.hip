@@ -41,12 +41,12 @@
 // does not depend on m beyond rounding.  m only ever grows, and starts from the true maximum of the
 // first keys or from the log-sum-exp of the partial result that is being resumed.  What rounding it depends on: the
 // key whose score is m has a weight of exactly 1, and the split kernel (attn_fwd_split.inc) has four such keys per row.  Where
-// single causal tiles of this kernel take its place, m follows the row maximum in a sequence's first tile (p.follow_max),
+// single causal tiles of this kernel take its place, m follows the row maximum in a sequence's first tile (FOLLOW),
 // whose rows of few keys are most of the error.  Error against float64 over that of the split kernel, without | with, 16-bit
 // types, N(0,1) and clustered data: d = 64, 100 heads of 600 rows to 32 of 4096 1.015 to 1.024 | 0.992 to 0.997, d = 128, 48 of
-// 685 to 16 of 4096 1.010 to 1.024 | 0.994 to 1.000.  It costs nothing where a launch has longer tiles than CUs to hide the
-// first ones behind (48 of 2048 rows 43 us, d = 128 44 of 1024 32) and up to 3 us elsewhere (d = 64 130 of 1024 35.3 -> 37.7,
-// 100 of 700 21.2 -> 23.8; the split kernel 59 and 27).
+// 685 to 16 of 4096 1.010 to 1.024 | 0.994 to 1.000.  It costs nothing where the first tiles run beside longer ones (48 of
+// 2048 rows 44 us, d = 128 44 of 1024 32) and up to 5 us where they are a round of their own (d = 64 130 of 1024 35.5 -> 38.1,
+// 100 of 700 21.0 -> 23.3, d = 128 96 of 520 26.4 -> 31.0; the split kernel 59, 27 and 37; 150 of 300 16.3 -> 18.9, split 17.0).
 #include "ha_common.h"
 #include "attn_tiles.h"
 #include "attn_fwd.h"
@@ -300,8 +300,10 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
   return r;
 }
 
+// FOLLOW (exact causal kernel, single tiles): the reference exponents of a sequence's first tile follow the row maxima.  An
+// instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
 template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D>
+          int DC = D, bool FOLLOW = false>
 __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   // head dim 64, where a CU holds two workgroups, the second 256 in reversed order (see ha_attn_fwd_split_kernel).
   constexpr bool PAIRED = CAUSAL && !GATHER;
   const int wg_per_seq = PAIRED ? (qtiles + 1) / 2 : qtiles;  // what p.div_qtiles divides by
-  const bool single = PAIRED && p.tiles_per_wg == 0;
+  const bool single = PAIRED && (FOLLOW || p.tiles_per_wg == 0);
   int hg, vseq, slot;
   if (single) {
     const int second = min((int)gridDim.x, 512);
@@ -388,9 +390,11 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
       const int qt = t_long;
 #include "attn_fwd_tile.inc"
     }
-    if (!single && slot != t_long && slot * WG_QUERIES < n_q) {  // an odd number of tiles: the middle one has no partner
-      const int qt = slot;
+    if constexpr (!FOLLOW) {
+      if (!single && slot != t_long && slot * WG_QUERIES < n_q) {  // an odd number of tiles: the middle one has no partner
+        const int qt = slot;
 #include "attn_fwd_tile.inc"
+      }
     }
   }
 }
@@ -401,9 +405,9 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
 namespace {
 
 template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D>
+          int DC = D, bool FOLLOW = false>
 int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT, DC>), dim3(grid),
+  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT, DC, FOLLOW>), dim3(grid),
                      dim3(WaveShape<D>::THREADS), 0, stream, p);
   return ha_launch_status(what);
 }
@@ -429,6 +433,7 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
   // the plain instance: d = 96, 16 heads of 32768 rows 205 -> 182 us, d = 40 98 -> 88
   if (gather && plain) return launch_one<T, D, true, false, true, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
   if (gather) return launch_one<T, D, true, false, false, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
+  if (causal && p.follow_max) return launch_one<T, D, false, true, false, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
   return launch_one<T, D, false, false, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
 }
@@ -460,6 +465,7 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
     if (plain) return launch_one<T, D, true, false, true>(p, grid, stream, "ha_block_attn_fwd");
     return launch_one<T, D, true, false>(p, grid, stream, "ha_block_attn_fwd");
   }
+  if (causal && p.follow_max) return launch_one<T, D, false, true, false, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
   return launch_one<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
 }
@@ -580,7 +586,7 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
   if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
   if (single && !p.split_keys) p.tiles_per_wg = 0;
-  p.follow_max = single && t.split < t.whole;
+  p.follow_max = single && !p.split_keys && t.split < t.whole;
   p.div_qtiles = make_divisor(p.split_keys == 2 || p.tiles_per_wg == 0 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);
