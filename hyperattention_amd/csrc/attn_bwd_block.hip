@@ -4,8 +4,8 @@
 // The passes gather a level's rows three times (4.0 GB at 24 heads of 65536 rows with gradients added to; dq 447 us, dk/dv of
 // the blocks 403, of the sampled keys 229) and compute the scores twice (7 products per pair).  Here a workgroup gathers the
 // q, k, v, dO, O rows of a block of 256 queries and 256 keys once, computes every score once (5 products) and leaves dq, dk,
-// dv of the block and adds to the sampled keys' sums: 2.9 GB, 875 us in the same launch (without adding, 24 heads of 16384:
-// 285 -> 250 us).  What bounds it now: the board's power limit (1.9 to 2.1 GHz); of a block's 73k cycles 50k are the steps.
+// dv of the block and adds to the sampled keys' sums: 2.9 GB, 810 to 826 us in the same launch (without adding, 24 heads
+// of 16384, the whole call: 269 -> 223 us).  What bounds it now: the board's power limit (2.1 GHz); of a block's 73k cycles 50k are the steps.
 //
 // A workgroup: 8 waves, a run of consecutive blocks of one (head, segment).  A block has a phase for its own keys and one
 // per 256 sampled keys.  In a phase a wave keeps 32 keys (k, v rows as MFMA B operands, sums of dK^T, dV^T in registers) and

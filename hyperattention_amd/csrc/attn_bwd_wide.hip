@@ -16,7 +16,7 @@
 //   - Causal tiles one by one, the ones with the most queries first.
 // Bound by the matrix cores and what does not overlap them: 32 products of 34 cycles and two waves on each SIMD are 0.9 us
 // at 2.4 GHz of a step's 1.3 us (half the chip at work) to 1.9 us (all of it).  Measured, bf16, 128 -> 256 keys: exact
-// causal, 8 segments of 2048 rows, 32 query heads on 8, 753 -> 540 us (1.0 PFLOP/s of the visible pairs); 32 heads of 4096
+// causal, 8 segments of 2048 rows, 32 query heads on 8, 753 -> 540 us (540 to 577 on other boxes; 1.0 PFLOP/s of the visible pairs); 32 heads of 4096
 // rows without mask 684 -> 477 (1.15); blocks of 256 of 16384 rows, 32 heads on 8, 225 -> 159; 256 sampled keys of 8192
 // queries, 32 heads, 128 -> 75 (with atomic adds instead of stores at the end 122).
 #include "ha_common.h"

@@ -10,7 +10,7 @@
 // two waves take 0.7 at 2.4 GHz, and 13 us a workgroup outside its loop, 6 to 7 of them for 240 KB of first loads of every CU
 // at once.  (Workgroups that take tile after tile and load the next one's rows beside the loop lost: their loop got as
 // much slower as the start got shorter, 493 against 467 us.  So did touching the next workgroup's rows, 513.)
-// Measured, bf16, 128 -> 256 queries: causal, 8 segments of 2048 rows, 32 heads, 480 -> 453 us; 32 heads of 4096 223 -> 190;
+// Measured, bf16, 128 -> 256 queries: causal, 8 segments of 2048 rows, 32 heads, 480 -> 453 us (444 to 456 on other boxes); 32 heads of 4096 223 -> 190;
 // without mask 376 -> 342 (1.2 PFLOP/s).
 #include "ha_common.h"
 #include "attn_tiles.h"
