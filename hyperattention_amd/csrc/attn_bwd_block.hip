@@ -539,8 +539,8 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 // (0.25 to 24 per CU): up to 256 samples it is the faster one at all (4 heads x 4096 rows 44 | 40, 24 x 4096 98 | 79, 24 x 8192
 // 156 | 131, 32 x 16384 361 | 267, 24 x 65536 1038 | 744; without samples 20.4 | 19.3 to 692 | 424; where it adds to them
 // too, but for 16 x 2048 without samples, 22.8 | 23.2); 512: 8 x 2048 51 | 54, 24 x 2048 82 | 79, 10 x 16384 172 | 178, 130 x 2048
-// 294 | 306, then within 5 % to both sides up to 1600 blocks, 28 x 16384 (1792) 453 | 382, 24 x 65536 1402 | 1118; 1024 never:
-// 8 x 2048 66 | 82, 24 x 65536 2027 | 2247.
+// 294 | 306, then within 5 % to both sides up to 1600 blocks, 28 x 16384 (1792) 453 | 382, 24 x 65536 1402 | 1118; 768: 24 x
+// 8192 254 | 306, 20 x 16384 373 | 405, 24 x 65536 1695 | 1633, not enough for a rule; 1024: 8 x 2048 66 | 82, 24 x 65536 2027 | 2247.
 bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d) {
   const int64_t blocks = (int64_t)p.batch * p.heads * p.segs * ((p.n_q + FUSED_ROWS - 1) / FUSED_ROWS);
   return d == FD && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
