@@ -5,9 +5,9 @@
 // bias "none" (src/flash_attn_triton.py:57-267); the resume-from-a-previous-partial-result mode
 // folds add_self_attentions (src/attn_utils.py:6-50) into the kernel.
 //
-// Work decomposition.  A workgroup owns 256 consecutive (sorted) query positions of one (virtual) head:
-// 4 waves of 64 queries (two 32-wide MFMA column blocks) at head dim 64, 8 waves of 32 queries at head
-// dim 128 (WaveShape below).  Query rows and key
+// Work decomposition.  A workgroup of 4 waves owns consecutive (sorted) query positions of one (virtual) head:
+// 256 at head dim 64, 64 queries (two 32-wide MFMA column blocks) per wave, 128 at head dim 128, 32 queries per
+// wave (WaveShape below), and a CU holds two workgroups.  Query rows and key
 // rows go from HBM straight into LDS (global_load_lds, 16 bytes per lane, whole rows per
 // instruction, no staging registers), row-major with their 16-byte pieces XOR-swizzled by the row
 // number (the swizzle is applied on the source side: a lane fetches the piece that belongs in its
@@ -58,7 +58,6 @@
 
 namespace {
 
-constexpr int WG_QUERIES = 256;  // sorted query positions per workgroup
 constexpr int KC = 64;           // keys per LDS tile
 constexpr float HALF_SUM_LIMIT = 16384.f;  // 2^14: a lane's half-step sum below this has no fp16 overflow
 // Reference exponent (log2 units) of a row that has seen no key yet.  Finite on purpose: a masked score
@@ -67,18 +66,23 @@ constexpr float HALF_SUM_LIMIT = 16384.f;  // 2^14: a lane's half-step sum below
 // which takes that path once and sets the row's true exponent.
 constexpr float M_FLOOR = -1e30f;
 
-// How a workgroup's 256 queries are split over its waves.  A wave's registers hold the output accumulators
+// A workgroup's waves and their queries.  A wave's registers hold the output accumulators
 // of its queries (queries x head dim floats over 64 lanes), their query fragments and two S^T buffers: 64
 // queries per wave fit 256 registers at head dim 64, at head dim 128 only 32 do.  256 registers is what lets
 // two waves share a SIMD, and a wave on its own leaves the matrix pipe idle through every stretch of vector
 // work and every wait (one wave per SIMD with 64 queries and 512 registers ran the d = 128 loop at 1170
-// cycles per 16 keys where its MFMAs alone take 512).  So: 4 waves x 64 queries at d = 64 (two workgroups per
-// CU), 8 waves x 32 queries at d = 128 (one workgroup per CU, LDS-bound), two waves per SIMD either way.
+// cycles per 16 keys where its MFMAs alone take 512).  The two waves of a SIMD belong to two workgroups: neither waits at the
+// other's barriers, and one's set-up and output stage run beside the other's loop.  With 8 waves of 32 queries at
+// d = 128 (256 queries, one workgroup per CU) a wave stood at the barrier of a 64-key iteration for a quarter of it: 2 x 32
+// heads of 65536 rows, smooth blocks of 512 2.80 -> 2.58 ms, 16 x 20479 causal, d = 96 508 -> 457 us (whole call, 2.5 rounds of 256
+// workgroups), leaves of 2048 rows, 32 x 32768 671 -> 650, 24 heads of 2048 causal 55 -> 38; a plain level of 32 x 16384
+// queries, before in runs of tiles per workgroup (attn_fwd_stream.inc), the same 200.
 template <int D>
 struct WaveShape {
   static constexpr int NB = D <= 64 ? 2 : 1;        // 32-query MFMA column blocks per wave
   static constexpr int QW = 32 * NB;                // queries per wave
-  static constexpr int WAVES = WG_QUERIES / QW;     // waves per workgroup
+  static constexpr int WAVES = 4;                   // waves per workgroup
+  static constexpr int QUERIES = QW * WAVES;        // sorted query positions per workgroup
   static constexpr int THREADS = 64 * WAVES;
 };
 
@@ -115,8 +119,13 @@ __device__ __forceinline__ void half_step_p(const f32x16 (&s_use)[NB], const flo
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      pn[nb][e] = (T)__builtin_amdgcn_exp2f(__builtin_fmaf(s_use[nb][H * 8 + e], scale_log2, -m[nb]));
+    for (int e = 0; e < 8; e += 2) {
+      const f32x2 two = {__builtin_amdgcn_exp2f(__builtin_fmaf(s_use[nb][H * 8 + e], scale_log2, -m[nb])),
+                         __builtin_amdgcn_exp2f(__builtin_fmaf(s_use[nb][H * 8 + e + 1], scale_log2, -m[nb]))};
+      const typename ElemTraits<T>::vec2 p2 = __builtin_convertvector(two, typename ElemTraits<T>::vec2);
+      pn[nb][e] = p2[0];
+      pn[nb][e + 1] = p2[1];
+    }
   half_step_sums<T, NB>(pn, sum);
 }
 
@@ -151,6 +160,25 @@ __device__ __forceinline__ void half_step_rescale(const f32x16 (&s_use)[NB], flo
   half_step_p<T, NB, H>(s_use, m_use, scale_log2, pn, sum);
 }
 
+// Issue order of a block: each of its NB*DC/16 large MFMAs is followed by a share of the P arithmetic (8 NB multiply-adds,
+// 4 NB conversions, 8 NB exponentials in all), so the soft-max fills the issue slots behind every MFMA instead of running as
+// one burst after the last of them.  Measured 3 % faster than the scheduler's own order at d = 64, 8 % at d = 128.
+// With one 32-query block per wave (d = 128) a block reads twice as much from LDS per MFMA, and the issue of 12 reads in a row
+// is half as long as its MFMAs: they are spread behind the first six, the K operands (needed by the second half of the MFMAs)
+// first.  32 x 32768 grouped: leaves 641 -> 617 us, a level 200 -> 198, smooth 2 x 32 x 65536 2.495 -> 2.455 ms.  At d = 64
+// (six reads) the same order measured 0 to 1 % slower; there they stay at the head of the block.
+template <int NB, int DC, int G = 0>
+__device__ __forceinline__ void half_step_order() {
+  constexpr int MFMAS = NB * DC / 16, DB = DC / 32;
+  constexpr int V_LEFT = 2 * DB - (G < 4 ? 2 * (G - 1) : G + 2);  // transposing V^T reads not issued yet (G > 0)
+  constexpr int READS = NB > 1 ? 0 : G == 0 ? DC / 32 : V_LEFT > (G < 4 ? 2 : 1) ? (G < 4 ? 2 : 1) : V_LEFT;
+  __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                // one MFMA
+  if constexpr (READS > 0) __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);   // LDS reads
+  __builtin_amdgcn_sched_group_barrier(0x002, (12 * NB + MFMAS - 1) / MFMAS, 0);    // its share of plain VALU
+  __builtin_amdgcn_sched_group_barrier(0x400, (8 * NB + MFMAS - 1) / MFMAS, 0);     // and of the transcendentals
+  if constexpr (G + 1 < MFMAS) half_step_order<NB, DC, G + 1>();
+}
+
 // One block of the pipeline: half-step H (16 keys) of the 32-key step whose S^T is s_use.
 //   MFMAs : P.V of the previous half-step (operands vf, pb, both in registers) and this half's share
 //           (k-steps H*KSTEPS/2 ..) of the next step's S^T, K rows k_row_off.. of k_tile
@@ -178,9 +206,9 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
   vec8 vf_next[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) vf_next[db] = lds_read_vt<T>(v_tile, lo.v[db] + v_key_off, D * 2);
-  // the LDS reads stay at the head of the block: their latency hides behind the P.V MFMAs and the
+  // d = 64: the LDS reads stay at the head of the block: their latency hides behind the P.V MFMAs and the
   // exponentials instead of being waited for where the compiler would sink them to
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NB > 1) __builtin_amdgcn_sched_barrier(0);
 
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -200,17 +228,7 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
   vec8 pn[NB];
   float sum[NB];
   half_step_p<T, NB, H>(s_use, m_run, scale_log2, pn, sum);
-  // Issue order of the block: each of its NB*DC/16 large MFMAs is followed by a share of the P arithmetic (8 NB
-  // multiply-adds, 4 NB conversions, 8 NB exponentials in all), so the soft-max fills the issue slots behind
-  // every MFMA instead of running as one burst after the last of them.  Measured 3 % faster than the
-  // scheduler's own order.
-  constexpr int MFMAS = NB * DC / 16;
-#pragma unroll
-  for (int g = 0; g < MFMAS; ++g) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
-    __builtin_amdgcn_sched_group_barrier(0x002, (12 * NB + MFMAS - 1) / MFMAS, 0);  // its share of plain VALU
-    __builtin_amdgcn_sched_group_barrier(0x400, (8 * NB + MFMAS - 1) / MFMAS, 0);             // and of the transcendentals
-  }
+  half_step_order<NB, DC>();
   // One compare for all query blocks: their sums are >= 0 or NaN, so the total is below the limit
   // only if every one is.  Not "total >= limit": a NaN (row that has seen nothing yet) must take the rare
   // path too.
@@ -243,8 +261,8 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB
 
 // PLAIN (gathered kernel only): the common configuration, for which the per-iteration bookkeeping of the
 // general one is compiled out: no smoothing, default samples (rows 0 .. sample_size-1), and both
-// 128-query tiles of the workgroup inside one key block, so no chunk is ever masked for half of it (where the second tile
-// is past the end, its waves work on row 0 and store nothing).
+// 128-query tiles of the workgroup inside one key block (d = 64; at d = 128 it has one), so no chunk is ever masked for half of it
+// (where the second tile is past the end, its waves work on row 0 and store nothing).
 // Head dims below the built width D (NARROW kernels): a row holds fewer 16-byte pieces than its LDS slot.
 // A lane whose piece lies past the end of the row fetches these zeros instead, so the tiles hold the rows
 // zero-padded to D: zero columns change neither q.k nor the other columns of the output.
@@ -310,6 +328,8 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   constexpr int NB = WaveShape<D>::NB;        // 32-query column blocks per wave
   constexpr int QW = WaveShape<D>::QW;        // queries per wave
   constexpr int WAVES = WaveShape<D>::WAVES;  // waves per workgroup
+  constexpr int WG_QUERIES = WaveShape<D>::QUERIES;
+  constexpr int REF_TILES = WG_QUERIES / 128;  // reference query tiles of 128 per workgroup
   constexpr int DV = D;
   constexpr int KSTEPS = DC / 16;  // MFMA k-steps of Q.K^T
   constexpr int DB = DC / 32;      // 32-row blocks of O^T
@@ -320,13 +340,16 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   // serialise them.  The query region (QW rows per wave) is reused for the output rows at the end.
   constexpr int TILE_BYTES = KC * D * 2;
   // The key tiles ask for the larger alignment only to be placed first: LDS offsets below 64 KB fit
-  // the immediate field of the LDS reads, which matters at d = 128 where the workgroup uses 130 KB.
+  // the immediate field of the LDS reads.
   constexpr int Q_WAVE_BYTES = QW * D * 2;  // a wave's part of the query region
+  // At d = 128 two workgroups fit a CU's 160 KB if most of the query region lies in tile space that is free before and
+  // after the loop: V tile 1 (waves 0, 1) and the first half of K tile 0 (wave 3).
+  constexpr bool OVERLAY = D == 128;
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_v1[TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) unsigned char lds_q[4 * TILE_BYTES];
+  __shared__ __attribute__((aligned(16))) unsigned char lds_q[OVERLAY ? Q_WAVE_BYTES : WAVES * Q_WAVE_BYTES];
   __shared__ int lds_qrow[WG_QUERIES];   // original row of every query position (-1: past the end)
   __shared__ float lds_w[WG_QUERIES];    // weight of the resumed partial result per query position
 
@@ -347,16 +370,16 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
   // launch has the same number of key chunks to go through.  The hardware hands out workgroups in order and
   // a slot freed by a short one stays empty until the ones queued before it are placed: with one tile per
   // workgroup (4 to 32 chunks in a 2048-row leaf) the slots of a CU stood empty for 8 us at a time.
-  // Few workgroups (p.tiles_per_wg == 0, see single_tiles): one tile each, the tiles of all sequences, longest first, at
-  // head dim 64, where a CU holds two workgroups, the second 256 in reversed order (see ha_attn_fwd_split_kernel).
+  // Few workgroups (p.tiles_per_wg == 0, see single_tiles): one tile each, the tiles of all sequences, longest first,
+  // the second 256 in reversed order: a CU holds two workgroups (see ha_attn_fwd_split_kernel).
   constexpr bool PAIRED = CAUSAL && !GATHER;
   const int wg_per_seq = PAIRED ? (qtiles + 1) / 2 : qtiles;  // what p.div_qtiles divides by
-  const bool single = PAIRED && (FOLLOW || p.tiles_per_wg == 0);
+  const bool single = PAIRED && (FOLLOW || (D <= 64 && p.tiles_per_wg == 0));  // d = 128: the FOLLOW instance's alone
   int hg, vseq, slot;
   if (single) {
     const int second = min((int)gridDim.x, 512);
     wg = blockIdx.x;
-    if (D <= 64 && wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
+    if (wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
     slot = fast_div(wg, p.div_qtiles);
     wg -= slot * (p.batch * p.heads * p.segs);  // what p.div_qtiles divides by here
     vseq = fast_div(wg, p.div_kv_group);
@@ -393,6 +416,8 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
     if constexpr (!FOLLOW) {
       if (!single && slot != t_long && slot * WG_QUERIES < n_q) {  // an odd number of tiles: the middle one has no partner
         const int qt = slot;
+        // the first tile's output rows were staged in tiles that the second's loads fill (LDS only: the stores need no wait)
+        if (OVERLAY) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #include "attn_fwd_tile.inc"
       }
     }
@@ -444,7 +469,7 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
     return launch_one<T, D, true, false, false, false, true>(p, grid, stream, "ha_block_attn_fwd");
   // also with an odd number of tiles: d = 128, 32 heads of 80000 rows in blocks of 512, the whole call 1907 us with the
   // general instance, 1827 with the plain one; d = 80, 24 of 110464, blocks of 256 1177 -> 1158
-  const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0;
+  const bool plain = !p.smooth && !p.sampled_idx && (p.block_tiles * 128) % WaveShape<D>::QUERIES == 0;
   if (p.qk_pieces != D / 8 || p.v_pieces != D / 8) {
     if constexpr (D == 128) {
       if (p.qk_pieces <= 12 && p.v_pieces <= 12) return launch_narrow<T, D, 96>(p, grid, gather, causal, plain, stream);
@@ -457,9 +482,9 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
     return launch_split<T, D, false, false, false, D>(p, grid, stream, "ha_flash_attn_fwd");
   }
   if (gather) {
-    if (p.tiles_per_wg > 1) {  // set by ha_attn_launch for the instances built below
-      if (plain) hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, true>), dim3(grid), dim3(WaveShape<D>::THREADS), 0, stream, p);
-      else hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, false>), dim3(grid), dim3(WaveShape<D>::THREADS), 0, stream, p);
+    if constexpr (D == 64) if (p.tiles_per_wg > 1) {  // set by ha_attn_launch for the instances built below
+      if (plain) hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, true>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
+      else hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, false>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
       return ha_launch_status("ha_block_attn_fwd");
     }
     if (plain) return launch_one<T, D, true, false, true>(p, grid, stream, "ha_block_attn_fwd");
@@ -484,46 +509,60 @@ static ha_divisor make_divisor(int64_t y) {
 
 // Whether a launch is better off with the keys of its query tiles split over waves (attn_fwd_split.inc): estimated
 // times in us of the two kernels, from how many steps a workgroup takes and how many workgroups a CU has to take.  A step
-// of the 256-query kernel is 64 keys, one of a split workgroup 64 queries x 128 keys.  What the estimates have to catch:
-// - 256-query workgroups: up to one per CU the launch takes as long as one of them; the first ones past 256 cost most
-//   of a second round (48 causal heads of 3000 rows, 288 pairs: 97 us, 24 heads 66).  At d = 64 a CU works on two at a
-//   time, so beyond that it is the CU's share that counts; at d = 128 equal workgroups go in whole rounds.
+// of the kernels that do not split is 64 keys, one of a split workgroup 64 queries x 128 keys.  What the estimates have to catch:
+// - workgroups of 256 queries (d = 64): up to one per CU the launch takes as long as one of them; the first ones past 256 cost most
+//   of a second round (48 causal heads of 3000 rows, 288 pairs: 97 us, 24 heads 66).  A CU works on two at a time, so beyond
+//   that it is the CU's share that counts.
 // - split workgroups: the longest one, or a CU's share of all; causal ones run longest first, so a CU's share ends with
 //   short ones and some of the set-up hides behind other workgroups; at d = 128 equal ones go in whole rounds.
-// Constants fitted to the kernels' times inside calls of the module, 645 launches at d <= 64 and 648 above (2 to 256
-// heads, grouped and not, 300 to 4133 rows exact, 2048 to 16384 rows hashed): the chosen kernel is within 3 % of the
-// better one at all but 10 of them, within 10 % at all.  Times whole | split in us, d = 64 causal: 24 heads of 1000
+// d = 64: constants fitted to the kernels' times inside calls of the module, 645 launches (2 to 256
+// heads, grouped and not, 300 to 4133 rows exact, 2048 to 16384 rows hashed).  Times whole | split in us, causal: 24 heads of 1000
 // rows 31 | 13, of 2048 39 | 28, of 4096 72 | 72; 48 of 2048 41 | 45, of 4096 116 | 143; without mask 16 of 4096 rows
-// 75 | 86; d = 128, 12 heads of 2048 rows, blocks and samples of 256: 20 | 26.
+// 75 | 86.
+// d = 128, causal: fitted to 64 launches, at which the choice is 1 % slower than the best one on average (worst: 32 heads of 520 rows, 14.9 |
+// 17.7, 12 of 3000 49.0 | 53.5; 4 % and less beyond 24 of 1000).  Single tiles of 128
+// queries | split: 12 heads of 1000 rows 20.7 | 17.2, 24 21.8 | 23.0, 48 25.1 | 37; 16 of 2048 35.3 | 34.3, 24 38.4 | 50; 8 of
+// 4096 65 | 51, 12 70 | 85.
+// d = 128, without mask or gathered: the estimate of `whole` is that of a kernel of 256-query tiles, which the present one outruns.  It
+// is kept because the split form is the closer one to float64 (four exact weights per row: 2 to 4 % for 256 to 1024 keys a row,
+// 0.2 to 2 % above), and the launches that it gives to it lose little: 8 heads of 2048 rows, blocks and samples of 128 10.7 | 12.2,
+// 256 14.5 | 14.5, 512 22.8 | 19.8; without mask 12 of 1000 19.8 | 17.1, 4 of 4096 57 | 44, but 8 of 4096 68 | 85.
 struct LaunchTimes {
-  double whole, single, split;  // the 256-query kernel (exact causal: pairs of tiles), its single tiles, the split kernel
+  double whole, single, split;  // a tile per workgroup (exact causal: pairs of tiles), single causal tiles, the split kernel
 };
 static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   struct Fit {
-    double step, pair, start, crowd, second, share, rest;    // 256-query kernel
+    double step, pair, start, crowd, second, share, rest;    // 256-query tiles
     double split_step, split_start, set_up, hidden;          // split kernel
   };
-  const Fit f = width == 64 ? Fit{0.97, 4.4, 6.2, 0.08, 1.85, 0.94, 0.45, 0.56, 5.6, 4.3, 0.34}
-                            : Fit{1.25, 2.0, 7.0, 0.37, 1.47, 1.58, 0.29, 1.23, 1.3, 5.4, 0.22};
   const bool paired = causal && !gather;
+  const Fit f = width == 64 ? Fit{0.97, 4.4, 6.2, 0.08, 1.85, 0.94, 0.45, 0.56, 5.6, 4.3, 0.34}
+                : paired    ? Fit{0, 0, 0, 0, 0, 0, 0, 1.03, 1.3, 7.9, 0.}
+                            : Fit{1.25, 2.0, 7.0, 0.37, 1.47, 1.58, 0.29, 1.23, 1.3, 5.4, 0.22};
   const double cus = 256., vheads = (double)p.batch * p.heads * p.segs;
-  const double tiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES, split_tiles = (p.n_q + 63) / 64;
+  const double tiles = (p.n_q + 255) / 256, split_tiles = (p.n_q + 63) / 64;
   const double keys = gather ? 128. * p.block_tiles + 64. * p.sample_chunks : p.n_k;
 
-  const double per_cu = vheads * (paired ? std::ceil(tiles / 2) : tiles) / cus;
-  const double one = paired ? 4. * (tiles + 1) * f.step + f.pair : std::ceil(keys / 64.) * f.step;  // a workgroup
-  double rounds;
-  if (per_cu <= 1) rounds = 1 + f.crowd * per_cu;
-  else if (width == 64 || paired) rounds = std::max(f.second, f.share * per_cu + f.rest);
-  else rounds = f.second * std::ceil(per_cu);
   LaunchTimes t;
-  t.whole = t.single = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
-  if (paired) {
-    // one tile per workgroup, longest first: the longest chain, slowed by its neighbours, or a CU's share of all
-    const double longest = 4. * tiles, share = vheads * 2. * tiles * (tiles + 1) / cus, wgs = vheads * tiles / cus;
-    const double crowd = width == 64 ? 0.1 * share : 0.3 * std::min(longest, share);
-    t.single = f.start + std::max(f.step * (longest + crowd), (width == 64 ? 0.97 : 1.9) * share + 2. * wgs);
-    if (width == 128) t.single *= 0.93;  // the other estimate is that much too low beside this one (48 heads of 685 rows: 24 us | split 30)
+  if (paired && width == 128) {
+    // two workgroups of 128 queries per CU: the longest chain, slowed by its neighbour, or a CU's share of all
+    const double tiles_128 = (p.n_q + 127) / 128, wgs = vheads * tiles_128 / cus;
+    const double longest = 2. * tiles_128 * (1 + 0.4 * std::min(1., wgs / 2)), share = wgs * (tiles_128 + 1);
+    t.single = 6.6 + std::max(0.78 * longest, 0.895 * share + 3.1 * wgs - 1.);
+    t.whole = t.single;  // pairs are for launches far larger than those the split kernel is for
+  } else {
+    const double per_cu = vheads * (paired ? std::ceil(tiles / 2) : tiles) / cus;
+    const double one = paired ? 4. * (tiles + 1) * f.step + f.pair : std::ceil(keys / 64.) * f.step;  // a workgroup
+    double rounds;
+    if (per_cu <= 1) rounds = 1 + f.crowd * per_cu;
+    else if (width == 64) rounds = std::max(f.second, f.share * per_cu + f.rest);
+    else rounds = f.second * std::ceil(per_cu);
+    t.whole = t.single = f.start + (gather ? 3.5 : 0.) + one * rounds;  // gathered: a chain of row numbers, then rows
+    if (paired) {
+      // one tile per workgroup, longest first: the longest chain, slowed by its neighbours, or a CU's share of all
+      const double longest = 4. * tiles, share = vheads * 2. * tiles * (tiles + 1) / cus, wgs = vheads * tiles / cus;
+      t.single = f.start + std::max(f.step * (longest + 0.1 * share), 0.97 * share + 2. * wgs);
+    }
   }
 
   const double chain = std::ceil(keys / 128.), split_per_cu = vheads * split_tiles / cus;
@@ -536,15 +575,19 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
 
 // Whether exact causal attention takes one query tile per workgroup, longest first, instead of a pair of tiles.  Pairs
 // leave CUs idle in a last round that is not full; single tiles fill it, but read a sequence's keys at times
-// far apart, which costs where there are many rounds.  At head dim 128, with one workgroup per CU, full rounds of pairs
-// are as fast or faster.  Times in us, pairs | single, 256-query pairs per CU in brackets: d = 64, 48 heads of 2048 rows
+// far apart, which costs where there are many rounds, and full rounds of pairs are as fast or faster.
+// Times in us, pairs | single.  d = 64, 256-query pairs per CU in brackets: 48 heads of 2048 rows
 // (0.75) 49.9 | 43.0, 80 (1.25) 74.1 | 58.1, 96 of 1024 (0.75) 32.8 | 26.8, 128 of 2048 (2) 82.9 | 81.2, 200 (3.1) 151 |
-// 130, 256 (4) 170 | 175, 700 (11) 448 | 490, 2048 (32) 1292 | 1462; d = 128, 24 of 2048 (0.38) 64 | 55, 64 (1) 78 | 78, 96
-// (1.5) 136 | 117, 128 (2) 154 | 156, 256 of 1024 (2) 99 | 106, 200 of 2048 (3.1) 285 | 263, 300 (4.7) 402 | 417, 512 (8)
-// 659 | 736.
+// 130, 256 (4) 170 | 175, 700 (11) 448 | 490, 2048 (32) 1292 | 1462.
+// d = 128, rounds of 512 pairs of 128-query tiles in brackets: 24 of 2048 (0.38) 41.0 | 38.4, 40 (0.62) 63.1 | 50.4, 64 (1) 73.7 |
+// 73.0, 80 (1.25) 104 | 92, 96 (1.5) 110 | 107, 160 (2.5) 181 | 184, 256 (4) 292 | 352; 48 of 3000 (1.12) 142 | 115; 150 of 300
+// (0.59) 22.9 | 18.4, 192 of 1024 (1.5) 67.6 | 70.7, 400 (3.1) 148 | 175; 8 of 8192 (0.5) 135 | 140.
 static bool single_tiles(const ha_attn_kernel_params& p, int width) {
-  const double pairs = (double)p.batch * p.heads * p.segs * ((p.n_q + 2 * WG_QUERIES - 1) / (2 * WG_QUERIES)) / 256.;
-  return width == 64 ? pairs <= 3.5 : pairs < 4 && std::ceil(pairs) > 1.05 * pairs;
+  const int64_t pair_rows = width == 64 ? 2 * WaveShape<64>::QUERIES : 2 * WaveShape<128>::QUERIES;
+  const double pairs = (double)p.batch * p.heads * p.segs * ((p.n_q + pair_rows - 1) / pair_rows) / 256.;
+  if (width == 64) return pairs <= 3.5;
+  const double rounds = pairs / 2;
+  return rounds < 1 || (rounds <= 1.5 && std::ceil(rounds) > 1.05 * rounds);
 }
 
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,
@@ -555,16 +598,14 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   const int width = d <= 64 && dv <= 64 ? 64 : 128;
   p.qk_pieces = d / 8;
   p.v_pieces = dv / 8;
-  int64_t qtiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES;
+  const int tile_rows = width == 64 ? WaveShape<64>::QUERIES : WaveShape<128>::QUERIES;
+  int64_t qtiles = (p.n_q + tile_rows - 1) / tile_rows;
   const bool single = causal && !gather && single_tiles(p, width);
   if (causal && !gather && !single) qtiles = (qtiles + 1) / 2;  // one workgroup per pair of tiles
-  // Gathered attention with whole 256-query tiles, whole key blocks and an even number of at least four key
+  // Gathered attention at head dim 64 with whole 256-query tiles, whole key blocks and an even number of at least four key
   // chunks per tile can run as a stream: a workgroup takes a run of tiles of its head
-  // (ha_attn_fwd_stream_kernel), as long a run as still leaves every CU its full set of resident workgroups.
-  // It is the default where it measured faster: head dim 128 (one workgroup per CU, nothing else covers a
-  // workgroup's set-up and output stage) in the plain configuration, 4 to 7 % on a level of 64 tiles per head
-  // at 8 chunks per tile.  At head dim 64 the second workgroup of the CU covers them already and the stream
-  // measured 2 to 5 % slower; with smooth windows (18 chunks per tile) it measured the same.
+  // (ha_attn_fwd_stream_kernel).  It measured 2 to 5 % slower than one tile per workgroup with two workgroups per CU,
+  // so only the measurement aid below asks for it.
   p.tiles_per_wg = 1;
   const char* stream_env = getenv("HA_STREAM_TILES");  // measurement aid: force the run length (1: off)
   const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0;
@@ -573,20 +614,19 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   // (a forced run length asks for the 256-query kernels)
   p.split_keys = !reweight && !(gather && stream_env) && (split_env ? atoi(split_env) != 0 : t.split < (single ? t.single : t.whole));
   if (p.split_keys) qtiles = (p.n_q + 63) / 64;
-  else if (gather && !reweight && p.qk_pieces == width / 8 && p.v_pieces == width / 8 && p.n_q % WG_QUERIES == 0 && qtiles >= 2 &&
-      p.sample_chunks % 2 == 0 && p.n_k % (p.block_tiles * 128) == 0 && 2 * p.block_tiles + p.sample_chunks >= 4 &&
-      (stream_env || (width == 128 && plain))) {
-    const int64_t slots = 256 * (width == 64 ? 2 : 1);  // workgroups the chip holds at once
-    int r = 16;
-    while (r > 1 && (r > qtiles || (qtiles / r) * p.batch * p.heads * p.segs < slots)) r /= 2;
-    if (stream_env) r = atoi(stream_env) < 1 ? 1 : (atoi(stream_env) > qtiles ? (int)qtiles : atoi(stream_env));
-    p.tiles_per_wg = r;
-    qtiles = (qtiles + r - 1) / r;
+  else if (stream_env && gather && !reweight && width == 64 && p.qk_pieces == width / 8 && p.v_pieces == width / 8 && p.n_q % STREAM_QUERIES == 0 &&
+           p.n_q >= 2 * STREAM_QUERIES && p.sample_chunks % 2 == 0 && p.n_k % (p.block_tiles * 128) == 0 &&
+           2 * p.block_tiles + p.sample_chunks >= 4) {
+    const int r = std::min(atoi(stream_env), p.n_q / STREAM_QUERIES);
+    if (r > 1) {  // else one tile per workgroup, whose tiles are not these
+      p.tiles_per_wg = r;
+      qtiles = (p.n_q / STREAM_QUERIES + r - 1) / r;
+    }
   }
   // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
   if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
   if (single && !p.split_keys) p.tiles_per_wg = 0;
-  p.follow_max = single && !p.split_keys && t.split < t.whole;
+  p.follow_max = single && !p.split_keys && (width == 128 || t.split < t.whole);
   p.div_qtiles = make_divisor(p.split_keys == 2 || p.tiles_per_wg == 0 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);

@@ -1,0 +1,35 @@
+"""Head dims above 64: workgroups of 128 queries, whose query and output rows are staged in tiles of keys and values.  Tile edges,
+ragged ends, pairs of causal tiles (the second tile's rows arrive where the first's were staged) and single ones."""
+import pytest
+import torch
+
+from oracle import hyper_oracle as O
+from test_gpu_ops import ha  # noqa: F401 (fixture)
+from _util import _randn, assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,d,h,hk,n,causal", [
+    (torch.bfloat16, 128, 2, 2, 1, False),
+    (torch.float16, 128, 2, 1, 127, False),
+    (torch.bfloat16, 96, 2, 2, 129, False),
+    (torch.bfloat16, 128, 3, 3, 385, False),
+    (torch.float16, 80, 2, 2, 640, False),
+    (torch.bfloat16, 128, 2, 2, 1, True),          # single tiles
+    (torch.float16, 128, 2, 1, 128, True),
+    (torch.bfloat16, 128, 2, 2, 257, True),
+    (torch.float16, 96, 5, 5, 1025, True),
+    (torch.bfloat16, 128, 150, 150, 510, True),    # 600 workgroups: 256, 256 reversed, the rest in order
+    (torch.bfloat16, 96, 1040, 1040, 130, True),   # pairs of tiles: one pair, the second of 2 rows
+    (torch.float16, 128, 520, 260, 500, True),     # two pairs
+    (torch.bfloat16, 128, 520, 520, 384, True),    # three tiles, the middle one alone
+])
+def test_exact(ha, monkeypatch, dtype, d, h, hk, n, causal):  # noqa: F811
+    monkeypatch.setenv("HA_SPLIT", "0")
+    q = _randn((1, h, n, d), 71, dtype)
+    k, v = (_randn((1, hk, n, d), s, dtype) for s in (72, 73))
+    o, lse = ha.flash_attn_func(*(x.cuda().transpose(1, 2) for x in (q, k, v)), None, causal)
+    ro, rl = O.exact_attention(q, *(x.repeat_interleave(h // hk, 1) for x in (k, v)), None, causal)
+    assert_close(o.transpose(1, 2), ro, "out", dtype)
+    assert_close(lse[:, :, :n], rl, "lse")
