@@ -2,16 +2,15 @@
 // Follows the definition in src/angular_lsh_triton.py:76-88 and :175-179 of the reference
 // (bit_j = [x . P[:, j] > 0], bin = sum_j bit_j << j, bucket = perm[bin], perm[i] = i ^ (i >> 1)).
 //
-// lsh_hash_mfma_kernel: a wave projects 16 rows at a time with v_mfma_f32_16x16x32 (rows x 16 projection
-// slots, fp32 accumulation), reading the rows straight from HBM as MFMA operands, so the kernel is purely
-// bandwidth bound.  Built for rows of 32, 64, 128 and 256 elements; a row of any other multiple of 8
-// elements runs in the next width with its missing elements (and the missing rows of the projection) read
-// as zeros.  fp32 accumulation cannot decide the
+// lsh_hash_mfma_kernel: a wave projects 16 rows at a time with v_mfma_f32_16x16x32 (16 projection slots x rows,
+// fp32 accumulation), reading the rows straight from HBM as MFMA operands: a stream of reads.  Built for rows of 32, 64,
+// 96, 128 and 256 elements; a row of any other multiple of 8 elements runs in the next width with its missing
+// elements (and the missing rows of the projection) read as zeros.  fp32 accumulation cannot decide the
 // sign of a projection that nearly cancels, so a second MFMA on |x| and |P| gives sum |x_k P_kj|, which
 // bounds the accumulation error of any summation order (d * 2^-23 * sum, used with a factor 2 margin;
 // fp16/bf16 products are exact in fp32 and subnormal inputs are not flushed).  Whenever some
-// |projection| is inside that bound, the 16-row tile is recomputed in fp64 (products exact, sum exact
-// to 2^-53), which happens for well under 1 % of the tiles on random data.
+// |projection| is inside that bound, that projection of the 16 rows is recomputed in fp64 (products exact, sum exact
+// to 2^-53): 2 % of the 16-row tiles on random data of 64 elements, 5 % of 128.
 #include "ha_common.h"
 #include "bucket_sort.h"
 
@@ -32,24 +31,21 @@ struct HashMfma<bf16_t> {
   }
 };
 
-// Tiles of 512 elements (16 MFMA rows of 32 elements) per wave: as many as a launch of that size can have with the
-// chip full of workgroups, so that the projection's set-up is shared; a wave's groups of tiles in flight are one
-// memory round trip after the other.  8 sequences of 4096 rows of 128 bytes at 32 tiles per wave: 32 workgroups, 18.3 us;
-// at 8: 8.3, at 4: 6.4, at 2: 6.0, at 1: 6.6; 48 of 2048 rows at 8: 9.8, at 4: 9.1, at 2: 8.3, at 1: 8.9.  On a full chip
-// the set-up counts: 64 of 32768 rows at 32: 57.5, at 4: 64.7, at 2: 81.2
+// Tiles of 16 rows per wave: 8 KB, in two groups of tiles whose rows are in flight together, and fewer where the launch would
+// not fill the chip with workgroups.  Short waves, many of them, read fastest: the projection's set-up of one runs beside the
+// loads of the others.  TB/s at 32, 8, 4, 2, 1 tiles per wave (the better group size of each): 64 x 131072 rows of 128
+// bytes 5.03, 5.60, 5.92, 5.78, 4.98; 64 x 32768 6.00, 6.52, 6.75, 6.43, 4.89; 128 x 65536 of 256 bytes 5.24, 5.82,
+// 5.84, 6.14, 5.54; 34 x 32768 4.81, 5.91, 6.46, 6.41, 5.56; 32 x 20480 of 192 bytes 5.47, 6.14, 6.16, 5.92, 5.48.
 constexpr int HASH_FULL_CHIP = 2048;  // workgroups
-constexpr int HASH_SHORT = 8;         // waves of up to this many tiles have them all in flight at once
-constexpr int HASH_LEAST = 2;         // tiles per wave of the smallest launches
-// tiles in flight per wave: at 8 the longer waves' registers cost them occupancy (4.2 M rows of 256 B: 4.1 TB/s
-// against 4.4 with 4, 16 tiles 3.1)
-template <int TILES>
-constexpr int hash_unroll() { return TILES <= HASH_SHORT ? TILES : 4; }
+template <int PARTS>
+constexpr int hash_group() { return PARTS <= 2 ? 2 : 1; }
 
-// A data row of D elements is cut into PARTS = D/32 MFMA rows of 32 elements, so that one load
-// instruction of the wave (16 bytes per lane) covers whole rows: 16/PARTS data rows of D*2 bytes.
-// MFMA row m = (data row)*PARTS + part; lane (m = lane%16, kg = lane/16) holds elements
-// part*32 + 8*kg .. +7 of its data row.  The C registers i = 0..3 of a lane are MFMA rows 4*kg + i
-// of projection slot lane%16; the partial projections of one data row are summed afterwards.
+// A row of up to PARTS*32 elements is PARTS k-steps of the MFMA: lane (m = lane%16, kg = lane/16) holds elements
+// 32*part + 8*kg .. +7 of row m of the tile (a load instruction covers 64 bytes of 16 rows, the part's neighbour the rest
+// of their lines) and of projection slot m, and gets the projections of row m on slots 4*kg .. +3.  (With the parts of a
+// row as rows of the MFMA, so that a load instruction covered whole rows, the other parts had to be zeroed and the
+// product repeated per part: 4 times the vector instructions at 128 elements, which bounded the launch: 40 x 16384 rows of
+// 256 bytes 44.6 -> 26.8 us, 128 x 65536 463 -> 353; of 128 bytes, 64 x 131072 218 -> 181, 8 x 4096 7.8 -> 4.3.)
 // Up to two tensors per launch (queries and keys of one forward): blockIdx.y + blockIdx.z * gridDim.y counts
 // the (batch, head) sequences of the first tensor, then those of the second (a grid dimension holds 65535).
 struct HashTensors {
@@ -63,15 +59,23 @@ struct HashTensors {
   int64_t first[2], end[2];  // rows of every sequence whose ids are wanted
 };
 
-template <typename T, int D, bool OUT8, int TILES>
+// the bits of c's signs, c[0]'s lowest
+__device__ __forceinline__ uint32_t sign_bits(f32x4 c) {
+  uint32_t bits = 0;
+#pragma unroll
+  for (int i = 3; i >= 0; --i) {
+    const float ci = c[i];
+    bits = __builtin_amdgcn_alignbit(bits, __builtin_bit_cast(uint32_t, ci), 31);
+  }
+  return bits;
+}
+
+template <typename T, int PARTS, bool OUT8, int GROUP>  // GROUP tiles (1 or 2) in flight together
 __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors ten, const T* __restrict__ proj, int64_t n,
-                                                            int r, int64_t psb, int64_t psh, int d_real) {
+                                                            int r, int64_t psb, int64_t psh, int d_real, int tiles) {
   typedef typename ElemTraits<T>::vec8 vec8;
-  constexpr int HASH_UNROLL = hash_unroll<TILES>();
-  constexpr int PARTS = D / 32;
-  constexpr int ROWS = 16 / PARTS;            // data rows per tile
-  constexpr int NS = PARTS >= 4 ? 1 : 4 / PARTS;  // data rows per lane (sums of C registers)
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int D = PARTS * 32;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int seq = (int)(blockIdx.y + blockIdx.z * gridDim.y);
   if (seq >= ten.seqs) return;  // the last layer of the grid may be partly empty
   const int which = seq >= ten.seqs0 ? 1 : 0;
@@ -84,169 +88,154 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   int32_t* obase = OUT8 ? nullptr : (int32_t*)ten.out[which] + (int64_t)bh * n;
   uint8_t* obase8 = OUT8 ? (uint8_t*)ten.out[which] + (int64_t)bh * n : nullptr;
   const int m = lane & 15, kg = lane >> 4;
-  const int my_row = m / PARTS, my_part = m % PARTS;  // data row inside a tile, 32-element part of it
-  const int j = m;                                    // projection slot of this lane's C registers
 
   const int64_t end = ten.end[which];
-  const int64_t wave_row0 = ten.first[which] + ((int64_t)blockIdx.x * 4 + wave) * TILES * ROWS;
+  const int64_t wave_row0 = ten.first[which] + ((int64_t)blockIdx.x * 4 + wave) * tiles * 16;
   // The loads of a group have no condition, so that all of them are in flight together: rows and pieces that do not
   // exist read the last row or the first piece, and are zeroed where the group is used (a condition on a load
   // made the compiler wait for it before the next one).
-  const bool piece_exists = my_part * 32 + 8 * kg < d_real;
-  const T* const xlane = xbase + (piece_exists ? my_part * 32 + 8 * kg : 0);
-  const int64_t last_row = ten.n_read - 1;
-  vec8 xf[HASH_UNROLL];
-  auto load_rows = [&](int t0) {
+  int piece[PARTS];
 #pragma unroll
-    for (int u = 0; u < HASH_UNROLL; ++u) {
-      const int64_t row = wave_row0 + (int64_t)(t0 + u) * ROWS + my_row;
-      xf[u] = *reinterpret_cast<const vec8*>(xlane + (row < last_row ? row : last_row) * sn);
+  for (int pt = 0; pt < PARTS; ++pt) piece[pt] = pt * 32 + 8 * kg < d_real ? pt * 32 + 8 * kg : 0;
+  const int64_t last_row = ten.n_read - 1;
+  vec8 xf[GROUP][PARTS];
+  auto load_rows = [&](int64_t row0) {
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u) {
+      const int64_t row = row0 + u * 16 + m;
+      const T* x = xbase + (row < last_row ? row : last_row) * sn;
+#pragma unroll
+      for (int pt = 0; pt < PARTS; ++pt) xf[u][pt] = *reinterpret_cast<const vec8*>(x + piece[pt]);
     }
   };
-  // a short wave's rows are in flight while the projection is set up
-  constexpr bool EARLY = TILES == HASH_UNROLL;
-  if (EARLY) load_rows(0);
+  // the first rows are in flight while the projection is set up
+  load_rows(wave_row0);
 
-  // the projection matrix goes through LDS once per block (one coalesced pass instead of a chain of
-  // dependent 2-byte loads per lane)
-  __shared__ T lds_p[D * 16];
-  // rows of d_real <= D elements: the missing elements of a row and the missing rows of the projection are
-  // zeros (they add nothing to a dot product)
-  for (int i = threadIdx.x; i < D * r; i += 256) {
-    const T v = pbase[i < d_real * r ? i : 0];
-    lds_p[i] = i < d_real * r ? v : (T)0.f;
+  // The projection matrix goes through LDS once per block, transposed: a lane's operand is 8 elements of one
+  // projection.  Rows of d_real <= D elements: the missing elements of a row, the missing rows of the projection and the
+  // projections past the last one are zeros (they add nothing to a dot product).
+  constexpr int PITCH = D + 8;  // 16 bytes more, so that the 16 projections' pieces lie on different banks
+  __shared__ __attribute__((aligned(16))) T lds_p[16 * PITCH];
+  {
+    const int j = threadIdx.x & 15, k0 = threadIdx.x >> 4;
+    T v[D / 16];
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) v[i] = pbase[j < r && k0 + 16 * i < d_real ? (k0 + 16 * i) * r + j : 0];
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) lds_p[j * PITCH + k0 + 16 * i] = j < r && k0 + 16 * i < d_real ? v[i] : (T)0.f;
   }
   __syncthreads();
-  // B operands: P and |P| for every part: slot j, group kg holds P[part*32 + 8*kg + e][j]; slots >= r are zero
+  // A operands: P and |P| for every part: slot m, group kg holds P[part*32 + 8*kg + e][m]
   vec8 pf[PARTS], pa[PARTS];
-  const int jc = j < r ? j : 0;
 #pragma unroll
-  for (int pt = 0; pt < PARTS; ++pt)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      // read by every lane (the slots past r a copy of slot 0) and then selected: a read under a condition waits for
-      // itself before the next one is issued
-      float v = ha_to_float(lds_p[(pt * 32 + 8 * kg + e) * r + jc]);
-      v = j < r ? v : 0.f;
-      pf[pt][e] = (T)v;
-      pa[pt][e] = (T)__builtin_fabsf(v);
-    }
+  for (int pt = 0; pt < PARTS; ++pt) {
+    pf[pt] = *reinterpret_cast<const vec8*>(&lds_p[m * PITCH + pt * 32 + 8 * kg]);
+    pa[pt] = __builtin_bit_cast(vec8, __builtin_bit_cast(u32x4, pf[pt]) & 0x7fff7fffu);
+  }
   const float tol = (float)(D + 8) * 4.76837158203125e-07f;  // 2 * (d + 8) * 2^-23
+  // a slot past the last projection starts at -1 and its products are zeros: never in doubt, its bit never set
+  f32x4 c_first;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c_first[i] = 4 * kg + i < r ? 0.f : -1.f;
 
-  // A row's parts meet different B operands, but an MFMA has one B operand per lane column, not per
-  // row: so the tile is multiplied once per part with the rows of the other parts zeroed.  (For
-  // PARTS == 1 this is a single MFMA.)
-#pragma unroll 1  // unrolled, four copies of the group overflow the instruction cache
-  for (int t0 = 0; t0 < TILES; t0 += HASH_UNROLL) {
-    if (wave_row0 + (int64_t)t0 * ROWS >= end) break;
-    if (!EARLY) load_rows(t0);
-    const bool all_exist = d_real == D && wave_row0 + (int64_t)(t0 + HASH_UNROLL) * ROWS <= ten.n_read;
+#pragma unroll 1
+  for (int64_t row0 = wave_row0, wave_end = wave_row0 + tiles * 16; row0 < end;) {
+    const bool all_exist = d_real == D && row0 + GROUP * 16 <= ten.n_read;
     if (!all_exist) {
 #pragma unroll
-      for (int u = 0; u < HASH_UNROLL; ++u) {
-        const bool exists = piece_exists && wave_row0 + (int64_t)(t0 + u) * ROWS + my_row <= last_row;
-        xf[u] = exists ? xf[u] : vec8{};
-      }
+      for (int u = 0; u < GROUP; ++u)
+#pragma unroll
+        for (int pt = 0; pt < PARTS; ++pt) {
+          const bool exists = pt * 32 + 8 * kg < d_real && row0 + u * 16 + m <= last_row;
+          xf[u][pt] = exists ? xf[u][pt] : vec8{};
+        }
+    }
+    f32x4 c[GROUP], ca[GROUP];
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u) {
+      c[u] = c_first;
+      ca[u] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int u = 0; u < HASH_UNROLL; ++u) {
-      const int64_t tile_row0 = wave_row0 + (int64_t)(t0 + u) * ROWS;
-      if (tile_row0 >= end) break;
-      f32x4 c = {0.f, 0.f, 0.f, 0.f}, ca = {0.f, 0.f, 0.f, 0.f};
-      const u32x4 raw = __builtin_bit_cast(u32x4, xf[u]);
+    for (int pt = 0; pt < PARTS; ++pt)
 #pragma unroll
-      for (int pt = 0; pt < PARTS; ++pt) {
-        const u32x4 sel = (PARTS == 1 || my_part == pt) ? raw : u32x4{0u, 0u, 0u, 0u};
-        c = HashMfma<T>::run(__builtin_bit_cast(vec8, sel), pf[pt], c);
-        ca = HashMfma<T>::run(__builtin_bit_cast(vec8, sel & 0x7fff7fffu), pa[pt], ca);
+      for (int u = 0; u < GROUP; ++u) {
+        const vec8 abs_x = __builtin_bit_cast(vec8, __builtin_bit_cast(u32x4, xf[u][pt]) & 0x7fff7fffu);
+        c[u] = HashMfma<T>::run(pf[pt], xf[u][pt], c[u]);
+        ca[u] = HashMfma<T>::run(pa[pt], abs_x, ca[u]);
       }
-      // sum the parts of each data row: C register i of this lane is MFMA row 4*kg + i
-      float s[NS], sa[NS];
-      if (PARTS <= 4) {
+    // slots 4*kg .. +3 of row m: set where the projection is negative
+    uint32_t nib[GROUP];
 #pragma unroll
-        for (int q = 0; q < NS; ++q) {
-          s[q] = 0.f;
-          sa[q] = 0.f;
+    for (int u = 0; u < GROUP; ++u) {
+      nib[u] = sign_bits(c[u]);
+      // what is left of |projection| above the bound of its error; a NaN stays one
+      float left[4];
 #pragma unroll
-          for (int i = 0; i < 4 / NS; ++i) {
-            s[q] += c[q * (4 / NS) + i];
-            sa[q] += ca[q * (4 / NS) + i];
-          }
-        }
-      } else {  // PARTS == 8: a data row spans the C registers of lanes kg and kg^1
-        s[0] = c[0] + c[1] + c[2] + c[3];
-        sa[0] = ca[0] + ca[1] + ca[2] + ca[3];
-        s[0] += __shfl_xor(s[0], 16);
-        sa[0] += __shfl_xor(sa[0], 16);
-      }
-      uint64_t pos[NS];
-      bool unsure = false;
+      for (int i = 0; i < 4; ++i) left[i] = __builtin_fmaf(-tol, ca[u][i], __builtin_fabsf(c[u][i]));
+      const float least = __builtin_elementwise_minimum(__builtin_elementwise_minimum(left[0], left[1]),
+                                                        __builtin_elementwise_minimum(left[2], left[3]));
+      if (__builtin_expect(__any(!(least > 0.f)), false)) {
+        uint32_t unsure = 0;
 #pragma unroll
-      for (int q = 0; q < NS; ++q) {
-        pos[q] = __ballot(s[q] > 0.f);
-        unsure = unsure || (j < r && __builtin_fabsf(s[q]) <= tol * sa[q]);
-      }
-      int bin;
-      if (__any(unsure)) {
-        // exact recomputation of the tile in fp64: this lane's 8 elements, then a sum over the lanes
-        // that share the data row (parts: lane bits 0..log2(PARTS)-1, groups kg: lane bits 4, 5)
-        const int64_t row = tile_row0 + my_row;
-        bin = 0;
+        for (int i = 0; i < 4; ++i) unsure |= left[i] > 0.f ? 0u : 1u << (4 * kg + i);
         for (int jj = 0; jj < r; ++jj) {
+          if (!__any((unsure >> jj) & 1u)) continue;
+          // this lane's elements of row m, then the sum over the four lanes that share the row
           double part = 0.0;
-          if (row < end)
+#pragma unroll
+          for (int pt = 0; pt < PARTS; ++pt) {
+            // converted where they are used (ahead of the loop, the doubles took 64 registers that are waves in flight)
+            u32x4 raw = __builtin_bit_cast(u32x4, xf[u][pt]);
+            asm volatile("" : "+v"(raw));
+            const vec8 x = __builtin_bit_cast(vec8, raw);
+            const vec8 p8 = *reinterpret_cast<const vec8*>(&lds_p[jj * PITCH + pt * 32 + 8 * kg]);
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-              part = __builtin_fma((double)ha_to_float(xf[u][e]),
-                                   (double)ha_to_float(lds_p[(my_part * 32 + 8 * kg + e) * r + jj]), part);
-          for (int off = 1; off < PARTS; off <<= 1) part += __shfl_xor(part, off);
+              part = __builtin_fma((double)ha_to_float(x[e]), (double)ha_to_float(p8[e]), part);
+            __builtin_amdgcn_sched_barrier(0);
+          }
           part += __shfl_xor(part, 16);
           part += __shfl_xor(part, 32);
-          bin |= (part > 0.0 ? 1 : 0) << jj;
+          const uint32_t bit = 1u << (jj & 3);
+          if (kg == jj >> 2) nib[u] = part > 0.0 ? nib[u] & ~bit : nib[u] | bit;
         }
-        // every lane of a data row now holds its bin; lane L < ROWS must hold the bin of row L
-        bin = __shfl(bin, (lane % ROWS) * PARTS);
-      } else {
-        // data row L of the tile sits in sum q = L % NS of the lanes with kg = L / NS (PARTS <= 4),
-        // or in the lanes with kg = 2*L (PARTS == 8); its bits are 16 consecutive ballot bits
-        const int L = lane % ROWS;
-        const int q = PARTS <= 4 ? L % NS : 0;
-        const int g = PARTS <= 4 ? L / NS : 2 * L;
-        uint64_t sel = pos[0];
-#pragma unroll
-        for (int qq = 1; qq < NS; ++qq) sel = q == qq ? pos[qq] : sel;
-        bin = (int)((sel >> (16 * g)) & ((1u << r) - 1u));
-      }
-      if (lane < ROWS && tile_row0 + lane < end) {
-        if (OUT8)
-          obase8[tile_row0 + lane] = (uint8_t)(bin ^ (bin >> 1));
-        else
-          obase[tile_row0 + lane] = bin ^ (bin >> 1);
       }
     }
+    // the nibbles of a row's slots meet in one lane, rows in order over the lanes, 16 for every tile; after the swap
+    // groups of 16 lanes hold (tile 0, tile 1) of slots 0..3 | 8..11, and of slots 4..7 | 12..15
+    const auto sw = __builtin_amdgcn_permlane16_swap(nib[0], GROUP == 2 ? nib[GROUP - 1] : 0u, false, false);
+    uint32_t bin = sw[0] | sw[1] << 4;
+    if (r > 8) bin |= (uint32_t)__shfl_xor((int)bin, 32) << 8;  // of use in the lower half of the lanes
+    bin = ~bin & ((1u << r) - 1u);
+    if (lane < 16 * GROUP && row0 + lane < end) {
+      if (OUT8)
+        obase8[row0 + lane] = (uint8_t)(bin ^ (bin >> 1));
+      else
+        obase[row0 + lane] = (int32_t)(bin ^ (bin >> 1));
+    }
+    row0 += GROUP * 16;
+    if (row0 >= wave_end) break;
+    load_rows(row0);
   }
 }
 
-template <typename T, int D, bool OUT8>
+template <typename T, int PARTS, bool OUT8>
 int launch_hash_mfma(HashTensors ten, int64_t seqs, const void* proj, int64_t n, int64_t r, int64_t psb, int64_t psh,
                      int64_t d_real, hipStream_t stream) {
   ten.seqs = (int)seqs;
   for (int i = 0; i < 2; ++i)
     if (ten.end[i] <= 0) ten.end[i] = n;
   const int64_t rows = ten.end[0] - ten.first[0] > ten.end[1] - ten.first[1] ? ten.end[0] - ten.first[0] : ten.end[1] - ten.first[1];
-  constexpr int MOST = D >= 128 ? 64 : 32;
-  int tiles = MOST;
-  while (tiles > HASH_LEAST && (rows + 4 * tiles * (16 / (D / 32)) - 1) / (4 * tiles * (16 / (D / 32))) * seqs < HASH_FULL_CHIP) tiles /= 2;
-  const int64_t rows_per_block = 4 * tiles * (16 / (D / 32));
+  constexpr int GROUP = hash_group<PARTS>();
+  int tiles = 2 * GROUP;
+  while (tiles > 1 && (rows + 64 * tiles - 1) / (64 * tiles) * seqs < HASH_FULL_CHIP) tiles /= 2;
+  const int64_t rows_per_block = 64 * tiles;
   if (ten.n_read <= 0 || ten.n_read > n) ten.n_read = n;
   const int64_t gy = seqs < 32768 ? seqs : 32768, gz = (seqs + gy - 1) / gy;
   dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block), (unsigned)gy, (unsigned)gz);
-  auto kernel = tiles == MOST ? lsh_hash_mfma_kernel<T, D, OUT8, MOST>
-                : tiles == 32 ? lsh_hash_mfma_kernel<T, D, OUT8, 32>
-                : tiles == 16 ? lsh_hash_mfma_kernel<T, D, OUT8, 16>
-                : tiles == 8  ? lsh_hash_mfma_kernel<T, D, OUT8, 8>
-                : tiles == 4  ? lsh_hash_mfma_kernel<T, D, OUT8, 4> : lsh_hash_mfma_kernel<T, D, OUT8, HASH_LEAST>;
-  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh, (int)d_real);
+  auto kernel = tiles % GROUP == 0 ? lsh_hash_mfma_kernel<T, PARTS, OUT8, GROUP> : lsh_hash_mfma_kernel<T, PARTS, OUT8, 1>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh, (int)d_real, tiles);
   return ha_launch_status("ha_lsh_hash");
 }
 
@@ -281,14 +270,14 @@ int ha_hash_i32(const void* x, const void* proj, int32_t* buckets, int64_t batch
   ten.heads[0] = ten.heads[1] = (int)heads;
   ten.seqs0 = (int)(batch * heads);
   ten.n_read = n_read;
-  // built for rows of 32, 64, 128 and 256 elements; a shorter row runs in the next width
+  // built for rows of 32, 64, 96, 128 and 256 elements; a shorter row runs in the next width
 #define HA_HASH_MFMA(DD)                                                                                              \
-  if (d <= DD) {                                                                                                      \
-    if (dtype == HA_F16)                                                                                              \
-      return launch_hash_mfma<f16_t, DD, false>(ten, batch * heads, proj, n, r, proj_stride_b, proj_stride_h, d, s);  \
-    return launch_hash_mfma<bf16_t, DD, false>(ten, batch * heads, proj, n, r, proj_stride_b, proj_stride_h, d, s);   \
+  if (d <= DD) {                                                                                                          \
+    if (dtype == HA_F16)                                                                                                  \
+      return launch_hash_mfma<f16_t, DD / 32, false>(ten, batch * heads, proj, n, r, proj_stride_b, proj_stride_h, d, s); \
+    return launch_hash_mfma<bf16_t, DD / 32, false>(ten, batch * heads, proj, n, r, proj_stride_b, proj_stride_h, d, s);  \
   }
-  HA_HASH_MFMA(32) HA_HASH_MFMA(64) HA_HASH_MFMA(128) HA_HASH_MFMA(256)
+  HA_HASH_MFMA(32) HA_HASH_MFMA(64) HA_HASH_MFMA(96) HA_HASH_MFMA(128) HA_HASH_MFMA(256)
 #undef HA_HASH_MFMA
   return ha_fail(HA_ERR_HEADDIM, "ha_lsh_hash: d must be a multiple of 8 in [8, 256]");
 }
@@ -314,11 +303,11 @@ int ha_hash_pair_u8(const void* q, const void* k, const void* proj, uint8_t* ids
   ten.first[1] = 0; ten.end[1] = k_end;
   const int64_t seqs = batch * (heads + kv_heads);
 #define HA_HASH_PAIR(DD)                                                                                  \
-  if (d <= DD) {                                                                                          \
-    if (dtype == HA_F16) return launch_hash_mfma<f16_t, DD, true>(ten, seqs, proj, n, r, 0, 0, d, stream); \
-    return launch_hash_mfma<bf16_t, DD, true>(ten, seqs, proj, n, r, 0, 0, d, stream);                    \
+  if (d <= DD) {                                                                                               \
+    if (dtype == HA_F16) return launch_hash_mfma<f16_t, DD / 32, true>(ten, seqs, proj, n, r, 0, 0, d, stream); \
+    return launch_hash_mfma<bf16_t, DD / 32, true>(ten, seqs, proj, n, r, 0, 0, d, stream);                    \
   }
-  HA_HASH_PAIR(32) HA_HASH_PAIR(64) HA_HASH_PAIR(128)
+  HA_HASH_PAIR(32) HA_HASH_PAIR(64) HA_HASH_PAIR(96) HA_HASH_PAIR(128)
 #undef HA_HASH_PAIR
   return ha_fail(HA_ERR_UNSUPPORTED, "ha_forward: paired hash not built for head dim %lld", (long long)d);
 }
