@@ -99,7 +99,7 @@ void fill_params(const ha_attn_operands& t, ha_attn_kernel_params& p) {
   p.n_q_last = (int)t.n_q;
   p.lse_rows = (int)t.lse_rows;
   p.tiles_per_wg = 1;
-  p.rag_levels = -1; p.rag_split = 0; p.rag_n = 0;
+  p.rag_levels = -1; p.rag_n = 0;
   for (int& c : p.rag_half) c = 0;
   p.scale_log2 = t.scale * LOG2E_F;
 }
@@ -135,8 +135,8 @@ int block_attn(const ha_block_attn_args& a, hipStream_t stream, int64_t n_q_last
 
 // Ragged segments of an exact launch inside a causal recursion with odd lengths (see ha_attn_kernel_params)
 struct Ragged {
-  int levels, split, n;
-  int half[HA_MAX_RAGGED_LEVELS + 1];
+  int levels, n;
+  int half[HA_MAX_RAGGED_LEVELS];
 };
 
 int flash_attn(const ha_attn_operands& t, int causal, int accumulate, hipStream_t stream, const Ragged* rag = nullptr) {
@@ -146,8 +146,8 @@ int flash_attn(const ha_attn_operands& t, int causal, int accumulate, hipStream_
   fill_params(t, p);
   p.accumulate = accumulate != 0;
   if (rag) {
-    p.rag_levels = rag->levels; p.rag_split = rag->split; p.rag_n = rag->n;
-    for (int i = 0; i <= HA_MAX_RAGGED_LEVELS; ++i) p.rag_half[i] = rag->half[i];
+    p.rag_levels = rag->levels; p.rag_n = rag->n;
+    for (int i = 0; i < HA_MAX_RAGGED_LEVELS; ++i) p.rag_half[i] = rag->half[i];
   }
   return ha_attn_launch(p, (int)t.d, (int)t.dv, t.dtype, false, causal != 0, false, stream);
 }
@@ -571,33 +571,36 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     return flash_attn(f, 0, 0, stream);
   }
 
-  // Exact launches over the segments of level `level` (leaves: level == pl.levels, whole segments with the
-  // causal mask; else the off-diagonal part of that level: second halves against first halves).  With an odd
-  // length somewhere the segments are ragged: the kernel finds each segment's rows from the plan.
-  auto exact_level = [&](int level, bool leaves) -> int {
+  // Exact causal attention on the segments of level `level`.  With an odd length somewhere the segments are ragged:
+  // the kernel finds each segment's rows from the plan.
+  auto exact_level = [&](int level) -> int {
     ha_attn_operands f = t;
-    const int64_t rows = leaves ? pl.len[level] : pl.half[level];
+    const int64_t rows = pl.len[level];
     f.n_q = f.n_k = rows;
     f.segs = 1ll << level;
-    f.seg_stride_rows = leaves ? rows : 2 * rows;
-    f.q_seg_offset = leaves ? 0 : rows;
-    f.k_seg_offset = 0;
+    f.seg_stride_rows = rows;
+    f.q_seg_offset = f.k_seg_offset = 0;
     if (pl.levels == 0) f.lse_rows = a.lse_rows;
-    if (!pl.ragged) return flash_attn(f, leaves ? 1 : 0, leaves ? 0 : 1, stream);
+    if (!pl.ragged || level == 0) return flash_attn(f, 1, 0, stream);
     Ragged rag = {};
     rag.levels = level;
-    rag.split = leaves ? 0 : 1;
     rag.n = (int)a.n;
-    for (int i = 0; i <= level && i < pl.levels; ++i) rag.half[i] = (int)pl.half[i];
-    return flash_attn(f, leaves ? 1 : 0, leaves ? 0 : 1, stream, &rag);
+    for (int i = 0; i < level; ++i) rag.half[i] = (int)pl.half[i];
+    return flash_attn(f, 1, 0, stream, &rag);
   };
 
-  // 3. leaves: exact causal attention on every segment of the deepest level
-  st = exact_level(pl.levels, true);
+  // 3. leaves: exact causal attention on every segment of the deepest level.  Where the deepest level's off-diagonal part is
+  // exact too (halves below min_seq_len: every length but powers of two times it), the two are one launch over
+  // that level's segments, which are exact causal attention as a whole: the same pairs, with the second halves' rows
+  // set up, merged and written once and one launch's last round of workgroups less.  Two launches | one, in us: 16 heads of 2100 rows
+  // 33.9 | 20.9, 24 of 5000 98.6 | 90.7, 96 of 6000 476 | 464, d = 128 24 of 2600 71.5 | 52.1, 64 of 7296 871 | 842; the worst of
+  // 176 sizes, 16 of 7296 at d = 64, 131.3 | 133.5.
+  const int leaf_level = pl.levels > 0 && !pl.level_hyper[pl.levels - 1] ? pl.levels - 1 : pl.levels;
+  st = exact_level(leaf_level);
   if (st != HA_OK) return st;
   // 4. off-diagonal parts, deepest level first, merged in place into the second halves
-  for (int j = pl.levels - 1; j >= 0; --j) {
-    st = pl.level_hyper[j] ? hyper_level(j, true) : exact_level(j, false);
+  for (int j = leaf_level - 1; j >= 0; --j) {
+    st = hyper_level(j, true);
     if (st != HA_OK) return st;
   }
   return HA_OK;

@@ -59,10 +59,9 @@ struct ha_attn_kernel_params {
   // segments of a level neither start at multiples of one stride nor hold the same number of rows: level i
   // cuts a segment of (padded) length 2*rag_half[i] into two, and the rows that exist are the first rag_n of
   // the whole sequence.  Segment number `seg` has rag_levels bits, most significant first: bit i says which
-  // half of its level-i ancestor it lies in.  rag_split: the launch is the off-diagonal part of the level
-  // below (queries = second half, keys = first half of the segment, halves of rag_half[rag_levels] rows).
-  int rag_levels, rag_split, rag_n;
-  int rag_half[HA_MAX_RAGGED_LEVELS + 1];
+  // half of its level-i ancestor it lies in.
+  int rag_levels, rag_n;
+  int rag_half[HA_MAX_RAGGED_LEVELS];
   // the divisors of the workgroup -> (head, segment, tile) decomposition as multiply-and-shift
   // constants (filled by ha_attn_launch): the kernel never divides
   ha_divisor div_qtiles, div_segs, div_heads, div_kv_heads, div_kv_group, div_block_tiles;

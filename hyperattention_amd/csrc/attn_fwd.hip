@@ -303,17 +303,8 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
         real = min(real, c);
       }
     }
-    if (p.rag_split) {
-      const int c = p.rag_half[p.rag_levels];
-      r.q_row = start + c;
-      r.k_row = start;
-      r.n_q = min(max(real - c, 0), c);
-      r.n_k = min(real, c);
-    } else {
-      r.q_row = r.k_row = start;
-      r.n_q = r.n_k = real;
-    }
-    r.o_row = r.q_row;
+    r.o_row = r.q_row = r.k_row = start;
+    r.n_q = r.n_k = real;
   }
   return r;
 }
