@@ -54,7 +54,8 @@ struct ha_attn_kernel_params {
   int tiles_per_wg;
   int split_keys;  // the keys of a query tile are split over the waves of a workgroup, 2: longest tiles first (filled by
                    // ha_attn_launch)
-  int follow_max;  // exact causal kernel: the FOLLOW instance (filled by ha_attn_launch)
+  int small_tiles;  // head dims up to 64: tiles of 128 queries (filled by ha_attn_launch)
+  int follow_max;  // the FOLLOW instances; gathered: in that many chunks (filled by ha_attn_launch)
   // Ragged segments (exact kernels; rag_levels < 0: regular).  Inside a causal recursion with odd lengths the
   // segments of a level neither start at multiples of one stride nor hold the same number of rows: level i
   // cuts a segment of (padded) length 2*rag_half[i] into two, and the rows that exist are the first rag_n of

@@ -185,18 +185,17 @@ __device__ __forceinline__ void half_step_order() {
 //   VALU  : P of this half-step from s_use -> pb (for the next block) and the row sums
 //   follow: the reference exponents follow the rows' maxima, raised at every step of 32 keys
 //   LDS   : V^T of this half-step's keys (v_key_off.. of v_tile) -> vf (for the next block)
-template <typename T, int D, int H, int DC>
-__device__ __forceinline__ void half_step(const f32x16 (&s_use)[WaveShape<D>::NB], f32x16 (&s_fill)[WaveShape<D>::NB],
+template <typename T, int D, int H, int DC, int NB>
+__device__ __forceinline__ void half_step(const f32x16 (&s_use)[NB], f32x16 (&s_fill)[NB],
                                           const unsigned char* k_tile, int k_row_off,
                                           const unsigned char* v_tile, int v_key_off, const LaneOffsets<DC>& lo,
-                                          const typename ElemTraits<T>::vec8 (&qf)[WaveShape<D>::NB][DC / 16],
-                                          f32x16 (&acc)[DC / 32][WaveShape<D>::NB], float (&m_run)[WaveShape<D>::NB],
-                                          float (&l_run)[WaveShape<D>::NB],
-                                          typename ElemTraits<T>::vec8 (&pb)[WaveShape<D>::NB],
+                                          const typename ElemTraits<T>::vec8 (&qf)[NB][DC / 16],
+                                          f32x16 (&acc)[DC / 32][NB], float (&m_run)[NB],
+                                          float (&l_run)[NB],
+                                          typename ElemTraits<T>::vec8 (&pb)[NB],
                                           typename ElemTraits<T>::vec8 (&vf)[DC / 32], float scale_log2,
                                           bool follow = false) {
   typedef typename ElemTraits<T>::vec8 vec8;
-  constexpr int NB = WaveShape<D>::NB;
   constexpr int KH = DC / 32;  // k-steps of this half
   constexpr int DB = DC / 32;
 
@@ -309,18 +308,19 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
   return r;
 }
 
-// FOLLOW (exact causal kernel, single tiles): the reference exponents of a sequence's first tile follow the row maxima.  An
+// FOLLOW (p.follow_max): the reference exponents follow the row maxima at every step of 32 keys, in exact causal single tiles in a
+// sequence's first tile, gathered (plain or not, tiles of 128 queries at head dim 64) in the first half of a row's keys.  An
 // instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
 template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D, bool FOLLOW = false>
-__global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
+__global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
-  constexpr int NB = WaveShape<D>::NB;        // 32-query column blocks per wave
-  constexpr int QW = WaveShape<D>::QW;        // queries per wave
+  constexpr int QW = 32 * NB;                 // queries per wave
   constexpr int WAVES = WaveShape<D>::WAVES;  // waves per workgroup
-  constexpr int WG_QUERIES = WaveShape<D>::QUERIES;
+  constexpr int WG_QUERIES = QW * WAVES;
   constexpr int REF_TILES = WG_QUERIES / 128;  // reference query tiles of 128 per workgroup
+  static_assert(!GATHER || PLAIN || REF_TILES == 1, "two reference tiles of a workgroup share their keys");
   constexpr int DV = D;
   constexpr int KSTEPS = DC / 16;  // MFMA k-steps of Q.K^T
   constexpr int DB = DC / 32;      // 32-row blocks of O^T
@@ -421,9 +421,9 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, 2) void ha_attn_fwd_kernel(c
 namespace {
 
 template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D, bool FOLLOW = false>
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
 int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT, DC, FOLLOW>), dim3(grid),
+  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT, DC, FOLLOW, NB>), dim3(grid),
                      dim3(WaveShape<D>::THREADS), 0, stream, p);
   return ha_launch_status(what);
 }
@@ -448,7 +448,7 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
   }
   // the plain instance: d = 96, 16 heads of 32768 rows 205 -> 182 us, d = 40 98 -> 88
   if (gather && plain) return launch_one<T, D, true, false, true, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
-  if (gather) return launch_one<T, D, true, false, false, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
+  if (gather) return launch_one<T, D, true, false, false, true, false, DC, false, 1>(p, grid, stream, "ha_block_attn_fwd");
   if (causal && p.follow_max) return launch_one<T, D, false, true, false, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
   return launch_one<T, D, false, false, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
@@ -457,7 +457,7 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
 template <typename T, int D>
 int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, bool reweight, hipStream_t stream) {
   if (gather && reweight)  // the entry point has checked that the head dims are the built ones
-    return launch_one<T, D, true, false, false, false, true>(p, grid, stream, "ha_block_attn_fwd");
+    return launch_one<T, D, true, false, false, false, true, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
   // also with an odd number of tiles: d = 128, 32 heads of 80000 rows in blocks of 512, the whole call 1907 us with the
   // general instance, 1827 with the plain one; d = 80, 24 of 110464, blocks of 256 1177 -> 1158
   const bool plain = !p.smooth && !p.sampled_idx && (p.block_tiles * 128) % WaveShape<D>::QUERIES == 0;
@@ -474,12 +474,20 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
   }
   if (gather) {
     if constexpr (D == 64) if (p.tiles_per_wg > 1) {  // set by ha_attn_launch for the instances built below
-      if (plain) hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, true>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
-      else hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D, false>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
+      hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
       return ha_launch_status("ha_block_attn_fwd");
     }
+    if constexpr (D == 64) {
+      if (plain && p.follow_max) return launch_one<T, D, true, false, true, false, false, D, true, 1>(p, grid, stream, "ha_block_attn_fwd");
+      if (p.follow_max) return launch_one<T, D, true, false, false, false, false, D, true, 1>(p, grid, stream, "ha_block_attn_fwd");
+      if (plain && p.small_tiles) return launch_one<T, D, true, false, true, false, false, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
+    }
     if (plain) return launch_one<T, D, true, false, true>(p, grid, stream, "ha_block_attn_fwd");
-    return launch_one<T, D, true, false>(p, grid, stream, "ha_block_attn_fwd");
+    return launch_one<T, D, true, false, false, false, false, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
+  }
+  if constexpr (D == 64) if (p.small_tiles) {
+    if (causal) return launch_one<T, D, false, true, false, false, false, D, true, 1>(p, grid, stream, "ha_flash_attn_fwd");
+    return launch_one<T, D, false, false, false, false, false, D, false, 1>(p, grid, stream, "ha_flash_attn_fwd");
   }
   if (causal && p.follow_max) return launch_one<T, D, false, true, false, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
@@ -518,8 +526,17 @@ static ha_divisor make_divisor(int64_t y) {
 // is kept because the split form is the closer one to float64 (four exact weights per row: 2 to 4 % for 256 to 1024 keys a row,
 // 0.2 to 2 % above), and the launches that it gives to it lose little: 8 heads of 2048 rows, blocks and samples of 128 10.7 | 12.2,
 // 256 14.5 | 14.5, 512 22.8 | 19.8; without mask 12 of 1000 19.8 | 17.1, 4 of 4096 57 | 44, but 8 of 4096 68 | 85.
+//
+// d = 64, tiles of 256 | 128 queries (`large`, `small`; 470 launches of 6 to 512 heads, 512 to 8192 rows, mean error 3 %; a choice that lost 2.5 % or more is not among them).  A
+// workgroup of 128 queries takes half as long, a CU holds three, and ragged rows waste less; its waves read the keys
+// for half as many queries, 10 % more time on a full chip.  Exact causal, us: 48 heads of 700 rows 16.8 | 13.4, of 2048 40.0 | 35.9, 32 of 3000 53.8 |
+// 48.6, 64 of 1000 23.2 | 18.6, 24 of 4096 70.3 | 64.5, but 48 of 4096 113 | 115.5, 160 of 4096 341 | 376; without mask 32 of 1000 21.0 |
+// 16.1, 48 of 2048 62 | 58, 64 of 2048 69 | 76; whole calls with blocks and samples of 256: 16 heads of 2560 rows 24.6 | 23.7, 24 of
+// 4096 37.0 | 36.0, 24 of 6144 54.5 | 51.2, 24 of 8192 58.3 | 59.4.
 struct LaunchTimes {
   double whole, single, split;  // a tile per workgroup (exact causal: pairs of tiles), single causal tiles, the split kernel
+  double large, small;          // d = 64: tiles of 256 and of 128 queries (exact causal: single ones)
+  double split_rounds;          // the split kernel's with whole rounds of workgroups per CU
 };
 static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   struct Fit {
@@ -556,11 +573,33 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
     }
   }
 
+  t.large = t.small = 0;
+  if (width == 64) {
+    // start, a chunk of 64 keys, its slowdown by the neighbours; causal: a CU's share of chunks and of workgroups,
+    // and what more than three of them cost (`less`: a CU holds three small ones); else a
+    // round's chunks and what it costs beside them, in whole rounds while they are few
+    struct TileFit {
+      double start, chunk, crowd, share, less, per_wg;
+    };
+    auto time = [&](double rows, const TileFit& c) {
+      const double count = std::ceil(p.n_q / rows), wgs = vheads * count / cus;
+      if (paired) {
+        const double longest = rows / 64 * count, share = wgs * (count + 1) * rows / 128;
+        return c.start + std::max(c.chunk * (longest + c.crowd * share), c.share * share + c.per_wg * wgs + (wgs > 3 ? c.less : 0));
+      }
+      const double rounds = wgs <= 1 ? 1 + c.crowd * wgs : c.share * (wgs <= 6 ? std::ceil(wgs) : wgs + 0.3) - c.less;
+      return c.start + (std::ceil(keys / 64.) * c.chunk + c.per_wg) * rounds;
+    };
+    t.large = time(256, paired ? TileFit{8.2, 0.783, 0.261, 0.912, 0., 2.2} : TileFit{5.85, 0.815, 0.156, 1.222, 0.33, 1.41});
+    t.small = time(128, paired ? TileFit{7.2, 0.51, 0.29, 0.524, 1.5, 1.2} : TileFit{5.05, 0.542, 0.139, 1.005, 0.235, 1.1});
+  }
+
   const double chain = std::ceil(keys / 128.), split_per_cu = vheads * split_tiles / cus;
   double all;
   if (paired) all = split_per_cu * (chain / 2 + 0.5 + f.set_up) - f.hidden * chain;
   else all = (width == 64 ? split_per_cu : std::ceil(split_per_cu)) * (chain + f.set_up);
   t.split = f.split_start + f.split_step * std::max(chain + f.set_up, all);
+  t.split_rounds = f.split_start + f.split_step * std::ceil(split_per_cu) * (chain + f.set_up);
   return t;
 }
 
@@ -589,23 +628,46 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   const int width = d <= 64 && dv <= 64 ? 64 : 128;
   p.qk_pieces = d / 8;
   p.v_pieces = dv / 8;
-  const int tile_rows = width == 64 ? WaveShape<64>::QUERIES : WaveShape<128>::QUERIES;
-  int64_t qtiles = (p.n_q + tile_rows - 1) / tile_rows;
   const bool single = causal && !gather && single_tiles(p, width);
-  if (causal && !gather && !single) qtiles = (qtiles + 1) / 2;  // one workgroup per pair of tiles
-  // Gathered attention at head dim 64 with whole 256-query tiles, whole key blocks and an even number of at least four key
-  // chunks per tile can run as a stream: a workgroup takes a run of tiles of its head
-  // (ha_attn_fwd_stream_kernel).  It measured 2 to 5 % slower than one tile per workgroup with two workgroups per CU,
-  // so only the measurement aid below asks for it.
   p.tiles_per_wg = 1;
   const char* stream_env = getenv("HA_STREAM_TILES");  // measurement aid: force the run length (1: off)
   const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0;
+  const bool full_rows = p.qk_pieces == width / 8 && p.v_pieces == width / 8;
   const LaunchTimes t = launch_times(p, width, gather, causal);
   const char* split_env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
   // (a forced run length asks for the 256-query kernels)
   p.split_keys = !reweight && !(gather && stream_env) && (split_env ? atoi(split_env) != 0 : t.split < (single ? t.single : t.whole));
+  // Head dims up to 64, tiles of 128 queries: gathered launches that are not plain always, since two tiles of 128 share neither
+  // their window nor a block of 128 (a workgroup of 256 queries went through what either has, 1.05 to 1.2 times the time from 4
+  // heads of 4096 rows to 128 of 32768, smooth blocks of 512 0.99 to 1.07); others of full rows by the estimates.
+  // Gathered ones take the place of the split kernel where that has more workgroups than CUs.  It is the closer one to float64, so the
+  // exponents follow the row maxima in half of the chunks: 0.97 to 0.99 of its error with blocks and samples of 128 and 256
+  // (without 1.01 and more), 12 heads of 2560 rows, blocks of 128 20.9 -> 19.7 us, 256 23.3 -> 22.4, 12 of 3072 25.8 -> 22.7
+  // and 29.1 -> 26.2.  With 1024 keys a row the half costs what the tiles gain.
+  p.small_tiles = p.follow_max = 0;
+  const bool choice = width == 64 && full_rows && !reweight && !(gather && stream_env);
+  const int chunks = 2 * p.block_tiles + p.sample_chunks;  // gathered: of a row's keys
+  if (choice && gather && p.split_keys && !split_env && chunks <= 8 && t.small + 1.5 < t.split_rounds) {
+    p.split_keys = 0;
+    p.small_tiles = 1;
+    p.follow_max = (chunks + 1) / 2;
+  } else if (width == 64 && gather && (!plain || reweight)) {
+    p.small_tiles = !p.split_keys;
+  } else if (choice && causal && !gather) {
+    p.small_tiles = single && !split_env && 1.01 * t.small < std::min(t.large, t.split);
+    if (p.small_tiles) p.split_keys = 0;
+  } else if (choice && !p.split_keys) {
+    p.small_tiles = 1.02 * t.small < t.large;
+  }
+  const int tile_rows = width == 64 && !p.small_tiles ? WaveShape<64>::QUERIES : WaveShape<128>::QUERIES;
+  int64_t qtiles = (p.n_q + tile_rows - 1) / tile_rows;
+  if (causal && !gather && !single) qtiles = (qtiles + 1) / 2;  // one workgroup per pair of tiles
   if (p.split_keys) qtiles = (p.n_q + 63) / 64;
-  else if (stream_env && gather && !reweight && width == 64 && p.qk_pieces == width / 8 && p.v_pieces == width / 8 && p.n_q % STREAM_QUERIES == 0 &&
+  // A plain gathered launch with whole 256-query tiles, whole key blocks and an even number of at least four key
+  // chunks per tile can run as a stream: a workgroup takes a run of tiles of its head
+  // (ha_attn_fwd_stream_kernel).  It measured 2 to 5 % slower than one tile per workgroup with two workgroups per CU,
+  // so only the measurement aid asks for it.
+  else if (stream_env && gather && !reweight && width == 64 && plain && full_rows && p.n_q % STREAM_QUERIES == 0 &&
            p.n_q >= 2 * STREAM_QUERIES && p.sample_chunks % 2 == 0 && p.n_k % (p.block_tiles * 128) == 0 &&
            2 * p.block_tiles + p.sample_chunks >= 4) {
     const int r = std::min(atoi(stream_env), p.n_q / STREAM_QUERIES);
@@ -617,7 +679,7 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
   if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
   if (single && !p.split_keys) p.tiles_per_wg = 0;
-  p.follow_max = single && !p.split_keys && (width == 128 || t.split < t.whole);
+  if (single && !p.split_keys) p.follow_max = width == 128 || t.split < t.whole;
   p.div_qtiles = make_divisor(p.split_keys == 2 || p.tiles_per_wg == 0 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);
