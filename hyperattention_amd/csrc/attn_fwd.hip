@@ -518,10 +518,10 @@ static ha_divisor make_divisor(int64_t y) {
 // heads, grouped and not, 300 to 4133 rows exact, 2048 to 16384 rows hashed).  Times whole | split in us, causal: 24 heads of 1000
 // rows 31 | 13, of 2048 39 | 28, of 4096 72 | 72; 48 of 2048 41 | 45, of 4096 116 | 143; without mask 16 of 4096 rows
 // 75 | 86.
-// d = 128, causal: fitted to 64 launches, at which the choice is 1 % slower than the best one on average (worst: 32 heads of 520 rows, 14.9 |
-// 17.7, 12 of 3000 49.0 | 53.5; 4 % and less beyond 24 of 1000).  Single tiles of 128
-// queries | split: 12 heads of 1000 rows 20.7 | 17.2, 24 21.8 | 23.0, 48 25.1 | 37; 16 of 2048 35.3 | 34.3, 24 38.4 | 50; 8 of
-// 4096 65 | 51, 12 70 | 85.
+// d = 128, causal: fitted to 93 launches each of 128 and of 96 columns (4 to 128 heads of 512 to 4096 rows), at which the choice
+// is 0.2 % slower than the best one on average (worst: 40 heads of 512 rows, 96 columns 10 %, 24 of 700, 128 columns 8 %).  Single tiles of 128
+// queries | split: 12 heads of 1000 rows 20.7 | 17.2, 24 of 1000 20.6 | 22.3, 48 25.1 | 37; 8 of 512 13.3 | 12.3, 96 columns 13.2 | 10.3;
+// 16 of 2048 35.3 | 34.3, 24 38.4 | 50; 8 of 4096 65 | 51, 12 70 | 85.
 // d = 128, without mask or gathered: the estimate of `whole` is that of a kernel of 256-query tiles, which the present one outruns.  It
 // is kept because the split form is the closer one to float64 (four exact weights per row: 2 to 4 % for 256 to 1024 keys a row,
 // 0.2 to 2 % above), and the launches that it gives to it lose little: 8 heads of 2048 rows, blocks and samples of 128 10.7 | 12.2,
@@ -541,12 +541,13 @@ struct LaunchTimes {
 static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool gather, bool causal) {
   struct Fit {
     double step, pair, start, crowd, second, share, rest;    // 256-query tiles
-    double split_step, split_start, set_up, hidden;          // split kernel
+    double split_step, split_start, set_up, share_up, hidden;  // split kernel; share_up: the set-up in a CU's share
   };
   const bool paired = causal && !gather;
-  const Fit f = width == 64 ? Fit{0.97, 4.4, 6.2, 0.08, 1.85, 0.94, 0.45, 0.56, 5.6, 4.3, 0.34}
-                : paired    ? Fit{0, 0, 0, 0, 0, 0, 0, 1.03, 1.3, 7.9, 0.}
-                            : Fit{1.25, 2.0, 7.0, 0.37, 1.47, 1.58, 0.29, 1.23, 1.3, 5.4, 0.22};
+  const bool columns_96 = p.qk_pieces <= 12 && p.v_pieces <= 12;
+  const Fit f = width == 64 ? Fit{0.97, 4.4, 6.2, 0.08, 1.85, 0.94, 0.45, 0.56, 5.6, 4.3, 4.3, 0.34}
+                : paired    ? (columns_96 ? Fit{0, 0, 0, 0, 0, 0, 0, 1.02, 4.0, 2.4, 4.9, 0.} : Fit{0, 0, 0, 0, 0, 0, 0, 1.07, 4.2, 3.5, 6.4, 0.})
+                            : Fit{1.25, 2.0, 7.0, 0.37, 1.47, 1.58, 0.29, 1.23, 1.3, 5.4, 5.4, 0.22};
   const double cus = 256., vheads = (double)p.batch * p.heads * p.segs;
   const double tiles = (p.n_q + 255) / 256, split_tiles = (p.n_q + 63) / 64;
   const double keys = gather ? 128. * p.block_tiles + 64. * p.sample_chunks : p.n_k;
@@ -555,8 +556,9 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
   if (paired && width == 128) {
     // two workgroups of 128 queries per CU: the longest chain, slowed by its neighbour, or a CU's share of all
     const double tiles_128 = (p.n_q + 127) / 128, wgs = vheads * tiles_128 / cus;
-    const double longest = 2. * tiles_128 * (1 + 0.4 * std::min(1., wgs / 2)), share = wgs * (tiles_128 + 1);
-    t.single = 6.6 + std::max(0.78 * longest, 0.895 * share + 3.1 * wgs - 1.);
+    const double longest = 2. * tiles_128, beside = std::min(1., wgs / 2), share = wgs * (tiles_128 + 1);
+    t.single = columns_96 ? 7.8 + std::max(0.638 * longest * (1 + 0.376 * beside), 0.748 * share + 2.57 * wgs)
+                          : 7.65 + std::max(0.688 * longest * (1 + 0.478 * beside), 0.929 * share + 1.71 * wgs + 2.3);
     t.whole = t.single;  // pairs are for launches far larger than those the split kernel is for
   } else {
     const double per_cu = vheads * (paired ? std::ceil(tiles / 2) : tiles) / cus;
@@ -596,8 +598,8 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
 
   const double chain = std::ceil(keys / 128.), split_per_cu = vheads * split_tiles / cus;
   double all;
-  if (paired) all = split_per_cu * (chain / 2 + 0.5 + f.set_up) - f.hidden * chain;
-  else all = (width == 64 ? split_per_cu : std::ceil(split_per_cu)) * (chain + f.set_up);
+  if (paired) all = split_per_cu * (chain / 2 + 0.5 + f.share_up) - f.hidden * chain;
+  else all = (width == 64 ? split_per_cu : std::ceil(split_per_cu)) * (chain + f.share_up);
   t.split = f.split_start + f.split_step * std::max(chain + f.set_up, all);
   t.split_rounds = f.split_start + f.split_step * std::ceil(split_per_cu) * (chain + f.set_up);
   return t;
