@@ -258,10 +258,13 @@ __device__ __forceinline__ void half_step(const f32x16 (&s_use)[NB], f32x16 (&s_
 
 }  // namespace
 
-// PLAIN (gathered kernel only): the common configuration, for which the per-iteration bookkeeping of the
-// general one is compiled out: no smoothing, default samples (rows 0 .. sample_size-1), and both
-// 128-query tiles of the workgroup inside one key block (d = 64; at d = 128 it has one), so no chunk is ever masked for half of it
-// (where the second tile is past the end, its waves work on row 0 and store nothing).
+// FORM (gathered kernel only): the common configurations, default samples (rows 0 .. sample_size-1), have instances in which the
+// general one's source of sampled rows and, for PLAIN blocks, the wrap of smooth windows are compiled out of every iteration.  Two 128-query
+// tiles of a workgroup (d = 64) share their keys: PLAIN with both inside one key block (where the second tile is past the end, its
+// waves work on row 0 and store nothing); the other forms have one.  SMOOTH against the general instance: 2 x 32 heads of 65536
+// rows, d = 128, blocks of 512, the whole call 2897 -> 2820 us; d = 64, 32 of 36352 437 -> 428.
+enum GatherForm { GENERAL = 0, PLAIN = 1, SMOOTH = 2 };
+
 // Head dims below the built width D (NARROW kernels): a row holds fewer 16-byte pieces than its LDS slot.
 // A lane whose piece lies past the end of the row fetches these zeros instead, so the tiles hold the rows
 // zero-padded to D: zero columns change neither q.k nor the other columns of the output.
@@ -311,7 +314,7 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
 // FOLLOW (p.follow_max): the reference exponents follow the row maxima at every step of 32 keys, in exact causal single tiles in a
 // sequence's first tile, gathered (plain or not, tiles of 128 queries at head dim 64) in the first half of a row's keys.  An
 // instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
-template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
+template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
           int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
 __global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) 
   constexpr int WAVES = WaveShape<D>::WAVES;  // waves per workgroup
   constexpr int WG_QUERIES = QW * WAVES;
   constexpr int REF_TILES = WG_QUERIES / 128;  // reference query tiles of 128 per workgroup
-  static_assert(!GATHER || PLAIN || REF_TILES == 1, "two reference tiles of a workgroup share their keys");
+  static_assert(!GATHER || FORM == PLAIN || REF_TILES == 1, "two reference tiles of a workgroup share their keys");
   constexpr int DV = D;
   constexpr int KSTEPS = DC / 16;  // MFMA k-steps of Q.K^T
   constexpr int DB = DC / 32;      // 32-row blocks of O^T
@@ -420,10 +423,10 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) 
 
 namespace {
 
-template <typename T, int D, bool GATHER, bool CAUSAL, bool PLAIN = false, bool NARROW = false, bool REWEIGHT = false,
+template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
           int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
 int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, PLAIN, NARROW, REWEIGHT, DC, FOLLOW, NB>), dim3(grid),
+  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, FORM, NARROW, REWEIGHT, DC, FOLLOW, NB>), dim3(grid),
                      dim3(WaveShape<D>::THREADS), 0, stream, p);
   return ha_launch_status(what);
 }
@@ -435,61 +438,64 @@ int launch_split(const ha_attn_kernel_params& p, int grid, hipStream_t stream, c
   return ha_launch_status(what);
 }
 
+// gathered launches in workgroups of 128 queries
+template <typename T, int D, bool NARROW, int DC, bool FOLLOW = false>
+int launch_gathered(const ha_attn_kernel_params& p, int grid, GatherForm form, hipStream_t stream) {
+  const char* const what = "ha_block_attn_fwd";
+  if (form == PLAIN) return launch_one<T, D, true, false, PLAIN, NARROW, false, DC, FOLLOW, 1>(p, grid, stream, what);
+  if (form == SMOOTH) return launch_one<T, D, true, false, SMOOTH, NARROW, false, DC, FOLLOW, 1>(p, grid, stream, what);
+  return launch_one<T, D, true, false, GENERAL, NARROW, false, DC, FOLLOW, 1>(p, grid, stream, what);
+}
+
 // Head dims below the built width.  At D = 128 the ones up to 96 (80 and 96 are models' head dims) compute with three
 // quarters of the row: a quarter of the MFMAs and LDS operand reads and 30 to 40 registers less.  16 heads of 20479
 // causal rows of d = 96: 546 -> 507 us (gathered level 87 -> 76, leaves 173 -> 151); 8 heads of 16384 rows without mask:
 // 896 -> 791 us.
 template <typename T, int D, int DC>
-int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, bool plain, hipStream_t stream) {
+int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, GatherForm form, hipStream_t stream) {
   if (p.split_keys) {
     if (gather) return launch_split<T, D, true, false, true, DC>(p, grid, stream, "ha_block_attn_fwd");
     if (causal) return launch_split<T, D, false, true, true, DC>(p, grid, stream, "ha_flash_attn_fwd");
     return launch_split<T, D, false, false, true, DC>(p, grid, stream, "ha_flash_attn_fwd");
   }
   // the plain instance: d = 96, 16 heads of 32768 rows 205 -> 182 us, d = 40 98 -> 88
-  if (gather && plain) return launch_one<T, D, true, false, true, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
-  if (gather) return launch_one<T, D, true, false, false, true, false, DC, false, 1>(p, grid, stream, "ha_block_attn_fwd");
-  if (causal && p.follow_max) return launch_one<T, D, false, true, false, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
-  if (causal) return launch_one<T, D, false, true, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
-  return launch_one<T, D, false, false, false, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
+  if (gather && D == 64 && !p.small_tiles) return launch_one<T, D, true, false, PLAIN, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
+  if (gather) return launch_gathered<T, D, true, DC>(p, grid, form, stream);
+  if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
+  if (causal) return launch_one<T, D, false, true, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
+  return launch_one<T, D, false, false, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
 }
 
 template <typename T, int D>
 int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, bool reweight, hipStream_t stream) {
   if (gather && reweight)  // the entry point has checked that the head dims are the built ones
-    return launch_one<T, D, true, false, false, false, true, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
-  // also with an odd number of tiles: d = 128, 32 heads of 80000 rows in blocks of 512, the whole call 1907 us with the
-  // general instance, 1827 with the plain one; d = 80, 24 of 110464, blocks of 256 1177 -> 1158
-  const bool plain = !p.smooth && !p.sampled_idx && (p.block_tiles * 128) % WaveShape<D>::QUERIES == 0;
+    return launch_one<T, D, true, false, GENERAL, false, true, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
+  const GatherForm form = p.sampled_idx ? GENERAL : p.smooth ? SMOOTH : PLAIN;
   if (p.qk_pieces != D / 8 || p.v_pieces != D / 8) {
     if constexpr (D == 128) {
-      if (p.qk_pieces <= 12 && p.v_pieces <= 12) return launch_narrow<T, D, 96>(p, grid, gather, causal, plain, stream);
+      if (p.qk_pieces <= 12 && p.v_pieces <= 12) return launch_narrow<T, D, 96>(p, grid, gather, causal, form, stream);
     }
-    return launch_narrow<T, D, D>(p, grid, gather, causal, plain, stream);
+    return launch_narrow<T, D, D>(p, grid, gather, causal, form, stream);
   }
   if (p.split_keys) {
     if (gather) return launch_split<T, D, true, false, false, D>(p, grid, stream, "ha_block_attn_fwd");
     if (causal) return launch_split<T, D, false, true, false, D>(p, grid, stream, "ha_flash_attn_fwd");
     return launch_split<T, D, false, false, false, D>(p, grid, stream, "ha_flash_attn_fwd");
   }
-  if (gather) {
-    if constexpr (D == 64) if (p.tiles_per_wg > 1) {  // set by ha_attn_launch for the instances built below
+  if constexpr (D == 64) {
+    if (gather && p.tiles_per_wg > 1) {  // set by ha_attn_launch for plain launches only
       hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
       return ha_launch_status("ha_block_attn_fwd");
     }
-    if constexpr (D == 64) {
-      if (plain && p.follow_max) return launch_one<T, D, true, false, true, false, false, D, true, 1>(p, grid, stream, "ha_block_attn_fwd");
-      if (p.follow_max) return launch_one<T, D, true, false, false, false, false, D, true, 1>(p, grid, stream, "ha_block_attn_fwd");
-      if (plain && p.small_tiles) return launch_one<T, D, true, false, true, false, false, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
+    if (gather && p.follow_max) return launch_gathered<T, D, false, D, true>(p, grid, form, stream);
+    if (gather && !p.small_tiles) return launch_one<T, D, true, false, PLAIN>(p, grid, stream, "ha_block_attn_fwd");
+    if (!gather && p.small_tiles) {
+      if (causal) return launch_one<T, D, false, true, GENERAL, false, false, D, true, 1>(p, grid, stream, "ha_flash_attn_fwd");
+      return launch_one<T, D, false, false, GENERAL, false, false, D, false, 1>(p, grid, stream, "ha_flash_attn_fwd");
     }
-    if (plain) return launch_one<T, D, true, false, true>(p, grid, stream, "ha_block_attn_fwd");
-    return launch_one<T, D, true, false, false, false, false, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
   }
-  if constexpr (D == 64) if (p.small_tiles) {
-    if (causal) return launch_one<T, D, false, true, false, false, false, D, true, 1>(p, grid, stream, "ha_flash_attn_fwd");
-    return launch_one<T, D, false, false, false, false, false, D, false, 1>(p, grid, stream, "ha_flash_attn_fwd");
-  }
-  if (causal && p.follow_max) return launch_one<T, D, false, true, false, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
+  if (gather) return launch_gathered<T, D, false, D>(p, grid, form, stream);
+  if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
   return launch_one<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
 }
