@@ -237,8 +237,12 @@ void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w) {
     ha_unit_grid& g = w.grid;
     g.n = nh;
     g.granule = pl.granule;
-    g.units_per_granule = (int)((g.granule + HA_SORT_CHUNK - 1) / HA_SORT_CHUNK);
-    g.unit = (int)std::min<int64_t>(g.granule, HA_SORT_CHUNK);
+    // the one segment of the one hashed level in one unit, without a placement launch, up to the length where that is
+    // faster (rank_units_kernel) and one workgroup per CU
+    const bool whole = nh / g.granule == (a.causal ? 2 : 1) && g.granule <= HA_SORT_WHOLE && a.batch * (a.heads + a.kv_heads) <= 256;
+    const int64_t most = whole ? HA_SORT_WHOLE : HA_SORT_CHUNK;
+    g.units_per_granule = (int)((g.granule + most - 1) / most);
+    g.unit = (int)std::min<int64_t>(g.granule, most);
     g.units_per_seq = (int)(nh / g.granule) * g.units_per_granule;
     int64_t longest = 0;
     for (int j = 0; j < nlev; ++j)

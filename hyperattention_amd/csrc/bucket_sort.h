@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #define HA_SORT_CHUNK 4096   // keys per workgroup
+#define HA_SORT_WHOLE 12288  // most rows of a unit that is a whole segment (ha_rank_units with `out`)
 #define HA_SORT_MAX_JOBS 40
 
 struct ha_sort_job {
@@ -39,7 +40,8 @@ int ha_sort_launch(const ha_sort_jobs& jobs, int total_blocks, int total_segment
 struct ha_unit_grid {
   int64_t n;            // rows per sequence
   int64_t granule;      // leaf length (n for the non-causal case); divides n
-  int unit;             // rows per unit, <= HA_SORT_CHUNK; the last unit of a granule may be shorter
+  int unit;             // rows per unit, <= HA_SORT_CHUNK (the only unit of a sequence: <= HA_SORT_WHOLE); the last unit of
+                        // a granule may be shorter
   int units_per_granule;
   int units_per_seq;
 };

@@ -15,6 +15,8 @@
 #include "ha_common.h"
 #include "bucket_sort.h"
 
+#include <type_traits>
+
 #include <mutex>
 
 namespace {
@@ -270,13 +272,18 @@ struct RankArgs {
 // scatter kernel above (a wave owns a contiguous run, ballot matching inside 64-row steps).  Launches
 // of at most one unit per CU take 1024 threads per unit: a wave then ranks 4 steps instead of 16, one after the
 // other (8 units of 4096 rows: 7.4 -> 6.1 us; 512 units: 11.9 -> 13.2).
-template <int THREADS>
+// ROWS > HA_SORT_CHUNK: units that are whole segments (a.out), whose longer chain of steps is shorter than the placement
+// launch that it saves.  Whole calls without mask, units and placement | whole, us: 4 heads of 4224 rows 28.3 | 23.0, of 8192
+// 29.6 | 25.5, of 12288 32.2 | 31.6, of 16384 35.1 | 35.8; 32 heads 52.4 | 47.3, 70.5 | 66.5, 94.7 | 93.1, 119.5 | 120.3.
+template <int THREADS, int ROWS>
 __global__ __launch_bounds__(THREADS) void rank_units_kernel(RankArgs a) {
   constexpr int WAVES = THREADS / HA_WAVE;
-  constexpr int STEPS = HA_SORT_CHUNK / THREADS;
+  constexpr int STEPS = ROWS / THREADS;
+  constexpr bool WHOLE = ROWS > HA_SORT_CHUNK;
+  typedef typename std::conditional<WHOLE, uint16_t, uint32_t>::type Entry;  // row, and above it the bucket if a placement follows
   __shared__ uint32_t wave_hist[WAVES][256];
   __shared__ uint32_t wave_totals[WAVES];
-  __shared__ uint32_t staged[HA_SORT_CHUNK];
+  __shared__ __attribute__((aligned(16))) Entry staged[ROWS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int which = (int)blockIdx.x >= a.units0 ? 1 : 0;
   const int local = (int)blockIdx.x - (which ? a.units0 : 0);
@@ -302,7 +309,7 @@ __global__ __launch_bounds__(THREADS) void rank_units_kernel(RankArgs a) {
   if (tid < 256) {
 #pragma unroll
     for (int k = 0; k < WAVES; ++k) total += wave_hist[k][tid];
-    if (!a.out[which]) a.hist[which][((int64_t)seq * g.units_per_seq + u) * 256 + tid] = total;
+    if (!WHOLE && !a.out[which]) a.hist[which][((int64_t)seq * g.units_per_seq + u) * 256 + tid] = total;
   }
   uint32_t run = block_exclusive_scan(total, wave_totals);
   if (tid < 256) {
@@ -322,13 +329,13 @@ __global__ __launch_bounds__(THREADS) void rank_units_kernel(RankArgs a) {
     const int digit = digit_all[s];
     const uint64_t m = match_digit(digit, valid);
     const uint32_t below = rank_below(m);
-    if (valid) staged[wave_hist[wave][digit] + below] = ((uint32_t)digit << 16) | (uint32_t)i;
+    if (valid) staged[wave_hist[wave][digit] + below] = (Entry)(WHOLE ? (uint32_t)i : ((uint32_t)digit << 16) | (uint32_t)i);
     __builtin_amdgcn_wave_barrier();
     if (valid && below == 0) wave_hist[wave][digit] += (uint32_t)__popcll(m);
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
-  if (a.out[which]) {
+  if (WHOLE || a.out[which]) {
     int32_t* out = a.out[which] + (int64_t)seq * len;
     for (int pos = tid; pos < len; pos += THREADS) out[pos] = (int32_t)(staged[pos] & 0xFFFFu);
     return;
@@ -353,6 +360,16 @@ __global__ __launch_bounds__(SORT_THREADS) void place_units_kernel(ha_place_jobs
   const int seq = seg / job.segs_per_seq, sis = seg % job.segs_per_seq;
   const int64_t first_row = job.seg_offset + (int64_t)sis * job.seg_stride;   // of the segment, in its sequence
   const int64_t first_unit = (int64_t)seq * g.units_per_seq + (first_row / g.granule) * g.units_per_granule;
+  // the unit's entries are asked for before the counts: their places need the counts, their loads do not
+  const int gran = u / g.units_per_granule, w = u % g.units_per_granule;
+  const int64_t row0 = (int64_t)gran * g.granule + (int64_t)w * g.unit;   // of the unit, in its segment
+  const int len = (int)min((int64_t)g.unit, g.granule - (int64_t)w * g.unit);
+  const uint32_t* src = job.sorted + (int64_t)seq * g.n + first_row + row0;
+  constexpr int ENTRIES = HA_SORT_CHUNK / SORT_THREADS;
+  uint32_t v[ENTRIES];
+#pragma unroll
+  for (int i = 0; i < ENTRIES; ++i)
+    if (i * SORT_THREADS < len) v[i] = src[min(tid + i * SORT_THREADS, len - 1)];
   const uint32_t* h = job.hist + first_unit * 256 + tid;
   // eight independent loads in flight at a time: one after the other, a segment of 32 units would cost the
   // workgroup 32 memory round trips before it moves a single row
@@ -372,20 +389,11 @@ __global__ __launch_bounds__(SORT_THREADS) void place_units_kernel(ha_place_jobs
   const uint32_t unit_first = block_exclusive_scan(mine, wave_totals);
   delta[tid] = (int32_t)(seg_first + before) - (int32_t)unit_first;
   __syncthreads();
-  const int gran = u / g.units_per_granule, w = u % g.units_per_granule;
-  const int64_t row0 = (int64_t)gran * g.granule + (int64_t)w * g.unit;   // of the unit, in its segment
-  const int len = (int)min((int64_t)g.unit, g.granule - (int64_t)w * g.unit);
-  const uint32_t* src = job.sorted + (int64_t)seq * g.n + first_row + row0;
   int32_t* out = job.out + (int64_t)seg * job.seg_len;
-  for (int pos0 = tid; pos0 < len; pos0 += 8 * SORT_THREADS) {
-    uint32_t v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = src[min(pos0 + i * SORT_THREADS, len - 1)];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int pos = pos0 + i * SORT_THREADS;
-      if (pos < len) out[pos + delta[v[i] >> 16]] = (int32_t)row0 + (int32_t)(v[i] & 0xFFFFu);
-    }
+  for (int i = 0; i < ENTRIES; ++i) {
+    const int pos = tid + i * SORT_THREADS;
+    if (pos < len) out[pos + delta[v[i] >> 16]] = (int32_t)row0 + (int32_t)(v[i] & 0xFFFFu);
   }
 }
 
@@ -405,11 +413,14 @@ int ha_rank_units(const uint8_t* const ids[2], uint32_t* const sorted[2], uint32
   a.grid = grid;
   a.num_units = num_units;
   const int64_t units = (seqs[0] + seqs[1]) * num_units;
-  HA_REQUIRE(units < (1ll << 31) && grid.unit >= 1 && grid.unit <= HA_SORT_CHUNK, HA_ERR_SHAPE,
+  HA_REQUIRE(units < (1ll << 31) && grid.unit >= 1 && grid.unit <= (out[0] && out[1] ? HA_SORT_WHOLE : HA_SORT_CHUNK), HA_ERR_SHAPE,
              "ha_forward: too many sort units");
   a.units0 = (int)(seqs[0] * num_units);
-  if (units <= 256) hipLaunchKernelGGL(rank_units_kernel<1024>, dim3((unsigned)units), dim3(1024), 0, stream, a);
-  else hipLaunchKernelGGL(rank_units_kernel<SORT_THREADS>, dim3((unsigned)units), dim3(SORT_THREADS), 0, stream, a);
+  const dim3 blocks((unsigned)units);
+  if (grid.unit > 2 * HA_SORT_CHUNK) hipLaunchKernelGGL((rank_units_kernel<1024, HA_SORT_WHOLE>), blocks, dim3(1024), 0, stream, a);
+  else if (grid.unit > HA_SORT_CHUNK) hipLaunchKernelGGL((rank_units_kernel<1024, 2 * HA_SORT_CHUNK>), blocks, dim3(1024), 0, stream, a);
+  else if (units <= 256) hipLaunchKernelGGL((rank_units_kernel<1024, HA_SORT_CHUNK>), blocks, dim3(1024), 0, stream, a);
+  else hipLaunchKernelGGL((rank_units_kernel<SORT_THREADS, HA_SORT_CHUNK>), blocks, dim3(SORT_THREADS), 0, stream, a);
   return ha_launch_status("ha_forward (rank)");
 }
 
