@@ -29,14 +29,14 @@ HIPCC_FLAGS = [
 # exported symbols, in the order of include/hyperattn.h
 SYMBOLS = [
     "ha_abi_version", "ha_last_error", "ha_lsh_hash", "ha_bucket_argsort_workspace_bytes",
-    "ha_bucket_argsort", "ha_bucket_argsort_static", "ha_gather_rows", "ha_block_attn_fwd", "ha_flash_attn_fwd",
+    "ha_bucket_argsort", "ha_bucket_argsort_static", "ha_gather_rows", "ha_copy_rows", "ha_block_attn_fwd", "ha_flash_attn_fwd",
     "ha_attn_bwd_workspace_bytes", "ha_block_attn_bwd", "ha_flash_attn_bwd", "ha_lse_merge",
     "ha_lse_merge_segments",
     "ha_forward_workspace_bytes", "ha_forward", "ha_forward_sort", "ha_lse_merge_levels", "ha_power_probe",
 ]
 
 HA_F16, HA_BF16 = 0, 1
-ABI_VERSION = 7
+ABI_VERSION = 8
 HA_IDX_I32, HA_IDX_I64 = 0, 1
 
 
@@ -141,7 +141,17 @@ class AttnGrads(ctypes.Structure):
         ("dk_stride_b", ctypes.c_int64), ("dk_stride_h", ctypes.c_int64), ("dk_stride_n", ctypes.c_int64),
         ("dv_stride_b", ctypes.c_int64), ("dv_stride_h", ctypes.c_int64), ("dv_stride_n", ctypes.c_int64),
         ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_int64),
-        ("accumulate", ctypes.c_int),
+        ("accumulate", ctypes.c_int), ("out_d", ctypes.c_int64),
+    ]
+
+
+class RowCopy(ctypes.Structure):
+    _fields_ = [
+        ("src", ctypes.c_void_p), ("dst", ctypes.c_void_p),
+        ("batch", ctypes.c_int64), ("heads", ctypes.c_int64), ("n", ctypes.c_int64),
+        ("src_d", ctypes.c_int64), ("dst_d", ctypes.c_int64),
+        ("src_stride_b", ctypes.c_int64), ("src_stride_h", ctypes.c_int64), ("src_stride_n", ctypes.c_int64),
+        ("dst_stride_b", ctypes.c_int64), ("dst_stride_h", ctypes.c_int64), ("dst_stride_n", ctypes.c_int64),
     ]
 
 
@@ -183,6 +193,8 @@ def _declare(lib):
     lib.ha_bucket_argsort_static.argtypes = [vp, vp, ci, i64, i64, i64, i64, i64, vp]
     lib.ha_gather_rows.restype = ci
     lib.ha_gather_rows.argtypes = [vp, vp, ci, vp] + [i64] * 9 + [ci, vp]
+    lib.ha_copy_rows.restype = ci
+    lib.ha_copy_rows.argtypes = [ctypes.POINTER(RowCopy), ci, vp]
     lib.ha_block_attn_fwd.restype = ci
     lib.ha_block_attn_fwd.argtypes = [ctypes.POINTER(BlockAttnArgs), vp]
     lib.ha_flash_attn_fwd.restype = ci

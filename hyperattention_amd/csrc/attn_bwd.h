@@ -46,6 +46,7 @@ struct ha_attn_bwd_params {
   int block_tiles;  // ceil(block_size / 128)
   int sample_size;
   int smooth, idx64;
+  int out_last;    // last 16-byte piece of an `out` row that exists
   int accumulate;  // add to dq / dk / dv instead of overwriting them
   int q_split;  // sampled-key pass: queries per workgroup
   int single_tiles;  // exact causal passes: one tile per workgroup, longest first, instead of pairs

@@ -332,6 +332,7 @@ int check_grads(const ha_attn_operands& t, int64_t sample_size, const ha_attn_gr
   HA_REQUIRE(g.dout && g.dq && g.dk && g.dv, HA_ERR_NULL, "%s: null gradient pointer", who);
   HA_REQUIRE((t.d == 64 || t.d == 128) && t.dv == t.d, HA_ERR_UNSUPPORTED,
              "%s: the backward is built for head dims 64 and 128 with a value dim equal to them", who);
+  HA_REQUIRE(g.out_d >= 0 && g.out_d <= t.d && g.out_d % 8 == 0, HA_ERR_SHAPE, "%s: out_d must be a multiple of 8 up to the head dim", who);
   const int64_t strides[] = {g.do_stride_b, g.do_stride_h, g.do_stride_n, g.dq_stride_b, g.dq_stride_h, g.dq_stride_n,
                              g.dk_stride_b, g.dk_stride_h, g.dk_stride_n, g.dv_stride_b, g.dv_stride_h, g.dv_stride_n};
   for (int64_t s : strides) HA_REQUIRE(s % 8 == 0, HA_ERR_SHAPE, "%s: gradient rows must be 16-byte aligned", who);
@@ -376,6 +377,7 @@ void fill_bwd_params(const ha_attn_operands& t, const ha_attn_grads& g, const Wo
   p.o_seg_off = t.o_seg_stride_rows > 0 ? t.o_seg_offset : t.q_seg_offset;
   p.n_q = (int)t.n_q; p.n_k = (int)t.n_k;
   p.block_tiles = 1; p.sample_size = 0; p.smooth = 0; p.idx64 = 0;
+  p.out_last = (int)((g.out_d ? g.out_d : t.d) / 8) - 1;
   p.accumulate = g.accumulate != 0;
   p.single_tiles = 0;
   p.q_split = (int)t.n_q;

@@ -543,7 +543,7 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 // 8192 254 | 306, 20 x 16384 373 | 405, 24 x 65536 1695 | 1633, not enough for a rule; 1024: 8 x 2048 66 | 82, 24 x 65536 2027 | 2247.
 bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d) {
   const int64_t blocks = (int64_t)p.batch * p.heads * p.segs * ((p.n_q + FUSED_ROWS - 1) / FUSED_ROWS);
-  return d == FD && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
+  return d == FD && p.out_last == FD / 8 - 1 && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
          (p.sample_size <= FUSED_ROWS || (p.sample_size <= FUSED_MAX_SAMPLES && blocks >= 1792));
 }
 

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_dq_kernel(co
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) {
         const uint32_t row = query_row(j * 4 + lane / 16);
-        of[j] = *reinterpret_cast<const vec8*>(row_address(ob, row, o_rb, (lane & 15) * 16));
+        of[j] = *reinterpret_cast<const vec8*>(row_address(ob, row, o_rb, min((int)lane & 15, p.out_last) * 16));  // (shorter rows: zeros of dO)
         df[j] = *reinterpret_cast<const vec8*>(row_address(dob, row, do_rb, (lane & 15) * 16));
       }
       lse2 = p.lse[b * p.lse_sb + h * p.lse_sh + o_row0 + q_row] * LOG2E;

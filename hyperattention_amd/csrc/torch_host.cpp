@@ -69,6 +69,15 @@ bool addressable(const Tensor& t) {
 }
 Tensor as_addressable(const Tensor& t) { return readable(t) && addressable(t) ? t : t.contiguous(); }
 
+// The backward is built for head dims 64 and 128; others up to 128 run in zero-padded copies of q, k, v and the output's
+// gradient, made for it in one launch, whose gradients' wanted columns are copied out in another.
+int64_t built_dim(int64_t d) { return d <= 64 ? 64 : 128; }
+Tensor rows_of(const Tensor& like, int64_t d) { return at::empty({like.size(0), like.size(1), like.size(2), d}, like.options()); }
+ha_row_copy row_copy(const Tensor& from, const Tensor& to) {
+  return {from.data_ptr(), to.data_ptr(), from.size(0), from.size(1), from.size(2), from.size(3), to.size(3),
+          from.stride(0), from.stride(1), from.stride(2), to.stride(0), to.stride(1), to.stride(2)};
+}
+
 struct Config {
   double scale;
   bool causal;
@@ -294,7 +303,7 @@ class Attention : public torch::autograd::Function<Attention> {
     Tensor dout = grads[0];
     if (!dout.defined()) return result;
     const variable_list saved = ctx->get_saved_variables();
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2];
+    Tensor q = saved[0], k = saved[1], v = saved[2];
     const auto s = c10::static_intrusive_pointer_cast<Saved>(ctx->saved_data["s"].toCapsule());
     const Config& c = s->c;
     c10::OptionalDeviceGuard guard(q.device());
@@ -302,6 +311,15 @@ class Attention : public torch::autograd::Function<Attention> {
     const int64_t n = q.size(2);
     dout = n != s->n ? at::constant_pad_nd(dout, {0, 0, 0, n - s->n}) : as_addressable(dout);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    const int64_t d = q.size(3), wide = built_dim(d);
+    Tensor dq_wide = dq, dk_wide = dk, dv_wide = dv;
+    if (d != wide) {
+      const Tensor pq = rows_of(q, wide), pk = rows_of(k, wide), pv = rows_of(v, wide), pdout = rows_of(dout, wide);
+      const ha_row_copy copies[] = {row_copy(q, pq), row_copy(k, pk), row_copy(v, pv), row_copy(dout, pdout)};
+      check(ha_copy_rows(copies, 4, stream));
+      q = pq; k = pk; v = pv; dout = pdout;
+      dq_wide = rows_of(q, wide); dk_wide = rows_of(k, wide); dv_wide = rows_of(v, wide);
+    }
     // A call's gradients are linear in the output gradient it is given, and that enters only through
     // P = exp(s - lse): weighting a row's output gradient by the call's merge weight w equals giving the call the
     // log-sum-exp lse - log(w).  So every call gets the output gradient as it is and the shifted log-sum-exps.
@@ -319,11 +337,12 @@ class Attention : public torch::autograd::Function<Attention> {
     Tensor ws = bytes_on(q, nbytes);  // one workspace for all calls: they run one after the other on the stream
     for (size_t i = 0; i < s->calls.size(); ++i) {
       ha_attn_grads g = {};
-      g.dout = dout.data_ptr(); g.dq = dq.data_ptr(); g.dk = dk.data_ptr(); g.dv = dv.data_ptr();
+      g.out_d = d;
+      g.dout = dout.data_ptr(); g.dq = dq_wide.data_ptr(); g.dk = dk_wide.data_ptr(); g.dv = dv_wide.data_ptr();
       g.do_stride_b = dout.stride(0); g.do_stride_h = dout.stride(1); g.do_stride_n = dout.stride(2);
-      g.dq_stride_b = dq.stride(0); g.dq_stride_h = dq.stride(1); g.dq_stride_n = dq.stride(2);
-      g.dk_stride_b = dk.stride(0); g.dk_stride_h = dk.stride(1); g.dk_stride_n = dk.stride(2);
-      g.dv_stride_b = dv.stride(0); g.dv_stride_h = dv.stride(1); g.dv_stride_n = dv.stride(2);
+      g.dq_stride_b = dq_wide.stride(0); g.dq_stride_h = dq_wide.stride(1); g.dq_stride_n = dq_wide.stride(2);
+      g.dk_stride_b = dk_wide.stride(0); g.dk_stride_h = dk_wide.stride(1); g.dk_stride_n = dk_wide.stride(2);
+      g.dv_stride_b = dv_wide.stride(0); g.dv_stride_h = dv_wide.stride(1); g.dv_stride_n = dv_wide.stride(2);
       g.accumulate = i > 0;
       g.workspace = ws.data_ptr();
       g.workspace_bytes = ws.numel();
@@ -333,6 +352,10 @@ class Attention : public torch::autograd::Function<Attention> {
       } else {
         check(ha_flash_attn_bwd(&ops[i], s->calls[i].causal, &g, stream));
       }
+    }
+    if (d != wide) {
+      const ha_row_copy copies[] = {row_copy(dq_wide, dq), row_copy(dk_wide, dk), row_copy(dv_wide, dv)};
+      check(ha_copy_rows(copies, 3, stream));
     }
     if (n != s->n) {
       dq = dq.narrow(2, 0, s->n);
@@ -351,7 +374,7 @@ bool wants_grad(const Tensor& q, const Tensor& k, const Tensor& v) {
 }
 
 // HyperAttention.forward without the residual estimator.  Returns (attn, lse), or nothing where the head dims have
-// to be padded first: not multiples of 8, or gradients wanted and not one of the backward's.
+// to be padded first: not multiples of 8, or gradients wanted and a value dim of its own.
 std::optional<std::pair<Tensor, Tensor>> forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& proj,
                                                  const std::optional<Tensor>& sampled_idx, double scale, bool causal,
                                                  int64_t projs, int64_t block, int64_t sample, int64_t min_seq, bool smooth) {
@@ -373,7 +396,7 @@ std::optional<std::pair<Tensor, Tensor>> forward(const Tensor& query, const Tens
           "All tensors must have the same type");
   const int64_t d = query.size(3), dv = value.size(3);
   require(d <= 128 && dv <= 128, "FlashAttention only support head dimensions up to 128");
-  if (d % 8 || dv % 8 || (grad && !(d == dv && (d == 64 || d == 128)))) return std::nullopt;
+  if (d % 8 || dv % 8 || (grad && d != dv)) return std::nullopt;
   // the runtime's device is the tensors' one in all but a few programs: ask before paying for a guard
   c10::OptionalDeviceGuard guard;
   if (c10::hip::current_device() != query.device().index()) guard.reset_device(query.device());

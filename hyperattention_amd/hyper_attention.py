@@ -69,10 +69,9 @@ class HyperAttention(torch.nn.Module):
         result = run(query, key, value, proj, sampled, scale or 0.0, causal is not False, self.lsh_num_projs,
                      self.block_size, self.sample_size, self.min_seq_len, bool(self.smooth_block))
         if result is None:
-            # The forward kernels take head dims that are multiples of 8 as they are, the value dim apart
-            # from the q/k dim.  Other head dims, and the backward for anything but 64 and 128 with equal
-            # dims, run zero-padded: zero columns change neither the projections, nor q.k, nor the wanted
-            # outputs
+            # Head dims that are multiples of 8 run as they are, without gradients with a value dim apart from the
+            # q/k dim.  Others run zero-padded: zero columns change neither the projections, nor q.k, nor the
+            # wanted outputs
             wide = ops.padded_head_dim(max(dim, dim_v))
             pad = lambda x: torch.nn.functional.pad(x, (0, wide - x.shape[-1]))
             attn, lse = run(pad(query), pad(key), pad(value), torch.nn.functional.pad(proj, (0, 0, 0, wide - dim)), sampled,

@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define HA_ABI_VERSION 7
+#define HA_ABI_VERSION 8
 
 typedef enum {
   HA_OK = 0,
@@ -98,6 +98,22 @@ int ha_gather_rows(const void* x, const void* idx, int idx_type, void* out,
                    int64_t batch, int64_t heads, int64_t n_src, int64_t n_idx, int64_t n_out, int64_t d,
                    int64_t x_stride_b, int64_t x_stride_h, int64_t x_stride_n,
                    int elem_bytes, void* stream);
+
+/* Copies rows of 2-byte elements into rows of another length, up to HA_ROW_COPIES tensors (batch, heads, n, d) in one
+ * launch: dst_d elements of every row are written, the first min(src_d, dst_d) from src, the others zeros.  Strides in
+ * elements; lengths and strides multiples of 8, tensors 16-byte aligned.  (What torch.nn.functional.pad and its backward do
+ * to the head dim around the reference's kernels, which mask columns instead.)
+ */
+#define HA_ROW_COPIES 4
+typedef struct {
+  const void* src;
+  void* dst;
+  int64_t batch, heads, n, src_d, dst_d;
+  int64_t src_stride_b, src_stride_h, src_stride_n;
+  int64_t dst_stride_b, dst_stride_h, dst_stride_n;
+} ha_row_copy;
+int ha_copy_rows(const ha_row_copy* copies, int count, void* stream);
+
 
 /* ---------------------------------------------------------------------------------------------
  * Attention operands.  All tensors are addressed as ptr + b*stride_b + h*stride_h + row*stride_n
@@ -215,6 +231,8 @@ typedef struct {
   void* workspace;
   int64_t workspace_bytes;
   int accumulate;    /* != 0: dq, dk, dv hold gradients already and the results are added to them   */
+  int64_t out_d;     /* columns of the operands' `out` that exist, a multiple of 8; 0: all of them.  The columns
+                      * of dout past them must be zeros                                              */
 } ha_attn_grads;
 
 int64_t ha_attn_bwd_workspace_bytes(const ha_attn_operands* t, int64_t sample_size);
