@@ -7,7 +7,8 @@
 //
 // Work decomposition.  A workgroup of 4 waves owns consecutive (sorted) query positions of one (virtual) head:
 // 256 at head dim 64, 64 queries (two 32-wide MFMA column blocks) per wave, 128 at head dim 128, 32 queries per
-// wave (WaveShape below), and a CU holds two workgroups.  Query rows and key
+// wave (WaveShape below), and a CU holds two workgroups; at head dim 64 launches of few workgroups and windows that neighbouring
+// reference tiles do not share take 128 queries too (NB = 1), three workgroups per CU.  Query rows and key
 // rows go from HBM straight into LDS (global_load_lds, 16 bytes per lane, whole rows per
 // instruction, no staging registers), row-major with their 16-byte pieces XOR-swizzled by the row
 // number (the swizzle is applied on the source side: a lane fetches the piece that belongs in its
