@@ -618,15 +618,19 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
 // Times in us, pairs | single.  d = 64, 256-query pairs per CU in brackets: 48 heads of 2048 rows
 // (0.75) 49.9 | 43.0, 80 (1.25) 74.1 | 58.1, 96 of 1024 (0.75) 32.8 | 26.8, 128 of 2048 (2) 82.9 | 81.2, 200 (3.1) 151 |
 // 130, 256 (4) 170 | 175, 700 (11) 448 | 490, 2048 (32) 1292 | 1462.
-// d = 128, rounds of 512 pairs of 128-query tiles in brackets: 24 of 2048 (0.38) 41.0 | 38.4, 40 (0.62) 63.1 | 50.4, 64 (1) 73.7 |
-// 73.0, 80 (1.25) 104 | 92, 96 (1.5) 110 | 107, 160 (2.5) 181 | 184, 256 (4) 292 | 352; 48 of 3000 (1.12) 142 | 115; 150 of 300
-// (0.59) 22.9 | 18.4, 192 of 1024 (1.5) 67.6 | 70.7, 400 (3.1) 148 | 175; 8 of 8192 (0.5) 135 | 140.
+// d = 128 (and 96): what a last round of pairs leaves idle against what reading the keys of many sequences at once costs, which
+// grows with their number times the columns (fewer tiles in flight share a key's read).  Fitted to 450 launches (128 and 96 columns, 8 to 512
+// heads, 512 to 11000 rows), 0.3 % slower than the better form on average (worst: 128 heads of 892 rows 9 %).  Rounds of 512 pairs of 128-query
+// tiles in brackets: 24 of 2365 (0.47) 50.3 | 47.5, 80 of 2560 (1.56) 163 | 142, 88 of 2120 (1.55) 129 | 117, 112 of 2560 (2.19) 215 |
+// 198, 200 of 892 (1.56) 71.4 | 63.0, 160 of 2572 (3.44) 321 | 309, 48 of 3000 (1.12) 148 | 123, but 256 of 1000 (2) 92 | 104, 288 of 768 (1.69) 72.9 |
+// 84.5, 256 of 512 (1) 37.4 | 45.0, 112 of 4096 (3.5) 477 | 498, 144 of 4512 (5.06) 781 | 837, 256 of 3584 (7) 854 | 1076; 96 columns: 160 of 2560 (3.12)
+// 257 | 236, 224 of 1403 (2.62) 140 | 121, 400 of 596 (2.34) 71.5 | 71.6.
 static bool single_tiles(const ha_attn_kernel_params& p, int width) {
   const int64_t pair_rows = width == 64 ? 2 * WaveShape<64>::QUERIES : 2 * WaveShape<128>::QUERIES;
-  const double pairs = (double)p.batch * p.heads * p.segs * ((p.n_q + pair_rows - 1) / pair_rows) / 256.;
+  const double vheads = (double)p.batch * p.heads * p.segs, pairs = vheads * ((p.n_q + pair_rows - 1) / pair_rows) / 256.;
   if (width == 64) return pairs <= 3.5;
-  const double rounds = pairs / 2;
-  return rounds < 1 || (rounds <= 1.5 && std::ceil(rounds) > 1.05 * rounds);
+  const double rounds = pairs / 2, columns = 8. * std::max(p.qk_pieces, p.v_pieces);
+  return rounds <= 3.8 && vheads * columns <= 18000 + 30000 * (std::ceil(rounds) / rounds - 1);
 }
 
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,

@@ -21,6 +21,8 @@ pytestmark = pytest.mark.gpu
     (torch.bfloat16, 128, 2, 2, 257, True),
     (torch.float16, 96, 5, 5, 1025, True),
     (torch.bfloat16, 128, 150, 150, 510, True),    # 600 workgroups: 256, 256 reversed, the rest in order
+    (torch.bfloat16, 128, 200, 200, 890, True),    # 1400: single ones in more than one round of pairs
+    (torch.float16, 96, 176, 88, 1025, True),      # a last tile of one row
     (torch.bfloat16, 96, 1040, 1040, 130, True),   # pairs of tiles: one pair, the second of 2 rows
     (torch.float16, 128, 520, 260, 500, True),     # two pairs
     (torch.bfloat16, 128, 520, 520, 384, True),    # three tiles, the middle one alone
