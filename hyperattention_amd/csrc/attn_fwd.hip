@@ -313,7 +313,7 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
 }
 
 // FOLLOW (p.follow_max): the reference exponents follow the row maxima at every step of 32 keys, in exact causal single tiles in a
-// sequence's first tile, gathered (plain or not, tiles of 128 queries at head dim 64) in the first half of a row's keys.  An
+// sequence's first tile, gathered (plain or not, tiles of 128 queries) and at head dims above 64 without mask in a row's first p.follow_max chunks.  An
 // instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
 template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
           int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
@@ -461,9 +461,15 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
   }
   // the plain instance: d = 96, 16 heads of 32768 rows 205 -> 182 us, d = 40 98 -> 88
   if (gather && D == 64 && !p.small_tiles) return launch_one<T, D, true, false, PLAIN, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
+  if constexpr (D == 128) {
+    if (gather && p.follow_max) return launch_gathered<T, D, true, DC, true>(p, grid, form, stream);
+  }
   if (gather) return launch_gathered<T, D, true, DC>(p, grid, form, stream);
   if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
+  if constexpr (D == 128) {
+    if (p.follow_max) return launch_one<T, D, false, false, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
+  }
   return launch_one<T, D, false, false, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
 }
 
@@ -495,9 +501,15 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
       return launch_one<T, D, false, false, GENERAL, false, false, D, false, 1>(p, grid, stream, "ha_flash_attn_fwd");
     }
   }
+  if constexpr (D == 128) {
+    if (gather && p.follow_max) return launch_gathered<T, D, false, D, true>(p, grid, form, stream);
+  }
   if (gather) return launch_gathered<T, D, false, D>(p, grid, form, stream);
   if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
+  if constexpr (D == 128) {
+    if (p.follow_max) return launch_one<T, D, false, false, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
+  }
   return launch_one<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
 }
 
@@ -532,7 +544,8 @@ static ha_divisor make_divisor(int64_t y) {
 // d = 128, without mask or gathered: the estimate of `whole` is that of a kernel of 256-query tiles, which the present one outruns.  It
 // is kept because the split form is the closer one to float64 (four exact weights per row: 2 to 4 % for 256 to 1024 keys a row,
 // 0.2 to 2 % above), and the launches that it gives to it lose little: 8 heads of 2048 rows, blocks and samples of 128 10.7 | 12.2,
-// 256 14.5 | 14.5, 512 22.8 | 19.8; without mask 12 of 1000 19.8 | 17.1, 4 of 4096 57 | 44, but 8 of 4096 68 | 85.
+// 256 14.5 | 14.5, 512 22.8 | 19.8; without mask 12 of 1000 19.8 | 17.1, 4 of 4096 57 | 44.  What it gives the split kernel beyond
+// one round ha_attn_launch takes back.
 //
 // d = 64, tiles of 256 | 128 queries (`large`, `small`; 470 launches of 6 to 512 heads, 512 to 8192 rows, mean error 3 %; a choice that lost 2.5 % or more is not among them).  A
 // workgroup of 128 queries takes half as long, a CU holds three, and ragged rows waste less; its waves read the keys
@@ -671,6 +684,21 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
     if (p.small_tiles) p.split_keys = 0;
   } else if (choice && !p.split_keys) {
     p.small_tiles = 1.02 * t.small < t.large;
+  } else if (width == 128 && p.split_keys && !split_env && (gather || !causal)) {
+    // Head dims above 64, exact without mask and gathered: split workgroups go in whole rounds, and from the second on tiles of 128
+    // queries are faster, but for tiles that just miss one per CU against two rounds (24 heads of 1300 rows 40.7 us, split
+    // 38.7).  The split form is the closer one to float64, so the exponents follow the row maxima: without mask in an eighth of
+    // the chunks, at least four (half of fewer than eight), 0.98 to 0.998 of its error from 520 to 4096 keys on normal and on
+    // clustered rows (1.001 to 1.015 without) for 4 to 12 % of the tiles' time; gathered in five eighths (1024 keys a row: 0.975 to 0.998, in half 0.98 to
+    // 1.002, without 1.04).  Split -> tiles, us, without mask: 16 heads of 2048 rows 53 -> 43, 8 of 3000 65 -> 54, 24 of 2676 122 -> 91, 96
+    // columns 48 -> 40, 59 -> 49, 110 -> 78; blocks and samples of 512: 12 heads of 2688 rows 50 -> 42, 24 87 -> 62, 96 columns 44 -> 37, 78 -> 54.
+    const int64_t vheads = (int64_t)p.batch * p.heads * p.segs;
+    const int64_t rounds = (vheads * ((p.n_q + 63) / 64) + 255) / 256, tiles = vheads * ((p.n_q + 127) / 128);
+    if (rounds > 2 || (rounds == 2 && tiles <= 256)) {
+      const int exact_chunks = (p.n_k + 63) / 64;
+      p.split_keys = 0;
+      p.follow_max = gather ? (5 * chunks + 7) / 8 : std::max(std::min(4, (exact_chunks + 1) / 2), 1 + exact_chunks / 8);
+    }
   }
   const int tile_rows = width == 64 && !p.small_tiles ? WaveShape<64>::QUERIES : WaveShape<128>::QUERIES;
   int64_t qtiles = (p.n_q + tile_rows - 1) / tile_rows;

@@ -5,7 +5,7 @@ import torch
 
 from oracle import hyper_oracle as O
 from test_gpu_ops import ha  # noqa: F401 (fixture)
-from _util import _randn, assert_close
+from _util import _gen, _randn, assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,32 @@ def test_exact(ha, monkeypatch, dtype, d, h, hk, n, causal):  # noqa: F811
     ro, rl = O.exact_attention(q, *(x.repeat_interleave(h // hk, 1) for x in (k, v)), None, causal)
     assert_close(o.transpose(1, 2), ro, "out", dtype)
     assert_close(lse[:, :, :n], rl, "lse")
+
+
+# more than one round of split workgroups by the launcher's estimates: tiles whose exponents follow the row maxima in the first chunks
+@pytest.mark.parametrize("dtype,d,h,hk,n,scale", [
+    (torch.bfloat16, 128, 16, 16, 2048, 1.), (torch.float16, 96, 12, 4, 2676, 1.), (torch.bfloat16, 120, 8, 8, 3001, 1.),
+    (torch.float16, 128, 16, 8, 2047, 12.),  # maxima that rise by hundreds
+])
+def test_exact_without_mask_in_rounds(ha, dtype, d, h, hk, n, scale):  # noqa: F811
+    q = _randn((1, h, n, d), 74, dtype) * scale
+    k, v = (_randn((1, hk, n, d), s, dtype) for s in (75, 76))
+    o, lse = ha.flash_attn_func(*(x.cuda().transpose(1, 2) for x in (q, k, v)), None, False)
+    ro, rl = O.exact_attention(q, *(x.repeat_interleave(h // hk, 1) for x in (k, v)), None, False)
+    assert_close(o.transpose(1, 2), ro, "out", dtype)
+    assert_close(lse[:, :, :n], rl, "lse")
+
+
+@pytest.mark.parametrize("dtype,d,h,hk,n,smooth", [
+    (torch.bfloat16, 128, 12, 12, 2688, False), (torch.float16, 96, 12, 4, 2688, False), (torch.bfloat16, 120, 12, 12, 2688, True),
+])
+def test_gathered_in_rounds(ha, dtype, d, h, hk, n, smooth):  # noqa: F811
+    q = _randn((1, h, n, d), 77, dtype)
+    k, v = (_randn((1, hk, n, d), s, dtype) for s in (78, 79))
+    kw = dict(block_size=512, sample_size=512, min_seq_len=1, smooth_block=smooth)
+    m = ha.HyperAttention(input_dim=d, rng=_gen(80), **kw).to(device="cuda", dtype=dtype)
+    attn, lse = m(q.cuda(), k.cuda(), v.cuda(), return_lse=True)
+    full = [x.repeat_interleave(h // hk, 1) for x in (k, v)]
+    ref, ref_lse = O.hyper_forward(q, *full, m.lsh.proj_dir[0, 0].cpu(), **kw)
+    assert_close(attn, ref, "attn", dtype)
+    assert_close(lse, ref_lse, "lse")
