@@ -138,7 +138,8 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
   auto load_stats = [&](uint32_t row) -> Stats {
     const uint32_t piece = (opaque_lane() & 15) * 8;
     Stats st;
-    st.o = *reinterpret_cast<const vec4*>(row_address(ob, row, o_rb, piece));
+    // O's rows may be shorter than dO's (p.out_last): the last 8 bytes stand in for those that are missing, which meet zeros of dO
+    st.o = *reinterpret_cast<const vec4*>(row_address(ob, row, o_rb, min(piece, (uint32_t)p.out_last * 16 + 8)));
     st.g = *reinterpret_cast<const vec4*>(row_address(dob, row, do_rb, piece));
     st.l = lseb[row];
     return st;
@@ -541,9 +542,11 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 // too, but for 16 x 2048 without samples, 22.8 | 23.2); 512: 8 x 2048 51 | 54, 24 x 2048 82 | 79, 10 x 16384 172 | 178, 130 x 2048
 // 294 | 306, then within 5 % to both sides up to 1600 blocks, 28 x 16384 (1792) 453 | 382, 24 x 65536 1402 | 1118; 768: 24 x
 // 8192 254 | 306, 20 x 16384 373 | 405, 24 x 65536 1695 | 1633, not enough for a rule; 1024: 8 x 2048 66 | 82, 24 x 65536 2027 | 2247.
+// Head dims below 64, padded for the backward (O as it is): forward and backward of 24 x 16384, d = 48 476 | 418, 512 x 3072, d = 32
+// 1570 | 1324, causal 24 x 65536, d = 40 5923 | 5340.
 bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d) {
   const int64_t blocks = (int64_t)p.batch * p.heads * p.segs * ((p.n_q + FUSED_ROWS - 1) / FUSED_ROWS);
-  return d == FD && p.out_last == FD / 8 - 1 && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
+  return d == FD && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
          (p.sample_size <= FUSED_ROWS || (p.sample_size <= FUSED_MAX_SAMPLES && blocks >= 1792));
 }
 

@@ -75,3 +75,26 @@ def test_adds_to_gradients_in_transposed_layout_and_keeps_an_explicit_list(ha, d
         err = (got.double().cpu().transpose(1, 2) - total).norm() / total.norm()
         assert err <= unit + (3e-3 if dtype == torch.float16 else 8e-3), f"{name}: {err:.2e}"
         assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype,h,n,out_d", [(torch.float16, 2, 640, 48), (torch.bfloat16, 3, 1024, 40), (torch.float16, 1, 256, 8)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_short_output_rows(ha, dtype, h, n, out_d, accumulate):  # noqa: F811
+    """Head dims below 64 padded for the backward, with the forward's output as it is: bit for bit the gradients of padded output
+    rows, from the same kernel (the three passes sum in another order)."""
+    from hyperattention_amd import _lib, ops
+    pad = lambda x: torch.nn.functional.pad(x, (0, 64 - out_d)).cuda()  # noqa: E731
+    q, k, v, do = (pad(_randn((1, n, h, out_d), s, dtype)) for s in (51, 52, 53, 54))
+    qi, ki = (_perms(1, h, n, s).cuda().int().transpose(1, 2) for s in (55, 56))
+    o, lse = ops.hyper_attn_func(q, k, v, qi, ki, 256, 0, 0.2, False)
+    there = [_randn((1, n, h, 64), s, dtype).cuda() for s in (57, 58, 59)]
+    results = []
+    for out, columns in ((o, 0), (o[..., :out_d].contiguous(), out_d)):
+        grads = [x.clone() for x in there]
+        a, _keep = ops._block_attn_args(q, k, v, out, lse, qi, ki, 256, 0, 0.2, False, None)
+        g, _ws = ops._attn_grads(a.t, do, *grads)
+        g.accumulate, g.out_d = int(accumulate), columns
+        _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), ops._stream(q)))
+        results.append(grads)
+    for padded, short, name in zip(*results, ("dq", "dk", "dv")):
+        assert torch.equal(padded, short), name
