@@ -55,6 +55,7 @@ struct ha_attn_kernel_params {
   int split_keys;  // the keys of a query tile are split over the waves of a workgroup, 2: longest tiles first (filled by
                    // ha_attn_launch)
   int small_tiles;  // head dims up to 64: tiles of 128 queries (filled by ha_attn_launch)
+  int large_tiles;  // head dims above 64: exact attention in tiles of 256 queries (filled by ha_attn_launch)
   int follow_max;  // the FOLLOW instances; gathered: in that many chunks (filled by ha_attn_launch)
   // Ragged segments (exact kernels; rag_levels < 0: regular).  Inside a causal recursion with odd lengths the
   // segments of a level neither start at multiples of one stride nor hold the same number of rows: level i

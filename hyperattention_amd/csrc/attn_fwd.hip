@@ -7,7 +7,8 @@
 //
 // Work decomposition.  A workgroup of 4 waves owns consecutive (sorted) query positions of one (virtual) head:
 // 256 at head dim 64, 64 queries (two 32-wide MFMA column blocks) per wave, 128 at head dim 128, 32 queries per
-// wave (WaveShape below), and a CU holds two workgroups; at head dim 64 launches of few workgroups and windows that neighbouring
+// wave (WaveShape below), and a CU holds two workgroups (exact attention at head dim 128 also 8 waves, 256 queries, one
+// workgroup: large_tiles); at head dim 64 launches of few workgroups and windows that neighbouring
 // reference tiles do not share take 128 queries too (NB = 1), three workgroups per CU.  Query rows and key
 // rows go from HBM straight into LDS (global_load_lds, 16 bytes per lane, whole rows per
 // instruction, no staging registers), row-major with their 16-byte pieces XOR-swizzled by the row
@@ -316,12 +317,11 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
 // sequence's first tile, gathered (plain or not, tiles of 128 queries) and at head dims above 64 without mask in a row's first p.follow_max chunks.  An
 // instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
 template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
-__global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
+__global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int QW = 32 * NB;                 // queries per wave
-  constexpr int WAVES = WaveShape<D>::WAVES;  // waves per workgroup
   constexpr int WG_QUERIES = QW * WAVES;
   constexpr int REF_TILES = WG_QUERIES / 128;  // reference query tiles of 128 per workgroup
   static_assert(!GATHER || FORM == PLAIN || REF_TILES == 1, "two reference tiles of a workgroup share their keys");
@@ -338,8 +338,8 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) 
   // the immediate field of the LDS reads.
   constexpr int Q_WAVE_BYTES = QW * D * 2;  // a wave's part of the query region
   // At d = 128 two workgroups fit a CU's 160 KB if most of the query region lies in tile space that is free before and
-  // after the loop: V tile 1 (waves 0, 1) and the first half of K tile 0 (wave 3).
-  constexpr bool OVERLAY = D == 128;
+  // after the loop: V tile 1 (waves 0, 1) and the first half of K tile 0 (wave 3).  (8 waves: one workgroup per CU.)
+  constexpr bool OVERLAY = D == 128 && WAVES == 4;
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[TILE_BYTES];
@@ -425,10 +425,10 @@ __global__ __launch_bounds__(WaveShape<D>::THREADS, D == 64 && NB == 1 ? 3 : 2) 
 namespace {
 
 template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB>
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
 int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, FORM, NARROW, REWEIGHT, DC, FOLLOW, NB>), dim3(grid),
-                     dim3(WaveShape<D>::THREADS), 0, stream, p);
+  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, FORM, NARROW, REWEIGHT, DC, FOLLOW, NB, WAVES>), dim3(grid),
+                     dim3(64 * WAVES), 0, stream, p);
   return ha_launch_status(what);
 }
 
@@ -468,6 +468,7 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
   if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
   if constexpr (D == 128) {
+    if (p.large_tiles) return launch_one<T, D, false, false, GENERAL, true, false, DC, false, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
     if (p.follow_max) return launch_one<T, D, false, false, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
   }
   return launch_one<T, D, false, false, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
@@ -508,6 +509,7 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
   if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
   if constexpr (D == 128) {
+    if (p.large_tiles) return launch_one<T, D, false, false, GENERAL, false, false, D, false, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
     if (p.follow_max) return launch_one<T, D, false, false, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
   }
   return launch_one<T, D, false, false>(p, grid, stream, "ha_flash_attn_fwd");
@@ -651,6 +653,24 @@ static bool single_tiles(const ha_attn_kernel_params& p, int width) {
   return rounds <= 3.8 && vheads * columns <= 18000 + 30000 * (std::ceil(rounds) / rounds - 1);
 }
 
+// Whether exact attention at head dims above 64 takes workgroups of 8 waves, 256 queries, one per CU, instead of two of 128
+// queries per CU.  Per CU both have 256 queries in flight, the larger ones read the keys once for all of them; the smaller ones fill a last
+// round of up to half of the CUs' places in less time, waste less of a ragged end, and at many rounds run without waiting for each other.
+// Without mask, 256 | 128 queries per workgroup in us, rounds of the chip in brackets (470 launches in all, the rule 0.4 % slower than the
+// better form on average): 24 heads of 1298 rows (0.56 | 0.52) 35.8 | 38.0, 24 of 1500 42.1 | 44.4, 35 of 827 (0.55 | 0.48) 24.6 | 19.7, 45 of
+// 2340 (1.76 | 1.67) 136 | 141, 25 of 7193 (2.83 | 2.78) 588 | 619, 73 of 2056 (2.57 | 2.42) 176 | 167, 90 of 3393 (4.92 | 4.75) 509 | 524,
+// 122 of 1328 (2.86 | 2.62) 129 | 129, 368 of 412 (2.88 | 2.88) 56 | 54; 96 columns: 9 of 3915 (0.56 | 0.54) 72 | 87, 12 of 3458 72.8 | 79.6, 40 of 4332 (2.66)
+// 301 | 321, 242 of 666 (2.84) 58 | 61, 620 of 387 (4.84) 74 | 72, 402 of 130 (1.57; three quarters of the queries exist) 18.8 | 19.9.
+static bool large_tiles(const ha_attn_kernel_params& p) {
+  const double vheads = (double)p.batch * p.heads * p.segs;
+  const double rounds_256 = vheads * ((p.n_q + 255) / 256) / 256, rounds_128 = vheads * ((p.n_q + 127) / 128) / 512;
+  const double rounds = std::ceil(rounds_128);
+  const int columns_96 = p.qk_pieces <= 12 && p.v_pieces <= 12;
+  if (rounds_128 <= rounds - 0.5 || std::ceil(rounds_256) != rounds) return false;
+  if (columns_96 && rounds <= 3 && p.n_q <= 192) return true;
+  return rounds == 1 || (rounds <= 6 && p.n_q >= (columns_96 ? 200 : 500) * rounds);
+}
+
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,
                    bool reweight, hipStream_t stream) {
   ha_attn_kernel_params p = params;
@@ -675,7 +695,7 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   // exponents follow the row maxima in half of the chunks: 0.97 to 0.99 of its error with blocks and samples of 128 and 256
   // (without 1.01 and more), 12 heads of 2560 rows, blocks of 128 20.9 -> 19.7 us, 256 23.3 -> 22.4, 12 of 3072 25.8 -> 22.7
   // and 29.1 -> 26.2.  With 1024 keys a row the half costs what the tiles gain.
-  p.small_tiles = p.follow_max = 0;
+  p.small_tiles = p.large_tiles = p.follow_max = 0;
   const bool choice = width == 64 && full_rows && !reweight && !(gather && stream_env);
   const int chunks = 2 * p.block_tiles + p.sample_chunks;  // gathered: of a row's keys
   if (choice && gather && p.split_keys && !split_env && chunks <= 8 && t.small + 1.5 < t.split_rounds) {
@@ -689,6 +709,8 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
     if (p.small_tiles) p.split_keys = 0;
   } else if (choice && !p.split_keys) {
     p.small_tiles = 1.02 * t.small < t.large;
+  } else if (width == 128 && !p.split_keys && !gather && !causal) {
+    p.large_tiles = large_tiles(p);
   } else if (width == 128 && p.split_keys && !split_env && (gather || !causal)) {
     // Head dims above 64, exact without mask and gathered: split workgroups go in whole rounds, and from the second on tiles of 128
     // queries are faster, but for tiles that just miss one per CU against two rounds (24 heads of 1300 rows 40.7 us, split
@@ -705,7 +727,7 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
       p.follow_max = gather ? (5 * chunks + 7) / 8 : std::max(std::min(4, (exact_chunks + 1) / 2), 1 + exact_chunks / 8);
     }
   }
-  const int tile_rows = width == 64 && !p.small_tiles ? WaveShape<64>::QUERIES : WaveShape<128>::QUERIES;
+  const int tile_rows = p.large_tiles || (width == 64 && !p.small_tiles) ? 256 : 128;
   int64_t qtiles = (p.n_q + tile_rows - 1) / tile_rows;
   if (causal && !gather && !single) qtiles = (qtiles + 1) / 2;  // one workgroup per pair of tiles
   if (p.split_keys) qtiles = (p.n_q + 63) / 64;

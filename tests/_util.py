@@ -50,3 +50,23 @@ def assert_close(got, ref, what, out_dtype=None, reference_arithmetic=None):
     bound = max(tol, REL_BY_DTYPE[out_dtype]) * ref.abs().max() + ulp * ref.abs()
     worst = ((got - ref).abs() - bound).max()
     assert worst <= 0, f"{what}: element-wise error exceeds bound by {worst:.3e}"
+
+
+def forward_kernels(call):
+    """What `call` launches of the forward attention kernels, in order: "split", or the queries per workgroup, with "follow" behind
+    it where the instance is one whose reference exponents can follow the row maxima."""
+    import re
+    from torch.profiler import ProfilerActivity, profile
+    call()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as trace:
+        call()
+        torch.cuda.synchronize()
+    names = [e.name for e in trace.events() if "ha_attn_fwd" in e.name]
+    assert names, "no attention kernel in the trace"
+    forms = []
+    for name in names:
+        # <type, D, GATHER, CAUSAL, FORM, NARROW, REWEIGHT, DC, FOLLOW, NB, WAVES>
+        m = re.search(r"ha_attn_fwd_kernelI.*ELb([01])ELi(\d+)ELi(\d+)EEv", name)
+        forms.append(f"{32 * int(m[2]) * int(m[3])}{' follow' if m[1] == '1' else ''}" if m else "split")
+    return forms
