@@ -366,7 +366,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   // a slot freed by a short one stays empty until the ones queued before it are placed: with one tile per
   // workgroup (4 to 32 chunks in a 2048-row leaf) the slots of a CU stood empty for 8 us at a time.
   // Few workgroups (p.tiles_per_wg == 0, see single_tiles): one tile each, the tiles of all sequences, longest first,
-  // the second 256 in reversed order: a CU holds two workgroups (see ha_attn_fwd_split_kernel).
+  // the second 256 in reversed order where a CU holds two workgroups (see ha_attn_fwd_split_kernel).
   constexpr bool PAIRED = CAUSAL && !GATHER;
   const int wg_per_seq = PAIRED ? (qtiles + 1) / 2 : qtiles;  // what p.div_qtiles divides by
   const bool single = PAIRED && (FOLLOW || (D <= 64 && p.tiles_per_wg == 0));  // d = 128: the FOLLOW instance's alone
@@ -374,7 +374,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   if (single) {
     const int second = min((int)gridDim.x, 512);
     wg = blockIdx.x;
-    if (wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
+    if (WAVES == 4 && wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
     slot = fast_div(wg, p.div_qtiles);
     wg -= slot * (p.batch * p.heads * p.segs);  // what p.div_qtiles divides by here
     vseq = fast_div(wg, p.div_kv_group);
@@ -465,6 +465,9 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
     if (gather && p.follow_max) return launch_gathered<T, D, true, DC, true>(p, grid, form, stream);
   }
   if (gather) return launch_gathered<T, D, true, DC>(p, grid, form, stream);
+  if constexpr (D == 128) {
+    if (causal && p.large_tiles) return launch_one<T, D, false, true, GENERAL, true, false, DC, true, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
+  }
   if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
   if (causal) return launch_one<T, D, false, true, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
   if constexpr (D == 128) {
@@ -504,6 +507,7 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
   }
   if constexpr (D == 128) {
     if (gather && p.follow_max) return launch_gathered<T, D, false, D, true>(p, grid, form, stream);
+    if (causal && p.large_tiles) return launch_one<T, D, false, true, GENERAL, false, false, D, true, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
   }
   if (gather) return launch_gathered<T, D, false, D>(p, grid, form, stream);
   if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
@@ -661,11 +665,25 @@ static bool single_tiles(const ha_attn_kernel_params& p, int width) {
 // 2340 (1.76 | 1.67) 136 | 141, 25 of 7193 (2.83 | 2.78) 588 | 619, 73 of 2056 (2.57 | 2.42) 176 | 167, 90 of 3393 (4.92 | 4.75) 509 | 524,
 // 122 of 1328 (2.86 | 2.62) 129 | 129, 368 of 412 (2.88 | 2.88) 56 | 54; 96 columns: 9 of 3915 (0.56 | 0.54) 72 | 87, 12 of 3458 72.8 | 79.6, 40 of 4332 (2.66)
 // 301 | 321, 242 of 666 (2.84) 58 | 61, 620 of 387 (4.84) 74 | 72, 402 of 130 (1.57; three quarters of the queries exist) 18.8 | 19.9.
-static bool large_tiles(const ha_attn_kernel_params& p) {
+// Causal, single tiles, longest first: a launch works on the same tile of all sequences at a time, and the tiles of a sequence meet
+// in one XCD's L2 only where the number of sequences is a multiple of the 8 XCDs (of 4: in two, of 2: in four).  With others the
+// smaller workgroups, which read the keys twice as often, wait for them.  256 | 128 queries, us (370 launches; where the rule chooses 256, they
+// are at most 1 % slower, on average 8 % faster): 127 heads of 1953 rows 150 | 177, 35 of 3574 121 | 139, 33 of 6382 339 | 396, 81 of 3581 271 |
+// 319, 181 of 935 71 | 78, 66 of 2013 88 | 97, 50 of 5022 316 | 338, 156 of 2514 285 | 311, but 88 of 2071 (a multiple of 8) 128 | 112, 132 of 1621 124 | 123, 46 of 2861 119 | 113,
+// 28 of 1185 30.9 | 24.5 (0.5 rounds), 141 of 795 (7 tiles of 128 in 4 of 256) 55.6 | 49.7; with 96 columns rarely (70 of 1873 74 | 71).  And up to one
+// per CU where a quarter of a sequence's 256 queries does not exist: 248 of 150 13.7 | 15.4, 125 of 426 19.3 | 21.2, 96 columns 256 of 180 12.8 | 14.4.
+static bool large_tiles(const ha_attn_kernel_params& p, bool causal) {
   const double vheads = (double)p.batch * p.heads * p.segs;
   const double rounds_256 = vheads * ((p.n_q + 255) / 256) / 256, rounds_128 = vheads * ((p.n_q + 127) / 128) / 512;
   const double rounds = std::ceil(rounds_128);
-  const int columns_96 = p.qk_pieces <= 12 && p.v_pieces <= 12;
+  const bool columns_96 = p.qk_pieces <= 12 && p.v_pieces <= 12;
+  if (causal) {
+    const int last = (p.n_q - 1) % 256 + 1;  // queries of the last tile
+    if (rounds_256 > 0.8 && rounds_256 <= 1 && p.n_q <= 448 && last > 128 && last <= 192) return true;
+    const int64_t seqs = (int64_t)p.batch * p.heads * p.segs;
+    const double least = seqs % 2 ? 1.5 : seqs % 4 ? (seqs >= 64 ? 1.5 : 3.5) : 5;
+    return !columns_96 && seqs % 8 != 0 && p.n_q >= 640 && rounds_128 >= least && rounds_256 <= 1.1 * rounds_128;
+  }
   if (rounds_128 <= rounds - 0.5 || std::ceil(rounds_256) != rounds) return false;
   if (columns_96 && rounds <= 3 && p.n_q <= 192) return true;
   return rounds == 1 || (rounds <= 6 && p.n_q >= (columns_96 ? 200 : 500) * rounds);
@@ -709,8 +727,8 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
     if (p.small_tiles) p.split_keys = 0;
   } else if (choice && !p.split_keys) {
     p.small_tiles = 1.02 * t.small < t.large;
-  } else if (width == 128 && !p.split_keys && !gather && !causal) {
-    p.large_tiles = large_tiles(p);
+  } else if (width == 128 && !p.split_keys && !gather && (single || !causal)) {
+    p.large_tiles = large_tiles(p, causal);
   } else if (width == 128 && p.split_keys && !split_env && (gather || !causal)) {
     // Head dims above 64, exact without mask and gathered: split workgroups go in whole rounds, and from the second on tiles of 128
     // queries are faster, but for tiles that just miss one per CU against two rounds (24 heads of 1300 rows 40.7 us, split

@@ -49,3 +49,11 @@ def test_many_short_causal_rows(ha, monkeypatch, dtype, data, d, h, n):  # noqa:
     """Without exponents that follow: 1.007 to 1.024."""
     q, k, v = _inputs(dtype, data, d, h, n)
     _as_close_as_split_keys(monkeypatch, lambda: ha.flash_attn_func(q, k, v, None, True)[0], _exact(q, k, v, True), 1.003)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("data", ["normal", "clusters"])
+@pytest.mark.parametrize("d,h,n", [(128, 129, 768), (128, 250, 150), (96, 250, 180)])
+def test_causal_tiles_of_256(ha, monkeypatch, dtype, data, d, h, n):  # noqa: F811
+    q, k, v = _inputs(dtype, data, d, h, n)
+    _as_close_as_split_keys(monkeypatch, lambda: ha.flash_attn_func(q, k, v, None, True)[0], _exact(q, k, v, True), 1.003)

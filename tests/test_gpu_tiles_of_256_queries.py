@@ -36,3 +36,20 @@ def _check(ha, dtype, d, h, hk, n, causal, form):  # noqa: F811
 ])
 def test_without_mask(ha, dtype, d, h, hk, n, form):  # noqa: F811
     _check(ha, dtype, d, h, hk, n, False, form)
+
+
+# (heads not a multiple of 8: an instance that follows in the first tile, one tile per workgroup, longest first)
+@pytest.mark.parametrize("dtype,d,h,hk,n,form", [
+    (torch.bfloat16, 128, 250, 125, 129, "256 follow"),   # one tile per sequence
+    (torch.float16, 96, 236, 236, 192, "256 follow"),
+    (torch.bfloat16, 80, 110, 110, 385, "256 follow"),    # two, the last of 129 rows
+    (torch.float16, 128, 129, 43, 768, "256 follow"),    # whole tiles, more workgroups than CUs
+    (torch.bfloat16, 104, 129, 129, 767, "256 follow"),    # a last row less
+    (torch.bfloat16, 128, 102, 102, 1000, "256 follow"),
+    (torch.float16, 128, 57, 19, 1700, "256 follow"),     # 14 tiles of 128 in 7 of 256
+    (torch.bfloat16, 128, 124, 124, 768, "128 follow"),
+    (torch.float16, 96, 121, 121, 768, "128 follow"),
+    (torch.bfloat16, 128, 200, 200, 129, "128 follow"),   # less than four of five CUs
+])
+def test_causal(ha, dtype, d, h, hk, n, form):  # noqa: F811
+    _check(ha, dtype, d, h, hk, n, True, form)
