@@ -644,15 +644,15 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
 // 198, 200 of 892 (1.56) 71.4 | 63.0, 160 of 2572 (3.44) 321 | 309, 48 of 3000 (1.12) 148 | 123, but 256 of 1000 (2) 92 | 104, 288 of 768 (1.69) 72.9 |
 // 84.5, 256 of 512 (1) 37.4 | 45.0, 112 of 4096 (3.5) 477 | 498, 144 of 4512 (5.06) 781 | 837, 256 of 3584 (7) 854 | 1076; 96 columns: 160 of 2560 (3.12)
 // 257 | 236, 224 of 1403 (2.62) 140 | 121, 400 of 596 (2.34) 71.5 | 71.6.
-// Rows of up to 192 are single tiles in any number: there the split kernel would be the faster one but for these tiles, and tiles without
-// FOLLOW have 1.007 to 1.024 times its error, with it less (300 to 2048 sequences, normal and clustered).  Split | pairs | single, us: 512 of
-// 65 28.3 | 12.1 | 13.0, of 128 35.6 | 17.0 | 17.2, of 150 26.5 | 25.7 | 27.6, 2048 of 150 95.6 | 82.2 | 86.2, of 192 107 | 94 | 93;
-// 96 columns: 512 of 128 28.1 | 13.7 | 13.9, 2048 of 150 82.1 | 69.5 | 76.6.
+// Rows of up to 128 are single tiles in any number, of up to 192 in less than 384: there the split kernel would be the faster one but for
+// these tiles, and tiles without FOLLOW have 1.007 to 1.024 times its error, with it less (300 to 2048 sequences, normal and clustered).
+// Split | pairs | single, us: 512 of 65 28.3 | 12.1 | 13.0, of 128 35.6 | 17.0 | 17.2, 320 of 150 26.0 | 20.4 | 21.3; 96 columns: 512 of 128 28.1 |
+// 13.7 | 13.9.  From 384 on two rounds of pairs are closer to full (480 of 172, 80 columns 22 | 20.5 | 23.5, 1016 of 172 50.5 | 45.4 | 47.8).
 static bool single_tiles(const ha_attn_kernel_params& p, int width) {
   const int64_t pair_rows = width == 64 ? 2 * WaveShape<64>::QUERIES : 2 * WaveShape<128>::QUERIES;
   const double vheads = (double)p.batch * p.heads * p.segs, pairs = vheads * ((p.n_q + pair_rows - 1) / pair_rows) / 256.;
   if (width == 64) return pairs <= 3.5;
-  if (p.n_q <= 192) return true;
+  if (p.n_q <= 128 || (p.n_q <= 192 && vheads < 384)) return true;
   const double rounds = pairs / 2, columns = 8. * std::max(p.qk_pieces, p.v_pieces);
   return rounds <= 3.8 && vheads * columns <= 18000 + 30000 * (std::ceil(rounds) / rounds - 1);
 }
