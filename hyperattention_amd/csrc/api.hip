@@ -98,7 +98,6 @@ void fill_params(const ha_attn_operands& t, ha_attn_kernel_params& p) {
   p.sampled_pos = nullptr; p.sample_bias_raw = 0.f;
   p.n_q_last = (int)t.n_q;
   p.lse_rows = (int)t.lse_rows;
-  p.tiles_per_wg = 1;
   p.rag_levels = -1; p.rag_n = 0;
   for (int& c : p.rag_half) c = 0;
   p.scale_log2 = t.scale * LOG2E_F;

@@ -48,15 +48,13 @@ struct ha_attn_kernel_params {
   // first row of segment g in the out / lse tensors: o_seg_off + g * o_seg_stride (= the query side's unless
   // the caller packs the rows a call writes)
   int64_t o_seg_off, o_seg_stride;
-  // Streaming gathered kernel: consecutive query tiles of one (virtual) head per workgroup (the last
-  // workgroup of a head may have fewer); 1: the one-tile kernels.  Exact causal kernel: 0 for one tile per
-  // workgroup, longest first, instead of pairs
-  int tiles_per_wg;
+  int single;      // exact causal kernel: one tile per workgroup, longest first, instead of pairs (filled by ha_attn_launch)
   int split_keys;  // the keys of a query tile are split over the waves of a workgroup, 2: longest tiles first (filled by
                    // ha_attn_launch)
   int small_tiles;  // head dims up to 64: tiles of 128 queries (filled by ha_attn_launch)
   int large_tiles;  // head dims above 64: exact attention in tiles of 256 queries (filled by ha_attn_launch)
-  int follow_max;  // the FOLLOW instances; gathered: in that many chunks (filled by ha_attn_launch)
+  int follow_max;  // the FOLLOW instances; gathered, and exact without mask at head dims above 64: in that many chunks of a row
+                   // (filled by ha_attn_launch)
   // Ragged segments (exact kernels; rag_levels < 0: regular).  Inside a causal recursion with odd lengths the
   // segments of a level neither start at multiples of one stride nor hold the same number of rows: level i
   // cuts a segment of (padded) length 2*rag_half[i] into two, and the rows that exist are the first rag_n of

@@ -77,8 +77,8 @@ constexpr float M_FLOOR = -1e30f;
 // other's barriers, and one's set-up and output stage run beside the other's loop.  With 8 waves of 32 queries at
 // d = 128 (256 queries, one workgroup per CU) a wave stood at the barrier of a 64-key iteration for a quarter of it: 2 x 32
 // heads of 65536 rows, smooth blocks of 512 2.80 -> 2.58 ms, 16 x 20479 causal, d = 96 508 -> 457 us (whole call, 2.5 rounds of 256
-// workgroups), leaves of 2048 rows, 32 x 32768 671 -> 650, 24 heads of 2048 causal 55 -> 38; a plain level of 32 x 16384
-// queries, before in runs of tiles per workgroup (attn_fwd_stream.inc), the same 200.
+// workgroups), leaves of 2048 rows, 32 x 32768 671 -> 650, 24 heads of 2048 causal 55 -> 38.  Exact attention still takes 8 waves where
+// that fills a last round better (large_tiles).
 template <int D>
 struct WaveShape {
   static constexpr int NB = D <= 64 ? 2 : 1;        // 32-query MFMA column blocks per wave
@@ -365,11 +365,11 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   // launch has the same number of key chunks to go through.  The hardware hands out workgroups in order and
   // a slot freed by a short one stays empty until the ones queued before it are placed: with one tile per
   // workgroup (4 to 32 chunks in a 2048-row leaf) the slots of a CU stood empty for 8 us at a time.
-  // Few workgroups (p.tiles_per_wg == 0, see single_tiles): one tile each, the tiles of all sequences, longest first,
+  // Few workgroups (p.single, see single_tiles): one tile each, the tiles of all sequences, longest first,
   // the second 256 in reversed order where a CU holds two workgroups (see ha_attn_fwd_split_kernel).
   constexpr bool PAIRED = CAUSAL && !GATHER;
   const int wg_per_seq = PAIRED ? (qtiles + 1) / 2 : qtiles;  // what p.div_qtiles divides by
-  const bool single = PAIRED && (FOLLOW || (D <= 64 && p.tiles_per_wg == 0));  // d = 128: the FOLLOW instance's alone
+  const bool single = PAIRED && (FOLLOW || (D <= 64 && p.single));  // d = 128: the FOLLOW instance's alone
   int hg, vseq, slot;
   if (single) {
     const int second = min((int)gridDim.x, 512);
@@ -419,7 +419,6 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   }
 }
 
-#include "attn_fwd_stream.inc"
 #include "attn_fwd_split.inc"
 
 namespace {
@@ -494,10 +493,6 @@ int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool c
     return launch_split<T, D, false, false, false, D>(p, grid, stream, "ha_flash_attn_fwd");
   }
   if constexpr (D == 64) {
-    if (gather && p.tiles_per_wg > 1) {  // set by ha_attn_launch for plain launches only
-      hipLaunchKernelGGL((ha_attn_fwd_stream_kernel<T, D>), dim3(grid), dim3(StreamShape<D>::THREADS), 0, stream, p);
-      return ha_launch_status("ha_block_attn_fwd");
-    }
     if (gather && p.follow_max) return launch_gathered<T, D, false, D, true>(p, grid, form, stream);
     if (gather && !p.small_tiles) return launch_one<T, D, true, false, PLAIN>(p, grid, stream, "ha_block_attn_fwd");
     if (!gather && p.small_tiles) {
@@ -698,14 +693,11 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   p.qk_pieces = d / 8;
   p.v_pieces = dv / 8;
   const bool single = causal && !gather && single_tiles(p, width);
-  p.tiles_per_wg = 1;
-  const char* stream_env = getenv("HA_STREAM_TILES");  // measurement aid: force the run length (1: off)
   const bool plain = !p.smooth && !p.sampled_idx && p.block_tiles % 2 == 0;
   const bool full_rows = p.qk_pieces == width / 8 && p.v_pieces == width / 8;
   const LaunchTimes t = launch_times(p, width, gather, causal);
   const char* split_env = getenv("HA_SPLIT");  // measurement aid: 1 forces the split kernel, 0 the other
-  // (a forced run length asks for the 256-query kernels)
-  p.split_keys = !reweight && !(gather && stream_env) && (split_env ? atoi(split_env) != 0 : t.split < (single ? t.single : t.whole));
+  p.split_keys = !reweight && (split_env ? atoi(split_env) != 0 : t.split < (single ? t.single : t.whole));
   // Head dims up to 64, tiles of 128 queries: gathered launches that are not plain always, since two tiles of 128 share neither
   // their window nor a block of 128 (a workgroup of 256 queries went through what either has, 1.05 to 1.2 times the time from 4
   // heads of 4096 rows to 128 of 32768, smooth blocks of 512 0.99 to 1.07); others of full rows by the estimates.
@@ -714,7 +706,7 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   // (without 1.01 and more), 12 heads of 2560 rows, blocks of 128 20.9 -> 19.7 us, 256 23.3 -> 22.4, 12 of 3072 25.8 -> 22.7
   // and 29.1 -> 26.2.  With 1024 keys a row the half costs what the tiles gain.
   p.small_tiles = p.large_tiles = p.follow_max = 0;
-  const bool choice = width == 64 && full_rows && !reweight && !(gather && stream_env);
+  const bool choice = width == 64 && full_rows && !reweight;
   const int chunks = 2 * p.block_tiles + p.sample_chunks;  // gathered: of a row's keys
   if (choice && gather && p.split_keys && !split_env && chunks <= 8 && t.small + 1.5 < t.split_rounds) {
     p.split_keys = 0;
@@ -749,24 +741,11 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   int64_t qtiles = (p.n_q + tile_rows - 1) / tile_rows;
   if (causal && !gather && !single) qtiles = (qtiles + 1) / 2;  // one workgroup per pair of tiles
   if (p.split_keys) qtiles = (p.n_q + 63) / 64;
-  // A plain gathered launch with whole 256-query tiles, whole key blocks and an even number of at least four key
-  // chunks per tile can run as a stream: a workgroup takes a run of tiles of its head
-  // (ha_attn_fwd_stream_kernel).  It measured 2 to 5 % slower than one tile per workgroup with two workgroups per CU,
-  // so only the measurement aid asks for it.
-  else if (stream_env && gather && !reweight && width == 64 && plain && full_rows && p.n_q % STREAM_QUERIES == 0 &&
-           p.n_q >= 2 * STREAM_QUERIES && p.sample_chunks % 2 == 0 && p.n_k % (p.block_tiles * 128) == 0 &&
-           2 * p.block_tiles + p.sample_chunks >= 4) {
-    const int r = std::min(atoi(stream_env), p.n_q / STREAM_QUERIES);
-    if (r > 1) {  // else one tile per workgroup, whose tiles are not these
-      p.tiles_per_wg = r;
-      qtiles = (p.n_q / STREAM_QUERIES + r - 1) / r;
-    }
-  }
   // causal launches of more split workgroups than CUs run longest first: tile number before sequence number
   if (p.split_keys && causal && !gather && qtiles * p.batch * p.heads * p.segs > 256) p.split_keys = 2;
-  if (single && !p.split_keys) p.tiles_per_wg = 0;
-  if (single && !p.split_keys) p.follow_max = width == 128 || t.split < t.whole;
-  p.div_qtiles = make_divisor(p.split_keys == 2 || p.tiles_per_wg == 0 ? (int64_t)p.batch * p.heads * p.segs : qtiles);
+  p.single = single && !p.split_keys;
+  if (p.single) p.follow_max = width == 128 || t.split < t.whole;
+  p.div_qtiles = make_divisor(p.split_keys == 2 || p.single ? (int64_t)p.batch * p.heads * p.segs : qtiles);
   p.div_segs = make_divisor(p.segs);
   p.div_heads = make_divisor(p.heads);
   p.div_kv_heads = make_divisor(p.heads / p.kv_group);

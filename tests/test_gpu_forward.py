@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import _gen, _randn, assert_close
+from _util import _gen, _randn, assert_close, forward_kernels
 from oracle import hyper_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -128,25 +128,26 @@ def test_causal_odd_lengths(ha, monkeypatch, n, msl, block):
     assert_close(lse, rl, "lse")
 
 
+@pytest.mark.parametrize("split", ["0", "1"])
 @pytest.mark.parametrize("d,dtype,kv_heads", [(128, torch.bfloat16, 1), (64, torch.float16, 2), (128, torch.float16, 2)])
-def test_one_call_forward_is_the_same_with_streaming_workgroups(ha, monkeypatch, d, dtype, kv_heads):
-    """The whole causal forward with the gathered levels run by workgroups that stream runs of query tiles
-    (forced by the library's measurement switch) equals the forward with one tile per workgroup bit for bit:
-    an odd length (the last query of the last segment of every hashed level is the appended row, which the
-    stream kernel has to drop), resumed partial results at every level, grouped-query heads."""
+def test_odd_length_with_levels_in_both_forms(ha, monkeypatch, split, d, dtype, kv_heads):
+    """The whole causal forward with its levels as tiles and with split keys (forced by the library's measurement switch): the
+    last query of the last segment of every hashed level is the appended row, which the kernels have to drop, a partial result is
+    resumed at every level, query heads share key heads."""
     n, msl = 9215, 2304   # -> 9216 -> halves of 4608 and 2304: two hashed levels of 18 and 9 tiles per segment
-    q = _randn((1, 2, n, d), 160, dtype).cuda()
-    k, v = (_randn((1, kv_heads, n, d), s, dtype).cuda() for s in (161, 162))
-    m, _ = _module(ha, d, dtype, 163, block_size=256, sample_size=256, min_seq_len=msl)
+    q = _randn((1, 2, n, d), 160, dtype)
+    k, v = (_randn((1, kv_heads, n, d), s, dtype) for s in (161, 162))
+    m, proj = _module(ha, d, dtype, 163, block_size=256, sample_size=256, min_seq_len=msl)
     _no_composed_path(m, monkeypatch)
-    out = {}
-    for tiles in (1, 4):
-        monkeypatch.setenv("HA_STREAM_TILES", str(tiles))
-        attn, lse = m(q, k, v, causal=True, return_lse=True)
-        torch.cuda.synchronize()
-        out[tiles] = (attn.clone(), lse.clone())
-    assert torch.isfinite(out[1][0].float()).all()
-    assert torch.equal(out[1][0], out[4][0]) and torch.equal(out[1][1], out[4][1])
+    monkeypatch.setenv("HA_SPLIT", split)
+    call = lambda: m(q.cuda(), k.cuda(), v.cuda(), causal=True, return_lse=True)  # noqa: E731
+    attn, lse = call()
+    full = (q, *(x.repeat_interleave(2 // kv_heads, 1) for x in (k, v)), proj, m, True)
+    ro, rl = _oracle(*full)
+    assert_close(attn, ro, "attn", dtype, _reference_arithmetic(dtype, *full))
+    assert_close(lse, rl, "lse")
+    forms = forward_kernels(call)  # leaves, two levels
+    assert len(forms) == 3 and all((f == "split") == (split == "1") for f in forms), forms
 
 
 def test_causal_odd_length_sort_places_the_appended_row(ha):
