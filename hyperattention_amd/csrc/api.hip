@@ -138,12 +138,11 @@ struct Ragged {
   int half[HA_MAX_RAGGED_LEVELS];
 };
 
-int flash_attn(const ha_attn_operands& t, int causal, int accumulate, hipStream_t stream, const Ragged* rag = nullptr) {
+int flash_attn(const ha_attn_operands& t, int causal, hipStream_t stream, const Ragged* rag = nullptr) {
   int st = ha_check_operands(t, "ha_flash_attn_fwd");
   if (st != HA_OK) return st;
   ha_attn_kernel_params p;
   fill_params(t, p);
-  p.accumulate = accumulate != 0;
   if (rag) {
     p.rag_levels = rag->levels; p.rag_n = rag->n;
     for (int i = 0; i < HA_MAX_RAGGED_LEVELS; ++i) p.rag_half[i] = rag->half[i];
@@ -457,7 +456,7 @@ extern "C" int ha_block_attn_fwd(const ha_block_attn_args* args, void* stream) {
 
 extern "C" int ha_flash_attn_fwd(const ha_attn_operands* t, int causal, void* stream) {
   HA_REQUIRE(t, HA_ERR_NULL, "ha_flash_attn_fwd: null argument block");
-  return flash_attn(*t, causal, 0, (hipStream_t)stream);
+  return flash_attn(*t, causal, (hipStream_t)stream);
 }
 
 extern "C" int64_t ha_forward_workspace_bytes(const ha_forward_args* args) {
@@ -571,7 +570,7 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     f.n_q = f.n_k = a.n;
     f.segs = 1; f.seg_stride_rows = a.n; f.q_seg_offset = f.k_seg_offset = 0;
     f.lse_rows = a.lse_rows;
-    return flash_attn(f, 0, 0, stream);
+    return flash_attn(f, 0, stream);
   }
 
   // Exact causal attention on the segments of level `level`.  With an odd length somewhere the segments are ragged:
@@ -584,12 +583,12 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     f.seg_stride_rows = rows;
     f.q_seg_offset = f.k_seg_offset = 0;
     if (pl.levels == 0) f.lse_rows = a.lse_rows;
-    if (!pl.ragged || level == 0) return flash_attn(f, 1, 0, stream);
+    if (!pl.ragged || level == 0) return flash_attn(f, 1, stream);
     Ragged rag = {};
     rag.levels = level;
     rag.n = (int)a.n;
     for (int i = 0; i < level; ++i) rag.half[i] = (int)pl.half[i];
-    return flash_attn(f, 1, 0, stream, &rag);
+    return flash_attn(f, 1, stream, &rag);
   };
 
   // 3. leaves: exact causal attention on every segment of the deepest level.  Where the deepest level's off-diagonal part is
