@@ -21,6 +21,7 @@
 #include "attn_bwd.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -54,7 +55,8 @@ constexpr uint32_t TILES = 0, DS = TILES + STEPS * 8192, KEYS = DS + 3 * 16384, 
                    ROWS = DELTA + 2 * FUSED_ROWS * 4, SAMPLE_ROWS = ROWS + 4 * FUSED_ROWS * 4, LDS_BYTES = SAMPLE_ROWS + FUSED_MAX_SAMPLES * 4;
 static_assert(LDS_BYTES <= 163840, "one workgroup per CU");
 
-template <typename T, bool ACC>
+// SHORT_O: O's rows are shorter than dO's (p.out_last), an instance of its own: as a clamp in every call 0.4 % of the kernel
+template <typename T, bool ACC, bool SHORT_O>
 __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(const ha_attn_bwd_params p) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
@@ -138,8 +140,8 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
   auto load_stats = [&](uint32_t row) -> Stats {
     const uint32_t piece = (opaque_lane() & 15) * 8;
     Stats st;
-    // O's rows may be shorter than dO's (p.out_last): the last 8 bytes stand in for those that are missing, which meet zeros of dO
-    st.o = *reinterpret_cast<const vec4*>(row_address(ob, row, o_rb, min(piece, (uint32_t)p.out_last * 16 + 8)));
+    // the last 8 bytes of a short row stand in for those that are missing, which meet zeros of dO
+    st.o = *reinterpret_cast<const vec4*>(row_address(ob, row, o_rb, SHORT_O ? min(piece, (uint32_t)p.out_last * 16 + 8) : piece));
     st.g = *reinterpret_cast<const vec4*>(row_address(dob, row, do_rb, piece));
     st.l = lseb[row];
     return st;
@@ -567,7 +569,12 @@ int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stre
   const int64_t grid = vseqs * ((blocks + p.run_blocks - 1) / p.run_blocks);
   if (grid >= (1ll << 31)) return ha_fail(HA_ERR_SHAPE, "ha_block_attn_bwd: grid of %lld workgroups", (long long)grid);
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FUSED_THREADS), LDS_BYTES, stream, p); };
-  if (is_f16) p.accumulate ? launch(ha_block_bwd_fused_kernel<f16_t, true>) : launch(ha_block_bwd_fused_kernel<f16_t, false>);
-  else p.accumulate ? launch(ha_block_bwd_fused_kernel<bf16_t, true>) : launch(ha_block_bwd_fused_kernel<bf16_t, false>);
+  auto launch_for = [&](auto short_o) {
+    constexpr bool SHORT_O = decltype(short_o)::value;
+    if (is_f16) p.accumulate ? launch(ha_block_bwd_fused_kernel<f16_t, true, SHORT_O>) : launch(ha_block_bwd_fused_kernel<f16_t, false, SHORT_O>);
+    else p.accumulate ? launch(ha_block_bwd_fused_kernel<bf16_t, true, SHORT_O>) : launch(ha_block_bwd_fused_kernel<bf16_t, false, SHORT_O>);
+  };
+  if (p.out_last < FD / 8 - 1) launch_for(std::true_type{});
+  else launch_for(std::false_type{});
   return ha_launch_status("ha_block_attn_bwd: blocks and sampled keys");
 }
