@@ -5,7 +5,7 @@ import torch
 
 from oracle import hyper_oracle as O
 from test_gpu_ops import ha  # noqa: F401 (fixture)
-from _util import _gen, _randn, assert_close
+from _util import _gen, _randn, assert_close, forward_kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -45,7 +45,10 @@ def test_exact(ha, monkeypatch, dtype, d, h, hk, n, causal):  # noqa: F811
 def test_exact_without_mask_in_rounds(ha, dtype, d, h, hk, n, scale):  # noqa: F811
     q = _randn((1, h, n, d), 74, dtype) * scale
     k, v = (_randn((1, hk, n, d), s, dtype) for s in (75, 76))
-    o, lse = ha.flash_attn_func(*(x.cuda().transpose(1, 2) for x in (q, k, v)), None, False)
+    on_gpu = [x.cuda().transpose(1, 2) for x in (q, k, v)]
+    call = lambda: ha.flash_attn_func(*on_gpu, None, False)  # noqa: E731
+    assert forward_kernels(call) == ["128 follow"]
+    o, lse = call()
     ro, rl = O.exact_attention(q, *(x.repeat_interleave(h // hk, 1) for x in (k, v)), None, False)
     assert_close(o.transpose(1, 2), ro, "out", dtype)
     assert_close(lse[:, :, :n], rl, "lse")
@@ -59,7 +62,9 @@ def test_gathered_in_rounds(ha, dtype, d, h, hk, n, smooth):  # noqa: F811
     k, v = (_randn((1, hk, n, d), s, dtype) for s in (78, 79))
     kw = dict(block_size=512, sample_size=512, min_seq_len=1, smooth_block=smooth)
     m = ha.HyperAttention(input_dim=d, rng=_gen(80), **kw).to(device="cuda", dtype=dtype)
-    attn, lse = m(q.cuda(), k.cuda(), v.cuda(), return_lse=True)
+    call = lambda: m(q.cuda(), k.cuda(), v.cuda(), return_lse=True)  # noqa: E731
+    assert forward_kernels(call) == ["128 follow"]
+    attn, lse = call()
     full = [x.repeat_interleave(h // hk, 1) for x in (k, v)]
     ref, ref_lse = O.hyper_forward(q, *full, m.lsh.proj_dir[0, 0].cpu(), **kw)
     assert_close(attn, ref, "attn", dtype)
