@@ -5,7 +5,9 @@
 // the blocks 403, of the sampled keys 229) and compute the scores twice (7 products per pair).  Here a workgroup gathers the
 // q, k, v, dO, O rows of a block of 256 queries and 256 keys once, computes every score once (5 products) and leaves dq, dk,
 // dv of the block and adds to the sampled keys' sums: 2.9 GB, 810 to 826 us in the same launch (without adding, 24 heads
-// of 16384, the whole call: 269 -> 223 us).  What bounds it now: the board's power limit (2.1 GHz); of a block's 73k cycles 50k are the steps.
+// of 16384, the whole call: 269 -> 223 us).  What bounds it now: not the board's power limit (2.21 to 2.28 GHz, matrix pipe busy 0.30 to 0.32 of
+// the time); of a block's 73k cycles 50k are the steps, the others the ends of its phases, where every wave does the same memory and vector
+// work with one workgroup per CU and nothing beside it.
 //
 // A workgroup: 8 waves, a run of consecutive blocks of one (head, segment).  A block has a phase for its own keys and one
 // per 256 sampled keys.  In a phase a wave keeps 32 keys (k, v rows as MFMA B operands, sums of dK^T, dV^T in registers) and

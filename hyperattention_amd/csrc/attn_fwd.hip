@@ -542,17 +542,17 @@ static ha_divisor make_divisor(int64_t y) {
 // is 0.2 % slower than the best one on average (worst: 40 heads of 512 rows, 96 columns 10 %, 24 of 700, 128 columns 8 %).  Single tiles of 128
 // queries | split: 12 heads of 1000 rows 20.7 | 17.2, 24 of 1000 20.6 | 22.3, 48 25.1 | 37; 8 of 512 13.3 | 12.3, 96 columns 13.2 | 10.3;
 // 16 of 2048 35.3 | 34.3, 24 38.4 | 50; 8 of 4096 65 | 51, 12 70 | 85.
-// d = 128, without mask or gathered: the estimate of `whole` is that of a kernel of 256-query tiles, which the present one outruns.  It
-// is kept because the split form is the closer one to float64 (four exact weights per row: 2 to 4 % for 256 to 1024 keys a row,
-// 0.2 to 2 % above), and the launches that it gives to it lose little: 8 heads of 2048 rows, blocks and samples of 128 10.7 | 12.2,
+// d = 128, without mask or gathered: the estimate of `whole` is that of 256-query tiles, which gathered launches no longer have and
+// exact ones take in few places (large_tiles); tiles of 128 outrun it.  It stays the line because the split form is the closer one to
+// float64 (four exact weights per row: 2 to 4 % for 256 to 1024 keys a row, 0.2 to 2 % above), and the launches that it gives to it lose little: 8 heads of 2048 rows, blocks and samples of 128 10.7 | 12.2,
 // 256 14.5 | 14.5, 512 22.8 | 19.8; without mask 12 of 1000 19.8 | 17.1, 4 of 4096 57 | 44.  What it gives the split kernel beyond
 // one round ha_attn_launch takes back.
 //
 // d = 64, tiles of 256 | 128 queries (`large`, `small`; 470 launches of 6 to 512 heads, 512 to 8192 rows, mean error 3 %; a choice that lost 2.5 % or more is not among them).  A
 // workgroup of 128 queries takes half as long, a CU holds three, and ragged rows waste less; its waves read the keys
-// for half as many queries, 10 % more time on a full chip.  Exact causal, us: 48 heads of 700 rows 16.8 | 13.4, of 2048 40.0 | 35.9, 32 of 3000 53.8 |
-// 48.6, 64 of 1000 23.2 | 18.6, 24 of 4096 70.3 | 64.5, but 48 of 4096 113 | 115.5, 160 of 4096 341 | 376; without mask 32 of 1000 21.0 |
-// 16.1, 48 of 2048 62 | 58, 64 of 2048 69 | 76; whole calls with blocks and samples of 256: 16 heads of 2560 rows 24.6 | 23.7, 24 of
+// for half as many queries, 10 % more time on a full chip.  Exact causal, us: 48 heads of 2048 rows 40.0 | 35.9, 32 of 3000 53.8 |
+// 48.6, 64 of 1000 23.2 | 18.6, 24 of 4096 70.3 | 64.5, but 48 of 4096 113 | 115.5, 160 of 4096 341 | 376; without mask 48 of
+// 2048 62 | 58, 64 of 2048 69 | 76 (what the split kernel takes from tiles of 256 without mask stays with it: the closer one to float64); whole calls with blocks and samples of 256: 16 heads of 2560 rows 24.6 | 23.7, 24 of
 // 4096 37.0 | 36.0, 24 of 6144 54.5 | 51.2, 24 of 8192 58.3 | 59.4.
 struct LaunchTimes {
   double whole, single, split;  // a tile per workgroup (exact causal: pairs of tiles), single causal tiles, the split kernel

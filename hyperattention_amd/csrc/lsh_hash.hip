@@ -283,7 +283,7 @@ int ha_hash_i32(const void* x, const void* proj, int32_t* buckets, int64_t batch
 }
 
 // Bucket ids of the queries and keys of one forward pass as one byte each (r <= 8 projections, one shared
-// projection matrix), in one launch.  q: (batch, heads, n_read, d), k: (batch, kv_heads, n_read, d), d in {64, 128};
+// projection matrix), in one launch.  q: (batch, heads, n_read, d), k: (batch, kv_heads, n_read, d), d a multiple of 8 up to 128;
 // ids: n >= n_read per sequence, the ids past n_read being those of zero rows.  Wanted are the queries' from row q_first
 // on and the keys' before row k_end.
 int ha_hash_pair_u8(const void* q, const void* k, const void* proj, uint8_t* ids_q, uint8_t* ids_k, int64_t batch,
