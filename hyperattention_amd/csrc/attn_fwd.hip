@@ -643,6 +643,8 @@ static LaunchTimes launch_times(const ha_attn_kernel_params& p, int width, bool 
 // these tiles, and tiles without FOLLOW have 1.007 to 1.024 times its error, with it less (300 to 2048 sequences, normal and clustered).
 // Split | pairs | single, us: 512 of 65 28.3 | 12.1 | 13.0, of 128 35.6 | 17.0 | 17.2, 320 of 150 26.0 | 20.4 | 21.3; 96 columns: 512 of 128 28.1 |
 // 13.7 | 13.9.  From 384 on two rounds of pairs are closer to full (480 of 172, 80 columns 22 | 20.5 | 23.5, 1016 of 172 50.5 | 45.4 | 47.8).
+// One round of sequences of 129 to 256 rows, which fill the chip with tiles that all follow, pays the most for it: up to 2 us against tiles of
+// 256 without, 256 of 200 16.7 | 18.7, of 130 12.3 | 13.4 (large_tiles), 200 of 200 14.4 | 15.1, 96 columns 248 of 220 14.3 | 15.4.
 static bool single_tiles(const ha_attn_kernel_params& p, int width) {
   const int64_t pair_rows = width == 64 ? 2 * WaveShape<64>::QUERIES : 2 * WaveShape<128>::QUERIES;
   const double vheads = (double)p.batch * p.heads * p.segs, pairs = vheads * ((p.n_q + pair_rows - 1) / pair_rows) / 256.;
