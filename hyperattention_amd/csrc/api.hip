@@ -138,7 +138,8 @@ struct Ragged {
   int half[HA_MAX_RAGGED_LEVELS];
 };
 
-int flash_attn(const ha_attn_operands& t, int causal, hipStream_t stream, const Ragged* rag = nullptr) {
+int flash_attn(const ha_attn_operands& t, int causal, hipStream_t stream, const Ragged* rag = nullptr,
+               const ha_rank_beside* ranking = nullptr) {
   int st = ha_check_operands(t, "ha_flash_attn_fwd");
   if (st != HA_OK) return st;
   ha_attn_kernel_params p;
@@ -147,7 +148,7 @@ int flash_attn(const ha_attn_operands& t, int causal, hipStream_t stream, const 
     p.rag_levels = rag->levels; p.rag_n = rag->n;
     for (int i = 0; i < HA_MAX_RAGGED_LEVELS; ++i) p.rag_half[i] = rag->half[i];
   }
-  return ha_attn_launch(p, (int)t.d, (int)t.dv, t.dtype, false, causal != 0, false, stream);
+  return ha_attn_launch(p, (int)t.d, (int)t.dv, t.dtype, false, causal != 0, false, stream, ranking);
 }
 
 inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
@@ -212,6 +213,7 @@ int make_plan(const ha_forward_args& a, Plan& pl) {
 
 struct Workspace {
   bool units;                          // one ranking for all levels (byte-sized ids), else a sort per level
+  bool beside;                         // with `units`: hashed and ranked beside the leaves, without ids in memory
   ha_unit_grid grid;
   int64_t buckets_q, buckets_k;        // byte offsets; one byte per id with `units`, else int32
   int64_t sorted_q, sorted_k;          // with `units`: per-unit orders
@@ -226,7 +228,8 @@ struct Workspace {
 // longest hashed segment may span this many units before the per-level sort is the better choice.
 inline int64_t max_units_per_segment(int unit) { return std::max<int64_t>(64, unit / 4); }
 
-void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w) {
+// leaves: an exact causal launch precedes the hashed levels, which units can be hashed and ranked beside
+void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w, bool leaves) {
   int64_t off = 0;
   memset(&w, 0, sizeof(w));
   const int nlev = a.causal ? pl.levels : 1;
@@ -235,10 +238,11 @@ void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w) {
     ha_unit_grid& g = w.grid;
     g.n = nh;
     g.granule = pl.granule;
-    // the one segment of the one hashed level in one unit, without a placement launch, up to the length where that is
-    // faster (rank_units_kernel) and one workgroup per CU
-    const bool whole = nh / g.granule == (a.causal ? 2 : 1) && g.granule <= HA_SORT_WHOLE && a.batch * (a.heads + a.kv_heads) <= 256;
-    const int64_t most = whole ? HA_SORT_WHOLE : HA_SORT_CHUNK;
+    // the one segment of the one hashed level in one unit, without a placement launch: up to the length where that is
+    // faster (rank_units_kernel) and one workgroup per CU, or, beside the leaves, where its rows' numbers and ids fit the tiles' LDS
+    const bool one = nh / g.granule == (a.causal ? 2 : 1);
+    const bool whole = one && (leaves ? g.granule <= HA_SORT_BESIDE : g.granule <= HA_SORT_WHOLE && a.batch * (a.heads + a.kv_heads) <= 256);
+    const int64_t most = whole ? g.granule : HA_SORT_CHUNK;
     g.units_per_granule = (int)((g.granule + most - 1) / most);
     g.unit = (int)std::min<int64_t>(g.granule, most);
     g.units_per_seq = (int)(nh / g.granule) * g.units_per_granule;
@@ -247,7 +251,8 @@ void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w) {
       if (pl.level_hyper[j]) longest = std::max<int64_t>(longest, a.causal ? pl.half[j] : a.n);
     w.units = a.lsh_num_projs <= 8 && longest / g.granule * g.units_per_granule <= max_units_per_segment(g.unit) &&
               nh % g.granule == 0;
-    const int64_t id_bytes = w.units ? 1 : 4;
+    w.beside = w.units && leaves;
+    const int64_t id_bytes = w.beside ? 0 : w.units ? 1 : 4;
     w.buckets_q = off; off += align256(a.batch * a.heads * nh * id_bytes);
     w.buckets_k = off; off += align256(a.batch * a.kv_heads * nh * id_bytes);
     if (w.units) {
@@ -330,6 +335,61 @@ int check_forward_layout(const ha_attn_operands& t, bool with_values, const char
   return HA_OK;
 }
 
+// The units that a ranking of the hashed levels takes, and where it leaves them in the workspace.
+struct Units {
+  uint32_t *sorted[2], *hist[2];
+  int32_t* whole[2];  // one unit per sequence is the one segment of the one hashed level: its rank is its order, nothing to place
+  int64_t seqs[2];
+  int first_unit[2], num_units;
+};
+Units units_of(const ha_forward_args& a, const Workspace& w) {
+  unsigned char* ws = (unsigned char*)a.workspace;
+  Units u = {};
+  u.sorted[0] = (uint32_t*)(ws + w.sorted_q); u.sorted[1] = (uint32_t*)(ws + w.sorted_k);
+  u.hist[0] = (uint32_t*)(ws + w.unit_hist_q); u.hist[1] = (uint32_t*)(ws + w.unit_hist_k);
+  u.seqs[0] = a.batch * a.heads; u.seqs[1] = a.batch * a.kv_heads;
+  u.first_unit[0] = a.causal ? w.grid.units_per_granule : 0;
+  u.num_units = w.grid.units_per_seq - u.first_unit[0];
+  if (u.num_units == 1) {
+    u.whole[0] = (int32_t*)(ws + w.qidx[0]);
+    u.whole[1] = (int32_t*)(ws + w.kidx[0]);
+  }
+  return u;
+}
+
+// The stable bucket order of every hashed level's segments from the units' orders and counts.
+int place_units(const ha_forward_args& a, const Plan& pl, const Workspace& w, hipStream_t stream) {
+  unsigned char* ws = (unsigned char*)a.workspace;
+  const int nlev = a.causal ? pl.levels : 1;
+  const Units u = units_of(a, w);
+  if (u.num_units == 1) return HA_OK;
+  ha_place_jobs jobs;
+  jobs.num_jobs = 0;
+  jobs.grid = w.grid;
+  int64_t blocks = 0;
+  for (int j = 0; j < nlev; ++j) {
+    if (!pl.level_hyper[j]) continue;
+    const int64_t seg_len = a.causal ? pl.half[j] : a.n;
+    const int64_t segs = a.causal ? (1ll << j) : 1;
+    for (int side = 0; side < 2; ++side) {
+      HA_REQUIRE(jobs.num_jobs < HA_SORT_MAX_JOBS, HA_ERR_SHAPE, "ha_forward: too many sort jobs");
+      ha_place_job& job = jobs.job[jobs.num_jobs++];
+      job.sorted = u.sorted[side];
+      job.hist = u.hist[side];
+      job.out = (int32_t*)(ws + (side == 0 ? w.qidx[j] : w.kidx[j]));
+      job.seg_stride = a.causal ? 2 * seg_len : a.n;
+      job.seg_offset = (a.causal && side == 0) ? seg_len : 0;  // queries: second halves, keys: first halves
+      job.seg_len = (int)seg_len;
+      job.segs_per_seq = (int)segs;
+      job.units_per_seg = (int)(seg_len / w.grid.granule) * w.grid.units_per_granule;
+      job.first_block = (int)blocks;
+      blocks += u.seqs[side] * segs * job.units_per_seg;
+      HA_REQUIRE(blocks < (1ll << 30), HA_ERR_SHAPE, "ha_forward: too many sort units");
+    }
+  }
+  return ha_place_units(jobs, (int)blocks, stream);
+}
+
 // Bucket ids of q and k, then the stable bucket order of the query and key segment of every hashed level
 // (hyper_attention.py:112-117 at every level of the recursion), as int32 rows local to the segment.
 int hash_and_sort(const ha_forward_args& a, const Plan& pl, const Workspace& w, const ha_attn_operands& t,
@@ -345,44 +405,9 @@ int hash_and_sort(const ha_forward_args& a, const Plan& pl, const Workspace& w, 
                          a.n, a.d, a.lsh_num_projs, qs, ks, unused, pl.n_hashed - unused, a.dtype, stream);
     if (st != HA_OK) return st;
     const uint8_t* ids[2] = {ws + w.buckets_q, ws + w.buckets_k};
-    uint32_t* sorted[2] = {(uint32_t*)(ws + w.sorted_q), (uint32_t*)(ws + w.sorted_k)};
-    uint32_t* hist[2] = {(uint32_t*)(ws + w.unit_hist_q), (uint32_t*)(ws + w.unit_hist_k)};
-    const int64_t seqs[2] = {a.batch * a.heads, a.batch * a.kv_heads};
-    const int first_unit[2] = {a.causal ? w.grid.units_per_granule : 0, 0};
-    const int num_units = w.grid.units_per_seq - first_unit[0];
-    // one unit per sequence is the one segment of the one hashed level: its rank is its order, nothing to place
-    int32_t* whole[2] = {nullptr, nullptr};
-    if (num_units == 1) {
-      whole[0] = (int32_t*)(ws + w.qidx[0]);
-      whole[1] = (int32_t*)(ws + w.kidx[0]);
-    }
-    st = ha_rank_units(ids, sorted, hist, seqs, w.grid, first_unit, num_units, whole, stream);
-    if (st != HA_OK || num_units == 1) return st;
-    ha_place_jobs jobs;
-    jobs.num_jobs = 0;
-    jobs.grid = w.grid;
-    int64_t blocks = 0;
-    for (int j = 0; j < nlev; ++j) {
-      if (!pl.level_hyper[j]) continue;
-      const int64_t seg_len = a.causal ? pl.half[j] : a.n;
-      const int64_t segs = a.causal ? (1ll << j) : 1;
-      for (int side = 0; side < 2; ++side) {
-        HA_REQUIRE(jobs.num_jobs < HA_SORT_MAX_JOBS, HA_ERR_SHAPE, "ha_forward: too many sort jobs");
-        ha_place_job& job = jobs.job[jobs.num_jobs++];
-        job.sorted = sorted[side];
-        job.hist = hist[side];
-        job.out = (int32_t*)(ws + (side == 0 ? w.qidx[j] : w.kidx[j]));
-        job.seg_stride = a.causal ? 2 * seg_len : a.n;
-        job.seg_offset = (a.causal && side == 0) ? seg_len : 0;  // queries: second halves, keys: first halves
-        job.seg_len = (int)seg_len;
-        job.segs_per_seq = (int)segs;
-        job.units_per_seg = (int)(seg_len / w.grid.granule) * w.grid.units_per_granule;
-        job.first_block = (int)blocks;
-        blocks += seqs[side] * segs * job.units_per_seg;
-        HA_REQUIRE(blocks < (1ll << 30), HA_ERR_SHAPE, "ha_forward: too many sort units");
-      }
-    }
-    return ha_place_units(jobs, (int)blocks, stream);
+    const Units u = units_of(a, w);
+    st = ha_rank_units(ids, u.sorted, u.hist, u.seqs, w.grid, u.first_unit, u.num_units, u.whole, stream);
+    return st != HA_OK ? st : place_units(a, pl, w, stream);
   }
 
   int32_t* bq = (int32_t*)(ws + w.buckets_q);
@@ -468,9 +493,10 @@ extern "C" int64_t ha_forward_workspace_bytes(const ha_forward_args* args) {
     return ha_fail(HA_ERR_SHAPE, "ha_forward_workspace_bytes: sizes must be positive");
   int st = make_plan(a, pl);
   if (st != HA_OK) return st;
-  Workspace w;
-  layout_workspace(a, pl, w);
-  return w.total;
+  Workspace w, with_leaves;
+  layout_workspace(a, pl, w, false);
+  layout_workspace(a, pl, with_leaves, a.causal);
+  return std::max(w.total, with_leaves.total);
 }
 
 extern "C" int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offset, int64_t* k_idx_offset,
@@ -488,7 +514,7 @@ extern "C" int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offse
   int st = make_plan(a, pl);
   if (st != HA_OK) return st;
   Workspace w;
-  layout_workspace(a, pl, w);
+  layout_workspace(a, pl, w, false);
   const int nlev = a.causal ? pl.levels : 1;
   *num_levels = nlev;
   for (int j = 0; j < nlev; ++j) {
@@ -517,7 +543,7 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   st = make_plan(a, pl);
   if (st != HA_OK) return st;
   Workspace w;
-  layout_workspace(a, pl, w);
+  layout_workspace(a, pl, w, a.causal);
   if (pl.any_hyper) {
     st = check_hashing(a, w, "ha_forward");
     if (st != HA_OK) return st;
@@ -532,10 +558,30 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   if (st != HA_OK) return st;
 
   // 1. bucket ids, once for the whole tensors (the projection does not depend on the level), and
-  // 2. the bucket order of every segment of every hashed level
-  if (pl.any_hyper) {
+  // 2. the bucket order of every segment of every hashed level; in a causal pass up to the units' orders beside the leaves, which
+  // need neither (24 heads of 4096 rows 63.3 -> 56.8 us: place_ranking in attn_fwd.hip)
+  if (pl.any_hyper && !w.beside) {
     st = hash_and_sort(a, pl, w, t, stream);
     if (st != HA_OK) return st;
+  }
+  ha_rank_beside ranking = {};
+  if (w.beside) {
+    const Units u = units_of(a, w);
+    ranking.proj = a.proj;
+    for (int i = 0; i < 2; ++i) {
+      ranking.sorted[i] = u.sorted[i];
+      ranking.hist[i] = u.hist[i];
+      ranking.out[i] = u.whole[i];
+      ranking.first_unit[i] = u.first_unit[i];
+    }
+    ranking.n_read = a.n;
+    ranking.num_projs = (int)a.lsh_num_projs;
+    ranking.num_units = u.num_units;
+    const int64_t units = (u.seqs[0] + u.seqs[1]) * u.num_units;
+    HA_REQUIRE(units < (1ll << 30), HA_ERR_SHAPE, "ha_forward: too many sort units");
+    ranking.units0 = (int)(u.seqs[0] * u.num_units);
+    ranking.units = (int)units;
+    ranking.grid = w.grid;
   }
 
   auto hyper_level = [&](int j, bool accumulate) -> int {
@@ -583,12 +629,12 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
     f.seg_stride_rows = rows;
     f.q_seg_offset = f.k_seg_offset = 0;
     if (pl.levels == 0) f.lse_rows = a.lse_rows;
-    if (!pl.ragged || level == 0) return flash_attn(f, 1, stream);
+    if (!pl.ragged || level == 0) return flash_attn(f, 1, stream, nullptr, w.beside ? &ranking : nullptr);
     Ragged rag = {};
     rag.levels = level;
     rag.n = (int)a.n;
     for (int i = 0; i < level; ++i) rag.half[i] = (int)pl.half[i];
-    return flash_attn(f, 1, stream, &rag);
+    return flash_attn(f, 1, stream, &rag, w.beside ? &ranking : nullptr);
   };
 
   // 3. leaves: exact causal attention on every segment of the deepest level.  Where the deepest level's off-diagonal part is
@@ -600,6 +646,10 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   const int leaf_level = pl.levels > 0 && !pl.level_hyper[pl.levels - 1] ? pl.levels - 1 : pl.levels;
   st = exact_level(leaf_level);
   if (st != HA_OK) return st;
+  if (w.beside) {
+    st = place_units(a, pl, w, stream);
+    if (st != HA_OK) return st;
+  }
   // 4. off-diagonal parts, deepest level first, merged in place into the second halves
   for (int j = leaf_level - 1; j >= 0; --j) {
     st = hyper_level(j, true);

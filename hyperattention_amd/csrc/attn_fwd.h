@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bucket_sort.h"
+
 // x / y for 0 <= x < 2^31 as (x * magic) >> shift, with shift = 31 + ceil(log2 y) and
 // magic = floor(2^shift / y) + 1 < 2^32 (exact for every such x)
 struct ha_divisor {
@@ -11,6 +13,24 @@ struct ha_divisor {
 };
 
 constexpr int HA_MAX_RAGGED_LEVELS = 30;
+
+// Workgroups of an exact causal launch that hash and rank units of the same tensors' rows for the hashed levels that follow
+// (unit_ranking.h).  They come in groups of eight, one per XCD, so that the others keep the XCD that their number gives them.
+struct ha_rank_beside {
+  const void* proj;       // (d, num_projs), num_projs <= 8
+  uint32_t* sorted[2];    // of q's and k's units: as ha_rank_units
+  uint32_t* hist[2];
+  int32_t* out[2];
+  int64_t n_read;         // rows of a sequence that exist; the others are zero rows
+  int num_projs;
+  int first_unit[2];
+  int num_units;          // of a sequence
+  int units0;             // of q
+  int units;              // of q and k
+  ha_unit_grid grid;
+  int tiles;              // workgroups of the attention (filled by ha_attn_launch)
+  int first_group, groups;  // groups of eight workgroups before the first ranking one, and of ranking ones (as well)
+};
 
 struct ha_attn_kernel_params {
   const void* q;
@@ -67,8 +87,9 @@ struct ha_attn_kernel_params {
   ha_divisor div_qtiles, div_segs, div_heads, div_kv_heads, div_kv_group, div_block_tiles;
 };
 
+// ranking: exact causal launches, or null
 int ha_attn_launch(const ha_attn_kernel_params& p, int d, int dv, int dtype, bool gather, bool causal, bool reweight,
-                   hipStream_t stream);
+                   hipStream_t stream, const ha_rank_beside* ranking = nullptr);
 
 // argument checks shared by the forward and backward entry points (defined in api.hip); `who` names
 // the entry point in the error message

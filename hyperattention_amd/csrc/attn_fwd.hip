@@ -52,6 +52,7 @@
 #include "ha_common.h"
 #include "attn_tiles.h"
 #include "attn_fwd.h"
+#include "unit_ranking.h"
 
 #include <stdlib.h>
 
@@ -90,6 +91,16 @@ struct WaveShape {
 
 // x / y for 0 <= x < 2^31 by the divisor's multiply-and-shift constants
 __device__ __forceinline__ int fast_div(int x, ha_divisor y) { return (int)(((uint64_t)(uint32_t)x * y.magic) >> y.shift); }
+
+// What workgroup `id` of a launch with ranking workgroups does: a unit's number, or -1; in `id` and `count` its number among
+// the others and how many they are, no less than which means that it is none of them.
+__device__ __forceinline__ int ranking_unit(const ha_rank_beside& a, int& id, int& count) {
+  const int unit = id - a.first_group * NUM_XCD, ranking = a.groups * NUM_XCD;
+  count = a.tiles;
+  if (unit < 0) return -1;
+  id = unit < ranking ? count : id - ranking;
+  return unit < a.units ? unit : -1;
+}
 
 // LDS byte offsets of one lane's operand reads, relative to a tile base (fixed for the whole kernel).
 template <int DC>
@@ -317,8 +328,9 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
 // sequence's first tile, gathered (plain or not, tiles of 128 queries) and at head dims above 64 without mask in a row's first p.follow_max chunks.  An
 // instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
 template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
-__global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES, typename... Ranking>
+__global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p,
+                                                                                          const Ranking... ranking) {
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int QW = 32 * NB;                 // queries per wave
@@ -348,6 +360,16 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   __shared__ int lds_qrow[WG_QUERIES];   // original row of every query position (-1: past the end)
   __shared__ float lds_w[WG_QUERIES];    // weight of the resumed partial result per query position
 
+  int wg_id = blockIdx.x, wg_count = gridDim.x;
+  if constexpr (sizeof...(Ranking) > 0) {
+    const int unit = ranking_unit(ranking..., wg_id, wg_count);
+    if (unit >= 0) {
+      if constexpr (D == 64) hash_and_rank_unit<T, DC / 32, WAVES>(p, ranking..., unit, lds_q, lds_k0, lds_v0, lds_v1);
+      else hash_and_rank_unit<T, DC / 32, WAVES>(p, ranking..., unit, lds_k0, lds_k1, lds_v0, lds_v1);
+    }
+    if (wg_id >= wg_count) return;
+  }
+
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   // the same number, known to the compiler to be wave-uniform: what the tile loads derive from it
@@ -359,7 +381,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   // Workgroup number = (((batch, kv head), segment), tile, query head inside the kv group), the last one
   // fastest: the query heads that share a kv head work on the same tile side by side, on one XCD, so that the
   // K and V rows of the tile (the same for all of them) come from HBM once and from L2 after that.
-  int wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
+  int wg = xcd_contiguous_id(wg_id, wg_count);
   const int qtiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES;
   // Exact causal attention, many workgroups: one takes the tile pair (qtiles-1-s, s), so that every workgroup of the
   // launch has the same number of key chunks to go through.  The hardware hands out workgroups in order and
@@ -372,8 +394,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_att
   const bool single = PAIRED && (FOLLOW || (D <= 64 && p.single));  // d = 128: the FOLLOW instance's alone
   int hg, vseq, slot;
   if (single) {
-    const int second = min((int)gridDim.x, 512);
-    wg = blockIdx.x;
+    const int second = min(wg_count, 512);
+    wg = wg_id;
     if (WAVES == 4 && wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
     slot = fast_div(wg, p.div_qtiles);
     wg -= slot * (p.batch * p.heads * p.segs);  // what p.div_qtiles divides by here
@@ -431,8 +453,26 @@ int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, con
   return ha_launch_status(what);
 }
 
+// exact causal, in instances of their own with ranking workgroups: the branch and the longer argument block cost every
+// other launch 0.2 to 0.3 us
+template <typename T, int D, bool NARROW, int DC, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
+int launch_causal(const ha_attn_kernel_params& p, const ha_rank_beside* r, int grid, hipStream_t stream) {
+  const char* const what = "ha_flash_attn_fwd";
+  if (!r) return launch_one<T, D, false, true, GENERAL, NARROW, false, DC, FOLLOW, NB, WAVES>(p, grid, stream, what);
+  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, false, true, GENERAL, NARROW, false, DC, FOLLOW, NB, WAVES, ha_rank_beside>), dim3(grid),
+                     dim3(64 * WAVES), 0, stream, p, *r);
+  return ha_launch_status(what);
+}
+
 template <typename T, int D, bool GATHER, bool CAUSAL, bool NARROW, int DC>
-int launch_split(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
+int launch_split(const ha_attn_kernel_params& p, const ha_rank_beside* r, int grid, hipStream_t stream, const char* what) {
+  if constexpr (CAUSAL) {
+    if (r) {
+      hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, NARROW, DC, ha_rank_beside>), dim3(grid),
+                         dim3(SplitShape<D>::THREADS), 0, stream, p, *r);
+      return ha_launch_status(what);
+    }
+  }
   hipLaunchKernelGGL((ha_attn_fwd_split_kernel<T, D, GATHER, CAUSAL, NARROW, DC>), dim3(grid), dim3(SplitShape<D>::THREADS), 0,
                      stream, p);
   return ha_launch_status(what);
@@ -452,11 +492,11 @@ int launch_gathered(const ha_attn_kernel_params& p, int grid, GatherForm form, h
 // causal rows of d = 96: 546 -> 507 us (gathered level 87 -> 76, leaves 173 -> 151); 8 heads of 16384 rows without mask:
 // 896 -> 791 us.
 template <typename T, int D, int DC>
-int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, GatherForm form, hipStream_t stream) {
+int launch_narrow(const ha_attn_kernel_params& p, const ha_rank_beside* r, int grid, bool gather, bool causal, GatherForm form, hipStream_t stream) {
   if (p.split_keys) {
-    if (gather) return launch_split<T, D, true, false, true, DC>(p, grid, stream, "ha_block_attn_fwd");
-    if (causal) return launch_split<T, D, false, true, true, DC>(p, grid, stream, "ha_flash_attn_fwd");
-    return launch_split<T, D, false, false, true, DC>(p, grid, stream, "ha_flash_attn_fwd");
+    if (gather) return launch_split<T, D, true, false, true, DC>(p, r, grid, stream, "ha_block_attn_fwd");
+    if (causal) return launch_split<T, D, false, true, true, DC>(p, r, grid, stream, "ha_flash_attn_fwd");
+    return launch_split<T, D, false, false, true, DC>(p, r, grid, stream, "ha_flash_attn_fwd");
   }
   // the plain instance: d = 96, 16 heads of 32768 rows 205 -> 182 us, d = 40 98 -> 88
   if (gather && D == 64 && !p.small_tiles) return launch_one<T, D, true, false, PLAIN, true, false, DC>(p, grid, stream, "ha_block_attn_fwd");
@@ -465,10 +505,10 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
   }
   if (gather) return launch_gathered<T, D, true, DC>(p, grid, form, stream);
   if constexpr (D == 128) {
-    if (causal && p.large_tiles) return launch_one<T, D, false, true, GENERAL, true, false, DC, true, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
+    if (causal && p.large_tiles) return launch_causal<T, D, true, DC, true, 1, 8>(p, r, grid, stream);
   }
-  if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
-  if (causal) return launch_one<T, D, false, true, GENERAL, true, false, DC>(p, grid, stream, "ha_flash_attn_fwd");
+  if (causal && p.follow_max) return launch_causal<T, D, true, DC, true>(p, r, grid, stream);
+  if (causal) return launch_causal<T, D, true, DC>(p, r, grid, stream);
   if constexpr (D == 128) {
     if (p.large_tiles) return launch_one<T, D, false, false, GENERAL, true, false, DC, false, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
     if (p.follow_max) return launch_one<T, D, false, false, GENERAL, true, false, DC, true>(p, grid, stream, "ha_flash_attn_fwd");
@@ -477,36 +517,36 @@ int launch_narrow(const ha_attn_kernel_params& p, int grid, bool gather, bool ca
 }
 
 template <typename T, int D>
-int launch_variant(const ha_attn_kernel_params& p, int grid, bool gather, bool causal, bool reweight, hipStream_t stream) {
+int launch_variant(const ha_attn_kernel_params& p, const ha_rank_beside* r, int grid, bool gather, bool causal, bool reweight, hipStream_t stream) {
   if (gather && reweight)  // the entry point has checked that the head dims are the built ones
     return launch_one<T, D, true, false, GENERAL, false, true, D, false, 1>(p, grid, stream, "ha_block_attn_fwd");
   const GatherForm form = p.sampled_idx ? GENERAL : p.smooth ? SMOOTH : PLAIN;
   if (p.qk_pieces != D / 8 || p.v_pieces != D / 8) {
     if constexpr (D == 128) {
-      if (p.qk_pieces <= 12 && p.v_pieces <= 12) return launch_narrow<T, D, 96>(p, grid, gather, causal, form, stream);
+      if (p.qk_pieces <= 12 && p.v_pieces <= 12) return launch_narrow<T, D, 96>(p, r, grid, gather, causal, form, stream);
     }
-    return launch_narrow<T, D, D>(p, grid, gather, causal, form, stream);
+    return launch_narrow<T, D, D>(p, r, grid, gather, causal, form, stream);
   }
   if (p.split_keys) {
-    if (gather) return launch_split<T, D, true, false, false, D>(p, grid, stream, "ha_block_attn_fwd");
-    if (causal) return launch_split<T, D, false, true, false, D>(p, grid, stream, "ha_flash_attn_fwd");
-    return launch_split<T, D, false, false, false, D>(p, grid, stream, "ha_flash_attn_fwd");
+    if (gather) return launch_split<T, D, true, false, false, D>(p, r, grid, stream, "ha_block_attn_fwd");
+    if (causal) return launch_split<T, D, false, true, false, D>(p, r, grid, stream, "ha_flash_attn_fwd");
+    return launch_split<T, D, false, false, false, D>(p, r, grid, stream, "ha_flash_attn_fwd");
   }
   if constexpr (D == 64) {
     if (gather && p.follow_max) return launch_gathered<T, D, false, D, true>(p, grid, form, stream);
     if (gather && !p.small_tiles) return launch_one<T, D, true, false, PLAIN>(p, grid, stream, "ha_block_attn_fwd");
     if (!gather && p.small_tiles) {
-      if (causal) return launch_one<T, D, false, true, GENERAL, false, false, D, true, 1>(p, grid, stream, "ha_flash_attn_fwd");
+      if (causal) return launch_causal<T, D, false, D, true, 1>(p, r, grid, stream);
       return launch_one<T, D, false, false, GENERAL, false, false, D, false, 1>(p, grid, stream, "ha_flash_attn_fwd");
     }
   }
   if constexpr (D == 128) {
     if (gather && p.follow_max) return launch_gathered<T, D, false, D, true>(p, grid, form, stream);
-    if (causal && p.large_tiles) return launch_one<T, D, false, true, GENERAL, false, false, D, true, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
+    if (causal && p.large_tiles) return launch_causal<T, D, false, D, true, 1, 8>(p, r, grid, stream);
   }
   if (gather) return launch_gathered<T, D, false, D>(p, grid, form, stream);
-  if (causal && p.follow_max) return launch_one<T, D, false, true, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
-  if (causal) return launch_one<T, D, false, true>(p, grid, stream, "ha_flash_attn_fwd");
+  if (causal && p.follow_max) return launch_causal<T, D, false, D, true>(p, r, grid, stream);
+  if (causal) return launch_causal<T, D, false, D>(p, r, grid, stream);
   if constexpr (D == 128) {
     if (p.large_tiles) return launch_one<T, D, false, false, GENERAL, false, false, D, false, 1, 8>(p, grid, stream, "ha_flash_attn_fwd");
     if (p.follow_max) return launch_one<T, D, false, false, GENERAL, false, false, D, true>(p, grid, stream, "ha_flash_attn_fwd");
@@ -686,8 +726,25 @@ static bool large_tiles(const ha_attn_kernel_params& p, bool causal) {
   return rounds == 1 || (rounds <= 6 && p.n_q >= (columns_96 ? 200 : 500) * rounds);
 }
 
+// Where a grid of `tiles` workgroups of exact causal attention, `per_cu` of which a CU holds, has its ranking workgroups.  Behind the
+// others where all of the grid is resident at once, and in launches of many rounds, whose last one they fill: there the
+// order of the tiles over the CUs stays what it is without them.  Else in front: a ranking workgroup takes about as
+// long as a short tile, and behind one or two rounds of tiles it would be what the launch ends with.  Whole calls, hash and rank
+// launches | in front | behind, us (36 drawn calls and 4 others, 1.035 times faster in the geometric mean in front, 1.022 behind, none slower
+// by this rule): 12 heads of 7167 rows (672 tiles on 768 places) 78.0 | 70.7 | 65.5, 8 of 9728 85.9 | 80.0 | 74.6; 24 of 4096 (768 on 768)
+// 63.3 | 56.8 | 59.8, 12 of 14335, d = 96 (2.6 rounds) 272 | 260 | 282, 32 of 11520, d = 128 (3) 558 | 553 | 579; pairs of tiles, d = 64: 16 of
+// 29696 (2) 380 | 371 | 360, 24 of 29184 (3) 848 | 830 | 817; d = 128, 16 of 77824 (10) 2010 | 1998 | 1969.
+static int64_t place_ranking(ha_rank_beside& a, int64_t tiles, int per_cu, bool pairs_64) {
+  const int64_t groups = (tiles + NUM_XCD - 1) / NUM_XCD, places = 256 * per_cu;
+  a.groups = (a.units + NUM_XCD - 1) / NUM_XCD;
+  const bool behind = (groups + a.groups) * NUM_XCD <= places || pairs_64 || tiles >= 4 * places;
+  a.first_group = behind ? (int)groups : 0;
+  a.tiles = (int)tiles;
+  return (groups + a.groups) * NUM_XCD;
+}
+
 int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype, bool gather, bool causal,
-                   bool reweight, hipStream_t stream) {
+                   bool reweight, hipStream_t stream, const ha_rank_beside* ranking) {
   ha_attn_kernel_params p = params;
   // the kernels are built for rows of 64 and 128 elements; other head dims (multiples of 8) run in the
   // next width with the missing pieces of every row read as zeros
@@ -753,12 +810,19 @@ int ha_attn_launch(const ha_attn_kernel_params& params, int d, int dv, int dtype
   p.div_kv_heads = make_divisor(p.heads / p.kv_group);
   p.div_kv_group = make_divisor(p.kv_group);
   p.div_block_tiles = make_divisor(p.block_tiles);
-  const int64_t grid = qtiles * p.batch * p.heads * p.segs;
+  int64_t grid = qtiles * p.batch * p.heads * p.segs;
+  ha_rank_beside beside;
+  if (ranking) {
+    beside = *ranking;
+    ranking = &beside;
+    const int per_cu = p.split_keys ? (width == 64 ? 2 : 1) : p.large_tiles ? 1 : p.small_tiles ? 3 : 2;
+    grid = place_ranking(beside, grid, per_cu, width == 64 && !p.single && !p.split_keys);
+  }
   if (grid <= 0 || grid >= (1ll << 31)) return ha_fail(HA_ERR_SHAPE, "attention: grid of %lld workgroups", (long long)grid);
   if (dtype == HA_F16) {
-    if (width == 64) return launch_variant<f16_t, 64>(p, (int)grid, gather, causal, reweight, stream);
-    return launch_variant<f16_t, 128>(p, (int)grid, gather, causal, reweight, stream);
+    if (width == 64) return launch_variant<f16_t, 64>(p, ranking, (int)grid, gather, causal, reweight, stream);
+    return launch_variant<f16_t, 128>(p, ranking, (int)grid, gather, causal, reweight, stream);
   }
-  if (width == 64) return launch_variant<bf16_t, 64>(p, (int)grid, gather, causal, reweight, stream);
-  return launch_variant<bf16_t, 128>(p, (int)grid, gather, causal, reweight, stream);
+  if (width == 64) return launch_variant<bf16_t, 64>(p, ranking, (int)grid, gather, causal, reweight, stream);
+  return launch_variant<bf16_t, 128>(p, ranking, (int)grid, gather, causal, reweight, stream);
 }

@@ -5,6 +5,7 @@
 
 #define HA_SORT_CHUNK 4096   // keys per workgroup
 #define HA_SORT_WHOLE 12288  // most rows of a unit that is a whole segment (ha_rank_units with `out`)
+#define HA_SORT_BESIDE 8192  // and beside an exact causal launch (unit_ranking.h)
 #define HA_SORT_MAX_JOBS 40
 
 struct ha_sort_job {

@@ -14,6 +14,7 @@
 // causal forward) share one launch through a small by-value job table.
 #include "ha_common.h"
 #include "bucket_sort.h"
+#include "rank_tiles.h"
 
 #include <type_traits>
 
@@ -59,27 +60,6 @@ __device__ __forceinline__ BlockRef locate_block(const ha_sort_jobs& jobs, int b
   return r;
 }
 
-// lanes of the wave holding the same digit as this lane, restricted to valid lanes.  Per bit: the
-// lane's own bit spread over a word (0 or ~0), one ballot, and per mask half one three-input bit
-// operation "keep the lanes whose bit equals mine".
-__device__ __forceinline__ uint64_t match_digit(int digit, bool valid) {
-  const uint64_t all = __ballot(valid);
-  uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
-#pragma unroll
-  for (int bit = 0; bit < 8; ++bit) {
-    const uint32_t mine = (uint32_t)((int32_t)((uint32_t)digit << (31 - bit)) >> 31);
-    const uint64_t b = __ballot(mine != 0u);
-    lo &= ~((uint32_t)b ^ mine);
-    hi &= ~((uint32_t)(b >> 32) ^ mine);
-  }
-  return ((uint64_t)hi << 32) | lo;
-}
-
-// number of set bits of `mask` below this lane
-__device__ __forceinline__ uint32_t rank_below(uint64_t mask) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 // Digits (and source rows) of positions first + s*stride (s < SORT_STEPS) of a segment.  Positions past the
 // end are clamped to the last one, so every load is unconditional and all of them are in flight
 // together: one memory round trip per pass instead of one per step.
@@ -113,23 +93,6 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_hist_kernel(ha_sort_jobs jo
     if (chunk_start + s * SORT_THREADS + tid < job.seg_len) atomicAdd(&hist[digit[s]], 1u);
   __syncthreads();
   job.hist[((int64_t)br.seg * job.chunks_per_seg + br.chunk) * 256 + tid] = hist[tid];
-}
-
-// exclusive scan of one value per thread over a block
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* wave_totals) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  uint32_t incl = v;
-#pragma unroll
-  for (int off = 1; off < HA_WAVE; off <<= 1) {
-    const uint32_t up = __shfl_up(incl, off);
-    if (lane >= off) incl += up;
-  }
-  if (lane == HA_WAVE - 1) wave_totals[wave] = incl;
-  __syncthreads();
-  uint32_t base = 0;
-  for (int w = 0; w < wave; ++w) base += wave_totals[w];
-  __syncthreads();
-  return base + incl - v;
 }
 
 // ---- per-segment scan: hist[c][k] -> first output slot of (chunk c, key k) -------------------

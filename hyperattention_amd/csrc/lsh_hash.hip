@@ -13,23 +13,9 @@
 // to 2^-53): 2 % of the 16-row tiles on random data of 64 elements, 5 % of 128.
 #include "ha_common.h"
 #include "bucket_sort.h"
+#include "lsh_tiles.h"
 
 namespace {
-
-template <typename T>
-struct HashMfma;
-template <>
-struct HashMfma<f16_t> {
-  static __device__ __forceinline__ f32x4 run(f16x8 a, f16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct HashMfma<bf16_t> {
-  static __device__ __forceinline__ f32x4 run(bf16x8 a, bf16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
 
 // Tiles of 16 rows per wave: 8 KB, in two groups of tiles whose rows are in flight together, and fewer where the launch would
 // not fill the chip with workgroups.  Short waves, many of them, read fastest: the projection's set-up of one runs beside the
@@ -58,17 +44,6 @@ struct HashTensors {
   int64_t n_read;      // rows of a sequence that exist; rows from there up to n hash as zero rows
   int64_t first[2], end[2];  // rows of every sequence whose ids are wanted
 };
-
-// the bits of c's signs, c[0]'s lowest
-__device__ __forceinline__ uint32_t sign_bits(f32x4 c) {
-  uint32_t bits = 0;
-#pragma unroll
-  for (int i = 3; i >= 0; --i) {
-    const float ci = c[i];
-    bits = __builtin_amdgcn_alignbit(bits, __builtin_bit_cast(uint32_t, ci), 31);
-  }
-  return bits;
-}
 
 template <typename T, int PARTS, bool OUT8, int GROUP>  // GROUP tiles (1 or 2) in flight together
 __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors ten, const T* __restrict__ proj, int64_t n,
@@ -111,32 +86,12 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   // the first rows are in flight while the projection is set up
   load_rows(wave_row0);
 
-  // The projection matrix goes through LDS once per block, transposed: a lane's operand is 8 elements of one
-  // projection.  Rows of d_real <= D elements: the missing elements of a row, the missing rows of the projection and the
-  // projections past the last one are zeros (they add nothing to a dot product).
-  constexpr int PITCH = D + 8;  // 16 bytes more, so that the 16 projections' pieces lie on different banks
-  __shared__ __attribute__((aligned(16))) T lds_p[16 * PITCH];
-  {
-    const int j = threadIdx.x & 15, k0 = threadIdx.x >> 4;
-    T v[D / 16];
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) v[i] = pbase[j < r && k0 + 16 * i < d_real ? (k0 + 16 * i) * r + j : 0];
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) lds_p[j * PITCH + k0 + 16 * i] = j < r && k0 + 16 * i < d_real ? v[i] : (T)0.f;
-  }
+  // the projection matrix goes through LDS once per block
+  typedef Projection<T, PARTS> P;
+  __shared__ __attribute__((aligned(16))) T lds_p[16 * P::PITCH];
+  P::stage(pbase, r, d_real, lds_p, threadIdx.x);
   __syncthreads();
-  // A operands: P and |P| for every part: slot m, group kg holds P[part*32 + 8*kg + e][m]
-  vec8 pf[PARTS], pa[PARTS];
-#pragma unroll
-  for (int pt = 0; pt < PARTS; ++pt) {
-    pf[pt] = *reinterpret_cast<const vec8*>(&lds_p[m * PITCH + pt * 32 + 8 * kg]);
-    pa[pt] = __builtin_bit_cast(vec8, __builtin_bit_cast(u32x4, pf[pt]) & 0x7fff7fffu);
-  }
-  const float tol = (float)(D + 8) * 4.76837158203125e-07f;  // 2 * (d + 8) * 2^-23
-  // a slot past the last projection starts at -1 and its products are zeros: never in doubt, its bit never set
-  f32x4 c_first;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) c_first[i] = 4 * kg + i < r ? 0.f : -1.f;
+  const P projection(lds_p, r, lane);
 
 #pragma unroll 1
   for (int64_t row0 = wave_row0, wave_end = wave_row0 + tiles * 16; row0 < end;) {
@@ -150,69 +105,14 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
           xf[u][pt] = exists ? xf[u][pt] : vec8{};
         }
     }
-    f32x4 c[GROUP], ca[GROUP];
-#pragma unroll
-    for (int u = 0; u < GROUP; ++u) {
-      c[u] = c_first;
-      ca[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int pt = 0; pt < PARTS; ++pt)
-#pragma unroll
-      for (int u = 0; u < GROUP; ++u) {
-        const vec8 abs_x = __builtin_bit_cast(vec8, __builtin_bit_cast(u32x4, xf[u][pt]) & 0x7fff7fffu);
-        c[u] = HashMfma<T>::run(pf[pt], xf[u][pt], c[u]);
-        ca[u] = HashMfma<T>::run(pa[pt], abs_x, ca[u]);
-      }
-    // slots 4*kg .. +3 of row m: set where the projection is negative
     uint32_t nib[GROUP];
-#pragma unroll
-    for (int u = 0; u < GROUP; ++u) {
-      nib[u] = sign_bits(c[u]);
-      // what is left of |projection| above the bound of its error; a NaN stays one
-      float left[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) left[i] = __builtin_fmaf(-tol, ca[u][i], __builtin_fabsf(c[u][i]));
-      const float least = __builtin_elementwise_minimum(__builtin_elementwise_minimum(left[0], left[1]),
-                                                        __builtin_elementwise_minimum(left[2], left[3]));
-      if (__builtin_expect(__any(!(least > 0.f)), false)) {
-        uint32_t unsure = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) unsure |= left[i] > 0.f ? 0u : 1u << (4 * kg + i);
-        for (int jj = 0; jj < r; ++jj) {
-          if (!__any((unsure >> jj) & 1u)) continue;
-          // this lane's elements of row m, then the sum over the four lanes that share the row
-          double part = 0.0;
-#pragma unroll
-          for (int pt = 0; pt < PARTS; ++pt) {
-            // converted where they are used (ahead of the loop, the doubles took 64 registers that are waves in flight)
-            u32x4 raw = __builtin_bit_cast(u32x4, xf[u][pt]);
-            asm volatile("" : "+v"(raw));
-            const vec8 x = __builtin_bit_cast(vec8, raw);
-            const vec8 p8 = *reinterpret_cast<const vec8*>(&lds_p[jj * PITCH + pt * 32 + 8 * kg]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              part = __builtin_fma((double)ha_to_float(x[e]), (double)ha_to_float(p8[e]), part);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          part += __shfl_xor(part, 16);
-          part += __shfl_xor(part, 32);
-          const uint32_t bit = 1u << (jj & 3);
-          if (kg == jj >> 2) nib[u] = part > 0.0 ? nib[u] & ~bit : nib[u] | bit;
-        }
-      }
-    }
-    // the nibbles of a row's slots meet in one lane, rows in order over the lanes, 16 for every tile; after the swap
-    // groups of 16 lanes hold (tile 0, tile 1) of slots 0..3 | 8..11, and of slots 4..7 | 12..15
-    const auto sw = __builtin_amdgcn_permlane16_swap(nib[0], GROUP == 2 ? nib[GROUP - 1] : 0u, false, false);
-    uint32_t bin = sw[0] | sw[1] << 4;
-    if (r > 8) bin |= (uint32_t)__shfl_xor((int)bin, 32) << 8;  // of use in the lower half of the lanes
-    bin = ~bin & ((1u << r) - 1u);
+    projection_signs<T, PARTS, GROUP>(xf, projection, r, lane, nib);
+    const uint32_t bucket = bucket_ids(nib[0], GROUP == 2 ? nib[GROUP - 1] : 0u, r);
     if (lane < 16 * GROUP && row0 + lane < end) {
       if (OUT8)
-        obase8[row0 + lane] = (uint8_t)(bin ^ (bin >> 1));
+        obase8[row0 + lane] = (uint8_t)bucket;
       else
-        obase[row0 + lane] = (int32_t)(bin ^ (bin >> 1));
+        obase[row0 + lane] = (int32_t)bucket;
     }
     row0 += GROUP * 16;
     if (row0 >= wave_end) break;

@@ -1,0 +1,81 @@
+"""Units hashed and ranked by workgroups of the exact causal launch: the forward pass in one call against the same launches with
+the orders of ha_forward_sort (hash, rank and placement launches), bit for bit."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from _util import _randn
+
+
+def _launch_by_launch(q, k, v, proj, projs, block, sample, msl):
+    """The leaves, then the hashed levels merged in place, as hyper_forward runs them; even lengths."""
+    from hyperattention_amd import _lib, ops
+    b, h, n, d = q.shape
+    hk = k.shape[1]
+    q_idx, k_idx = ops.forward_sort(q, k, proj, causal=True, lsh_num_projs=projs, min_seq_len=msl)
+    halves, leaf = ops.causal_plan(n, msl)
+    hashed = [j for j, x in enumerate(q_idx) if x is not None]
+    out, lse = torch.empty_like(q), torch.empty((b, h, n), device=q.device, dtype=torch.float32)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def operands(segs, rows, stride, q_off):
+        t = _lib.AttnOperands()
+        t.q, t.k, t.v, t.out, t.lse = (x.data_ptr() for x in (q, k, v, out, lse))
+        t.batch, t.heads, t.n_q, t.n_k, t.d, t.dv = b, h, rows, rows, d, d
+        for name, x in (("q", q), ("k", k), ("v", v), ("o", out)):
+            for i, axis in enumerate("bhn"):
+                setattr(t, f"{name}_stride_{axis}", x.stride(i))
+        t.lse_stride_b, t.lse_stride_h = h * n, n
+        t.segs, t.seg_stride_rows, t.q_seg_offset, t.k_seg_offset = segs, stride, q_off, 0
+        t.kv_group, t.scale, t.dtype = h // hk, d ** -0.5, ops._dtype_code(q)
+        return t
+
+    levels = len(hashed)  # a deepest level that is not hashed is exact as a whole
+    rows = n if not halves else halves[levels - 1]
+    _lib.check(_lib.lib().ha_flash_attn_fwd(ctypes.byref(operands(1 << levels, rows, rows, 0)), 1, stream))
+    for j in reversed(hashed):
+        a = _lib.BlockAttnArgs()
+        half = halves[j]
+        a.t = operands(1 << j, half, 2 * half, half)
+        a.q_idx, a.k_idx = q_idx[j].data_ptr(), k_idx[j].data_ptr()
+        a.q_idx_stride_b, a.q_idx_stride_h, a.q_idx_stride_n = h * (half << j), half << j, 1
+        a.k_idx_stride_b, a.k_idx_stride_h, a.k_idx_stride_n = hk * (half << j), half << j, 1
+        a.block_size, a.sample_size, a.accumulate = block, sample, 1
+        _lib.check(_lib.lib().ha_block_attn_fwd(ctypes.byref(a), stream))
+    return out, lse
+
+
+@pytest.mark.parametrize("b,h,hk,n,msl,d,projs,dtype", [
+    (1, 2, 2, 256, 128, 64, 8, torch.float16),        # one segment of 128 rows, less than a step per wave
+    (1, 3, 1, 1536, 512, 64, 8, torch.bfloat16),      # the deepest level, of 384 rows, is exact
+    (1, 24, 24, 4096, 2048, 64, 8, torch.bfloat16),   # in front of the tiles: they take every place
+    (2, 4, 2, 8448, 4200, 64, 6, torch.float16),      # a unit of 4224 rows, a whole segment
+    (1, 2, 1, 16384, 8192, 64, 8, torch.bfloat16),    # the longest such one
+    (1, 2, 1, 16640, 8300, 64, 8, torch.bfloat16),    # three units and their placement
+    (1, 8, 8, 15360, 1024, 64, 8, torch.float16),     # four levels, one unit per granule of 1920
+    (4, 24, 24, 10240, 2048, 64, 8, torch.float16),   # pairs of tiles
+    (1, 2, 2, 9216, 4100, 128, 8, torch.bfloat16),    # two units of 4608 rows in a granule, the second of 512
+    (1, 2, 2, 4096, 512, 128, 8, torch.float16),      # the split kernel
+    (1, 16, 2, 8192, 2048, 128, 7, torch.bfloat16),
+    (1, 35, 35, 4096, 2048, 128, 8, torch.float16),   # eight waves per workgroup
+    (1, 4, 2, 4096, 1024, 40, 8, torch.bfloat16),     # rows shorter than their place
+    (1, 24, 12, 8192, 2048, 96, 8, torch.float16),
+    (2, 8, 8, 4096, 512, 80, 5, torch.bfloat16),
+    (1, 4, 4, 2048, 256, 112, 8, torch.float16),
+])
+def test_orders_are_those_of_the_sort(b, h, hk, n, msl, d, projs, dtype):
+    from hyperattention_amd import ops
+    q, v = (_randn((b, x, n, d), s, dtype).cuda() for x, s in ((h, 610), (hk, 612)))
+    k = _randn((b, hk, n, d), 611, dtype).cuda()
+    # equal rows tie, and their places in the order show in what they attend to
+    q[:, :, torch.arange(n) % 3 > 0] = q[:, :, :1].clone()
+    k[:, :, torch.arange(n) % 5 > 2] = k[:, :, :1].clone()
+    proj = _randn((1, 1, d, projs), 613, dtype).cuda()
+    got = ops.hyper_forward(q, k, v, proj, scale=d ** -0.5, causal=True, lsh_num_projs=projs, block_size=128, sample_size=128,
+                            min_seq_len=msl, smooth_block=False)
+    want = _launch_by_launch(q, k, v, proj, projs, 128, 128, msl)
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
