@@ -54,8 +54,15 @@ struct ha_attn_bwd_params {
   float scale, scale_log2, neg_inv_scale;  // scale * log2(e), -1 / scale
 };
 
-// dq, dk, dv of blocks and the sums of the sampled keys (dk32, dv32, cleared before) in one launch (attn_bwd_block.hip)
-bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d);
+// dq, dk, dv of blocks and the sums of the sampled keys in one launch (attn_bwd_block.hip).  Every workgroup leaves a share of
+// the sums, in the order of its registers (ha_fused_share_at) and dk's without their factor `scale`, in dk32, dv32.
+bool ha_block_bwd_fused_shape(const ha_attn_operands& t, int64_t sample_size);  // the other options apart
+bool ha_block_bwd_fused_takes(const ha_block_attn_args& a);
+int64_t ha_block_bwd_fused_shares(int64_t vseqs, int64_t n);  // of a (head, segment)
+// where elements 4 * piece .. +3 of sampled key `slot` lie in a share: [32 keys][half of the head dim][eight elements][four of them][key]
+__host__ __device__ __forceinline__ int ha_fused_share_at(int slot, int piece) {
+  return (slot >> 5) * 2048 + (piece >> 1) * 256 + (piece & 1) * 128 + (slot & 31) * 4;
+}
 int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream);
 
 // dk, dv of exact attention or of plain blocks (multiples of 256 keys) at head dim 128, 256 keys per workgroup

@@ -218,22 +218,22 @@ __global__ __launch_bounds__(256) void ha_bwd_zero_kernel(f32x4* __restrict__ bu
   if (i < n4) buf[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// Sums of the sampled keys (fp32, `shares` rows per slot of the sample list) added to the rows of dk (blockIdx.y = 0) or dv,
-// 4 elements per lane.  A row that is listed several times is handled by its first slot alone, which adds
+// Sums of the sampled keys (fp32, `shares` of them, rows by slot of the sample list or (FUSED) as ha_fused_share_at has them)
+// added to the rows of dk (blockIdx.y = 0; times k_factor) or dv, 4 elements per lane, lanes in the order of a share.  A row that is listed several times is handled by its first slot alone, which adds
 // the sums of all of them: no two lanes write the same row, whatever the list holds.
-template <typename T, int D>
+template <typename T, int D, bool FUSED>
 __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __restrict__ sk32, const float* __restrict__ sv32,
                                                                  T* __restrict__ dk, T* __restrict__ dv,
                                                                  const void* __restrict__ sampled_idx, int idx64,
                                                                  int64_t si_sb, int64_t si_sh, int kv_heads, int sample_size,
                                                                  int shares, int64_t dk_sb, int64_t dk_sh, int64_t dk_sn,
                                                                  int64_t dv_sb, int64_t dv_sh, int64_t dv_sn, int64_t total_slots,
-                                                                 int segs, int64_t seg_stride, int64_t k_seg_off) {
+                                                                 int segs, int64_t seg_stride, int64_t k_seg_off, float k_factor) {
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int PR = D / 4;
   const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t gslot = item / PR;
-  const int piece = (int)(item % PR);
+  const int64_t gslot = FUSED ? item / (32 * PR) * 32 + item % 32 : item / PR;
+  const int piece = (int)(FUSED ? item / 32 % PR : item % PR);
   if (gslot >= total_slots) return;
   const bool is_v = blockIdx.y != 0;
   const int64_t bhs = gslot / sample_size;   // (batch, kv head, segment)
@@ -243,10 +243,11 @@ __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __
   const int64_t row0 = k_seg_off + seg * seg_stride;
   int row = slot;
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-  const float* const base = (is_v ? sv32 : sk32) + bhs * shares * sample_size * D + piece * 4;
+  const float* const base = (is_v ? sv32 : sk32) + bhs * shares * sample_size * D;
   auto add_slot = [&](int s2) {
+    const float* const at = base + (FUSED ? ha_fused_share_at(s2, piece) : s2 * D + piece * 4);
 #pragma unroll 8
-    for (int k = 0; k < shares; ++k) sum += *reinterpret_cast<const f32x4*>(base + ((int64_t)k * sample_size + s2) * D);
+    for (int k = 0; k < shares; ++k) sum += *reinterpret_cast<const f32x4*>(at + (int64_t)k * sample_size * D);
   };
   if (sampled_idx) {
     const int64_t list = b * si_sb + h * si_sh;
@@ -263,7 +264,7 @@ __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __
                                                  : dk + b * dk_sb + h * dk_sh + (row0 + row) * dk_sn + piece * 4);
   vec4 o = *dst;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = (T)((float)o[e] + sum[e]);
+  for (int e = 0; e < 4; ++e) o[e] = (T)((float)o[e] + (FUSED && !is_v ? sum[e] * k_factor : sum[e]));
   *dst = o;
 }
 
@@ -387,17 +388,17 @@ void fill_bwd_params(const ha_attn_operands& t, const ha_attn_grads& g, const Wo
 }
 
 // the sampled keys' sums onto their rows of dk, dv
-template <typename T, int D>
+template <typename T, int D, bool FUSED = false>
 int launch_add_samples(const ha_block_attn_args& a, const ha_attn_grads& g, const Workspace& w, int64_t shares, hipStream_t stream) {
   const ha_attn_operands& t = a.t;
   const int64_t kv_heads = t.heads / t.kv_group;
   const int64_t slots = t.batch * kv_heads * t.segs * a.sample_size;
   const int64_t items = slots * (D / 4);
-  hipLaunchKernelGGL((ha_bwd_add_samples_kernel<T, D>), dim3((unsigned)((items + 255) / 256), 2), dim3(256), 0, stream,
+  hipLaunchKernelGGL((ha_bwd_add_samples_kernel<T, D, FUSED>), dim3((unsigned)((items + 255) / 256), 2), dim3(256), 0, stream,
                      w.dk32, w.dv32, (T*)g.dk, (T*)g.dv, a.sampled_idx, (int)(a.idx_type == HA_IDX_I64),
                      a.sampled_stride_b, a.sampled_stride_h, (int)kv_heads, (int)a.sample_size, (int)shares, g.dk_stride_b,
                      g.dk_stride_h, g.dk_stride_n, g.dv_stride_b, g.dv_stride_h, g.dv_stride_n, slots, (int)t.segs,
-                     t.seg_stride_rows, t.k_seg_offset);
+                     t.seg_stride_rows, t.k_seg_offset, t.scale);
   return ha_launch_status("attention backward: sampled keys");
 }
 
@@ -405,11 +406,12 @@ template <typename T, int D>
 int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream_t stream) {
   const ha_attn_operands& t = a.t;
   QueryRanges ranges;
-  const bool shared_out = writes_shares(t, a.sample_size, ranges);
-  const int64_t wanted = shared_out ? t.kv_group * ranges.count : 1;
-  // (a workspace for the sums alone takes the atomics)
-  const int64_t shares = carve(t, a.sample_size, wanted, nullptr).bytes <= g.workspace_bytes ? wanted : 1;
-  const bool wide_samples = shared_out && shares == wanted;
+  const bool shared_out = writes_shares(t, a.sample_size, ranges), one_kernel = ha_block_bwd_fused_takes(a);
+  const int64_t wanted = shared_out ? t.kv_group * ranges.count : one_kernel ? ha_block_bwd_fused_shares(t.batch * t.heads * t.segs, t.n_q) : 1;
+  // (a workspace for the sums alone takes the passes that add them with atomics)
+  const bool room = carve(t, a.sample_size, wanted, nullptr).bytes <= g.workspace_bytes;
+  const int64_t shares = room ? wanted : 1;
+  const bool wide_samples = shared_out && room;
   const Workspace w = carve(t, a.sample_size, shares, g.workspace);
   int st;
   ha_attn_bwd_params p;
@@ -423,17 +425,17 @@ int run_block_bwd(const ha_block_attn_args& a, const ha_attn_grads& g, hipStream
   p.smooth = a.smooth_block != 0;
   p.idx64 = a.idx_type == HA_IDX_I64;
   const int64_t bh = t.batch * t.heads * t.segs, bhk = t.batch * (t.heads / t.kv_group) * t.segs;
+  if (one_kernel && room) {
+    st = ha_launch_block_bwd_fused(p, std::is_same<T, f16_t>::value, stream);
+    if (st != HA_OK || a.sample_size == 0) return st;
+    if constexpr (D == 64) return launch_add_samples<T, D, true>(a, g, w, shares, stream);
+  }
   if (a.sample_size > 0 && !wide_samples) {
     // the two arrays of sums lie one behind the other in the workspace (each a multiple of 256 bytes): one fill
     const int64_t n4 = (int64_t)(((char*)w.dv32 - (char*)w.dk32) + align256(w.acc_floats * 4)) / 16;
     hipLaunchKernelGGL(ha_bwd_zero_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, (f32x4*)w.dk32, n4);
     st = ha_launch_status("attention backward: clear");
     if (st != HA_OK) return st;
-  }
-  if (ha_block_bwd_fused_takes(p, D)) {
-    st = ha_launch_block_bwd_fused(p, std::is_same<T, f16_t>::value, stream);
-    if (st != HA_OK || a.sample_size == 0) return st;
-    return launch_add_samples<T, D>(a, g, w, shares, stream);
   }
   st = launch_pass<T, D, HA_BWD_DQ_BLOCK, false>(p, bh * (t.n_q / ST_ROWS), stream, "ha_block_attn_bwd: dq");
   if (st != HA_OK) return st;
@@ -580,7 +582,10 @@ extern "C" int64_t ha_attn_bwd_workspace_bytes(const ha_attn_operands* t, int64_
       t->heads % t->kv_group != 0 || sample_size < 0 || t->segs < 1)
     return ha_fail(HA_ERR_SHAPE, "ha_attn_bwd_workspace_bytes: sizes must be positive, kv_group dividing heads, segs >= 1");
   QueryRanges r;
-  return carve(*t, sample_size, writes_shares(*t, sample_size, r) ? t->kv_group * r.count : 1, nullptr).bytes;
+  int64_t shares = 1;
+  if (writes_shares(*t, sample_size, r)) shares = t->kv_group * r.count;
+  else if (ha_block_bwd_fused_shape(*t, sample_size)) shares = ha_block_bwd_fused_shares(t->batch * t->heads * t->segs, t->n_q);
+  return carve(*t, sample_size, shares, nullptr).bytes;
 }
 
 extern "C" int ha_block_attn_bwd(const ha_block_attn_args* args, const ha_attn_grads* grads, void* stream) {

@@ -4,17 +4,20 @@
 // The passes gather a level's rows three times (4.0 GB at 24 heads of 65536 rows with gradients added to; dq 447 us, dk/dv of
 // the blocks 403, of the sampled keys 229) and compute the scores twice (7 products per pair).  Here a workgroup gathers the
 // q, k, v, dO, O rows of a block of 256 queries and 256 keys once, computes every score once (5 products) and leaves dq, dk,
-// dv of the block and adds to the sampled keys' sums: 2.9 GB, 810 to 826 us in the same launch (without adding, 24 heads
+// dv of the block and its share of the sampled keys' sums: 3.4 GB, 735 to 766 us in the same launch (without adding, 24 heads
 // of 16384, the whole call: 269 -> 223 us).  What bounds it now: not the board's power limit (2.21 to 2.28 GHz, matrix pipe busy 0.30 to 0.32 of
-// the time); of a block's 73k cycles 50k are the steps, the others the ends of its phases, where every wave does the same memory and vector
-// work with one workgroup per CU and nothing beside it.
+// the time); of a block's 65k cycles (57k where nothing is added to) 43k are the steps, bound by the LDS (1750 of a step's 2700 cycles), the others the ends
+// of its phases, where every wave does the same memory and vector work with one workgroup per CU and nothing beside it.
 //
 // A workgroup: 8 waves, a run of consecutive blocks of one (head, segment).  A block has a phase for its own keys and one
 // per 256 sampled keys.  In a phase a wave keeps 32 keys (k, v rows as MFMA B operands, sums of dK^T, dV^T in registers) and
 // goes through the block's queries in 8 steps of 32, their q and dO rows in LDS for the whole block (64 KB: 256 queries are
 // what fits).  dS of a step, 32 queries x 256 keys, goes through LDS once; of dq^T = sum K^T dS^T a wave sums 16 elements of
 // the head dim of 16 queries of every step over all keys.  All sums of a block are complete in registers: 64 (dk, dv) and 32
-// (dq) of them.  Of the sampled keys' sums a flush costs 64 KB of atomics per tensor, so two blocks in a row share one.
+// (dq) of them.  The sampled keys' sums, 64 KB per tensor and phase, stay in the registers over two blocks in a row and
+// else wait in memory of the workgroup's own, in the order of its registers, until ha_bwd_add_samples_kernel adds up the workgroups' shares.
+// (Added to one array with atomics, each time, they took 10 to 16 thousand cycles of every second block, and a launch to
+// clear it: 24 heads of 16384 rows 225 -> 215 us the call, of 4096 74 -> 64, 8 of 8192 67 -> 50, 24 of 65536 745 -> 735, with 512 samples 1148 -> 1099.)
 // The next block's rows come in while this one is worked on: q and dO rows into a step's place once the step is done for the
 // last time, k rows into an LDS stage, v rows through registers, O rows (for D) four queries of a step per wave.
 #include "ha_common.h"
@@ -30,7 +33,7 @@ namespace {
 constexpr int FUSED_WAVES = 8, FUSED_THREADS = 64 * FUSED_WAVES;
 constexpr int FUSED_ROWS = 256;  // queries, and keys of a phase, per workgroup
 constexpr int FD = 64;           // head dim
-constexpr int FUSED_MAX_SAMPLES = 512;  // their row numbers are kept in LDS
+constexpr int FUSED_MAX_SAMPLES = 1024;  // their row numbers are kept in LDS
 constexpr int STEPS = FUSED_ROWS / 32;
 
 template <typename T>
@@ -92,7 +95,8 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
   const uint32_t q_rb = (uint32_t)p.q_sn * 2, k_rb = (uint32_t)p.k_sn * 2, v_rb = (uint32_t)p.v_sn * 2,
                  do_rb = (uint32_t)p.do_sn * 2, o_rb = (uint32_t)p.o_sn * 2, dq_rb = (uint32_t)p.dq_sn * 2,
                  dk_rb = (uint32_t)p.dk_sn * 2, dv_rb = (uint32_t)p.dv_sn * 2;
-  const int64_t sums0 = (((int64_t)b * p.heads + h) * p.segs + seg) * p.sample_size * FD;
+  // the workgroup's own sums of the sampled keys in memory: [256 keys][wave][quarter of a sum's registers][lane], 16 bytes each
+  const int64_t sums0 = (((((int64_t)b * p.heads + h) * p.segs + seg) * runs + run) * p.sample_size + wave * 32) * FD;
 
   // ---- row numbers: of a block and the next one, of the sampled keys ----
   const int idx_shift = p.idx64 ? 3 : 2;
@@ -246,11 +250,24 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
           for (int ks = STEPS / 2; ks < STEPS; ++ks) kt[ks] = vec8{};
         }
       }
-      if (i_ph > 0 || ph == 0 || bl == first_block) {
+      // Sums of a phase: of the block's own keys from zero; of sampled keys as the block before left them in registers
+      // (a backward block's first phase), else as the last block left them in memory
+      if (ph == 0 || bl == first_block) {
 #pragma unroll
         for (int d2 = 0; d2 < 2; ++d2)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc1[d2][i] = acc2[d2][i] = 0.f;
+      } else if (i_ph > 0) {
+        const int64_t at = sums0 + (int64_t)(ph - 1) * FUSED_ROWS * FD + opaque_lane() * 4;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const f32x4 a1 = *reinterpret_cast<const f32x4*>(p.dk32 + at + i * 256), a2 = *reinterpret_cast<const f32x4*>(p.dv32 + at + i * 256);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc1[i >> 2][(i & 3) * 4 + e] = a1[e];
+            acc2[i >> 2][(i & 3) * 4 + e] = a2[e];
+          }
+        }
       }
 
       // ---- 32 queries a step ----
@@ -477,30 +494,13 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
           store(acc2, 1.f, dvb, dv_rb, old2);
         }
       } else if (!last_phase || !more_blocks) {  // else the next block goes on with the same sampled keys
-        const int64_t slot0 = sums0 + (int64_t)((ph - 1) * FUSED_ROWS + wave * 32) * FD;
+        const int64_t at = sums0 + (int64_t)(ph - 1) * FUSED_ROWS * FD + ln * 4;
 #pragma unroll
-        for (int which = 0; which < 2; ++which) {
-          float* const dst = (which == 0 ? p.dk32 : p.dv32) + slot0;
-          const float factor = which == 0 ? p.scale : 1.f;
-#pragma unroll
-          for (uint32_t part = 0; part < 2; ++part) {  // 16 keys at a time
-            if ((ln & 31) >> 4 == part) {
-#pragma unroll
-              for (int d2 = 0; d2 < 2; ++d2)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                  const f32x16& a = which == 0 ? acc1[d2] : acc2[d2];
-                  const uint32_t piece = (8 * d2 + 2 * g + (ln >> 5)) ^ (ln & 15);
-                  lds_put<f32x4>(turn + (ln & 15) * (FD * 4) + piece * 16,
-                                 f32x4{a[g * 4] * factor, a[g * 4 + 1] * factor, a[g * 4 + 2] * factor, a[g * 4 + 3] * factor});
-                }
-            }
-            wave_lds_order();
-#pragma unroll
-            for (uint32_t r = 0; r < 16; ++r)
-              unsafeAtomicAdd(dst + (part * 16 + r) * FD + ln, lds_get<float>(turn + r * (FD * 4) + (((ln >> 2) ^ r) << 4) + (ln & 3) * 4));
-            wave_lds_order();
-          }
+        for (int i = 0; i < 8; ++i) {
+          const f32x16 &a1 = acc1[i >> 2], &a2 = acc2[i >> 2];
+          const int g = (i & 3) * 4;
+          *reinterpret_cast<f32x4*>(p.dk32 + at + i * 256) = f32x4{a1[g], a1[g + 1], a1[g + 2], a1[g + 3]};
+          *reinterpret_cast<f32x4*>(p.dv32 + at + i * 256) = f32x4{a2[g], a2[g + 1], a2[g + 2], a2[g + 3]};
         }
       }
       // ---- dq ----
@@ -538,37 +538,46 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 }  // namespace
 
 // What the registers and LDS are laid out for: 256 keys and queries per block; with grouped queries a block's dk, dv would
-// have to be kept over the query heads beside the sampled keys' sums.  How many sampled keys: two blocks in a row share the
-// sums of one phase, those of the others are added to memory by every block, while the passes add them once per range of
-// queries.  Three passes | this kernel, the whole call in us where it writes the gradients, 38 launches of 64 to 6144 blocks
-// (0.25 to 24 per CU): up to 256 samples it is the faster one at all (4 heads x 4096 rows 44 | 40, 24 x 4096 98 | 79, 24 x 8192
-// 156 | 131, 32 x 16384 361 | 267, 24 x 65536 1038 | 744; without samples 20.4 | 19.3 to 692 | 424; where it adds to them
-// too, but for 16 x 2048 without samples, 22.8 | 23.2); 512: 8 x 2048 51 | 54, 24 x 2048 82 | 79, 10 x 16384 172 | 178, 130 x 2048
-// 294 | 306, then within 5 % to both sides up to 1600 blocks, 28 x 16384 (1792) 453 | 382, 24 x 65536 1402 | 1118; 768: 24 x
-// 8192 254 | 306, 20 x 16384 373 | 405, 24 x 65536 1695 | 1633, not enough for a rule; 1024: 8 x 2048 66 | 82, 24 x 65536 2027 | 2247.
+// have to be kept over the query heads beside the sampled keys' sums.  Three passes | this kernel, the whole call in us where it
+// writes the gradients: 256 samples (38 launches of 64 to 6144 blocks) 4 heads x 4096 rows 44 | 35, 24 x 4096 98 | 64, 24 x 8192
+// 156 | 113, 32 x 16384 361 | 259, 24 x 65536 1038 | 735; without samples 20.4 | 19.3 to 692 | 424 (where it adds to them
+// too, but for 16 x 2048 without samples, 22.8 | 23.2); 512: 2 x 512 43.7 | 39.5, 8 x 2048 50 | 48, 24 x 2048 79 | 56, 10 x 16384 165 | 132, 24 x
+// 16384 350 | 297, 130 x 2048 296 | 263, 24 x 65536 1402 | 1099; 768: 8 x 2048 56.8 | 57.6, 24 x 8192 232 | 202, 24 x 65536 1688 | 1434; 1024: 24 x
+// 2048 104 | 84, 130 x 2048 426 | 421, 24 x 65536 1994 | 1798.
 // Head dims below 64, padded for the backward (O as it is): forward and backward of 24 x 16384, d = 48 476 | 418, 512 x 3072, d = 32
 // 1570 | 1324, causal 24 x 65536, d = 40 5923 | 5340.
-bool ha_block_bwd_fused_takes(const ha_attn_bwd_params& p, int d) {
-  const int64_t blocks = (int64_t)p.batch * p.heads * p.segs * ((p.n_q + FUSED_ROWS - 1) / FUSED_ROWS);
-  return d == FD && p.kv_group == 1 && !p.smooth && p.block_tiles * 128 == FUSED_ROWS && p.n_q == p.n_k && p.sample_size % FUSED_ROWS == 0 &&
-         (p.sample_size <= FUSED_ROWS || (p.sample_size <= FUSED_MAX_SAMPLES && blocks >= 1792));
+static int64_t fused_blocks(int64_t n) { return (n + FUSED_ROWS - 1) / FUSED_ROWS; }
+bool ha_block_bwd_fused_shape(const ha_attn_operands& t, int64_t sample_size) {
+  return t.d == FD && t.kv_group == 1 && t.n_q == t.n_k && sample_size % FUSED_ROWS == 0 && sample_size <= FUSED_MAX_SAMPLES;
+}
+bool ha_block_bwd_fused_takes(const ha_block_attn_args& a) {
+  return !a.smooth_block && (a.block_size + 127) / 128 * 128 == FUSED_ROWS && ha_block_bwd_fused_shape(a.t, a.sample_size);
 }
 
-int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream) {
-  const int64_t vseqs = (int64_t)p.batch * p.heads * p.segs, blocks = (p.n_q + FUSED_ROWS - 1) / FUSED_ROWS;
-  // Blocks per workgroup, one workgroup per CU: the run with the least time by the rounds of workgroups; starting and ending
-  // one takes as long as two thirds of a block.  Within 0.2 % of the best run of 1 to 8, 10 and 12 at every one of those
-  // launches, samples or not; as two fifths of a block it chose three rounds of one block for 24 x 8192, 175 us.
-  int64_t best = INT64_MAX;
-  p.run_blocks = 1;
+// Blocks per workgroup, one workgroup per CU: the run with the least time by the rounds of workgroups; starting and ending
+// one takes as long as two thirds of a block.  Within 0.2 % of the best run of 1 to 8, 10 and 12 at every one of those
+// launches, samples or not; as two fifths of a block it chose three rounds of one block for 24 x 8192, 175 us.
+static int64_t fused_run(int64_t vseqs, int64_t n) {
+  int64_t best = INT64_MAX, run = 1;
+  const int64_t blocks = fused_blocks(n);
   for (int64_t r = 1; r <= std::min<int64_t>(blocks, 12); ++r) {
     const int64_t cost = (vseqs * ((blocks + r - 1) / r) + 255) / 256 * (3 * r + 2);
     if (cost < best) {
       best = cost;
-      p.run_blocks = (int)r;
+      run = r;
     }
   }
-  const int64_t grid = vseqs * ((blocks + p.run_blocks - 1) / p.run_blocks);
+  return run;
+}
+int64_t ha_block_bwd_fused_shares(int64_t vseqs, int64_t n) {
+  const int64_t run = fused_run(vseqs, n);
+  return (fused_blocks(n) + run - 1) / run;
+}
+
+int ha_launch_block_bwd_fused(ha_attn_bwd_params p, int is_f16, hipStream_t stream) {
+  const int64_t vseqs = (int64_t)p.batch * p.heads * p.segs;
+  p.run_blocks = (int)fused_run(vseqs, p.n_q);
+  const int64_t grid = vseqs * ha_block_bwd_fused_shares(vseqs, p.n_q);
   if (grid >= (1ll << 31)) return ha_fail(HA_ERR_SHAPE, "ha_block_attn_bwd: grid of %lld workgroups", (long long)grid);
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FUSED_THREADS), LDS_BYTES, stream, p); };
   auto launch_for = [&](auto short_o) {

@@ -17,8 +17,10 @@ pytestmark = pytest.mark.gpu
     (torch.float16, 1, 128, 0, torch.int64),       # half a block, nothing else
     (torch.bfloat16, 2, 256, 256, torch.int32),    # one block
     (torch.float16, 1, 384, 256, torch.int32),     # the last block is half
-    (torch.bfloat16, 3, 1152, 512, torch.int64),   # two phases of sampled keys: few blocks take the three passes
-    (torch.float16, 1, 1024, 1024, torch.int32),   # and so does what is above
+    (torch.bfloat16, 3, 1152, 512, torch.int64),   # two phases of sampled keys
+    (torch.float16, 1, 1024, 1024, torch.int32),   # the most
+    (torch.bfloat16, 1, 1280, 1280, torch.int32),  # three passes above
+    (torch.float16, 66, 1152, 768, torch.int32),   # three phases, runs of blocks that end with half of one
     (torch.float16, 5, 16512, 256, torch.int32),   # 65 blocks in runs of two: the last run has one, of half the rows
 ])
 def test_blocks_and_samples(ha, dtype, h, n, sample, idx):  # noqa: F811
@@ -32,7 +34,7 @@ def test_blocks_and_samples(ha, dtype, h, n, sample, idx):  # noqa: F811
 
 
 @pytest.mark.parametrize("dtype,h,n,idx", [
-    (torch.float16, 896, 512, torch.int32),   # 1792 blocks, the fewest with two phases of sampled keys; runs of two
+    (torch.float16, 896, 512, torch.int32),   # runs of two
     (torch.bfloat16, 600, 640, torch.int64),  # runs of three: the last block has half the rows
 ])
 def test_two_phases_of_samples(ha, dtype, h, n, idx):  # noqa: F811
@@ -98,3 +100,25 @@ def test_short_output_rows(ha, dtype, h, n, out_d, accumulate):  # noqa: F811
         results.append(grads)
     for padded, short, name in zip(*results, ("dq", "dk", "dv")):
         assert torch.equal(padded, short), name
+
+
+def test_small_workspace_takes_the_passes(ha):  # noqa: F811
+    """A workspace without room for the workgroups' shares of the sampled keys' sums, as large as one of the sums alone."""
+    from hyperattention_amd import _lib, ops
+    h, n, sample = 24, 1024, 256
+    q, k, v, do = (_randn((1, n, h, 64), s, torch.float16).cuda() for s in (61, 62, 63, 64))
+    qi, ki = (_perms(1, h, n, s).cuda().int().transpose(1, 2) for s in (65, 66))
+    o, lse = ops.hyper_attn_func(q, k, v, qi, ki, 256, sample, 0.125, False)
+    a, _keep = ops._block_attn_args(q, k, v, o, lse, qi, ki, 256, sample, 0.125, False, None)
+    results = []
+    for small in (False, True):
+        grads = [torch.empty_like(x) for x in (q, k, v)]
+        g, ws = ops._attn_grads(a.t, do, *grads, sample_size=sample)
+        if small:
+            g.workspace_bytes = h * n * 8 + 2 * h * sample * 64 * 4
+            assert g.workspace_bytes < ws.numel()
+        _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), ops._stream(q)))
+        results.append(grads)
+    for x, y, name in zip(*results, ("dq", "dk", "dv")):
+        # the same sums in another order, each rounded to fp16: half a unit of its last place on either side
+        assert (x.double() - y.double()).norm() / y.double().norm() <= 2.0 ** -10, name
