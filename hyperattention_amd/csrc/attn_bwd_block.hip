@@ -396,9 +396,7 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
         add_dkv(1, 3);
         read(-1, -1, 2);
         if (u + 1 == STEPS) {
-          // the scores are done: their registers take the v rows of the next phase and what this one adds to
-          load_v(more ? next_bl : bl, next_ph);
-          if (ACC && ph == 0) load_old(old1, dkb, dk_rb, FUSED_ROWS);
+          if (ACC && ph == 0) load_old(old2, dvb, dv_rb, FUSED_ROWS);
           in_order();
         }
         dq_of(6);
@@ -420,8 +418,15 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
         if (u == 1 && more) stage_keys(next_bl, next_ph);  // every wave is done with the keys of this phase
         if (u > 0 && __builtin_expect(last_phase && more_blocks, true)) fill_tile(u - 1, frow);  // every wave is done with step u-1
         in_order();
-        if (u + 1 == STEPS) {
-          if (ACC && ph == 0) load_old(old2, dvb, dv_rb, FUSED_ROWS);
+        if (u + 2 == STEPS) {
+          // the last scores are done: their operands' registers take the v rows of the next phase and dk rows that this one
+          // adds to, the scores' dv and dq rows (adding, 24 x 65536 812 -> 804 us; dv rows here too 808)
+          load_v(more ? next_bl : bl, next_ph);
+          if (ACC && ph == 0) load_old(old1, dkb, dk_rb, FUSED_ROWS);
+          in_order();
+        }
+        if (ACC && u + 1 == STEPS && last_phase) {
+          load_old(old3, dqb, dq_rb, 0);
           in_order();
         }
       };
@@ -449,7 +454,6 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 #pragma unroll
       for (int ks = 0; ks < STEPS; ++ks) add_dq(STEPS - 1, ks);
       if (i_ph == 0) keep_stats(bl + 1, STEPS - 1, st);
-      if (ACC && last_phase) load_old(old3, dqb, dq_rb, 0);
       // the next phase's v rows have landed, and with them all loads into LDS; not to be waited for behind the stores
 #pragma unroll
       for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(x2f[ks]));
