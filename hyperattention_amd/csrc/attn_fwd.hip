@@ -328,117 +328,18 @@ __device__ __forceinline__ SegmentRows segment_rows(const ha_attn_kernel_params&
 // sequence's first tile, gathered (plain or not, tiles of 128 queries) and at head dims above 64 without mask in a row's first p.follow_max chunks.  An
 // instance of its own: as an argument's value it cost every pair of tiles 0.5 %.
 template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
-          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES, typename... Ranking>
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
+__global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p) {
+#include "attn_fwd_body.inc"
+}
+// exact causal, with workgroups that hash and rank (place_ranking)
+template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
+          int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
 __global__ __launch_bounds__(64 * WAVES, D == 64 && NB == 1 ? 3 : 2) void ha_attn_fwd_kernel(const ha_attn_kernel_params p,
-                                                                                          const Ranking... ranking) {
-  typedef typename ElemTraits<T>::vec8 vec8;
-  typedef typename ElemTraits<T>::vec4 vec4;
-  constexpr int QW = 32 * NB;                 // queries per wave
-  constexpr int WG_QUERIES = QW * WAVES;
-  constexpr int REF_TILES = WG_QUERIES / 128;  // reference query tiles of 128 per workgroup
-  static_assert(!GATHER || FORM == PLAIN || REF_TILES == 1, "two reference tiles of a workgroup share their keys");
-  constexpr int DV = D;
-  constexpr int KSTEPS = DC / 16;  // MFMA k-steps of Q.K^T
-  constexpr int DB = DC / 32;      // 32-row blocks of O^T
-  constexpr int PR = D / 8;        // 16-byte pieces per row
-
-  // Separate LDS objects (two K tiles, two V tiles of KC rows, the query rows): the compiler then
-  // knows that a tile being filled from HBM and a tile being read do not alias, and does not
-  // serialise them.  The query region (QW rows per wave) is reused for the output rows at the end.
-  constexpr int TILE_BYTES = KC * D * 2;
-  // The key tiles ask for the larger alignment only to be placed first: LDS offsets below 64 KB fit
-  // the immediate field of the LDS reads.
-  constexpr int Q_WAVE_BYTES = QW * D * 2;  // a wave's part of the query region
-  // At d = 128 two workgroups fit a CU's 160 KB if most of the query region lies in tile space that is free before and
-  // after the loop: V tile 1 (waves 0, 1) and the first half of K tile 0 (wave 3).  (8 waves: one workgroup per CU.)
-  constexpr bool OVERLAY = D == 128 && WAVES == 4;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_v1[TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) unsigned char lds_q[OVERLAY ? Q_WAVE_BYTES : WAVES * Q_WAVE_BYTES];
-  __shared__ int lds_qrow[WG_QUERIES];   // original row of every query position (-1: past the end)
-  __shared__ float lds_w[WG_QUERIES];    // weight of the resumed partial result per query position
-
-  int wg_id = blockIdx.x, wg_count = gridDim.x;
-  if constexpr (sizeof...(Ranking) > 0) {
-    const int unit = ranking_unit(ranking..., wg_id, wg_count);
-    if (unit >= 0) {
-      if constexpr (D == 64) hash_and_rank_unit<T, DC / 32, WAVES>(p, ranking..., unit, lds_q, lds_k0, lds_v0, lds_v1);
-      else hash_and_rank_unit<T, DC / 32, WAVES>(p, ranking..., unit, lds_k0, lds_k1, lds_v0, lds_v1);
-    }
-    if (wg_id >= wg_count) return;
-  }
-
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  // the same number, known to the compiler to be wave-uniform: what the tile loads derive from it
-  // (chunk numbers, index array addresses, LDS destinations) then stays in scalar registers
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-  const int hi = lane >> 5, col = lane & 31;
-
-  // ---- which (virtual) head and query tile -----------------------------------------------------
-  // Workgroup number = (((batch, kv head), segment), tile, query head inside the kv group), the last one
-  // fastest: the query heads that share a kv head work on the same tile side by side, on one XCD, so that the
-  // K and V rows of the tile (the same for all of them) come from HBM once and from L2 after that.
-  int wg = xcd_contiguous_id(wg_id, wg_count);
-  const int qtiles = (p.n_q + WG_QUERIES - 1) / WG_QUERIES;
-  // Exact causal attention, many workgroups: one takes the tile pair (qtiles-1-s, s), so that every workgroup of the
-  // launch has the same number of key chunks to go through.  The hardware hands out workgroups in order and
-  // a slot freed by a short one stays empty until the ones queued before it are placed: with one tile per
-  // workgroup (4 to 32 chunks in a 2048-row leaf) the slots of a CU stood empty for 8 us at a time.
-  // Few workgroups (p.single, see single_tiles): one tile each, the tiles of all sequences, longest first,
-  // the second 256 in reversed order where a CU holds two workgroups (see ha_attn_fwd_split_kernel).
-  constexpr bool PAIRED = CAUSAL && !GATHER;
-  const int wg_per_seq = PAIRED ? (qtiles + 1) / 2 : qtiles;  // what p.div_qtiles divides by
-  const bool single = PAIRED && (FOLLOW || (D <= 64 && p.single));  // d = 128: the FOLLOW instance's alone
-  int hg, vseq, slot;
-  if (single) {
-    const int second = min(wg_count, 512);
-    wg = wg_id;
-    if (WAVES == 4 && wg >= 256 && wg < second) wg = 256 + second - 1 - wg;
-    slot = fast_div(wg, p.div_qtiles);
-    wg -= slot * (p.batch * p.heads * p.segs);  // what p.div_qtiles divides by here
-    vseq = fast_div(wg, p.div_kv_group);
-    hg = wg - vseq * p.kv_group;
-  } else {
-    const int wg_tile = fast_div(wg, p.div_kv_group);
-    hg = wg - wg_tile * p.kv_group;
-    vseq = fast_div(wg_tile, p.div_qtiles);
-    slot = wg_tile - vseq * wg_per_seq;
-  }
-  const int bhk = fast_div(vseq, p.div_segs);
-  const int seg = vseq - bhk * p.segs;
-  const int b = fast_div(bhk, p.div_kv_heads), hk = bhk - b * fast_div(p.heads, p.div_kv_group);
-  const int h = hk * p.kv_group + hg;
-
-  const SegmentRows rows = segment_rows<GATHER>(p, seg);
-  const int n_q = rows.n_q, n_k = rows.n_k;
-  const int64_t seg_q_row = rows.q_row, seg_k_row = rows.k_row, seg_o_row = rows.o_row;
-  // gathered kernel: entries of the query order from this number on name a row that does not exist
-  const int q_rows_exist = (GATHER && seg == p.segs - 1) ? p.n_q_last : n_q;
-
-  if constexpr (!PAIRED) {
-    const int qt = slot;
-    if (qt * WG_QUERIES >= n_q) return;  // ragged launches: the grid is sized for the longest segment
-#include "attn_fwd_tile.inc"
-  } else {
-    // the long tile first.  No barrier between the two: the last iteration of a tile ends with one, and after
-    // it a wave touches only its own part of the query region.
-    const int t_long = qtiles - 1 - slot;
-    if (t_long * WG_QUERIES < n_q) {  // ragged launches: the grid is sized for the longest segment
-      const int qt = t_long;
-#include "attn_fwd_tile.inc"
-    }
-    if constexpr (!FOLLOW) {
-      if (!single && slot != t_long && slot * WG_QUERIES < n_q) {  // an odd number of tiles: the middle one has no partner
-        const int qt = slot;
-        // the first tile's output rows were staged in tiles that the second's loads fill (LDS only: the stores need no wait)
-        if (OVERLAY) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#include "attn_fwd_tile.inc"
-      }
-    }
-  }
+                                                                                          const ha_rank_beside ranking) {
+#define HA_WITH_RANKING
+#include "attn_fwd_body.inc"
+#undef HA_WITH_RANKING
 }
 
 #include "attn_fwd_split.inc"
@@ -448,8 +349,8 @@ namespace {
 template <typename T, int D, bool GATHER, bool CAUSAL, int FORM = GENERAL, bool NARROW = false, bool REWEIGHT = false,
           int DC = D, bool FOLLOW = false, int NB = WaveShape<D>::NB, int WAVES = WaveShape<D>::WAVES>
 int launch_one(const ha_attn_kernel_params& p, int grid, hipStream_t stream, const char* what) {
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, FORM, NARROW, REWEIGHT, DC, FOLLOW, NB, WAVES>), dim3(grid),
-                     dim3(64 * WAVES), 0, stream, p);
+  void (*const kernel)(ha_attn_kernel_params) = ha_attn_fwd_kernel<T, D, GATHER, CAUSAL, FORM, NARROW, REWEIGHT, DC, FOLLOW, NB, WAVES>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WAVES), 0, stream, p);
   return ha_launch_status(what);
 }
 
@@ -459,8 +360,9 @@ template <typename T, int D, bool NARROW, int DC, bool FOLLOW = false, int NB = 
 int launch_causal(const ha_attn_kernel_params& p, const ha_rank_beside* r, int grid, hipStream_t stream) {
   const char* const what = "ha_flash_attn_fwd";
   if (!r) return launch_one<T, D, false, true, GENERAL, NARROW, false, DC, FOLLOW, NB, WAVES>(p, grid, stream, what);
-  hipLaunchKernelGGL((ha_attn_fwd_kernel<T, D, false, true, GENERAL, NARROW, false, DC, FOLLOW, NB, WAVES, ha_rank_beside>), dim3(grid),
-                     dim3(64 * WAVES), 0, stream, p, *r);
+  void (*const kernel)(ha_attn_kernel_params, ha_rank_beside) =
+      ha_attn_fwd_kernel<T, D, false, true, GENERAL, NARROW, false, DC, FOLLOW, NB, WAVES>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WAVES), 0, stream, p, *r);
   return ha_launch_status(what);
 }
 

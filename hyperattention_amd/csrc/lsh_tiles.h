@@ -49,11 +49,17 @@ struct Projection {
   // by the first 256 threads; a barrier belongs between this and the constructor
   static __device__ __forceinline__ void stage(const T* proj, int r, int d_real, T* lds, int tid) {
     const int j = tid & 15, k0 = tid >> 4;
+    // selects, not branches: behind one the compiler waits for the loads ahead of it, the rows'
     T v[D / 16];
+    bool wanted[D / 16];
 #pragma unroll
-    for (int i = 0; i < D / 16; ++i) v[i] = proj[j < r && k0 + 16 * i < d_real ? (k0 + 16 * i) * r + j : 0];
+    for (int i = 0; i < D / 16; ++i) {
+      const int k = k0 + 16 * i, at = __mul24(k, r) + j;
+      wanted[i] = (j < r) & (k < d_real);
+      v[i] = proj[wanted[i] ? at : 0];
+    }
 #pragma unroll
-    for (int i = 0; i < D / 16; ++i) lds[j * PITCH + k0 + 16 * i] = j < r && k0 + 16 * i < d_real ? v[i] : (T)0.f;
+    for (int i = 0; i < D / 16; ++i) lds[j * PITCH + k0 + 16 * i] = wanted[i] ? v[i] : (T)0.f;
   }
   __device__ __forceinline__ Projection(const T* staged, int r, int lane) : lds(staged) {
     const int m = lane & 15, kg = lane >> 4;
