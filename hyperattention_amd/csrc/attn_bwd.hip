@@ -71,6 +71,7 @@ __device__ __forceinline__ float row16_sum(float v) {
 
 template <typename T, int D, int PASS, bool CAUSAL, int HALVES>
 __global__ __launch_bounds__(WG_THREADS, (D <= 64 || PASS == HA_BWD_DQ_BLOCK || (PASS == HA_BWD_DQ_EXACT && HALVES == 1) ? 2 : 1)) void ha_attn_bwd_kernel(const ha_attn_bwd_params p) {
+  ha_load_arguments<(int)sizeof(ha_attn_bwd_params)>();
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr bool KEY_ST = PASS == HA_BWD_DKV_EXACT || PASS == HA_BWD_DKV_BLOCK || PASS == HA_BWD_DKV_SAMPLED;
@@ -229,6 +230,7 @@ __global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __
                                                                  int shares, int64_t dk_sb, int64_t dk_sh, int64_t dk_sn,
                                                                  int64_t dv_sb, int64_t dv_sh, int64_t dv_sn, int64_t total_slots,
                                                                  int segs, int64_t seg_stride, int64_t k_seg_off, float k_factor) {
+  ha_load_arguments<172>();
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int PR = D / 4;
   const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

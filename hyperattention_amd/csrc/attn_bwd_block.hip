@@ -63,6 +63,7 @@ static_assert(LDS_BYTES <= 163840, "one workgroup per CU");
 // SHORT_O: O's rows are shorter than dO's (p.out_last), an instance of its own: as a clamp in every call 0.4 % of the kernel
 template <typename T, bool ACC, bool SHORT_O>
 __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(const ha_attn_bwd_params p) {
+  ha_load_arguments<(int)sizeof(ha_attn_bwd_params)>();
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int KSTEPS = FD / 16;

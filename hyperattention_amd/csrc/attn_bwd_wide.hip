@@ -38,6 +38,7 @@ constexpr uint32_t LSE = STAGE + 65536, DELTA = LSE + 4 * 128, RAW = DELTA + 4 *
 
 template <typename T, int PASS, bool CAUSAL>
 __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_kernel(const ha_attn_bwd_params p) {
+  ha_load_arguments<(int)sizeof(ha_attn_bwd_params)>();
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int KSTEPS = WD / 16, DB = WD / 32;

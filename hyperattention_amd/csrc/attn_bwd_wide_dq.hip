@@ -31,6 +31,7 @@ constexpr uint32_t WIDE_LDS_BYTES = STAGE + 65536;
 
 template <typename T, bool CAUSAL>
 __global__ __launch_bounds__(WIDE_THREADS, 2) void ha_attn_bwd_wide_dq_kernel(const ha_attn_bwd_params p) {
+  ha_load_arguments<(int)sizeof(ha_attn_bwd_params)>();
   typedef typename ElemTraits<T>::vec8 vec8;
   typedef typename ElemTraits<T>::vec4 vec4;
   constexpr int KSTEPS = WD / 16, DB = WD / 32;

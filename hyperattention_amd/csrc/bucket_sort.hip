@@ -240,6 +240,7 @@ struct RankArgs {
 // 29.6 | 25.5, of 12288 32.2 | 31.6, of 16384 35.1 | 35.8; 32 heads 52.4 | 47.3, 70.5 | 66.5, 94.7 | 93.1, 119.5 | 120.3.
 template <int THREADS, int ROWS>
 __global__ __launch_bounds__(THREADS) void rank_units_kernel(RankArgs a) {
+  ha_load_arguments<(int)sizeof(RankArgs)>();
   constexpr int WAVES = THREADS / HA_WAVE;
   constexpr int STEPS = ROWS / THREADS;
   constexpr bool WHOLE = ROWS > HA_SORT_CHUNK;
@@ -310,6 +311,7 @@ __global__ __launch_bounds__(THREADS) void rank_units_kernel(RankArgs a) {
 // One workgroup per (job, segment, unit): where the unit's rows of every bucket start in the segment's
 // order, then a copy of the unit's order to those places.
 __global__ __launch_bounds__(SORT_THREADS) void place_units_kernel(ha_place_jobs jobs) {
+  if (blockIdx.x < 512) ha_load_arguments<16 * (int)sizeof(ha_place_job)>();  // of at most eight levels; as in the hash launch
   __shared__ uint32_t wave_totals[SORT_WAVES];
   __shared__ int32_t delta[256];   // segment slot minus unit slot, per bucket
   const int block = xcd_contiguous_block();

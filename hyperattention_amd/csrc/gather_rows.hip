@@ -40,6 +40,7 @@ struct RowCopies {
   int src_pieces[HA_ROW_COPIES], dst_pieces[HA_ROW_COPIES];
 };
 __global__ __launch_bounds__(256) void copy_rows_kernel(const RowCopies c) {
+  ha_load_arguments<(int)sizeof(RowCopies)>();
   const int job = blockIdx.z;
   const uint32_t pieces = c.dst_pieces[job], have = c.src_pieces[job];
   const uint32_t first = blockIdx.x * (256 * ROW_COPY_PIECES) + threadIdx.x, end = (uint32_t)c.rows[job] * pieces;

@@ -66,6 +66,23 @@ struct ElemTraits<bf16_t> {
 __device__ __forceinline__ float ha_to_float(f16_t v) { return (float)v; }
 __device__ __forceinline__ float ha_to_float(bf16_t v) { return (float)v; }
 
+// Asks for every 64-byte line of a kernel's first BYTES of arguments at once.  The argument block is new to the caches in every
+// launch, and the compiler loads a field where it is used: six to nine misses one after the other before a kernel's
+// first row is asked for.  24 heads of 1000 causal rows 12.3 -> 11.4 us, 4 of 4096 hashed (three launches) 19.7 -> 18.8.
+template <int BYTES>
+__device__ __forceinline__ void ha_load_arguments() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef const __attribute__((address_space(4))) uint32_t* words;
+  const words a = (words)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int LINES = (BYTES + 63) / 64;
+  uint32_t line[LINES];
+#pragma unroll
+  for (int i = 0; i < LINES; ++i) line[i] = a[16 * i];
+#pragma unroll
+  for (int i = 0; i < LINES; ++i) asm volatile("" ::"s"(line[i]));
+#endif
+}
+
 // index loads of either width
 __device__ __forceinline__ int ha_load_idx(const void* base, int64_t off, int is64) {
   // one load either way (row numbers fit the low word of a little-endian int64), so that the value

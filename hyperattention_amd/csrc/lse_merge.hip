@@ -163,6 +163,7 @@ __global__ __launch_bounds__(256) void lse_merge_levels_kernel(const T* __restri
                                                                T* __restrict__ out, float* __restrict__ lse_out,
                                                                float* __restrict__ leaf_shifted, MergeLevels lv,
                                                                int64_t rows, int64_t n, int pieces, int packed) {
+  ha_load_arguments<5 * 8 + (int)sizeof(MergeLevels) + 24>();
   typedef typename ElemTraits<T>::vec8 vec8;
   const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t row = item / pieces;

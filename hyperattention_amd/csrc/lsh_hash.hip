@@ -48,6 +48,8 @@ struct HashTensors {
 template <typename T, int PARTS, bool OUT8, int GROUP>  // GROUP tiles (1 or 2) in flight together
 __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors ten, const T* __restrict__ proj, int64_t n,
                                                             int r, int64_t psb, int64_t psh, int d_real, int tiles) {
+  // the first workgroups alone: in those that follow, which find the arguments in the caches, it cost 6 % of a long launch
+  if (blockIdx.y < 8 && blockIdx.z == 0) ha_load_arguments<(int)sizeof(HashTensors) + 48>();
   typedef typename ElemTraits<T>::vec8 vec8;
   constexpr int D = PARTS * 32;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
