@@ -32,7 +32,8 @@ SYMBOLS = [
     "ha_bucket_argsort", "ha_bucket_argsort_static", "ha_gather_rows", "ha_copy_rows", "ha_block_attn_fwd", "ha_flash_attn_fwd",
     "ha_attn_bwd_workspace_bytes", "ha_block_attn_bwd", "ha_flash_attn_bwd", "ha_lse_merge",
     "ha_lse_merge_segments",
-    "ha_forward_workspace_bytes", "ha_forward", "ha_forward_sort", "ha_lse_merge_levels", "ha_power_probe",
+    "ha_forward_workspace_bytes", "ha_forward", "ha_forward_sort", "ha_forward_sort_leaves",
+    "ha_lse_merge_levels", "ha_power_probe",
 ]
 
 HA_F16, HA_BF16 = 0, 1
@@ -221,6 +222,9 @@ def _declare(lib):
     lib.ha_forward_sort.restype = ci
     lib.ha_forward_sort.argtypes = [ctypes.POINTER(ForwardArgs), ctypes.POINTER(i64), ctypes.POINTER(i64),
                                     ctypes.POINTER(ci), vp]
+    lib.ha_forward_sort_leaves.restype = ci
+    lib.ha_forward_sort_leaves.argtypes = [ctypes.POINTER(ForwardArgs), ctypes.POINTER(AttnOperands), ctypes.POINTER(i64),
+                                           ctypes.POINTER(i64), ctypes.POINTER(ci), vp]
 
 
 def lib():

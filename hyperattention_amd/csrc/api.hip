@@ -357,6 +357,28 @@ Units units_of(const ha_forward_args& a, const Workspace& w) {
   return u;
 }
 
+// What the exact causal launch that hashes and ranks the units beside its tiles is given.
+int rank_beside(const ha_forward_args& a, const Workspace& w, ha_rank_beside& ranking) {
+  const Units u = units_of(a, w);
+  ranking = {};
+  ranking.proj = a.proj;
+  for (int i = 0; i < 2; ++i) {
+    ranking.sorted[i] = u.sorted[i];
+    ranking.hist[i] = u.hist[i];
+    ranking.out[i] = u.whole[i];
+    ranking.first_unit[i] = u.first_unit[i];
+  }
+  ranking.n_read = a.n;
+  ranking.num_projs = (int)a.lsh_num_projs;
+  ranking.num_units = u.num_units;
+  const int64_t units = (u.seqs[0] + u.seqs[1]) * u.num_units;
+  HA_REQUIRE(units < (1ll << 30), HA_ERR_SHAPE, "ha_forward: too many sort units");
+  ranking.units0 = (int)(u.seqs[0] * u.num_units);
+  ranking.units = (int)units;
+  ranking.grid = w.grid;
+  return HA_OK;
+}
+
 // The stable bucket order of every hashed level's segments from the units' orders and counts.
 int place_units(const ha_forward_args& a, const Plan& pl, const Workspace& w, hipStream_t stream) {
   unsigned char* ws = (unsigned char*)a.workspace;
@@ -499,8 +521,9 @@ extern "C" int64_t ha_forward_workspace_bytes(const ha_forward_args* args) {
   return std::max(w.total, with_leaves.total);
 }
 
-extern "C" int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offset, int64_t* k_idx_offset,
-                               int* num_levels, void* stream) {
+// leaves: or null, the exact causal call to run as well
+static int forward_sort(const ha_forward_args* args, const ha_attn_operands* leaves, int64_t* q_idx_offset, int64_t* k_idx_offset,
+                        int* num_levels, hipStream_t stream) {
   HA_REQUIRE(args && q_idx_offset && k_idx_offset && num_levels, HA_ERR_NULL, "ha_forward_sort: null argument");
   const ha_forward_args& a = *args;
   HA_REQUIRE(a.q && a.k, HA_ERR_NULL, "ha_forward_sort: null tensor pointer");
@@ -514,14 +537,14 @@ extern "C" int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offse
   int st = make_plan(a, pl);
   if (st != HA_OK) return st;
   Workspace w;
-  layout_workspace(a, pl, w, false);
+  layout_workspace(a, pl, w, leaves && a.causal);
   const int nlev = a.causal ? pl.levels : 1;
   *num_levels = nlev;
   for (int j = 0; j < nlev; ++j) {
     q_idx_offset[j] = pl.level_hyper[j] ? w.qidx[j] : -1;
     k_idx_offset[j] = pl.level_hyper[j] ? w.kidx[j] : -1;
   }
-  if (!pl.any_hyper) return HA_OK;
+  if (!pl.any_hyper) return leaves ? flash_attn(*leaves, 1, stream) : HA_OK;
   st = check_hashing(a, w, "ha_forward_sort");
   if (st != HA_OK) return st;
   ha_attn_operands t;
@@ -530,8 +553,34 @@ extern "C" int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offse
   forward_operands(b, t);
   st = check_forward_layout(t, false, "ha_forward_sort");
   if (st != HA_OK) return st;
-  return hash_and_sort(a, pl, w, t, (hipStream_t)stream);
+  if (leaves) {  // the ranking workgroups read q and k as the launch's operands describe them
+    const ha_attn_operands& f = *leaves;
+    HA_REQUIRE(f.q == t.q && f.k == t.k && f.batch == t.batch && f.heads == t.heads && f.kv_group == t.kv_group && f.d == t.d &&
+                   f.dtype == t.dtype && f.q_stride_b == t.q_stride_b && f.q_stride_h == t.q_stride_h && f.q_stride_n == t.q_stride_n &&
+                   f.k_stride_b == t.k_stride_b && f.k_stride_h == t.k_stride_h && f.k_stride_n == t.k_stride_n,
+               HA_ERR_SHAPE, "ha_forward_sort_leaves: the leaves' q and k are not those of the pass");
+  }
+  if (!w.beside) {
+    st = hash_and_sort(a, pl, w, t, stream);
+    return st != HA_OK || !leaves ? st : flash_attn(*leaves, 1, stream);
+  }
+  ha_rank_beside ranking;
+  st = rank_beside(a, w, ranking);
+  if (st == HA_OK) st = flash_attn(*leaves, 1, stream, nullptr, &ranking);
+  return st == HA_OK ? place_units(a, pl, w, stream) : st;
 }
+
+extern "C" int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offset, int64_t* k_idx_offset,
+                               int* num_levels, void* stream) {
+  return forward_sort(args, nullptr, q_idx_offset, k_idx_offset, num_levels, (hipStream_t)stream);
+}
+
+extern "C" int ha_forward_sort_leaves(const ha_forward_args* args, const ha_attn_operands* leaves, int64_t* q_idx_offset,
+                                      int64_t* k_idx_offset, int* num_levels, void* stream) {
+  HA_REQUIRE(leaves, HA_ERR_NULL, "ha_forward_sort_leaves: null argument");
+  return forward_sort(args, leaves, q_idx_offset, k_idx_offset, num_levels, (hipStream_t)stream);
+}
+
 
 extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   HA_REQUIRE(args, HA_ERR_NULL, "ha_forward: null argument block");
@@ -566,22 +615,8 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   }
   ha_rank_beside ranking = {};
   if (w.beside) {
-    const Units u = units_of(a, w);
-    ranking.proj = a.proj;
-    for (int i = 0; i < 2; ++i) {
-      ranking.sorted[i] = u.sorted[i];
-      ranking.hist[i] = u.hist[i];
-      ranking.out[i] = u.whole[i];
-      ranking.first_unit[i] = u.first_unit[i];
-    }
-    ranking.n_read = a.n;
-    ranking.num_projs = (int)a.lsh_num_projs;
-    ranking.num_units = u.num_units;
-    const int64_t units = (u.seqs[0] + u.seqs[1]) * u.num_units;
-    HA_REQUIRE(units < (1ll << 30), HA_ERR_SHAPE, "ha_forward: too many sort units");
-    ranking.units0 = (int)(u.seqs[0] * u.num_units);
-    ranking.units = (int)units;
-    ranking.grid = w.grid;
+    st = rank_beside(a, w, ranking);
+    if (st != HA_OK) return st;
   }
 
   auto hyper_level = [&](int j, bool accumulate) -> int {

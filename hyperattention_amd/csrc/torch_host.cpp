@@ -228,20 +228,6 @@ class Attention : public torch::autograd::Function<Attention> {
     const bool any_hashed = std::any_of(s->calls.begin(), s->calls.end(), [](const Call& x) { return x.hashed; });
     s->q_idx_at.assign(s->calls.size(), -1);
     s->k_idx_at.assign(s->calls.size(), -1);
-    Tensor ws;
-    if (any_hashed) {
-      ha_forward_args a = forward_args(q, k, v, s->proj, s->sampled, c);
-      ws = attach_workspace(a, q);
-      int64_t at_q[48], at_k[48];
-      int nlev = 0;
-      check(ha_forward_sort(&a, at_q, at_k, &nlev, stream));
-      for (size_t i = 0; i < s->calls.size(); ++i)
-        if (s->calls[i].hashed) {
-          const int j = std::max(s->calls[i].level, 0);
-          s->q_idx_at[i] = at_q[j];
-          s->k_idx_at[i] = at_k[j];
-        }
-    }
     const auto f32 = q.options().dtype(at::kFloat);
     // the first call's result; the levels' results packed: a level writes the second halves of its segments, n/2
     // rows per head
@@ -251,7 +237,27 @@ class Attention : public torch::autograd::Function<Attention> {
       o_un = at::empty({levels, b, h, n / 2, d}, q.options());
       lse_un = at::empty({levels, b, h, n / 2}, f32);
     }
-    for (size_t i = 0; i < s->calls.size(); ++i) {
+    Tensor ws;
+    if (any_hashed) {
+      ha_forward_args a = forward_args(q, k, v, s->proj, s->sampled, c);
+      ws = attach_workspace(a, q);
+      int64_t at_q[48], at_k[48];
+      int nlev = 0;
+      if (c.causal) {  // with the leaves, beside which rows are hashed and ranked: forward + backward of 24 x 4096 234.6 -> 231.6 us,
+                       // 8 x 32768 862 -> 850, 4 x 12 x 10240 1432 -> 1401; d = 128 and long sequences the same
+        const ha_attn_operands t = operands(q, k, v, o0, lse0, c, s->calls[0]);
+        check(ha_forward_sort_leaves(&a, &t, at_q, at_k, &nlev, stream));
+      } else {
+        check(ha_forward_sort(&a, at_q, at_k, &nlev, stream));
+      }
+      for (size_t i = 0; i < s->calls.size(); ++i)
+        if (s->calls[i].hashed) {
+          const int j = std::max(s->calls[i].level, 0);
+          s->q_idx_at[i] = at_q[j];
+          s->k_idx_at[i] = at_k[j];
+        }
+    }
+    for (size_t i = any_hashed && c.causal ? 1 : 0; i < s->calls.size(); ++i) {
       const Call& call = s->calls[i];
       Tensor o = i ? o_un.select(0, call.level) : o0, l = i ? lse_un.select(0, call.level) : lse0;
       ha_attn_operands t = operands(q, k, v, o, l, c, call);

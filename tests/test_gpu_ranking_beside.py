@@ -79,3 +79,54 @@ def test_orders_are_those_of_the_sort(b, h, hk, n, msl, d, projs, dtype):
     want = _launch_by_launch(q, k, v, proj, projs, 128, 128, msl)
     for x, y in zip(got, want):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("b,h,hk,n,msl,d,projs,dtype", [
+    (1, 2, 2, 256, 128, 64, 8, torch.float16),        # one segment, no placement
+    (1, 24, 24, 4096, 2048, 64, 8, torch.bfloat16),
+    (1, 3, 1, 3072, 512, 64, 8, torch.bfloat16),      # two hashed levels and an exact one
+    (2, 4, 2, 8192, 1024, 128, 7, torch.float16),
+    (1, 4, 2, 4096, 1024, 80, 8, torch.bfloat16),
+    (1, 2, 2, 2048, 512, 64, 9, torch.float16),       # more buckets than a unit's ranking takes: launches of their own
+    (1, 2, 2, 1000, 1024, 64, 8, torch.float16),      # no level at all
+])
+def test_sort_with_the_leaves(b, h, hk, n, msl, d, projs, dtype):
+    """ha_forward_sort_leaves on transposed views: the orders of ha_forward_sort, the leaves of ha_flash_attn_fwd, bit for bit."""
+    from hyperattention_amd import _lib, ops
+    q, k, v = (_randn((b, n, x, d), s, dtype).cuda().transpose(1, 2) for x, s in ((h, 620), (hk, 621), (hk, 622)))
+    k[:, :, torch.arange(n) % 5 > 2] = k[:, :, :1].clone()  # ties
+    proj = _randn((1, 1, d, projs), 623, dtype).cuda()
+    want_q, want_k = ops.forward_sort(q, k, proj, causal=True, lsh_num_projs=projs, min_seq_len=msl)
+    halves, leaf = ops.causal_plan(n, msl)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    t = _lib.AttnOperands()
+    t.batch, t.heads, t.n_q, t.n_k, t.d, t.dv = b, h, leaf, leaf, d, d
+    t.segs, t.seg_stride_rows, t.kv_group, t.scale, t.dtype = 1 << len(halves), leaf, h // hk, d ** -0.5, ops._dtype_code(q)
+    t.lse_stride_b, t.lse_stride_h = h * n, n
+    results = []
+    for with_sort in (False, True):
+        out, lse = torch.zeros((b, h, n, d), device="cuda", dtype=dtype), torch.zeros((b, h, n), device="cuda")
+        for name, x in (("q", q), ("k", k), ("v", v), ("o", out)):
+            for i, axis in enumerate("bhn"):
+                setattr(t, f"{name}_stride_{axis}", x.stride(i))
+        t.q, t.k, t.v, t.out, t.lse = (x.data_ptr() for x in (q, k, v, out, lse))
+        if with_sort:
+            a, keep = ops._forward_args(q, k, None, None, None, proj, scale=1.0, causal=True, lsh_num_projs=projs, block_size=128,
+                                        sample_size=0, min_seq_len=msl, smooth_block=False)
+            q_at, k_at, levels = (ctypes.c_int64 * 48)(), (ctypes.c_int64 * 48)(), ctypes.c_int(0)
+            _lib.check(_lib.lib().ha_forward_sort_leaves(ctypes.byref(a), ctypes.byref(t), q_at, k_at, ctypes.byref(levels), stream))
+            assert levels.value == len(want_q)
+            for at, want in ((q_at, want_q), (k_at, want_k)):
+                for j, w in enumerate(want):
+                    assert (at[j] < 0) == (w is None)
+                    if w is not None:
+                        got = keep[-1][at[j]:at[j] + 4 * w.numel()].view(torch.int32).view(w.shape)
+                        assert torch.equal(got, w)
+            t.k = t.v  # another tensor than the one that is hashed: refused before any launch
+            if want_q and want_q[0] is not None:
+                assert _lib.lib().ha_forward_sort_leaves(ctypes.byref(a), ctypes.byref(t), q_at, k_at, ctypes.byref(levels), stream) == -3
+        else:
+            _lib.check(_lib.lib().ha_flash_attn_fwd(ctypes.byref(t), 1, stream))
+        results.append((out, lse))
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
