@@ -5,6 +5,8 @@
 // the rest is fp32, with the same eps = 2^-23 inside the log.  One 8-element piece (16 bytes) per lane.
 #include "ha_common.h"
 
+#include <algorithm>
+
 namespace {
 
 template <typename T>
@@ -157,72 +159,128 @@ struct MergeLevels {
   int levels;
 };
 
-// MAXL: levels the instance is unrolled for (the recursion rarely goes deeper than 8)
-template <typename T, int MAXL>
-__global__ __launch_bounds__(256) void lse_merge_levels_kernel(const T* __restrict__ o_leaf, const float* __restrict__ lse_leaf,
-                                                               T* __restrict__ out, float* __restrict__ lse_out,
-                                                               float* __restrict__ leaf_shifted, MergeLevels lv,
-                                                               int64_t rows, int64_t n, int pieces, int packed) {
-  ha_load_arguments<5 * 8 + (int)sizeof(MergeLevels) + 24>();
+constexpr int MERGE_THREADS = 256;
+
+struct MergeLevelsParams {
+  const void* o_leaf;
+  const float* lse_leaf;
+  void* out;
+  float *lse_out, *leaf_shifted;
+  MergeLevels lv;
+  int64_t n;
+  uint32_t leaf_len, chunks, chunk_rows, pieces;
+  uint32_t row_of_item;  // ceil(2^22 / pieces), 0 where a chunk is one row: item * that >> 22 is the item's row in its chunk
+  int packed;
+};
+
+// A workgroup merges up to 256 * UNROLL pieces of 16 bytes of consecutive rows of one leaf (more where a row alone has more): which
+// levels they take part in and where those results lie is the same for all, in scalar registers.  A row's chain of weights is
+// one thread's, while the pieces' loads are in flight; its pieces' threads read the weights from LDS.
+// HBM-bound.  With a thread's row, its halves and its weights found by each of its pieces' threads (64-bit divisions, every
+// weight 8 to 16 times) it was bound by instructions: 24 x 131072 rows of 128 bytes, six levels, 443 -> 366 us (5.5 TB/s), 32 x 16384
+// of 256 bytes, three levels, 94 -> 83, 48 x 10240 of 128, two levels, 40 -> 36, 8 x 65536, nine levels, 171 -> 118.
+// GROUP: levels whose pieces are loaded at once, all of them unless MORE.
+template <typename T, int GROUP, int UNROLL, bool MORE>
+__global__ __launch_bounds__(MERGE_THREADS) void lse_merge_levels_kernel(const MergeLevelsParams p) {
+  ha_load_arguments<(int)sizeof(MergeLevelsParams)>();
   typedef typename ElemTraits<T>::vec8 vec8;
-  const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t row = item / pieces;
-  const int piece = (int)(item % pieces);
-  if (row >= rows) return;
-  // leaf number of the row inside its sequence: its bit (levels - 1 - j) says which half of its level-j
-  // segment the row is in (such a half is 2^(levels - 1 - j) leaves long)
-  const uint32_t leaf_no = (uint32_t)(row % n) / (uint32_t)(n >> lv.levels);
-  const int64_t at = row * pieces * 8 + piece * 8;
-  float x = lse_leaf[row];
-  const float x_leaf = x;
-  vec8 r = *reinterpret_cast<const vec8*>(o_leaf + at);
-  float c_of[MAXL], x_of[MAXL];
-  vec8 v_of[MAXL];
-  // Row of the level-j arrays that holds this row's result.  Packed arrays keep only the rows a level writes,
+  extern __shared__ float weight[];  // [level][row of the chunk]
+  const MergeLevels& lv = p.lv;
+  const uint32_t in_leaf = blockIdx.x / p.chunks, chunk = blockIdx.x - in_leaf * p.chunks;
+  // leaf number of the rows inside their sequence: its bit (levels - 1 - j) says which half of its level-j
+  // segment a row is in (such a half is 2^(levels - 1 - j) leaves long)
+  const uint32_t leaf_no = in_leaf & ((1u << lv.levels) - 1), row_in_leaf = chunk * p.chunk_rows;
+  const int64_t seq = in_leaf >> lv.levels, row_in_seq = (int64_t)leaf_no * p.leaf_len + row_in_leaf, row0 = seq * p.n + row_in_seq;
+  const uint32_t rows = min(p.chunk_rows, p.leaf_len - row_in_leaf), items = rows * p.pieces;
+  auto takes_part = [&](int j) -> bool { return j < lv.levels && ((leaf_no >> (lv.levels - 1 - j)) & 1u); };
+  // Row of the level-j arrays that holds the first row's result.  Packed arrays keep only the rows a level writes,
   // the second halves of its segments of n >> j rows one after the other: (batch * heads, n / 2) rows.
-  const int64_t seq = row / n;
-  const uint32_t r_in = (uint32_t)(row - seq * n);
   auto level_row = [&](int j) -> int64_t {
-    if (!packed) return row;
-    // the segment number from the leaf number: shifts only (the leaf length need not be a power of two)
-    const uint32_t len = (uint32_t)(n >> j), half = len >> 1, sg = leaf_no >> (lv.levels - j);
-    return seq * (n >> 1) + (int64_t)sg * half + (r_in - sg * len - half);
+    const int64_t half = p.n >> (j + 1), segment = leaf_no >> (lv.levels - j);
+    return p.packed ? seq * (p.n >> 1) + row_in_seq - (segment + 1) * half : row0;
   };
-  // every load first, so that they are all in flight before the chain of weights (each level's weight needs
-  // the log-sum-exp the deeper levels left) starts
+  const int64_t row_bytes = (int64_t)p.pieces * 16;
+  const bool own_row = threadIdx.x < rows;
+  const float x_leaf = own_row ? p.lse_leaf[row0 + threadIdx.x] : 0.f;
+  float x = x_leaf, x_of[GROUP];
+  for (uint32_t base = 0; base < items; base += MERGE_THREADS * UNROLL) {
+    vec8 r[UNROLL], v[GROUP][UNROLL];
+    uint32_t item[UNROLL], row[UNROLL];
 #pragma unroll
-  for (int j = MAXL - 1; j >= 0; --j) {
-    c_of[j] = 1.0f;
-    x_of[j] = 0.0f;
-    if (j < lv.levels && ((leaf_no >> (lv.levels - 1 - j)) & 1u)) {
-      const int64_t lr = level_row(j);
-      x_of[j] = lv.lse_un[j][lr];
-      v_of[j] = *reinterpret_cast<const vec8*>((const T*)lv.o_un[j] + lr * pieces * 8 + piece * 8);
+    for (int u = 0; u < UNROLL; ++u) {
+      item[u] = base + u * MERGE_THREADS + threadIdx.x;
+      row[u] = min(item[u], items - 1) * p.row_of_item >> 22;
     }
-  }
+    auto load = [&](vec8 (&to)[UNROLL], const void* from, int64_t first_row) {
+      const char* const rows0 = (const char*)from + first_row * row_bytes;
 #pragma unroll
-  for (int j = MAXL - 1; j >= 0; --j) {
-    if (j < lv.levels && ((leaf_no >> (lv.levels - 1 - j)) & 1u)) {
-      const float c = (float)(T)(1.0f / (1.0f + __expf(x_of[j] - x)));
+      for (int u = 0; u < UNROLL; ++u) to[u] = *reinterpret_cast<const vec8*>(rows0 + min(item[u], items - 1) * 16);
+    };
+    for (int first = MORE ? (lv.levels - 1) / GROUP * GROUP : 0; first >= 0; first -= GROUP) {  // deepest levels first
+      // the log-sum-exps before the pieces, so that they are back before those are
+      if (base == 0 && own_row) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[e] = (T)(c * (float)r[e] + (1.0f - c) * (float)v_of[j][e]);
-      x = x - __logf(c + 1.1920929e-07f);
-      c_of[j] = c;
+        for (int j = GROUP - 1; j >= 0; --j) {
+          x_of[j] = 0.f;
+          if (takes_part(first + j)) x_of[j] = lv.lse_un[first + j][level_row(first + j) + threadIdx.x];
+        }
+      }
+      if (!MORE || first + GROUP >= lv.levels) load(r, p.o_leaf, row0);
+#pragma unroll
+      for (int j = GROUP - 1; j >= 0; --j)
+        if (takes_part(first + j)) load(v[j], lv.o_un[first + j], level_row(first + j));
+      if (base == 0) {
+        if (own_row) {
+          // each level's weight needs the log-sum-exp the deeper levels left
+#pragma unroll
+          for (int j = GROUP - 1; j >= 0; --j) {
+            if (takes_part(first + j)) {
+              const float c = (float)(T)(1.0f / (1.0f + __expf(x_of[j] - x)));
+              weight[(first + j) * p.chunk_rows + threadIdx.x] = c;
+              x = x - __logf(c + 1.1920929e-07f);
+            }
+          }
+        }
+        __syncthreads();
+      }
+#pragma unroll
+      for (int j = GROUP - 1; j >= 0; --j) {
+        if (takes_part(first + j)) {
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) {
+            const float c = weight[(first + j) * p.chunk_rows + row[u]];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              float sum = __builtin_fmaf(c, (float)r[u][e], (1.0f - c) * (float)v[j][u][e]);
+              asm volatile("" : "+v"(sum));  // rounded to fp32 before T, as in the other merges
+              r[u][e] = (T)sum;
+            }
+          }
+        }
+      }
     }
-  }
-  *reinterpret_cast<vec8*>(out + at) = r;
-  if (piece != 0) return;
-  lse_out[row] = x;
-  if (!leaf_shifted) return;
-  float log_w = 0.0f;  // log of the product of the weights c of the shallower levels
 #pragma unroll
-  for (int j = 0; j < MAXL; ++j) {
-    if (j < lv.levels && ((leaf_no >> (lv.levels - 1 - j)) & 1u)) {
-      lv.shifted[j][level_row(j)] = x_of[j] - log1pf(-c_of[j]) - log_w;
-      log_w += logf(c_of[j]);
-    }
+    for (int u = 0; u < UNROLL; ++u)
+      if (item[u] < items) *reinterpret_cast<vec8*>((char*)p.out + row0 * row_bytes + item[u] * 16) = r[u];
   }
-  leaf_shifted[row] = x_leaf - log_w;
+  if (!own_row) return;
+  p.lse_out[row0 + threadIdx.x] = x;
+  if (!p.leaf_shifted) return;
+  float log_w = 0.f;  // log of the product of the weights c of the shallower levels
+  auto shift = [&](int j, float x_un) {
+    const float c = weight[j * p.chunk_rows + threadIdx.x];
+    lv.shifted[j][level_row(j) + threadIdx.x] = x_un - log1pf(-c) - log_w;
+    log_w += logf(c);
+  };
+  if constexpr (MORE) {
+    for (int j = 0; j < lv.levels; ++j)
+      if (takes_part(j)) shift(j, lv.lse_un[j][level_row(j) + threadIdx.x]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < GROUP; ++j)
+      if (takes_part(j)) shift(j, x_of[j]);
+  }
+  p.leaf_shifted[row0 + threadIdx.x] = x_leaf - log_w;
 }
 
 }  // namespace
@@ -257,19 +315,35 @@ extern "C" int ha_lse_merge_levels(const void* o_leaf, const float* lse_leaf, co
     lv.lse_un[j] = lse_un[j];
     lv.shifted[j] = leaf_shifted ? lse_shifted[j] : nullptr;
   }
-  const int pieces = (int)(d / 8);
-  const int64_t rows = batch_heads * n, items = rows * pieces;
+  MergeLevelsParams p;
+  p.o_leaf = o_leaf; p.lse_leaf = lse_leaf; p.out = out; p.lse_out = lse_out; p.leaf_shifted = leaf_shifted;
+  p.lv = lv;
+  p.n = n;
+  p.packed = packed;
+  const int64_t leaf_len = n >> levels, pieces = d / 8, items = batch_heads * n * pieces;
   HA_REQUIRE((items + 255) / 256 < (1ll << 31), HA_ERR_SHAPE, "ha_lse_merge_levels: too many rows");
-  dim3 grid((unsigned)((items + 255) / 256));
-  hipStream_t s = (hipStream_t)stream;
-#define HA_MERGE_LEVELS(TT, LL)                                                                                  \
-  hipLaunchKernelGGL((lse_merge_levels_kernel<TT, LL>), grid, dim3(256), 0, s, (const TT*)o_leaf, lse_leaf, (TT*)out, \
-                     lse_out, leaf_shifted, lv, rows, n, pieces, packed)
-  if (dtype == HA_F16) {
-    if (levels <= 8) HA_MERGE_LEVELS(f16_t, 8); else HA_MERGE_LEVELS(f16_t, MERGE_MAX_LEVELS);
-  } else {
-    if (levels <= 8) HA_MERGE_LEVELS(bf16_t, 8); else HA_MERGE_LEVELS(bf16_t, MERGE_MAX_LEVELS);
-  }
-#undef HA_MERGE_LEVELS
+  // chunks of a leaf: as few as there can be, of equal lengths but for the last
+  const int unroll = levels > 4 && levels <= 8 ? 2 : 1;
+  const int64_t most = std::min<int64_t>(std::max<int64_t>(1, MERGE_THREADS * unroll / pieces), MERGE_THREADS), chunks = (leaf_len + most - 1) / most;
+  p.leaf_len = (uint32_t)leaf_len;
+  p.chunks = (uint32_t)chunks;
+  p.chunk_rows = (uint32_t)((leaf_len + chunks - 1) / chunks);
+  p.pieces = (uint32_t)pieces;
+  p.row_of_item = p.chunk_rows == 1 ? 0 : (uint32_t)(((1 << 22) + pieces - 1) / pieces);
+  HA_REQUIRE(leaf_len < (1ll << 32) && (batch_heads << levels) * chunks < (1ll << 31), HA_ERR_SHAPE, "ha_lse_merge_levels: too many rows");
+  dim3 grid((unsigned)((batch_heads << levels) * chunks));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(MERGE_THREADS), levels * p.chunk_rows * 4, (hipStream_t)stream, p);
+  };
+  // Two pieces per thread from five levels on (24 x 131072 rows of 128 bytes, six levels, one | two 377 | 366 us, 8 x 65536 of 256, five,
+  // 113 | 110), one below (32 x 16384 of 256, three, 83 | 88, 48 x 10240 of 128, two, 35.9 | 37.2)
+  auto launch_for = [&](auto element) {
+    typedef decltype(element) T;
+    if (levels <= 4) launch(lse_merge_levels_kernel<T, 4, 1, false>);
+    else if (levels <= 8) launch(lse_merge_levels_kernel<T, 8, 2, false>);
+    else launch(lse_merge_levels_kernel<T, 8, 1, true>);
+  };
+  if (dtype == HA_F16) launch_for(f16_t());
+  else launch_for(bf16_t());
   return ha_launch_status("ha_lse_merge_levels");
 }

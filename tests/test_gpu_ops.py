@@ -567,6 +567,41 @@ def test_merge_levels_equals_the_chain_of_segment_merges(ha, dtype, levels, pack
         assert torch.isinf(leaf_shifted).any() and torch.isinf(shifted[levels - 1][~torch.isnan(shifted[levels - 1])]).any()
 
 
+@pytest.mark.parametrize("b,h,leaf,d,levels,dtype", [
+    (1, 3, 129, 64, 2, torch.bfloat16),   # three chunks of 43 rows
+    (2, 1, 100, 96, 3, torch.float16),    # twelve pieces a row, chunks of 34, 34 and 32 rows
+    (1, 2, 600, 8, 1, torch.bfloat16),    # one piece a row: more rows than threads
+    (1, 2, 7, 1032, 1, torch.float16),    # chunks of three rows
+    (1, 1, 3, 2056, 2, torch.bfloat16),   # one row a chunk
+    (1, 1, 2, 4104, 1, torch.float16),    # one row is more than a trip of its workgroup
+    (1, 1, 3, 80, 9, torch.bfloat16),     # the instance for more than eight levels
+])
+def test_merge_levels_chunks_of_leaves(ha, b, h, leaf, d, levels, dtype):
+    """Rows of packed levels against one merge launch per level and segment half, bit for bit."""
+    import ctypes
+    from hyperattention_amd import _lib
+    n, bh, lib, code = leaf << levels, b * h, _lib.lib(), 0 if dtype == torch.float16 else 1
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    o_leaf, lse_leaf = _randn((bh, n, d), 85, dtype).cuda(), _randn((bh, n), 86, torch.float32).cuda() * 4
+    o_un, lse_un = _randn((levels, bh, n // 2, d), 87, dtype).cuda(), _randn((levels, bh, n // 2), 88, torch.float32).cuda() * 4
+    out, lse = o_leaf.clone(), lse_leaf.clone()
+    for j in reversed(range(levels)):
+        H, half = bh << j, n >> (j + 1)
+        o1, l1 = out.view(H, 2, half, d)[:, 1].contiguous(), lse.view(H, 2, half)[:, 1].contiguous()
+        o2, l2, c = torch.empty_like(o1), torch.empty_like(l1), torch.empty_like(l1)
+        _lib.check(lib.ha_lse_merge_segments(
+            o1.data_ptr(), l1.data_ptr(), o_un[j].data_ptr(), lse_un[j].data_ptr(), o2.data_ptr(), l2.data_ptr(), c.data_ptr(), H, half, d,
+            half * d, d, half * d, d, half * d, d, half, half, half, half, code, stream))
+        out.view(H, 2, half, d)[:, 1], lse.view(H, 2, half)[:, 1] = o2, l2
+    got, got_lse, leaf_shifted, shifted = torch.empty_like(out), torch.empty_like(lse), torch.empty_like(lse), torch.full_like(lse_un, float("nan"))
+    ptrs = lambda x: (ctypes.c_void_p * levels)(*[y.data_ptr() for y in x])
+    _lib.check(lib.ha_lse_merge_levels(o_leaf.data_ptr(), lse_leaf.data_ptr(), ptrs(o_un), ptrs(lse_un), ptrs(shifted), leaf_shifted.data_ptr(),
+                                       got.data_ptr(), got_lse.data_ptr(), levels, bh, n, d, code, 1, stream))
+    assert torch.equal(got, out) and torch.equal(got_lse, lse)
+    assert not torch.isnan(shifted).any() and not torch.isnan(leaf_shifted).any()
+
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_merge_segments_in_place(ha, dtype):
     """ha_lse_merge_segments on the second halves of every head, in place, with the weight written out:
