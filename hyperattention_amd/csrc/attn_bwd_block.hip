@@ -562,10 +562,12 @@ bool ha_block_bwd_fused_takes(const ha_block_attn_args& a) {
 // Blocks per workgroup, one workgroup per CU: the run with the least time by the rounds of workgroups; starting and ending
 // one takes as long as two thirds of a block.  Within 0.2 % of the best run of 1 to 8, 10 and 12 at every one of those
 // launches, samples or not; as two fifths of a block it chose three rounds of one block for 24 x 8192, 175 us.
+// Runs of more than 12 blocks, which save whole starts and shares where that leaves one round or two, forward and backward without mask,
+// up to 12 | 64: 32 heads x 65536 1422 | 1399 us, 16 x 65536 727 | 714, 12 x 65536 575 | 557, 24 x 40960 703 | 682, 64 x 24576 1068 | 1057.
 static int64_t fused_run(int64_t vseqs, int64_t n) {
   int64_t best = INT64_MAX, run = 1;
   const int64_t blocks = fused_blocks(n);
-  for (int64_t r = 1; r <= std::min<int64_t>(blocks, 12); ++r) {
+  for (int64_t r = 1; r <= std::min<int64_t>(blocks, 64); ++r) {
     const int64_t cost = (vseqs * ((blocks + r - 1) / r) + 255) / 256 * (3 * r + 2);
     if (cost < best) {
       best = cost;
