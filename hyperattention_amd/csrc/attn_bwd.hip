@@ -219,54 +219,76 @@ __global__ __launch_bounds__(256) void ha_bwd_zero_kernel(f32x4* __restrict__ bu
   if (i < n4) buf[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// Sums of the sampled keys (fp32, `shares` of them, rows by slot of the sample list or (FUSED) as ha_fused_share_at has them)
-// added to the rows of dk (blockIdx.y = 0; times k_factor) or dv, 4 elements per lane, lanes in the order of a share.  A row that is listed several times is handled by its first slot alone, which adds
-// the sums of all of them: no two lanes write the same row, whatever the list holds.
+struct AddSamplesParams {
+  const float* sums[2];  // of dk (times k_factor) and dv: `shares` of them, rows by slot of the sample list or (FUSED) as ha_fused_share_at has them
+  void* grad[2];         // dk, dv
+  int64_t sb[2], sh[2], sn[2];
+  const void* sampled_idx;
+  int64_t si_sb, si_sh, seg_stride, k_seg_off;
+  int idx64, kv_heads, sample_size, shares, segs;
+  float k_factor;
+};
+
+// Sums of the sampled keys added to the rows of dk (blockIdx.y = 0) or dv.  A workgroup has 2048 elements of one (batch, kv head,
+// segment), 8 per thread, so that rows are read and written whole; FUSED sums, which lie as the products leave them, are
+// turned around in LDS.  A row that is listed several times is handled by its first slot alone, which adds the sums of all of
+// them: no two lanes write the same row, whatever the list holds.
+// HBM-bound.  With 4 elements per thread, FUSED rows written 8 bytes at a time and three 64-bit divisions a thread it took 56.7 us and takes 30.9
+// for 768 segments of one share at d = 64 (6.5 TB/s), for 24 of 32 shares 21.0 | 20.9, 48 of 10 and 96 of 5 11.0 | 8.4, 16.6 | 14.2; d = 128,
+// 8 segments of 16 shares 16.5 | 12.6.
 template <typename T, int D, bool FUSED>
-__global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const float* __restrict__ sk32, const float* __restrict__ sv32,
-                                                                 T* __restrict__ dk, T* __restrict__ dv,
-                                                                 const void* __restrict__ sampled_idx, int idx64,
-                                                                 int64_t si_sb, int64_t si_sh, int kv_heads, int sample_size,
-                                                                 int shares, int64_t dk_sb, int64_t dk_sh, int64_t dk_sn,
-                                                                 int64_t dv_sb, int64_t dv_sh, int64_t dv_sn, int64_t total_slots,
-                                                                 int segs, int64_t seg_stride, int64_t k_seg_off, float k_factor) {
-  ha_load_arguments<172>();
-  typedef typename ElemTraits<T>::vec4 vec4;
-  constexpr int PR = D / 4;
-  const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t gslot = FUSED ? item / (32 * PR) * 32 + item % 32 : item / PR;
-  const int piece = (int)(FUSED ? item / 32 % PR : item % PR);
-  if (gslot >= total_slots) return;
-  const bool is_v = blockIdx.y != 0;
-  const int64_t bhs = gslot / sample_size;   // (batch, kv head, segment)
-  const int slot = (int)(gslot - bhs * sample_size);
-  const int64_t bh = bhs / segs, seg = bhs - bh * segs;
-  const int64_t b = bh / kv_heads, h = bh - b * kv_heads;
-  const int64_t row0 = k_seg_off + seg * seg_stride;
+__global__ __launch_bounds__(256) void ha_bwd_add_samples_kernel(const AddSamplesParams p) {
+  ha_load_arguments<(int)sizeof(AddSamplesParams)>();
+  typedef typename ElemTraits<T>::vec8 vec8;
+  constexpr int PR = D / 8, ROWS = 256 / PR;
+  static_assert(!FUSED || ROWS == 32, "FUSED sums come in groups of 32 keys");
+  const int tiles = p.sample_size / ROWS, bhs = blockIdx.x / tiles, slot0 = (blockIdx.x - bhs * tiles) * ROWS;
+  const int bh = bhs / p.segs, seg = bhs - bh * p.segs, b = bh / p.kv_heads, h = bh - b * p.kv_heads, is_v = blockIdx.y;
+  const int tid = threadIdx.x, r = tid / PR, piece = tid % PR, slot = slot0 + r;
+  const int64_t share = (int64_t)p.sample_size * D;
+  const float* const base = p.sums[is_v] + (int64_t)bhs * p.shares * share;
+  T* const rows = (T*)p.grad[is_v] + b * p.sb[is_v] + h * p.sh[is_v] + (p.k_seg_off + (int64_t)seg * p.seg_stride) * p.sn[is_v] + piece * 8;
+  const int64_t list = b * p.si_sb + h * p.si_sh;
   int row = slot;
-  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-  const float* const base = (is_v ? sv32 : sk32) + bhs * shares * sample_size * D;
-  auto add_slot = [&](int s2) {
-    const float* const at = base + (FUSED ? ha_fused_share_at(s2, piece) : s2 * D + piece * 4);
-#pragma unroll 8
-    for (int k = 0; k < shares; ++k) sum += *reinterpret_cast<const f32x4*>(at + (int64_t)k * sample_size * D);
-  };
-  if (sampled_idx) {
-    const int64_t list = b * si_sb + h * si_sh;
-    row = ha_load_idx(sampled_idx, list + slot, idx64);
-    for (int s2 = 0; s2 < slot; ++s2)
-      if (ha_load_idx(sampled_idx, list + s2, idx64) == row) return;  // an earlier slot owns this row
-    add_slot(slot);
-    for (int s2 = slot + 1; s2 < sample_size; ++s2)
-      if (ha_load_idx(sampled_idx, list + s2, idx64) == row) add_slot(s2);
-  } else {
-    add_slot(slot);
+  bool owner = true;  // no earlier slot has the row
+  if (p.sampled_idx) {
+    row = ha_load_idx(p.sampled_idx, list + slot, p.idx64);
+    for (int s2 = 0; s2 < slot && owner; ++s2) owner = ha_load_idx(p.sampled_idx, list + s2, p.idx64) != row;
   }
-  vec4* const dst = reinterpret_cast<vec4*>(is_v ? dv + b * dv_sb + h * dv_sh + (row0 + row) * dv_sn + piece * 4
-                                                 : dk + b * dk_sb + h * dk_sh + (row0 + row) * dk_sn + piece * 4);
-  vec4 o = *dst;
+  vec8* const dst = reinterpret_cast<vec8*>(rows + row * p.sn[is_v]);
+  vec8 o = *dst;
+  f32x4 sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  auto add_shares = [&](const float* at0, const float* at1) {
+#pragma unroll 8
+    for (int k = 0; k < p.shares; ++k) {
+      sum[0] += *reinterpret_cast<const f32x4*>(at0 + k * share);
+      sum[1] += *reinterpret_cast<const f32x4*>(at1 + k * share);
+    }
+  };
+  auto at = [&](int s2, int half) -> const float* {
+    return base + (FUSED ? ha_fused_share_at(s2, 2 * piece + half) : s2 * D + piece * 8 + half * 4);
+  };
+  if constexpr (FUSED) {
+    __shared__ f32x4 turn[512];  // [key][four elements]
+    const float* const mine = base + (slot0 >> 5) * 2048 + tid * 4;
+    add_shares(mine, mine + 1024);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = (T)((float)o[e] + (FUSED && !is_v ? sum[e] * k_factor : sum[e]));
+    for (int i = 0; i < 2; ++i) {
+      const int key = tid & 31, four = i * 8 + tid / 32;
+      turn[key * 16 + (four ^ (key & 15))] = sum[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sum[i] = turn[r * 16 + ((2 * piece + i) ^ (r & 15))];
+  } else {
+    add_shares(at(slot, 0), at(slot, 1));
+  }
+  if (!owner) return;
+  if (p.sampled_idx)
+    for (int s2 = slot + 1; s2 < p.sample_size; ++s2)
+      if (ha_load_idx(p.sampled_idx, list + s2, p.idx64) == row) add_shares(at(s2, 0), at(s2, 1));
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = (T)((float)o[e] + (FUSED && !is_v ? sum[e >> 2][e & 3] * p.k_factor : sum[e >> 2][e & 3]));
   *dst = o;
 }
 
@@ -394,13 +416,20 @@ template <typename T, int D, bool FUSED = false>
 int launch_add_samples(const ha_block_attn_args& a, const ha_attn_grads& g, const Workspace& w, int64_t shares, hipStream_t stream) {
   const ha_attn_operands& t = a.t;
   const int64_t kv_heads = t.heads / t.kv_group;
-  const int64_t slots = t.batch * kv_heads * t.segs * a.sample_size;
-  const int64_t items = slots * (D / 4);
-  hipLaunchKernelGGL((ha_bwd_add_samples_kernel<T, D, FUSED>), dim3((unsigned)((items + 255) / 256), 2), dim3(256), 0, stream,
-                     w.dk32, w.dv32, (T*)g.dk, (T*)g.dv, a.sampled_idx, (int)(a.idx_type == HA_IDX_I64),
-                     a.sampled_stride_b, a.sampled_stride_h, (int)kv_heads, (int)a.sample_size, (int)shares, g.dk_stride_b,
-                     g.dk_stride_h, g.dk_stride_n, g.dv_stride_b, g.dv_stride_h, g.dv_stride_n, slots, (int)t.segs,
-                     t.seg_stride_rows, t.k_seg_offset, t.scale);
+  AddSamplesParams p;
+  p.sums[0] = w.dk32; p.sums[1] = w.dv32;
+  p.grad[0] = g.dk; p.grad[1] = g.dv;
+  p.sb[0] = g.dk_stride_b; p.sh[0] = g.dk_stride_h; p.sn[0] = g.dk_stride_n;
+  p.sb[1] = g.dv_stride_b; p.sh[1] = g.dv_stride_h; p.sn[1] = g.dv_stride_n;
+  p.sampled_idx = a.sampled_idx;
+  p.si_sb = a.sampled_stride_b; p.si_sh = a.sampled_stride_h;
+  p.seg_stride = t.seg_stride_rows; p.k_seg_off = t.k_seg_offset;
+  p.idx64 = a.idx_type == HA_IDX_I64;
+  p.kv_heads = (int)kv_heads; p.sample_size = (int)a.sample_size; p.shares = (int)shares; p.segs = (int)t.segs;
+  p.k_factor = t.scale;
+  const int64_t workgroups = t.batch * kv_heads * t.segs * a.sample_size * (D / 8) / 256;  // sample_size is a multiple of 128
+  if (workgroups >= (1ll << 31)) return ha_fail(HA_ERR_SHAPE, "attention backward: %lld workgroups", (long long)workgroups);
+  hipLaunchKernelGGL((ha_bwd_add_samples_kernel<T, D, FUSED>), dim3((unsigned)workgroups, 2), dim3(256), 0, stream, p);
   return ha_launch_status("attention backward: sampled keys");
 }
 

@@ -122,3 +122,24 @@ def test_small_workspace_takes_the_passes(ha):  # noqa: F811
     for x, y, name in zip(*results, ("dq", "dk", "dv")):
         # the same sums in another order, each rounded to fp16: half a unit of its last place on either side
         assert (x.double() - y.double()).norm() / y.double().norm() <= 2.0 ** -10, name
+
+
+def test_runs_of_sixteen_blocks(ha):  # noqa: F811
+    """One round of workgroups, each with 16 blocks: the passes' gradients (see above: the sums' order, each rounded to fp16)."""
+    from hyperattention_amd import _lib, ops
+    h, n, sample = 64, 16384, 256
+    g = torch.Generator(device="cuda").manual_seed(71)
+    q, k, v, do = (torch.randn((1, n, h, 64), generator=g, device="cuda", dtype=torch.float16) for _ in range(4))
+    qi, ki = (torch.rand((1, h, n), generator=g, device="cuda").argsort(-1).int().transpose(1, 2) for _ in range(2))
+    o, lse = ops.hyper_attn_func(q, k, v, qi, ki, 256, sample, 0.125, False)
+    a, _keep = ops._block_attn_args(q, k, v, o, lse, qi, ki, 256, sample, 0.125, False, None)
+    results = []
+    for small in (False, True):
+        grads = [torch.empty_like(x) for x in (q, k, v)]
+        args, _ws = ops._attn_grads(a.t, do, *grads, sample_size=sample)
+        if small:
+            args.workspace_bytes = h * n * 8 + 2 * h * sample * 64 * 4
+        _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(args), ops._stream(q)))
+        results.append(grads)
+    for x, y, name in zip(*results, ("dq", "dk", "dv")):
+        assert (x.double() - y.double()).norm() / y.double().norm() <= 2.0 ** -10, name
