@@ -636,6 +636,8 @@ static bool large_tiles(const ha_attn_kernel_params& p, bool causal) {
 // by this rule): 12 heads of 7167 rows (672 tiles on 768 places) 78.0 | 70.7 | 65.5, 8 of 9728 85.9 | 80.0 | 74.6; 24 of 4096 (768 on 768)
 // 63.3 | 56.8 | 59.8, 12 of 14335, d = 96 (2.6 rounds) 272 | 260 | 282, 32 of 11520, d = 128 (3) 558 | 553 | 579; pairs of tiles, d = 64: 16 of
 // 29696 (2) 380 | 371 | 360, 24 of 29184 (3) 848 | 830 | 817; d = 128, 16 of 77824 (10) 2010 | 1998 | 1969.
+// Spread between the tiles of launches of many rounds, a group after every few groups of tiles, they cost the tiles more than hashing beside them
+// hides, behind | spread: 4 heads of 131072 474 | 498 us, 8 of 65536 422 | 443, d = 96, 16 of 20479 364 | 371, 32 of 131072 3900 | 3910.
 static int64_t place_ranking(ha_rank_beside& a, int64_t tiles, int per_cu, bool pairs_64) {
   const int64_t groups = (tiles + NUM_XCD - 1) / NUM_XCD, places = 256 * per_cu;
   a.groups = (a.units + NUM_XCD - 1) / NUM_XCD;
