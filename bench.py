@@ -58,7 +58,7 @@ def kernel_source_digest():
     record the digest of the sources they were measured on."""
     h = hashlib.sha256()
     try:
-        for name in ("attn_fwd.hip", "attn_fwd_tile.inc", "attn_tiles.h"):
+        for name in ("attn_fwd.hip", "attn_fwd_body.inc", "attn_fwd_tile.inc", "attn_tiles.h"):
             h.update(open(os.path.join(ROOT, "hyperattention_amd", "csrc", name), "rb").read())
     except OSError:
         return None
