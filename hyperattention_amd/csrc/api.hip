@@ -238,6 +238,10 @@ void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w, bo
     ha_unit_grid& g = w.grid;
     g.n = nh;
     g.granule = pl.granule;
+    // Not beside launches of so many rounds that their ends do not count: there the rows, hashed behind the tiles, come slower than in a launch
+    // of nothing else.  Whole calls, beside | apart, us: 32 heads of 131072 3809 | 3794, 4 x 32 of 32768 2995 | 2993, 32 of 65536 (half as many
+    // rows) 1709 | 1721, at d = 128 3340 | 3338, 16 of 131072 1912 | 1921, 8 971 | 991, 32 of 32768 767 | 789.
+    leaves = leaves && a.batch * (a.heads + a.kv_heads) * nh < (1ll << 23);
     // the one segment of the one hashed level in one unit, without a placement launch: up to the length where that is
     // faster (rank_units_kernel) and one workgroup per CU, or, beside the leaves, where its rows' numbers and ids fit the tiles' LDS
     const bool one = nh / g.granule == (a.causal ? 2 : 1);

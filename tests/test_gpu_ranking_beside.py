@@ -65,6 +65,7 @@ def _launch_by_launch(q, k, v, proj, projs, block, sample, msl):
     (1, 24, 12, 8192, 2048, 96, 8, torch.float16),
     (2, 8, 8, 4096, 512, 80, 5, torch.bfloat16),
     (1, 4, 4, 2048, 256, 112, 8, torch.float16),
+    (64, 32, 32, 2048, 1024, 16, 8, torch.float16),   # so many rows that they are hashed ahead of the leaves
 ])
 def test_orders_are_those_of_the_sort(b, h, hk, n, msl, d, projs, dtype):
     from hyperattention_amd import ops
