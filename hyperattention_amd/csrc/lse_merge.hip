@@ -167,7 +167,7 @@ struct MergeLevelsParams {
   void* out;
   float *lse_out, *leaf_shifted;
   MergeLevels lv;
-  int64_t n;
+  int64_t n, rows;  // rows of a sequence, of all of them
   uint32_t leaf_len, chunks, chunk_rows, pieces;
   uint32_t row_of_item;  // ceil(2^22 / pieces), 0 where a chunk is one row: item * that >> 22 is the item's row in its chunk
   int packed;
@@ -176,7 +176,7 @@ struct MergeLevelsParams {
 // A workgroup merges up to 256 * UNROLL pieces of 16 bytes of consecutive rows of one leaf (more where a row alone has more): which
 // levels they take part in and where those results lie is the same for all, in scalar registers.  A row's chain of weights is
 // one thread's, while the pieces' loads are in flight; its pieces' threads read the weights from LDS.
-// HBM-bound.  With a thread's row, its halves and its weights found by each of its pieces' threads (64-bit divisions, every
+// HBM-bound.  With a thread's row, its halves and its weights found by each of its pieces' threads (lse_merge_rows_kernel: 64-bit divisions, every
 // weight 8 to 16 times) it was bound by instructions: 24 x 131072 rows of 128 bytes, six levels, 443 -> 366 us (5.5 TB/s), 32 x 16384
 // of 256 bytes, three levels, 94 -> 83, 48 x 10240 of 128, two levels, 40 -> 36, 8 x 65536, nine levels, 171 -> 118.
 // GROUP: levels whose pieces are loaded at once, all of them unless MORE.
@@ -283,6 +283,76 @@ __global__ __launch_bounds__(MERGE_THREADS) void lse_merge_levels_kernel(const M
   p.leaf_shifted[row0 + threadIdx.x] = x_leaf - log_w;
 }
 
+// One piece of a row per thread, whatever leaf it lies in: for leaves that whole workgroups do not fit (merge_by_leaf).
+// MAXL: levels the instance is unrolled for (the recursion rarely goes deeper than 8)
+template <typename T, int MAXL>
+__global__ __launch_bounds__(MERGE_THREADS) void lse_merge_rows_kernel(const MergeLevelsParams p) {
+  ha_load_arguments<(int)sizeof(MergeLevelsParams)>();
+  typedef typename ElemTraits<T>::vec8 vec8;
+  const MergeLevels& lv = p.lv;
+  const int64_t item = (int64_t)blockIdx.x * MERGE_THREADS + threadIdx.x;
+  const int64_t row = item / p.pieces;
+  if (row >= p.rows) return;
+  const int64_t seq = row / p.n;
+  const uint32_t row_in_seq = (uint32_t)(row - seq * p.n), leaf_no = row_in_seq / p.leaf_len;
+  float x = p.lse_leaf[row];
+  const float x_leaf = x;
+  vec8 r = *reinterpret_cast<const vec8*>((const char*)p.o_leaf + item * 16);
+  float c_of[MAXL], x_of[MAXL];
+  vec8 v_of[MAXL];
+  auto takes_part = [&](int j) -> bool { return j < lv.levels && ((leaf_no >> (lv.levels - 1 - j)) & 1u); };
+  auto level_row = [&](int j) -> int64_t {
+    const int64_t half = p.n >> (j + 1), segment = leaf_no >> (lv.levels - j);
+    return p.packed ? seq * (p.n >> 1) + row_in_seq - (segment + 1) * half : row;
+  };
+  // every load first, so that they are all in flight before the chain of weights (each level's weight needs
+  // the log-sum-exp the deeper levels left) starts
+#pragma unroll
+  for (int j = MAXL - 1; j >= 0; --j) {
+    c_of[j] = 1.f;
+    x_of[j] = 0.f;
+    if (takes_part(j)) {
+      const int64_t at = level_row(j);
+      x_of[j] = lv.lse_un[j][at];
+      v_of[j] = *reinterpret_cast<const vec8*>((const char*)lv.o_un[j] + (item + (at - row) * p.pieces) * 16);
+    }
+  }
+#pragma unroll
+  for (int j = MAXL - 1; j >= 0; --j) {
+    if (takes_part(j)) {
+      const float c = (float)(T)(1.0f / (1.0f + __expf(x_of[j] - x)));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[e] = (T)(c * (float)r[e] + (1.0f - c) * (float)v_of[j][e]);
+      x = x - __logf(c + 1.1920929e-07f);
+      c_of[j] = c;
+    }
+  }
+  *reinterpret_cast<vec8*>((char*)p.out + item * 16) = r;
+  if (item != row * p.pieces) return;
+  p.lse_out[row] = x;
+  if (!p.leaf_shifted) return;
+  float log_w = 0.f;
+#pragma unroll
+  for (int j = 0; j < MAXL; ++j) {
+    if (takes_part(j)) {
+      lv.shifted[j][level_row(j)] = x_of[j] - log1pf(-c_of[j]) - log_w;
+      log_w += logf(c_of[j]);
+    }
+  }
+  p.leaf_shifted[row] = x_leaf - log_w;
+}
+
+// Whether a workgroup's rows lie in one leaf.  `full`: the part of the workgroups' threads that have a piece; a leaf that a chunk's rows do
+// not divide, and a short one above all, leaves some without, and chunks that do not start at multiples of 32 rows share lines of log-sum-exps.
+// Rows | by leaf, us (1300 launches of leaves of 1 to 4096 rows, 2^13 to 2^21 in all; where the rule takes the leaves they are 0.82 to 2 times as fast,
+// 1.23 at the median, the others 0.6 to 1.7, 0.84): one level, 2^20 sequences of d = 64: leaves of 1 row 139 | 3402, of 16 124 | 223, of 65 124 | 167, of 822 182 | 191,
+// of 64 (full) 145 | 128; three levels, 2^17 rows: leaves of 34 18 | 19, of 75 18 | 14; 3 * 2^20 rows, which no cache holds, of 41, d = 128, 561 | 586, of 392 287 | 276; six: 2^17
+// rows, leaves of 43 (0.67) 27.4 | 25.1, 3 * 2^20 of 135 (0.7) 463 | 473, of 230 (0.9) 464 | 454.
+static bool merge_by_leaf(int levels, double full, double bytes) {
+  if (levels < 2) return full == 1;
+  return full >= (bytes > 256e6 ? 0.9 : levels == 2 ? 0.8 : 0.7);
+}
+
 }  // namespace
 
 extern "C" int ha_lse_merge_levels(const void* o_leaf, const float* lse_leaf, const void* const* o_un,
@@ -319,9 +389,10 @@ extern "C" int ha_lse_merge_levels(const void* o_leaf, const float* lse_leaf, co
   p.o_leaf = o_leaf; p.lse_leaf = lse_leaf; p.out = out; p.lse_out = lse_out; p.leaf_shifted = leaf_shifted;
   p.lv = lv;
   p.n = n;
+  p.rows = batch_heads * n;
   p.packed = packed;
-  const int64_t leaf_len = n >> levels, pieces = d / 8, items = batch_heads * n * pieces;
-  HA_REQUIRE((items + 255) / 256 < (1ll << 31), HA_ERR_SHAPE, "ha_lse_merge_levels: too many rows");
+  const int64_t leaf_len = n >> levels, pieces = d / 8, items = p.rows * pieces;
+  HA_REQUIRE((items + 255) / 256 < (1ll << 31) && n < (1ll << 32), HA_ERR_SHAPE, "ha_lse_merge_levels: too many rows");
   // chunks of a leaf: as few as there can be, of equal lengths but for the last
   const int unroll = levels > 4 && levels <= 8 ? 2 : 1;
   const int64_t most = std::min<int64_t>(std::max<int64_t>(1, MERGE_THREADS * unroll / pieces), MERGE_THREADS), chunks = (leaf_len + most - 1) / most;
@@ -330,16 +401,21 @@ extern "C" int ha_lse_merge_levels(const void* o_leaf, const float* lse_leaf, co
   p.chunk_rows = (uint32_t)((leaf_len + chunks - 1) / chunks);
   p.pieces = (uint32_t)pieces;
   p.row_of_item = p.chunk_rows == 1 ? 0 : (uint32_t)(((1 << 22) + pieces - 1) / pieces);
-  HA_REQUIRE(leaf_len < (1ll << 32) && (batch_heads << levels) * chunks < (1ll << 31), HA_ERR_SHAPE, "ha_lse_merge_levels: too many rows");
-  dim3 grid((unsigned)((batch_heads << levels) * chunks));
+  const int64_t leaf_groups = (batch_heads << levels) * chunks, trip = MERGE_THREADS * unroll;
+  const double full = (double)items / ((double)leaf_groups * ((p.chunk_rows * pieces + trip - 1) / trip * trip));
+  const bool by_leaf = leaf_groups < (1ll << 24) &&  // a launch has less than 2^32 threads
+                       merge_by_leaf(levels, full, (double)items * 16 * (2 + 0.5 * levels));
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(MERGE_THREADS), levels * p.chunk_rows * 4, (hipStream_t)stream, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(by_leaf ? leaf_groups : (items + MERGE_THREADS - 1) / MERGE_THREADS)), dim3(MERGE_THREADS),
+                       by_leaf ? levels * p.chunk_rows * 4 : 0, (hipStream_t)stream, p);
   };
   // Two pieces per thread from five levels on (24 x 131072 rows of 128 bytes, six levels, one | two 377 | 366 us, 8 x 65536 of 256, five,
   // 113 | 110), one below (32 x 16384 of 256, three, 83 | 88, 48 x 10240 of 128, two, 35.9 | 37.2)
   auto launch_for = [&](auto element) {
     typedef decltype(element) T;
-    if (levels <= 4) launch(lse_merge_levels_kernel<T, 4, 1, false>);
+    if (!by_leaf && levels <= 8) launch(lse_merge_rows_kernel<T, 8>);
+    else if (!by_leaf) launch(lse_merge_rows_kernel<T, MERGE_MAX_LEVELS>);
+    else if (levels <= 4) launch(lse_merge_levels_kernel<T, 4, 1, false>);
     else if (levels <= 8) launch(lse_merge_levels_kernel<T, 8, 2, false>);
     else launch(lse_merge_levels_kernel<T, 8, 1, true>);
   };

@@ -568,13 +568,26 @@ def test_merge_levels_equals_the_chain_of_segment_merges(ha, dtype, levels, pack
 
 
 @pytest.mark.parametrize("b,h,leaf,d,levels,dtype", [
-    (1, 3, 129, 64, 2, torch.bfloat16),   # three chunks of 43 rows
-    (2, 1, 100, 96, 3, torch.float16),    # twelve pieces a row, chunks of 34, 34 and 32 rows
-    (1, 2, 600, 8, 1, torch.bfloat16),    # one piece a row: more rows than threads
-    (1, 2, 7, 1032, 1, torch.float16),    # chunks of three rows
-    (1, 1, 3, 2056, 2, torch.bfloat16),   # one row a chunk
-    (1, 1, 2, 4104, 1, torch.float16),    # one row is more than a trip of its workgroup
-    (1, 1, 3, 80, 9, torch.bfloat16),     # the instance for more than eight levels
+    (1, 3, 129, 64, 2, torch.bfloat16),   # five chunks of 26 rows in a leaf, the last of 25
+    (2, 1, 100, 96, 3, torch.float16),    # twelve pieces a row, five chunks of 20 rows
+    (1, 2, 600, 8, 1, torch.bfloat16),    # one level and threads without a piece: by rows
+    (1, 2, 7, 1032, 1, torch.float16),    # the same, 129 pieces a row
+    (1, 1, 3, 2056, 2, torch.bfloat16),   # 257 pieces
+    (1, 1, 2, 4104, 1, torch.float16),    # 513 pieces
+    (1, 1, 3, 80, 9, torch.bfloat16),     # by rows, more than eight levels
+    (1, 2, 128, 64, 9, torch.float16),    # the leaves' instance for those: four chunks of 32 rows
+    (1, 2, 512, 64, 1, torch.bfloat16),   # one level, every thread with a piece
+    (2, 1, 511, 8, 2, torch.float16),     # two chunks of 256 rows, the second of 255
+    (1, 2, 128, 64, 5, torch.bfloat16),   # two pieces a thread from five levels on: two chunks of 64 rows
+    (1, 3, 129, 64, 6, torch.float16),    # by rows, more than four levels
+    (2, 1, 100, 96, 5, torch.bfloat16),   # chunks of 34, 34 and 32 rows
+    (1, 1, 70, 112, 8, torch.float16),    # two chunks of 35 rows
+    (1, 1, 6, 1032, 6, torch.bfloat16),   # two chunks of three rows
+    (1, 1, 7, 1032, 6, torch.bfloat16),   # by rows
+    (1, 1, 2, 4088, 6, torch.float16),    # one row of 511 pieces a chunk
+    (1, 1, 2, 8128, 6, torch.bfloat16),   # of 1016, two trips
+    (300, 1, 1, 8, 1, torch.bfloat16),    # by rows: sequences of two rows
+    (7, 5, 3, 64, 1, torch.float16),
 ])
 def test_merge_levels_chunks_of_leaves(ha, b, h, leaf, d, levels, dtype):
     """Rows of packed levels against one merge launch per level and segment half, bit for bit."""
@@ -600,6 +613,25 @@ def test_merge_levels_chunks_of_leaves(ha, b, h, leaf, d, levels, dtype):
     assert torch.equal(got, out) and torch.equal(got_lse, lse)
     assert not torch.isnan(shifted).any() and not torch.isnan(leaf_shifted).any()
 
+
+def test_merge_levels_of_many_leaves(ha):
+    """2^24 leaves of one row: as one launch of one workgroup each they would be more threads than a launch may have."""
+    import ctypes
+    from hyperattention_amd import _lib
+    bh, d, lib = 1 << 23, 8, _lib.lib()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(89)
+    o_leaf = torch.randn((bh, 2, d), generator=g, device="cuda", dtype=torch.float16)
+    o_un = torch.randn((1, bh, 1, d), generator=g, device="cuda", dtype=torch.float16)
+    lse_leaf, lse_un = (torch.randn(x, generator=g, device="cuda") for x in ((bh, 2), (1, bh, 1)))
+    out, lse = torch.empty_like(o_leaf), torch.empty_like(lse_leaf)
+    ptrs = lambda x: (ctypes.c_void_p * 1)(x.data_ptr())
+    _lib.check(lib.ha_lse_merge_levels(o_leaf.data_ptr(), lse_leaf.data_ptr(), ptrs(o_un), ptrs(lse_un), None, None, out.data_ptr(),
+                                       lse.data_ptr(), 1, bh, 2, d, 0, 1, stream))
+    assert torch.equal(out[:, 0], o_leaf[:, 0]) and torch.equal(lse[:, 0], lse_leaf[:, 0])
+    want, want_lse = ha.add_self_attentions(o_leaf[:, 1:].unsqueeze(0).contiguous(), lse_leaf[:, 1:].unsqueeze(0).unsqueeze(-1).contiguous(),
+                                            o_un, lse_un.unsqueeze(-1))
+    assert torch.equal(out[:, 1:], want[0]) and torch.equal(lse[:, 1:], want_lse[0, ..., 0])
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
