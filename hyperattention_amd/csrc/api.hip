@@ -228,6 +228,19 @@ struct Workspace {
 // longest hashed segment may span this many units before the per-level sort is the better choice.
 inline int64_t max_units_per_segment(int unit) { return std::max<int64_t>(64, unit / 4); }
 
+// Whether units are hashed and ranked beside the exact causal launch (`granules` hashed ones in each of `seqs` sequences, whole if there is
+// `one` and it fits).  What that saves is two launches and their ends, 6 to 12 us.  Beyond a round or two of tiles the rows are not hidden: the launch grows
+// by about what hashing alone takes, and by more where a workgroup has few rows, since each one sets up the projection and adds up its
+// counts by itself.  Whole calls, apart | beside, us, units in brackets (110 launches of 80 to 57400 units; where the rule says beside they are 0.99 to 1.5
+// times as fast), rows a unit 128: 8 x 32 + 32 heads (1536) 86.5 | 85.4, 6 x 32 + 8 (1680) 116 | 117, 64 x 32 + 32 (12288, d = 128) 653 | 725, 205 x 32 + 8 (57400)
+// 3303 | 3629; 256: 8 x 32 + 32 (512) 47.2 | 44.2, 32 x 32 + 32 (2048) 130 | 133, 256 x 8 + 8 (12288) 761 | 818; 512: 64 x 8 + 8 (1024) 144 | 142, 16 x 32 + 32 (3072,
+// d = 128) 772 | 782; 1024: 51 x 32 + 8 (2040) 962 | 954, 64 x 32 + 32 (4096, d = 128) 2515 | 2544; 2048: 16 x 8 + 8 of 16384 (1792) 1354 | 1348, 102 x 16 + 4 (2040)
+// 2676 | 2649, 64 x 32 + 32 (4096) 3551 | 3551, 32 + 32 of 131072 (4032) 3925 | 3921, 64 + 64 (8064) 7778 | 7813; 4096: 8 x 32 + 32 of 16384 (1536) 3231 | 3191.
+bool rank_beside_leaves(int64_t seqs, int64_t granules, int64_t granule, bool one) {
+  const int64_t unit = one && granule <= HA_SORT_BESIDE ? granule : std::min<int64_t>(granule, HA_SORT_CHUNK);
+  return seqs * granules * ((granule + unit - 1) / unit) <= (unit >= 1024 ? 2048 : 1536);
+}
+
 // leaves: an exact causal launch precedes the hashed levels, which units can be hashed and ranked beside
 void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w, bool leaves) {
   int64_t off = 0;
@@ -238,13 +251,10 @@ void layout_workspace(const ha_forward_args& a, const Plan& pl, Workspace& w, bo
     ha_unit_grid& g = w.grid;
     g.n = nh;
     g.granule = pl.granule;
-    // Not beside launches of so many rounds that their ends do not count: there the rows, hashed behind the tiles, come slower than in a launch
-    // of nothing else.  Whole calls, beside | apart, us: 32 heads of 131072 3809 | 3794, 4 x 32 of 32768 2995 | 2993, 32 of 65536 (half as many
-    // rows) 1709 | 1721, at d = 128 3340 | 3338, 16 of 131072 1912 | 1921, 8 971 | 991, 32 of 32768 767 | 789.
-    leaves = leaves && a.batch * (a.heads + a.kv_heads) * nh < (1ll << 23);
     // the one segment of the one hashed level in one unit, without a placement launch: up to the length where that is
     // faster (rank_units_kernel) and one workgroup per CU, or, beside the leaves, where its rows' numbers and ids fit the tiles' LDS
     const bool one = nh / g.granule == (a.causal ? 2 : 1);
+    leaves = leaves && rank_beside_leaves(a.batch * (a.heads + a.kv_heads), nh / g.granule - 1, g.granule, one);
     const bool whole = one && (leaves ? g.granule <= HA_SORT_BESIDE : g.granule <= HA_SORT_WHOLE && a.batch * (a.heads + a.kv_heads) <= 256);
     const int64_t most = whole ? g.granule : HA_SORT_CHUNK;
     g.units_per_granule = (int)((g.granule + most - 1) / most);

@@ -629,8 +629,8 @@ static bool large_tiles(const ha_attn_kernel_params& p, bool causal) {
 }
 
 // Where a grid of `tiles` workgroups of exact causal attention, `per_cu` of which a CU holds, has its ranking workgroups.  Behind the
-// others where all of the grid is resident at once, and in launches of many rounds, whose last one they fill: there the
-// order of the tiles over the CUs stays what it is without them.  Else in front: a ranking workgroup takes about as
+// others where all of the grid is resident at once, and in launches of many rounds: there the order of the tiles over the CUs stays what
+// it is without them (the launch grows by about what hashing takes alone all the same: unit_ranking.h).  Else in front: a ranking workgroup takes about as
 // long as a short tile, and behind one or two rounds of tiles it would be what the launch ends with.  Whole calls, hash and rank
 // launches | in front | behind, us (36 drawn calls and 4 others, 1.035 times faster in the geometric mean in front, 1.022 behind, none slower
 // by this rule): 12 heads of 7167 rows (672 tiles on 768 places) 78.0 | 70.7 | 65.5, 8 of 9728 85.9 | 80.0 | 74.6; 24 of 4096 (768 on 768)

@@ -4,7 +4,9 @@
 // The exact causal launch of a forward pass needs neither, so its grid carries these workgroups along (ha_rank_beside in
 // attn_fwd.h) and the two launches with their start-up and their idle CUs are gone from the chain.  A unit is bound by the time
 // its rows take to arrive, 4 waves asking for 16 or 32 KB each at a time; a launch of nothing but these workgroups would
-// be slower than the two launches that it replaces, beside the exact tiles nobody waits for it.
+// be slower than the two launches that it replaces.  The exact tiles hide it where they are about one round (24 heads of 4096 rows: launch 36 -> 42 us, hash
+// and ranking 10); a launch of several rounds grows by what hashing takes alone (16 of 20479, d = 96: 177 -> 205 us, hash and ranking 27; 32 on 2 of
+// 32768, d = 128: 545 -> 611, 67), and what is saved is the launches themselves (rank_beside_leaves in api.hip).
 #pragma once
 
 #include "attn_fwd.h"

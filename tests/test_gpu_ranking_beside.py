@@ -65,7 +65,7 @@ def _launch_by_launch(q, k, v, proj, projs, block, sample, msl):
     (1, 24, 12, 8192, 2048, 96, 8, torch.float16),
     (2, 8, 8, 4096, 512, 80, 5, torch.bfloat16),
     (1, 4, 4, 2048, 256, 112, 8, torch.float16),
-    (64, 32, 32, 2048, 1024, 16, 8, torch.float16),   # so many rows that they are hashed ahead of the leaves
+    (64, 32, 32, 2048, 1024, 16, 8, torch.float16),   # so many units that they are hashed ahead of the leaves
 ])
 def test_orders_are_those_of_the_sort(b, h, hk, n, msl, d, projs, dtype):
     from hyperattention_amd import ops
@@ -131,3 +131,29 @@ def test_sort_with_the_leaves(b, h, hk, n, msl, d, projs, dtype):
         results.append((out, lse))
     for x, y in zip(*results):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("b,n,msl,beside", [
+    (24, 512, 256, True),      # 1536 units of 256 rows
+    (25, 512, 256, False),     # more of so few rows are hashed in a launch of their own
+    (32, 2048, 1024, True),    # 2048 units of 1024 rows
+    (33, 2048, 1024, False),
+])
+def test_many_units_are_hashed_ahead(b, n, msl, beside):
+    from torch.profiler import ProfilerActivity, profile
+    from hyperattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(630)
+    q, k, v = (torch.randn((b, 32, n, 16), generator=g, device="cuda", dtype=torch.float16) for _ in range(3))
+    proj = torch.randn((1, 1, 16, 8), generator=g, device="cuda", dtype=torch.float16)
+
+    def call():
+        ops.hyper_forward(q, k, v, proj, scale=0.25, causal=True, lsh_num_projs=8, block_size=128, sample_size=128,
+                          min_seq_len=msl, smooth_block=False)
+        torch.cuda.synchronize()
+
+    call()
+    with profile(activities=[ProfilerActivity.CUDA]) as trace:
+        call()
+    names = [e.name for e in trace.events()]
+    assert any("ha_attn_fwd" in x for x in names), "no attention kernel in the trace"
+    assert any("lsh_hash" in x for x in names) == (not beside)
