@@ -45,7 +45,8 @@ struct HashTensors {
   int64_t first[2], end[2];  // rows of every sequence whose ids are wanted
 };
 
-template <typename T, int PARTS, bool OUT8, int GROUP>  // GROUP tiles (1 or 2) in flight together
+// GROUP tiles (1 or 2) in flight together.  ROWS_FIRST: the first rows are asked for ahead of the projection, as the compiler does not by itself
+template <typename T, int PARTS, bool OUT8, int GROUP, bool ROWS_FIRST>
 __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors ten, const T* __restrict__ proj, int64_t n,
                                                             int r, int64_t psb, int64_t psh, int d_real, int tiles) {
   // the first workgroups alone: in those that follow, which find the arguments in the caches, it cost 6 % of a long launch
@@ -87,6 +88,7 @@ __global__ __launch_bounds__(256) void lsh_hash_mfma_kernel(const HashTensors te
   };
   // the first rows are in flight while the projection is set up
   load_rows(wave_row0);
+  if constexpr (ROWS_FIRST) __builtin_amdgcn_sched_barrier(0);
 
   // the projection matrix goes through LDS once per block
   typedef Projection<T, PARTS> P;
@@ -136,7 +138,13 @@ int launch_hash_mfma(HashTensors ten, int64_t seqs, const void* proj, int64_t n,
   if (ten.n_read <= 0 || ten.n_read > n) ten.n_read = n;
   const int64_t gy = seqs < 32768 ? seqs : 32768, gz = (seqs + gy - 1) / gy;
   dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block), (unsigned)gy, (unsigned)gz);
-  auto kernel = tiles % GROUP == 0 ? lsh_hash_mfma_kernel<T, PARTS, OUT8, GROUP> : lsh_hash_mfma_kernel<T, PARTS, OUT8, 1>;
+  // Rows from memory are worth asking for first, of those in the caches the projection is the later one.  Hash to placement, projection | rows first, us: 128
+  // heads of 65536 rows of 256 bytes 396 | 389, 4 of 524288 114.3 | 113.4, 64 of 131072 of 128 bytes 227 | 225; 34 of 32768 of 256 (280 MB) 54.1 | 55.7,
+  // 64 of 32768 of 128 (268 MB) 55.6 | 56.3; 32768 of 128 rows, which leave half of the waves idle, 160 | 163.5.
+  const bool rows_first = rows >= 1024 && (double)rows * seqs * PARTS * 64 > 400e6;
+  auto kernel = rows_first && tiles % GROUP == 0 ? lsh_hash_mfma_kernel<T, PARTS, OUT8, GROUP, true>
+                : tiles % GROUP == 0             ? lsh_hash_mfma_kernel<T, PARTS, OUT8, GROUP, false>
+                                                 : lsh_hash_mfma_kernel<T, PARTS, OUT8, 1, false>;
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ten, (const T*)proj, n, (int)r, psb, psh, (int)d_real, tiles);
   return ha_launch_status("ha_lsh_hash");
 }

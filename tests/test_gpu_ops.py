@@ -45,6 +45,18 @@ def test_hash_bit_exact(ha, dtype, b, h, n, d, r):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("n,d,dtype", [(900003, 64, torch.bfloat16), (850001, 40, torch.float16), (450002, 128, torch.float16), (600007, 96, torch.bfloat16),
+                                       (230001, 256, torch.bfloat16)])
+def test_hash_of_many_rows(ha, n, d, dtype):
+    """More than 400 MB of rows are asked for ahead of the projection: the ids of single heads, which are not that many."""
+    g = torch.Generator(device="cuda").manual_seed(91)
+    x = torch.randn((1, 4, n, d), generator=g, device="cuda", dtype=dtype)
+    proj = torch.randn((1, 1, d, 8), generator=g, device="cuda", dtype=dtype)
+    got = ha.lsh_hash(x, proj)
+    for h in range(4):
+        assert torch.equal(got[:, h:h + 1], ha.lsh_hash(x[:, h:h + 1], proj))
+
+
 def test_hash_reference_test_shape(ha):
     # unit_tests/test_lsh.py:25-31: fp16, (4, 32, 2048, 128), 8 projections
     x = _randn((4, 32, 2048, 128), 3, torch.float16)
