@@ -547,13 +547,16 @@ __global__ __launch_bounds__(FUSED_THREADS, 2) void ha_block_bwd_fused_kernel(co
 // writes the gradients: 256 samples (38 launches of 64 to 6144 blocks) 4 heads x 4096 rows 44 | 35, 24 x 4096 98 | 64, 24 x 8192
 // 156 | 113, 32 x 16384 361 | 259, 24 x 65536 1038 | 735; without samples 20.4 | 19.3 to 692 | 424 (where it adds to them
 // too, but for 16 x 2048 without samples, 22.8 | 23.2); 512: 2 x 512 43.7 | 39.5, 8 x 2048 50 | 48, 24 x 2048 79 | 56, 10 x 16384 165 | 132, 24 x
-// 16384 350 | 297, 130 x 2048 296 | 263, 24 x 65536 1402 | 1099; 768: 8 x 2048 56.8 | 57.6, 24 x 8192 232 | 202, 24 x 65536 1688 | 1434; 1024: 24 x
-// 2048 104 | 84, 130 x 2048 426 | 421, 24 x 65536 1994 | 1798.
+// 16384 350 | 297, 130 x 2048 296 | 263, 24 x 65536 1402 | 1099.  With more samples a workgroup's four or five phases are a chain that the passes spread over CUs
+// which up to 64 blocks leave idle: 768: 1 x 1024 44.8 | 47.9, 2 x 4096 48.8 | 53.0, 8 x 2048 (64 blocks) 54.8 | 56.3, 4 x 4096 56.8 | 56.2, 18 x 1024 (72) 59.5 | 55.2, 24 x 2048 93 |
+// 66, 24 x 8192 236 | 205, 24 x 65536 1737 | 1469; 1024: 1 x 1024 47.8 | 56.8, 2 x 4096 54.0 | 63.5, 8 x 2048 61.8 | 64.9, 2 x 8192 63.1 | 65.2, 3 x 6144 (72) 69.6 | 64.6, 5 x
+// 4096 67.7 | 65.1, 24 x 2048 107 | 79, 130 x 2048 439 | 409, 24 x 65536 2079 | 1847.
 // Head dims below 64, padded for the backward (O as it is): forward and backward of 24 x 16384, d = 48 476 | 418, 512 x 3072, d = 32
 // 1570 | 1324, causal 24 x 65536, d = 40 5923 | 5340.
 static int64_t fused_blocks(int64_t n) { return (n + FUSED_ROWS - 1) / FUSED_ROWS; }
 bool ha_block_bwd_fused_shape(const ha_attn_operands& t, int64_t sample_size) {
-  return t.d == FD && t.kv_group == 1 && t.n_q == t.n_k && sample_size % FUSED_ROWS == 0 && sample_size <= FUSED_MAX_SAMPLES;
+  return t.d == FD && t.kv_group == 1 && t.n_q == t.n_k && sample_size % FUSED_ROWS == 0 && sample_size <= FUSED_MAX_SAMPLES &&
+         (sample_size <= 512 || t.batch * t.heads * t.segs * fused_blocks(t.n_q) > 64);
 }
 bool ha_block_bwd_fused_takes(const ha_block_attn_args& a) {
   return !a.smooth_block && (a.block_size + 127) / 128 * 128 == FUSED_ROWS && ha_block_bwd_fused_shape(a.t, a.sample_size);

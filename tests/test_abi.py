@@ -224,6 +224,20 @@ def test_backward_argument_errors_before_any_launch(lib):
     assert lib.ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), None) == -1
 
 
+@pytest.mark.parametrize("heads,n,sample,shares", [
+    (16, 1024, 512, 4),    # a workgroup per block
+    (16, 1024, 768, 1),    # 64 blocks with more than 512 samples: the passes, which keep one array of sums
+    (17, 1024, 768, 4),
+    (16, 1024, 1024, 1),
+    (17, 1024, 1024, 4),
+    (17, 1024, 1280, 1),   # more than the one kernel takes
+])
+def test_backward_workspace_follows_the_kernel(lib, heads, n, sample, shares):
+    t = _lib.AttnOperands()
+    t.batch, t.heads, t.n_q, t.n_k, t.d, t.dv, t.kv_group, t.segs = 1, heads, n, n, 64, 64, 1, 1
+    assert lib.ha_attn_bwd_workspace_bytes(ctypes.byref(t), sample) == heads * n * 8 + 2 * shares * heads * sample * 64 * 4
+
+
 def test_python_layer_fails_loudly_without_library(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "missing.so"))
     monkeypatch.setattr(_lib, "_lib", None)

@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (torch.bfloat16, 2, 256, 256, torch.int32),    # one block
     (torch.float16, 1, 384, 256, torch.int32),     # the last block is half
     (torch.bfloat16, 3, 1152, 512, torch.int64),   # two phases of sampled keys
-    (torch.float16, 1, 1024, 1024, torch.int32),   # the most
+    (torch.float16, 1, 1024, 1024, torch.int32),   # few blocks and many samples: three passes
+    (torch.bfloat16, 17, 1024, 1024, torch.int64), # the most samples
     (torch.bfloat16, 1, 1280, 1280, torch.int32),  # three passes above
     (torch.float16, 66, 1152, 768, torch.int32),   # three phases, runs of blocks that end with half of one
     (torch.float16, 5, 16512, 256, torch.int32),   # 65 blocks in runs of two: the last run has one, of half the rows
