@@ -30,7 +30,7 @@ HIPCC_FLAGS = [
 SYMBOLS = [
     "ha_abi_version", "ha_last_error", "ha_lsh_hash", "ha_bucket_argsort_workspace_bytes",
     "ha_bucket_argsort", "ha_bucket_argsort_static", "ha_gather_rows", "ha_copy_rows", "ha_block_attn_fwd", "ha_flash_attn_fwd",
-    "ha_attn_bwd_workspace_bytes", "ha_block_attn_bwd", "ha_flash_attn_bwd", "ha_lse_merge",
+    "ha_attn_bwd_workspace_bytes", "ha_block_attn_bwd_workspace_bytes", "ha_block_attn_bwd", "ha_flash_attn_bwd", "ha_lse_merge",
     "ha_lse_merge_segments",
     "ha_forward_workspace_bytes", "ha_forward", "ha_forward_sort", "ha_forward_sort_leaves",
     "ha_lse_merge_levels", "ha_power_probe",
@@ -202,6 +202,8 @@ def _declare(lib):
     lib.ha_flash_attn_fwd.argtypes = [ctypes.POINTER(AttnOperands), ci, vp]
     lib.ha_attn_bwd_workspace_bytes.restype = i64
     lib.ha_attn_bwd_workspace_bytes.argtypes = [ctypes.POINTER(AttnOperands), i64]
+    lib.ha_block_attn_bwd_workspace_bytes.restype = i64
+    lib.ha_block_attn_bwd_workspace_bytes.argtypes = [ctypes.POINTER(BlockAttnArgs)]
     lib.ha_block_attn_bwd.restype = ci
     lib.ha_block_attn_bwd.argtypes = [ctypes.POINTER(BlockAttnArgs), ctypes.POINTER(AttnGrads), vp]
     lib.ha_flash_attn_bwd.restype = ci

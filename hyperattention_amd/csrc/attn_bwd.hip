@@ -619,6 +619,15 @@ extern "C" int64_t ha_attn_bwd_workspace_bytes(const ha_attn_operands* t, int64_
   return carve(*t, sample_size, shares, nullptr).bytes;
 }
 
+extern "C" int64_t ha_block_attn_bwd_workspace_bytes(const ha_block_attn_args* args) {
+  if (!args) return ha_fail(HA_ERR_NULL, "ha_block_attn_bwd_workspace_bytes: null argument block");
+  const ha_block_attn_args& a = *args;
+  const int64_t most = ha_attn_bwd_workspace_bytes(&a.t, a.sample_size);
+  QueryRanges r;
+  if (most < 0 || writes_shares(a.t, a.sample_size, r) || ha_block_bwd_fused_takes(a)) return most;
+  return carve(a.t, a.sample_size, 1, nullptr).bytes;
+}
+
 extern "C" int ha_block_attn_bwd(const ha_block_attn_args* args, const ha_attn_grads* grads, void* stream) {
   HA_REQUIRE(args && grads, HA_ERR_NULL, "ha_block_attn_bwd: null argument");
   const ha_block_attn_args& a = *args;

@@ -336,7 +336,13 @@ class Attention : public torch::autograd::Function<Attention> {
       const Call& call = s->calls[i];
       ops.push_back(operands(q, k, v, i ? saved[5].select(0, call.level) : saved[3],
                              i ? saved[6].select(0, call.level) : saved[4], c, call));
-      const int64_t m = ha_attn_bwd_workspace_bytes(&ops.back(), call.hashed ? c.sample : 0);
+      int64_t m;
+      if (call.hashed) {
+        const ha_block_attn_args a = block_args(ops.back(), saved[7], s->q_idx_at[i], s->k_idx_at[i], saved[8], c);
+        m = ha_block_attn_bwd_workspace_bytes(&a);
+      } else {
+        m = ha_attn_bwd_workspace_bytes(&ops.back(), 0);
+      }
       if (m < 0) check((int)m);
       nbytes = std::max(nbytes, m);
     }

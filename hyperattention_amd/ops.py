@@ -378,8 +378,9 @@ def _wants_grad(*tensors):
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
-def _attn_grads(t, dout, dq, dk, dv, layout_bnhd=True, accumulate=False, sample_size=0):
-    """AttnGrads for (b,n,h,d) [layout_bnhd] or (b,h,n,d) gradient tensors plus the workspace the C side asks for."""
+def _attn_grads(t, dout, dq, dk, dv, layout_bnhd=True, accumulate=False, sample_size=0, block=None):
+    """AttnGrads for (b,n,h,d) [layout_bnhd] or (b,h,n,d) gradient tensors plus the workspace the C side asks for; with
+    `block`, the BlockAttnArgs of the call, for its options."""
     sn, sh = (1, 2) if layout_bnhd else (2, 1)
     g = AttnGrads()
     g.dout, g.dq, g.dk, g.dv = dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
@@ -388,7 +389,10 @@ def _attn_grads(t, dout, dq, dk, dv, layout_bnhd=True, accumulate=False, sample_
     g.dk_stride_b, g.dk_stride_h, g.dk_stride_n = dk.stride(0), dk.stride(sh), dk.stride(sn)
     g.dv_stride_b, g.dv_stride_h, g.dv_stride_n = dv.stride(0), dv.stride(sh), dv.stride(sn)
     g.accumulate = int(bool(accumulate))
-    nbytes = _lib.lib().ha_attn_bwd_workspace_bytes(ctypes.byref(t), sample_size)
+    if block is not None:
+        nbytes = _lib.lib().ha_block_attn_bwd_workspace_bytes(ctypes.byref(block))
+    else:
+        nbytes = _lib.lib().ha_attn_bwd_workspace_bytes(ctypes.byref(t), sample_size)
     if nbytes <= 0:
         _lib.check(int(nbytes) if nbytes < 0 else -3)
     ws = torch.empty((nbytes,), device=dout.device, dtype=torch.uint8)
@@ -421,7 +425,7 @@ class HyperAttnFunc(torch.autograd.Function):
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         a, keep = _block_attn_args(q, k, v, o, lse, q_sort_idx, k_sort_idx, block_size, sample_size, softmax_scale,
                                    smooth_block, sampled_idx)
-        g, ws = _attn_grads(a.t, do, dq, dk, dv, sample_size=sample_size)
+        g, ws = _attn_grads(a.t, do, dq, dk, dv, block=a)
         with torch.cuda.device(q.device):
             _lib.check(_lib.lib().ha_block_attn_bwd(ctypes.byref(a), ctypes.byref(g), _stream(q)))
         return dq, dk, dv, None, None, None, None, None, None, None

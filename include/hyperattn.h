@@ -216,8 +216,10 @@ int ha_flash_attn_fwd(const ha_attn_operands* t, int causal, void* stream);
  * Segments (segs, seg_stride_rows and the offsets) as in the forward; dout, dq follow q's segment
  * layout, dk, dv that of k, v.  Built for d == dv in {64, 128} (HA_ERR_UNSUPPORTED otherwise).
  * workspace: ha_attn_bwd_workspace_bytes(t, sample_size) bytes (sample_size = 0 for exact attention),
- * 256-byte aligned: two floats per query, and fp32 sums of the sampled keys (at d = 128 shares of them, added up
- * by the call; a workspace with room for the sums alone is accepted and takes atomics), overwritten by the call.
+ * 256-byte aligned: two floats per query, and fp32 sums of the sampled keys (at d = 128, and at d = 64 in the one kernel for
+ * plain blocks of 256, shares of them, added up by the call; a workspace with room for the sums alone is accepted and takes
+ * atomics), overwritten by the call.  That is the most that any block_size and smooth_block need;
+ * ha_block_attn_bwd_workspace_bytes(args) is what the call with these options does.
  */
 typedef struct {
   const void* dout;  /* (.., n_q, dv)                          */
@@ -236,6 +238,7 @@ typedef struct {
 } ha_attn_grads;
 
 int64_t ha_attn_bwd_workspace_bytes(const ha_attn_operands* t, int64_t sample_size);
+int64_t ha_block_attn_bwd_workspace_bytes(const ha_block_attn_args* args);
 
 /* replaces: HyperAttnFunc.backward -> _hyper_attn_backward with _bwd_preprocess_do_o_dot,
  *           _bwd_permuted_block_diagonal_kernel, _bwd_sampled_col_kernel

@@ -238,6 +238,25 @@ def test_backward_workspace_follows_the_kernel(lib, heads, n, sample, shares):
     assert lib.ha_attn_bwd_workspace_bytes(ctypes.byref(t), sample) == heads * n * 8 + 2 * shares * heads * sample * 64 * 4
 
 
+@pytest.mark.parametrize("options,shares", [
+    (dict(), 4), (dict(block_size=200), 4),                                          # blocks are counted in tiles of 128
+    (dict(block_size=128), 1), (dict(block_size=512), 1), (dict(smooth_block=1), 1),   # not in the one kernel
+])
+def test_backward_workspace_of_a_call_follows_its_options(lib, options, shares):
+    a = _lib.BlockAttnArgs()
+    heads, n, a.sample_size, a.block_size = 24, 1024, 256, 256
+    t = a.t
+    t.batch, t.heads, t.n_q, t.n_k, t.d, t.dv, t.kv_group, t.segs = 1, heads, n, n, 64, 64, 1, 1
+    for name, x in options.items():
+        setattr(a, name, x)
+    of = lambda shares: heads * n * 8 + 2 * shares * heads * a.sample_size * 64 * 4
+    assert lib.ha_block_attn_bwd_workspace_bytes(ctypes.byref(a)) == of(shares)
+    assert lib.ha_attn_bwd_workspace_bytes(ctypes.byref(t), a.sample_size) == of(4)
+    t.segs = 0
+    assert lib.ha_block_attn_bwd_workspace_bytes(ctypes.byref(a)) == -3
+    assert lib.ha_block_attn_bwd_workspace_bytes(None) == -1
+
+
 def test_python_layer_fails_loudly_without_library(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "missing.so"))
     monkeypatch.setattr(_lib, "_lib", None)
