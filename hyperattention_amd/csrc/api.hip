@@ -372,8 +372,11 @@ Units units_of(const ha_forward_args& a, const Workspace& w) {
 }
 
 // What the exact causal launch that hashes and ranks the units beside its tiles is given.
-int rank_beside(const ha_forward_args& a, const Workspace& w, ha_rank_beside& ranking) {
+int rank_beside(const ha_forward_args& a, const Workspace& w, const ha_attn_operands& t, ha_rank_beside& ranking) {
   const Units u = units_of(a, w);
+  // a row's place is its unit's plus 32 bits, as in the attention kernels, whose segments may be half as long
+  HA_REQUIRE((w.grid.unit - 1) * std::max(t.q_stride_n, t.k_stride_n) * 2 + 128 * 2 <= (1ll << 32), HA_ERR_UNSUPPORTED,
+             "ha_forward: one head of a tensor may span 4 GiB at most");
   ranking = {};
   ranking.proj = a.proj;
   for (int i = 0; i < 2; ++i) {
@@ -547,11 +550,19 @@ static int forward_sort(const ha_forward_args* args, const ha_attn_operands* lea
   HA_REQUIRE(a.n < (1ll << 30), HA_ERR_SHAPE, "ha_forward_sort: sequence too long");
   HA_REQUIRE(a.d >= 8 && a.d <= 128 && a.d % 8 == 0, HA_ERR_UNSUPPORTED,
              "ha_forward_sort: head dim must be a multiple of 8 up to 128 (got %lld)", (long long)a.d);
+  HA_REQUIRE(!leaves || a.causal, HA_ERR_UNSUPPORTED, "ha_forward_sort_leaves: a pass without causal mask has no leaves");
   Plan pl;
   int st = make_plan(a, pl);
   if (st != HA_OK) return st;
+  if (leaves) {
+    const ha_attn_operands& f = *leaves;
+    HA_REQUIRE(!pl.ragged, HA_ERR_UNSUPPORTED, "ha_forward_sort_leaves: odd lengths are for the caller to pad");
+    HA_REQUIRE(f.n_q == pl.len[pl.levels] && f.n_k == f.n_q && f.segs == 1ll << pl.levels && f.q_seg_offset == 0 && f.k_seg_offset == 0 &&
+                   (f.segs == 1 || f.seg_stride_rows == f.n_q),
+               HA_ERR_SHAPE, "ha_forward_sort_leaves: the leaves are not those of the pass");
+  }
   Workspace w;
-  layout_workspace(a, pl, w, leaves && a.causal);
+  layout_workspace(a, pl, w, leaves != nullptr);
   const int nlev = a.causal ? pl.levels : 1;
   *num_levels = nlev;
   for (int j = 0; j < nlev; ++j) {
@@ -579,7 +590,7 @@ static int forward_sort(const ha_forward_args* args, const ha_attn_operands* lea
     return st != HA_OK || !leaves ? st : flash_attn(*leaves, 1, stream);
   }
   ha_rank_beside ranking;
-  st = rank_beside(a, w, ranking);
+  st = rank_beside(a, w, t, ranking);
   if (st == HA_OK) st = flash_attn(*leaves, 1, stream, nullptr, &ranking);
   return st == HA_OK ? place_units(a, pl, w, stream) : st;
 }
@@ -594,7 +605,6 @@ extern "C" int ha_forward_sort_leaves(const ha_forward_args* args, const ha_attn
   HA_REQUIRE(leaves, HA_ERR_NULL, "ha_forward_sort_leaves: null argument");
   return forward_sort(args, leaves, q_idx_offset, k_idx_offset, num_levels, (hipStream_t)stream);
 }
-
 
 extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   HA_REQUIRE(args, HA_ERR_NULL, "ha_forward: null argument block");
@@ -629,7 +639,7 @@ extern "C" int ha_forward(const ha_forward_args* args, void* stream_) {
   }
   ha_rank_beside ranking = {};
   if (w.beside) {
-    st = rank_beside(a, w, ranking);
+    st = rank_beside(a, w, t, ranking);
     if (st != HA_OK) return st;
   }
 

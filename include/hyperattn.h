@@ -363,8 +363,10 @@ int ha_forward_sort(const ha_forward_args* args, int64_t* q_idx_offset, int64_t*
                     void* stream);
 
 /* ha_forward_sort and, in front of the levels, the exact causal call of the recursion's leaves (as
- * ha_flash_attn_fwd(leaves, 1, stream)), whose q, k, sizes, strides and type are those of `args`.  The rows are hashed and
- * ranked beside the leaves, in the same launch, wherever ha_forward does that; the orders are those of ha_forward_sort. */
+ * ha_flash_attn_fwd(leaves, 1, stream)), whose q, k, sizes, strides and type are those of `args`: 2^levels segments
+ * of n / 2^levels rows, one after the other.  The rows are hashed and ranked beside the leaves, in the same launch, wherever
+ * ha_forward does that; the orders are those of ha_forward_sort.  Refused: a pass without causal mask, an odd length at any
+ * level (the caller pads), leaves other than the pass's. */
 int ha_forward_sort_leaves(const ha_forward_args* args, const ha_attn_operands* leaves, int64_t* q_idx_offset,
                            int64_t* k_idx_offset, int* num_levels, void* stream);
 

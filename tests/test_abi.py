@@ -257,6 +257,42 @@ def test_backward_workspace_of_a_call_follows_its_options(lib, options, shares):
     assert lib.ha_block_attn_bwd_workspace_bytes(None) == -1
 
 
+def test_sort_with_leaves_argument_errors(lib):
+    """A pass of two levels: leaves that are not its own are refused before any launch."""
+    q_at, k_at, levels = (ctypes.c_int64 * 48)(), (ctypes.c_int64 * 48)(), ctypes.c_int(0)
+
+    def call(leaves=None, stride=64, **args):
+        a = _lib.ForwardArgs()
+        a.q = a.k = a.proj = a.workspace = 4096
+        a.workspace_bytes = 1 << 40
+        a.batch, a.heads, a.kv_heads, a.n, a.d, a.dv, a.causal = 1, 2, 2, 4096, 64, 64, 1
+        a.lsh_num_projs, a.block_size, a.min_seq_len, a.dtype = 8, 256, 1024, 0
+        t = _operands(batch=1, heads=2, n_q=1024, n_k=1024, segs=4, seg_stride_rows=1024)
+        t.q = t.k = 4096
+        for x, row in ((a, stride), (t, stride)):
+            x.q_stride_b = x.k_stride_b = 2 * 4096 * row
+            x.q_stride_h = x.k_stride_h = 4096 * row
+            x.q_stride_n = x.k_stride_n = row
+        for x, changes in ((a, args), (t, leaves or {})):
+            for name, value in changes.items():
+                setattr(x, name, value)
+        return lib.ha_forward_sort_leaves(ctypes.byref(a), ctypes.byref(t), q_at, k_at, ctypes.byref(levels), None)
+
+    assert lib.ha_forward_sort_leaves(None, None, q_at, k_at, ctypes.byref(levels), None) == -1
+    assert call(q=None) == -1
+    assert call(causal=0) == -5 and b"without causal mask" in lib.ha_last_error()
+    assert call(n=4095) == -5 and b"odd" in lib.ha_last_error()   # its leaves would end a row past the tensors
+    for leaves in (dict(n_q=512), dict(n_k=512), dict(n_q=2048, n_k=2048), dict(segs=2), dict(segs=8), dict(seg_stride_rows=2048),
+                   dict(q_seg_offset=1024), dict(k_seg_offset=1024), dict(k=8192), dict(q=8192), dict(heads=4), dict(kv_group=2),
+                   dict(d=128), dict(dtype=1), dict(q_stride_n=128), dict(k_stride_h=64)):
+        assert call(leaves) == -3, leaves
+    assert call(min_seq_len=8192) == -3                            # no level: one leaf of 4096 rows
+    assert call(workspace_bytes=1024) == -6
+    # units of 4096 rows of 1.5 MiB: 6 GiB, their leaves (half as long: the deepest level is exact) 3 GiB
+    assert call(dict(n_q=2048, n_k=2048, seg_stride_rows=2048), stride=786432, n=8192, min_seq_len=3000) == -5
+    assert b"4 GiB" in lib.ha_last_error()
+
+
 def test_python_layer_fails_loudly_without_library(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "missing.so"))
     monkeypatch.setattr(_lib, "_lib", None)
