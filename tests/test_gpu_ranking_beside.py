@@ -1,5 +1,5 @@
 """Units hashed and ranked by workgroups of the exact causal launch: the forward pass in one call against the same launches with
-the orders of ha_forward_sort (hash, rank and placement launches), bit for bit."""
+the orders of ha_forward_sort (hash, rank and placement launches), and at odd lengths its orders themselves, bit for bit."""
 import ctypes
 
 import pytest
@@ -131,6 +131,60 @@ def test_sort_with_the_leaves(b, h, hk, n, msl, d, projs, dtype):
         results.append((out, lse))
     for x, y in zip(*results):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("b,h,hk,n,msl,d,projs,dtype", [
+    (1, 2, 2, 255, 128, 64, 8, torch.float16),        # a unit is a whole segment, its last row the appended one
+    (1, 24, 24, 4095, 2048, 64, 8, torch.bfloat16),
+    (2, 4, 2, 8447, 4200, 64, 6, torch.float16),
+    (1, 2, 1, 16639, 8300, 64, 8, torch.bfloat16),    # three units per granule, the last of 128 rows
+    (1, 8, 8, 15359, 1024, 64, 8, torch.float16),     # ragged leaves under three hashed levels
+    (1, 4, 2, 4095, 1024, 40, 8, torch.bfloat16),
+    (1, 2, 1, 12287, 6000, 96, 8, torch.bfloat16),
+    (1, 12, 4, 5119, 1024, 96, 7, torch.float16),
+    (1, 2, 2, 9215, 4100, 128, 8, torch.bfloat16),    # units of 4096 and 512 rows
+    (1, 16, 2, 8191, 2048, 128, 8, torch.float16),
+])
+def test_odd_lengths_place_the_appended_row(b, h, hk, n, msl, d, projs, dtype):
+    """The orders that ha_forward leaves in its workspace against ha_forward_sort's of the same rows, bit for bit.  Where they lie is
+    asked of ha_forward_sort_leaves, for the rows with the zero row that the recursion appends; its orders are the same too."""
+    from hyperattention_amd import _lib, ops
+    q, k, v = (_randn((b, x, n, d), s, dtype).cuda() for x, s in ((h, 640), (hk, 641), (hk, 642)))
+    q[:, :, torch.arange(n) % 4 > 1] = q[:, :, :1].clone()
+    k[:, :, torch.arange(n) % 3 > 1] = k[:, :, :1].clone()
+    for x in (q, k):  # rows that tie with the appended one, at the end and before
+        x[:, :, n - 5:n - 2] = 0
+        x[:, :, n // 3] = 0
+    proj = _randn((1, 1, d, projs), 643, dtype).cuda()
+    want = ops.forward_sort(q, k, proj, causal=True, lsh_num_projs=projs, min_seq_len=msl)
+    opts = dict(scale=d ** -0.5, causal=True, lsh_num_projs=projs, block_size=128, sample_size=128, min_seq_len=msl, smooth_block=False)
+    lib, stream = _lib.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    out, lse = torch.empty_like(q), torch.empty((b, h, n), device="cuda")
+    a, keep = ops._forward_args(q, k, v, out, lse, proj, **opts)
+    _lib.check(lib.ha_forward(ctypes.byref(a), stream))
+
+    pq, pk, pv = (torch.nn.functional.pad(x, (0, 0, 0, 1)) for x in (q, k, v))
+    halves, leaf = ops.causal_plan(n + 1, msl)
+    pa, pkeep = ops._forward_args(pq, pk, None, None, None, proj, **opts)
+    po, pl = torch.empty_like(pq), torch.empty((b, h, n + 1), device="cuda")
+    t = _lib.AttnOperands()
+    t.batch, t.heads, t.n_q, t.n_k, t.d, t.dv = b, h, leaf, leaf, d, d
+    t.segs, t.seg_stride_rows, t.kv_group, t.scale, t.dtype = 1 << len(halves), leaf, h // hk, d ** -0.5, ops._dtype_code(q)
+    t.lse_stride_b, t.lse_stride_h = h * (n + 1), n + 1
+    for name, x in (("q", pq), ("k", pk), ("v", pv), ("o", po)):
+        for i, axis in enumerate("bhn"):
+            setattr(t, f"{name}_stride_{axis}", x.stride(i))
+    t.q, t.k, t.v, t.out, t.lse = (x.data_ptr() for x in (pq, pk, pv, po, pl))
+    at = (ctypes.c_int64 * 48)(), (ctypes.c_int64 * 48)()
+    levels = ctypes.c_int(0)
+    _lib.check(lib.ha_forward_sort_leaves(ctypes.byref(pa), ctypes.byref(t), *at, ctypes.byref(levels), stream))
+    for side in (0, 1):
+        for j, w in enumerate(want[side]):
+            assert (at[side][j] < 0) == (w is None)
+            if w is not None:
+                for ws in (keep[-1], pkeep[-1]):
+                    got = ws[at[side][j]:at[side][j] + 4 * w.numel()].view(torch.int32).view(w.shape)
+                    assert torch.equal(got, w), (side, j)
 
 
 @pytest.mark.parametrize("b,n,msl,beside", [
