@@ -68,7 +68,8 @@ __device__ __forceinline__ float ha_to_float(bf16_t v) { return (float)v; }
 
 // Asks for every 64-byte line of a kernel's first BYTES of arguments at once.  The argument block is new to the caches in every
 // launch, and the compiler loads a field where it is used: six to nine misses one after the other before a kernel's
-// first row is asked for.  24 heads of 1000 causal rows 12.3 -> 11.4 us, 4 of 4096 hashed (three launches) 19.7 -> 18.8.
+// first row is asked for.  24 heads of 1000 causal rows 12.3 -> 11.4 us, 4 of 4096 hashed (three launches) 19.7 -> 18.8; each call on
+// inputs that no cache holds 13.7 -> 12.5 and 21.6 -> 20.3.
 template <int BYTES>
 __device__ __forceinline__ void ha_load_arguments() {
 #if defined(__HIP_DEVICE_COMPILE__)
