@@ -5,8 +5,8 @@
 // the blocks 403, of the sampled keys 229) and compute the scores twice (7 products per pair).  Here a workgroup gathers the
 // q, k, v, dO, O rows of a block of 256 queries and 256 keys once, computes every score once (5 products) and leaves dq, dk,
 // dv of the block and its share of the sampled keys' sums: 3.4 GB, 735 to 766 us in the same launch (without adding, 24 heads
-// of 16384, the whole call: 269 -> 223 us).  What bounds it now: not the board's power limit (2.21 to 2.28 GHz, matrix pipe busy 0.30 to 0.32 of
-// the time); of a block's 65k cycles (57k where nothing is added to) 43k are the steps, bound by the LDS (1750 of a step's 2700 cycles), the others the ends
+// of 16384, the whole call: 269 -> 215 us).  What bounds it now: not the board's power limit (2.18 to 2.39 GHz, matrix pipe busy 0.33 of
+// the time, 0.37 where nothing is added to); of a block's 65k cycles (57k where nothing is added to) 43k are the steps, bound by the LDS (1750 of a step's 2700 cycles), the others the ends
 // of its phases, where every wave does the same memory and vector work with one workgroup per CU and nothing beside it.
 //
 // A workgroup: 8 waves, a run of consecutive blocks of one (head, segment).  A block has a phase for its own keys and one

@@ -345,7 +345,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void lse_merge_rows_kernel(const Mer
 // Whether a workgroup's rows lie in one leaf.  `full`: the part of the workgroups' threads that have a piece; a leaf that a chunk's rows do
 // not divide, and a short one above all, leaves some without, and chunks that do not start at multiples of 32 rows share lines of log-sum-exps.
 // Rows | by leaf, us (1300 launches of leaves of 1 to 4096 rows, 2^13 to 2^21 in all; where the rule takes the leaves they are 0.82 to 2 times as fast,
-// 1.23 at the median; of the others a few are up to 1.7 times as fast by leaf, 0.84 at the median): one level, 2^20 sequences of d = 64: leaves of 1 row 139 | 3402, of 16 124 | 223, of 65 124 | 167, of 822 182 | 191,
+// 1.23 at the median; of the others a few are up to 1.7 times as fast by leaf, 0.84 at the median): one level, 2^21 rows of d = 64: leaves of 1 row 139 | 3402, of 16 124 | 223, of 65 124 | 167, of 822 182 | 191,
 // of 64 (full) 145 | 128; three levels, 2^17 rows: leaves of 34 18 | 19, of 75 18 | 14; 3 * 2^20 rows, which no cache holds, of 41, d = 128, 561 | 586, of 392 287 | 276; six: 2^17
 // rows, leaves of 43 (0.67) 27.4 | 25.1, 3 * 2^20 of 135 (0.7) 463 | 473, of 230 (0.9) 464 | 454.
 static bool merge_by_leaf(int levels, double full, double bytes) {
